@@ -39,6 +39,10 @@ struct DevGrid {
        lanes of consecutive cells read consecutive addresses:
        ipwT[(l*8 + j)*nsh + h] = ipw[8*(l*nsh + h) + j] */
     const double *ipwT;
+    /* terrain grids: -0.5*ipw*slope of every cell's edges in the terrain
+       layers, vcw[(k*6 + j)*nsh + h] for layer L - n_oro + k and slot j (the
+       weights of the vertical contravariant correction); null when flat */
+    const double *vcw;
     const double *tw, *drw, *dnd, *dzv, *darea, *fvec;
     const int *from, *to, *adj, *sgn, *ti, *tmc, *dri, *dfrom, *dto, *vit, *vst;
     /* per-edge differences that calc_pot_vort forms for its density
@@ -51,11 +55,11 @@ struct DevGrid {
        solver's implicit weight times dt over the volume); the runtime refills
        it when dt changes */
     double *idv;
-    /* number of layer chunks the per-cell kernels split a column into
-       (gridDim.y); more chunks give more waves to hide gather latency */
-    int split_cell;
-    /* the same for the per-edge kernels */
-    int split_edge;
+    /* numbers of layer chunks (gridDim.y) of the kernels that walk a column:
+       per cell (scalar transport, kinetic energy; the vertical TRSK flux's
+       levels), per edge (PV, TRSK flux, mass flux; the gradients), per
+       triangle, and of the terrain levels of the vertical corrections */
+    int split_cell, split_cell_w, split_edge, split_grad, split_tri, split_vcc;
     /* 1: tracer solver with one (column, tracer) per lane in registers; 0: LDS-staged */
     int gd_streaming;
     /* one tracer per block in the LDS-staged tracer solve instead of all five */

@@ -9,6 +9,8 @@
  * changed.  All kernels are HBM-bandwidth bound gathers/stencils; there is no
  * dense contraction, hence no MFMA.
  */
+#include <type_traits>
+
 #include "rkhevi_dev.h"
 #include "rkhevi_kernels.h"
 
@@ -53,16 +55,18 @@ __device__ __forceinline__ double grad_w_raw(const DevGrid &G, const TF *f, int 
     return ((double)f[h + (i64)(lev - 1)*G.nsh] - (double)f[h + (i64)lev*G.nsh])/G.nd[vi];
 }
 
-/* averaging.c:14-39 on a stored vector field */
+/* averaging.c:14-39 on a stored vector field.  The weights come from the
+   cell-major copy ipwT: consecutive cells' weights are consecutive words,
+   where ipw holds a cell's eight together (one 64-byte line per lane) */
 __device__ __forceinline__ double remap_verpri2horpri(const DevGrid &G, const double *f, int l, int e)
 {
-    int fr = G.from[e], to = G.to[e];
-    const double *ipw = G.ipw;
-    double c = ipw[8*((i64)l*G.nsh + fr) + 6]*f[(i64)l*G.vpl + fr];
-    c += ipw[8*((i64)l*G.nsh + to) + 6]*f[(i64)l*G.vpl + to];
+    const int fr = G.from[e], to = G.to[e];
+    const double *w6 = G.ipwT + ((i64)l*8 + 6)*G.nsh, *w7 = w6 + G.nsh;
+    double c = w6[fr]*f[(i64)l*G.vpl + fr];
+    c += w6[to]*f[(i64)l*G.vpl + to];
     if (l < G.L - 1) {
-        c += ipw[8*((i64)l*G.nsh + fr) + 7]*f[(i64)(l + 1)*G.vpl + fr];
-        c += ipw[8*((i64)l*G.nsh + to) + 7]*f[(i64)(l + 1)*G.vpl + to];
+        c += w7[fr]*f[(i64)(l + 1)*G.vpl + fr];
+        c += w7[to]*f[(i64)(l + 1)*G.vpl + to];
     }
     return 0.5*c;
 }
@@ -139,12 +143,12 @@ __device__ __forceinline__ double grad_edge_t(const DevGrid &G, const TF *f, int
     i64 vi = G.nsh + (i64)l*G.vpl + e;
     double g = ((double)f[to + (i64)l*G.nsh] - (double)f[fr + (i64)l*G.nsh])/G.nd[vi];
     if (!FLAT && l >= G.L - G.n_oro) {
-        const double *ipw = G.ipw;
-        double c = ipw[8*((i64)l*G.nsh + fr) + 6]*grad_w_raw(G, f, l, fr);
-        c += ipw[8*((i64)l*G.nsh + to) + 6]*grad_w_raw(G, f, l, to);
+        const double *w6 = G.ipwT + ((i64)l*8 + 6)*G.nsh, *w7 = w6 + G.nsh;
+        double c = w6[fr]*grad_w_raw(G, f, l, fr);
+        c += w6[to]*grad_w_raw(G, f, l, to);
         if (l < G.L - 1) {
-            c += ipw[8*((i64)l*G.nsh + fr) + 7]*grad_w_raw(G, f, l + 1, fr);
-            c += ipw[8*((i64)l*G.nsh + to) + 7]*grad_w_raw(G, f, l + 1, to);
+            c += w7[fr]*grad_w_raw(G, f, l + 1, fr);
+            c += w7[to]*grad_w_raw(G, f, l + 1, to);
         }
         c = 0.5*c;
         g += -G.slope[vi]*c;
@@ -180,15 +184,15 @@ __device__ __forceinline__ double grad_edge_walk(const DevGrid &G, const TF *f, 
         /* grad_w_raw at level l of both cells: carried unless layer l - 1
            had no terrain term or lies in another chunk */
         if (l == l0 || l == lt) { c.gwf = grad_w_raw(G, f, l, fr); c.gwt = grad_w_raw(G, f, l, to); }
-        const double *ipw = G.ipw;
-        double s = ipw[8*((i64)l*nsh + fr) + 6]*c.gwf;
-        s += ipw[8*((i64)l*nsh + to) + 6]*c.gwt;
+        const double *w6 = G.ipwT + ((i64)l*8 + 6)*nsh, *w7 = w6 + nsh;
+        double s = w6[fr]*c.gwf;
+        s += w6[to]*c.gwt;
         if (l < L - 1) {
             /* grad_w_raw at level l + 1 */
             const double gf1 = (c.ff - nff)/G.nd[fr + (i64)(l + 1)*G.vpl];
             const double gt1 = (c.ft - nft)/G.nd[to + (i64)(l + 1)*G.vpl];
-            s += ipw[8*((i64)l*nsh + fr) + 7]*gf1;
-            s += ipw[8*((i64)l*nsh + to) + 7]*gt1;
+            s += w7[fr]*gf1;
+            s += w7[to]*gt1;
             c.gwf = gf1;
             c.gwt = gt1;
         }
@@ -286,7 +290,8 @@ __global__ void __launch_bounds__(TPB) k_mass_flux(DevGrid G, const double *rho_
 template <typename TW>
 __global__ void __launch_bounds__(TPB) k_rel_vort_tri(DevGrid G, const double *w, TW *res)
 {
-    int h = xcd_block().x*TPB + threadIdx.x;
+    const Blk bk = xcd_block();
+    const int h = bk.x*TPB + threadIdx.x;
     if (h >= G.nt) return;
     const int L = G.L, lt = L - G.n_oro, nsh = G.nsh, vpl = G.vpl, nvh = G.nvh;
     const i64 dvpl = G.dvpl;
@@ -309,9 +314,17 @@ __global__ void __launch_bounds__(TPB) k_rel_vort_tri(DevGrid G, const double *w
         x.da = G.darea[di];
         return x;
     };
-    double wp[3] = {0.0, 0.0, 0.0}, zp[3] = {0.0, 0.0, 0.0};   /* layer l - 1 */
-    Lay cur = load(0);
-    for (int l = 0; l < L; ++l) {
+    int l0, l1;
+    layer_chunk(L, bk.y, l0, l1);
+    double wp[3], zp[3];   /* layer l - 1 (layer 0, unused, at the top) */
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const i64 vi = nsh + (i64)(l0 > 0 ? l0 - 1 : 0)*vpl + vit[j];
+        wp[j] = w[vi];
+        zp[j] = G.zv[vi];
+    }
+    Lay cur = load(l0);
+    for (int l = l0; l < l1; ++l) {
         const Lay nxt = load(l + 1 < L ? l + 1 : l);
         double r = 0;
 #pragma unroll
@@ -507,7 +520,7 @@ k_vorticity_flux_e(DevGrid G, const TW *F, const TW *pv, TW *out)
 }
 
 /* vorticity_flux.c:373-417, vertical part: one thread per cell, levels 0..L */
-template <typename TW>
+template <typename TW, int RUN>
 __global__ void __launch_bounds__(TPB) k_vorticity_flux_w(DevGrid G, const TW *F, const TW *pv, TW *out)
 {
     const Blk bk = xcd_block();
@@ -563,22 +576,22 @@ __global__ void __launch_bounds__(TPB) k_vorticity_flux_w(DevGrid G, const TW *F
         for (int j = 0; j < 6; ++j) { Fm[j] = Fc[j]; Wm[j] = Wc[j]; }
         return o;
     };
-    if (l1 - l0 <= 3) {
-        /* a short chunk: every level before any store, so no store orders a
-           later level's loads (a step past the chunk repeats its last level) */
-        double o3[3];
+    if constexpr (RUN > 0) {
+        /* chunks of at most RUN levels: every level before any store, so no
+           store orders a later level's loads (a step past the chunk repeats
+           its last level) */
+        double o[RUN];
 #pragma unroll
-        for (int t = 0; t < 3; ++t) o3[t] = level(l0 + t < l1 ? l0 + t : l1 - 1);
+        for (int t = 0; t < RUN; ++t) o[t] = level(l0 + t < l1 ? l0 + t : l1 - 1);
 #pragma unroll
-        for (int t = 0; t < 3; ++t)
-            if (l0 + t < l1) out[(i64)(l0 + t)*vpl + h] = (TW)o3[t];
-        return;
-    }
-    for (int l = l0; l < l1; ++l) out[(i64)l*vpl + h] = (TW)level(l);
+        for (int t = 0; t < RUN; ++t)
+            if (l0 + t < l1) out[(i64)(l0 + t)*vpl + h] = (TW)o[t];
+    } else
+        for (int l = l0; l < l1; ++l) out[(i64)l*vpl + h] = (TW)level(l);
 }
 
 /* inner_product.c:13-43, one thread per cell, all layers */
-template <typename TW>
+template <typename TW, int RUN>
 __global__ void __launch_bounds__(TPB) k_inner_product(DevGrid G, const double *a, const double *b, TW *out)
 {
     const Blk bk = xcd_block();
@@ -611,18 +624,18 @@ __global__ void __launch_bounds__(TPB) k_inner_product(DevGrid G, const double *
         bu = bl;
         return o;
     };
-    if (l1 - l0 <= 3) {
-        /* a short chunk: every layer before any store, so no store orders a
-           later layer's loads (a step past the chunk repeats its last layer) */
-        double o3[3];
+    if constexpr (RUN > 0) {
+        /* chunks of at most RUN layers: every layer before any store, so no
+           store orders a later layer's loads (a step past the chunk repeats
+           its last layer) */
+        double o[RUN];
 #pragma unroll
-        for (int t = 0; t < 3; ++t) o3[t] = layer(l0 + t < l1 ? l0 + t : l1 - 1);
+        for (int t = 0; t < RUN; ++t) o[t] = layer(l0 + t < l1 ? l0 + t : l1 - 1);
 #pragma unroll
-        for (int t = 0; t < 3; ++t)
-            if (l0 + t < l1) out[(i64)(l0 + t)*G.nsh + h] = (TW)o3[t];
-        return;
-    }
-    for (int l = l0; l < l1; ++l) out[(i64)l*G.nsh + h] = (TW)layer(l);
+        for (int t = 0; t < RUN; ++t)
+            if (l0 + t < l1) out[(i64)(l0 + t)*G.nsh + h] = (TW)o[t];
+    } else
+        for (int l = l0; l < l1; ++l) out[(i64)l*G.nsh + h] = (TW)layer(l);
 }
 
 /* grad (gradient_operators.c:56-74) of a scalar field: edges (one thread per
@@ -693,6 +706,18 @@ __global__ void __launch_bounds__(TPB) k_vector_tend(DevGrid G, DevWorkT<TW> W, 
    the wind (tracers, divergences.c:94-145), the gas mass flux and its
    rhotheta_v flux (divergences.c:41-59); the fluxes are formed on the fly
    exactly as scalar_times_vector_h forms them (multiplications.c:45-67). */
+/* the weights -0.5*ipw*slope of the corrections, cell-major per terrain level
+   and edge slot (a pentagon's sixth slot holds its first edge's, unused):
+   grid constants, formed once */
+__global__ void __launch_bounds__(TPB) k_vcc_weights(DevGrid G, double *vcw)
+{
+    const i64 t = (i64)blockIdx.x*TPB + threadIdx.x;
+    if (t >= (i64)G.n_oro*6*G.nsh) return;
+    const int q = (int)(t/G.nsh), h = (int)(t - (i64)q*G.nsh), k = q/6, j = q - 6*k, l = G.L - G.n_oro + k;
+    const int jj = j < (h < GAME_N_PENT ? 5 : 6) ? j : 0;
+    vcw[t] = -0.5*G.ipwT[((i64)l*8 + jj)*G.nsh + h]*G.slope[G.nsh + (i64)l*G.vpl + G.adj[6*h + jj]];
+}
+
 __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
 {
     /* one thread per cell walks a chunk of the terrain levels.  The
@@ -722,9 +747,10 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
     int c0, c1;
     layer_chunk(no, bk.y, c0, c1);
     /* one layer's inputs: the cell's density and rhotheta_v, and per edge
-       the wind, the neighbour's density and rhotheta_v, the weight (from the
-       cell-major copy of ipw: coalesced) and the slope */
-    struct In { double rh, rt, u[6], rn[6], rtn[6], w[6], sl[6]; };
+       the wind, the neighbour's density and rhotheta_v and the weight
+       -0.5*ipw*slope, a grid constant kept cell-major (coalesced, where the
+       slope is a gather) */
+    struct In { double rh, rt, u[6], rn[6], rtn[6], c[6]; };
     auto load = [&](int l) {
         In x;
         const i64 si = (i64)l*nsh + h;
@@ -736,8 +762,7 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
             x.u[j] = s.wind[vi];
             x.rn[j] = rg[sn];
             x.rtn[j] = s.rt[sn];
-            x.w[j] = G.ipwT[((i64)l*8 + (j < ne ? j : 0))*nsh + h];
-            x.sl[j] = G.slope[vi];
+            x.c[j] = G.vcw[((i64)(l - top)*6 + j)*nsh + h];
         }
         return x;
     };
@@ -751,7 +776,7 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
             const double rn = x.rn[j];
             const double f1 = (0.5*(rh + rn))*u;
             const double f2 = (0.5*(th + x.rtn[j]/rn))*f1;
-            const double c = -0.5*x.w[j]*x.sl[j];
+            const double c = x.c[j];
             tw[j] = c*u;
             t1[j] = c*f1;
             t2[j] = c*f2;
@@ -793,7 +818,7 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
    their divergences (divergences.c:14-148) and the RK-weighted tendencies.
    One thread per cell walks all layers; the edge fluxes are formed on the fly
    from the reference's own formulas, so no flux array is written. */
-template <bool FLAT, typename TW, int NC>
+template <bool FLAT, typename TW, int NC, int RUN>
 __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevWorkT<TW> W, double *td_rho,
                                                      double *td_rt, int rk)
 {
@@ -802,8 +827,8 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
     if (h >= G.nsh) return;
     /* NC: the number of constituents as a compile-time constant (1 dry, 6 moist),
        so the constituent loop unrolls and all neighbour loads can be in flight together */
-    const int nsh = G.nsh, vpl = G.vpl, L = G.L, no = G.n_oro, ncc = NC > 0 ? (NC > 1 ? NC - 2 : 0) : G.n_cond;
-    const int nc = NC > 0 ? NC : G.n_const;
+    const int nsh = G.nsh, vpl = G.vpl, L = G.L, no = G.n_oro;
+    constexpr int ncc = NC > 1 ? NC - 2 : 0, nc = NC;
     const i64 S = G.s, nvcc = (i64)no*nsh;
     const int ne = h < GAME_N_PENT ? 5 : 6;
     /* each edge as (edge, the cell across it, whether h is its from-cell);
@@ -825,8 +850,7 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
     }
     int l0, l1;
     layer_chunk(L, bk.y, l0, l1);
-    /* one layer's tendencies: with NC known they are returned in orho/ort
-       (stored by the caller), otherwise stored here */
+    /* one layer's tendencies, returned in orho/ort and stored by the caller */
     auto layer = [&](int l, double *orho, double &ort) {
         const i64 i = (i64)l*nsh + h;
         double a[6], u[6];
@@ -847,9 +871,8 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
         const double area_u = has_u ? G.area[h + (i64)l*vpl] : 0.0;
         const double area_l = has_l ? G.area[h + (i64)(l + 1)*vpl] : 0.0;
         const i64 vu = (i64)(l - (L - no))*nsh + h, vl = (i64)(l + 1 - (L - no))*nsh + h;
-        /* with NC known the new tendencies are kept in registers and stored
-           after every load of the layer, so no store orders the loads */
-        double out_rho[NC > 0 ? NC : 1];
+        /* the new tendencies are kept in registers and stored after every
+           load of the layer, so no store orders the loads */
         double out_rt = 0.0;
 #pragma unroll
         for (int k = 0; k < nc; ++k) {
@@ -947,39 +970,32 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
                 res = new_w*(-div + (double)W.ptr[shift_pt + i]);
                 if (old_w != 0.0) res = old_w*td_rho[shift + i] + res;
             }
-            if (NC > 0) out_rho[NC > 0 ? k : 0] = res;
-            else td_rho[shift + i] = res;
+            orho[k] = res;
         }
-        if (NC > 0) {
-#pragma unroll
-            for (int k = 0; k < (NC > 0 ? NC : 1); ++k) orho[k] = out_rho[k];
-            ort = out_rt;
-        } else td_rt[i] = out_rt;
+        ort = out_rt;
     };
     auto store = [&](int l, const double *orho, double ort) {
         const i64 i = (i64)l*nsh + h;
 #pragma unroll
-        for (int k = 0; k < (NC > 0 ? NC : 1); ++k) td_rho[(i64)k*S + i] = orho[k];
+        for (int k = 0; k < NC; ++k) td_rho[(i64)k*S + i] = orho[k];
         td_rt[i] = ort;
     };
-    constexpr int RUN = 3;
-    if (NC > 0 && l1 - l0 <= RUN) {
-        /* a short chunk: the loads and arithmetic of all its layers come
+    if constexpr (RUN > 0) {
+        /* chunks of at most RUN layers: the loads and arithmetic of all its layers come
            before any store, so no store orders a later layer's loads (a step
            past the chunk repeats its last layer and stores nothing) */
-        double orho[RUN][NC > 0 ? NC : 1], ort[RUN];
+        double orho[RUN][NC], ort[RUN];
 #pragma unroll
         for (int t = 0; t < RUN; ++t) layer(l0 + t < l1 ? l0 + t : l1 - 1, orho[t], ort[t]);
 #pragma unroll
         for (int t = 0; t < RUN; ++t)
             if (l0 + t < l1) store(l0 + t, orho[t], ort[t]);
-        return;
-    }
-    for (int l = l0; l < l1; ++l) {
-        double orho[NC > 0 ? NC : 1], ort = 0.0;
-        layer(l, orho, ort);
-        if (NC > 0) store(l, orho, ort);
-    }
+    } else
+        for (int l = l0; l < l1; ++l) {
+            double orho[NC], ort = 0.0;
+            layer(l, orho, ort);
+            store(l, orho, ort);
+        }
 }
 
 /* three_band_solver_ver_waves (column_solvers.c:19-383), one column per lane.
@@ -2463,6 +2479,19 @@ namespace hor {
         else LAUNCH(NAME, (KERNEL<false, TW, NC>), GRIDDIM, dim3(TPB), st, __VA_ARGS__);      \
     } while (0)
 
+/* launches f for the longest chunk of n layers or levels in `chunks` chunks:
+   1, 2 or 3 (the kernel holds a chunk's results until its last load), or 0
+   for longer chunks, which store layer by layer */
+template <class F>
+static void run_dispatch(int n, int chunks, F f)
+{
+    const int run = (n + chunks - 1)/chunks;
+    if (run == 1) f(std::integral_constant<int, 1>());
+    else if (run == 2) f(std::integral_constant<int, 2>());
+    else if (run == 3) f(std::integral_constant<int, 3>());
+    else f(std::integral_constant<int, 0>());
+}
+
 template <typename TW>
 static void pgrad_t(const DevGrid &G, const DevState &s, const DevWorkT<TW> &W, int first, double itw, hipStream_t st)
 {
@@ -2471,17 +2500,12 @@ static void pgrad_t(const DevGrid &G, const DevState &s, const DevWorkT<TW> &W, 
     if (G.n_const == 6) {
         LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 6>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, first, 1,
                (const double *)W.gas_frac, cvw);
-        FLAT_DISPATCH_NC("k_pgrad_e", k_pgrad_e, 6, GRID2(G.nvh, G.split_edge), G, s, W, first,
-                         (const double *)W.gas_frac, chw, ohw);
-    } else if (G.n_const == 1) {
-        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 1>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, first, 1,
-               (const double *)W.gas_frac, cvw);
-        FLAT_DISPATCH_NC("k_pgrad_e", k_pgrad_e, 1, GRID2(G.nvh, G.split_edge), G, s, W, first,
+        FLAT_DISPATCH_NC("k_pgrad_e", k_pgrad_e, 6, GRID2(G.nvh, G.split_grad), G, s, W, first,
                          (const double *)W.gas_frac, chw, ohw);
     } else {
-        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 0>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, first, 1,
+        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 1>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, first, 1,
                (const double *)W.gas_frac, cvw);
-        FLAT_DISPATCH_NC("k_pgrad_e", k_pgrad_e, 0, GRID2(G.nvh, G.split_edge), G, s, W, first,
+        FLAT_DISPATCH_NC("k_pgrad_e", k_pgrad_e, 1, GRID2(G.nvh, G.split_grad), G, s, W, first,
                          (const double *)W.gas_frac, chw, ohw);
     }
 }
@@ -2489,13 +2513,30 @@ static void pgrad_t(const DevGrid &G, const DevState &s, const DevWorkT<TW> &W, 
 template <typename TW>
 static void pgc_v_t(const DevGrid &G, const DevState &s, const DevWorkT<TW> &W, hipStream_t st)
 {
-    /* the constituent count as a compile-time constant where it is 6 or 1, so
-       the density sums unroll and their loads issue together */
+    /* the constituent count (6 or 1) as a compile-time constant, so the
+       density sums unroll and their loads issue together */
     if (G.n_const == 6)
         LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 6>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, 0, 0, nullptr, 0.0);
-    else if (G.n_const == 1)
+    else
         LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 1>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, 0, 0, nullptr, 0.0);
-    else LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 0>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, 0, 0, nullptr, 0.0);
+}
+
+template <typename TW>
+static void vorticity_flux_w_t(const DevGrid &G, const TW *F, const TW *pv, TW *out, hipStream_t st)
+{
+    run_dispatch(G.L + 1, G.split_cell_w, [&](auto r) {
+        LAUNCH("k_vorticity_flux_w", (k_vorticity_flux_w<TW, decltype(r)::value>), GRID2(G.nsh, G.split_cell_w), dim3(TPB),
+               st, G, F, pv, out);
+    });
+}
+
+template <typename TW>
+static void inner_product_t(const DevGrid &G, const double *a, const double *b, TW *out, hipStream_t st)
+{
+    run_dispatch(G.L, G.split_cell, [&](auto r) {
+        LAUNCH("k_inner_product", (k_inner_product<TW, decltype(r)::value>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G,
+               a, b, out);
+    });
 }
 
 template <typename TW>
@@ -2504,19 +2545,18 @@ static void advection_pv_t(const DevGrid &G, const double *wind, const double *r
 {
     LAUNCH("k_mass_flux", k_mass_flux<TW>, GRID2(G.nvh > G.nsh ? G.nvh : G.nsh, G.split_edge), dim3(TPB), st, G,
            rho_gas, wind, W.flux);
-    LAUNCH("k_rel_vort_tri", k_rel_vort_tri<TW>, GRID1(G.nt), dim3(TPB), st, G, wind, W.rvt);
+    LAUNCH("k_rel_vort_tri", k_rel_vort_tri<TW>, GRID2(G.nt, G.split_tri), dim3(TPB), st, G, wind, W.rvt);
     FLAT_DISPATCH("k_pot_vort", k_pot_vort, GRID2(G.nvh, G.split_edge), G, wind, rho_gas, (const TW *)W.rvt, W.pv);
     LAUNCH("k_vorticity_flux_e", k_vorticity_flux_e<TW>, GRID2(G.nvh, G.split_edge), dim3(TPB), st, G, (const TW *)W.flux,
            (const TW *)W.pv, W.pvt);
-    LAUNCH("k_vorticity_flux_w", k_vorticity_flux_w<TW>, GRID2(G.nsh, G.split_cell), dim3(TPB), st, G,
-           (const TW *)W.flux, (const TW *)W.pv, W.pvt);
+    vorticity_flux_w_t<TW>(G, W.flux, W.pv, W.pvt, st);
 }
 
 template <typename TW>
 static void advection_kinetic_t(const DevGrid &G, const double *wind, const DevWorkT<TW> &W, hipStream_t st)
 {
-    LAUNCH("k_inner_product", k_inner_product<TW>, GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, wind, wind, W.vsq);
-    FLAT_DISPATCH("k_grad_e", k_grad_e, GRID2(G.nvh, G.split_edge), G, (const TW *)W.vsq, W.vsq_grad);
+    inner_product_t<TW>(G, wind, wind, W.vsq, st);
+    FLAT_DISPATCH("k_grad_e", k_grad_e, GRID2(G.nvh, G.split_grad), G, (const TW *)W.vsq, W.vsq_grad);
     LAUNCH("k_grad_w", k_grad_w<TW>, GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, (const TW *)W.vsq, W.vsq_grad);
 }
 
@@ -2562,30 +2602,24 @@ static void scalar_tend_t(const DevGrid &G, const DevState &s, const DevState &t
                           hipStream_t st)
 {
     if (!G.flat)
-        /* chunks of three terrain levels (res 6 x 26, 23 terrain layers: 68 us
-           per launch; chunks of 2, 4 and 8 levels 77, 73 and 82 us).  Loading
-           each layer before the one above it is summed took the kernel's time
-           in the mountain window's gradient from 5.98 to 5.46 ms (176
-           registers, two waves per SIMD); chunks of six levels then 6.87 ms,
-           and the weights from ipw's interleaved
-           layout (eight per box) 5.68 ms */
-        LAUNCH("k_vcc", k_vcc, GRID2(G.nsh, (G.n_oro + 2)/3), dim3(TPB), st, G, s, W.vcc);
-    if (G.n_const == 6) {
-        if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 6>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, s,
-                           W, td.rho, td.rt, rk);
-        else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 6>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, s,
-                    W, td.rho, td.rt, rk);
-    } else if (G.n_const == 1) {
-        if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 1>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, s,
-                           W, td.rho, td.rt, rk);
-        else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 1>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, s,
-                    W, td.rho, td.rt, rk);
-    } else {
-        if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 0>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, s,
-                           W, td.rho, td.rt, rk);
-        else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 0>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, s,
-                    W, td.rho, td.rt, rk);
-    }
+        /* the chunks of terrain levels: set_layer_splits.  Loading each layer
+           before the one above it is summed took the kernel's time in the
+           mountain window's gradient from 5.98 to 5.46 ms; with the weights
+           -0.5*ipw*slope as a grid constant (one coalesced load for a
+           coalesced load and a gather) it takes 49.6 us per launch at
+           res 6 x 26 where it took 58.9 */
+        LAUNCH("k_vcc", k_vcc, GRID2(G.nsh, G.split_vcc), dim3(TPB), st, G, s, W.vcc);
+    run_dispatch(G.L, G.split_cell, [&](auto r) {
+        constexpr int RUN = decltype(r)::value;
+        const dim3 g = GRID2(G.nsh, G.split_cell), b(TPB);
+        if (G.n_const == 6) {
+            if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 6, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
+            else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 6, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
+        } else {
+            if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 1, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
+            else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 1, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
+        }
+    });
     scalar_tend_probe<TW>(G, td, st);
 }
 
@@ -2619,23 +2653,26 @@ void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const 
 { scalar_tend_t<float>(G, s, td, W, rk, st); }
 
 void inner_product(const DevGrid &G, const double *a, const double *b, double *out, hipStream_t st)
-{ LAUNCH("k_inner_product", k_inner_product<double>, GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, a, b, out); }
+{ inner_product_t<double>(G, a, b, out, st); }
 
 /* single operators (FP64), for the operator-level interface and its adjoints */
 void grad(const DevGrid &G, const double *f, double *out, hipStream_t st)
 {
     typedef double TW;
-    FLAT_DISPATCH("k_grad_e", k_grad_e, GRID2(G.nvh, G.split_edge), G, f, out);
+    FLAT_DISPATCH("k_grad_e", k_grad_e, GRID2(G.nvh, G.split_grad), G, f, out);
     LAUNCH("k_grad_w", k_grad_w<double>, GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, f, out);
 }
 
 void curl_triangles(const DevGrid &G, const double *wind, double *out, hipStream_t st)
-{ LAUNCH("k_rel_vort_tri", k_rel_vort_tri<double>, GRID1(G.nt), dim3(TPB), st, G, wind, out); }
+{ LAUNCH("k_rel_vort_tri", k_rel_vort_tri<double>, GRID2(G.nt, G.split_tri), dim3(TPB), st, G, wind, out); }
+
+void vcc_weights(const DevGrid &G, double *vcw, hipStream_t st)
+{ LAUNCH("k_vcc_weights", k_vcc_weights, GRID1((i64)G.n_oro*6*G.nsh), dim3(TPB), st, G, vcw); }
 
 void vorticity_flux(const DevGrid &G, const double *F, const double *pv, double *out, hipStream_t st)
 {
     LAUNCH("k_vorticity_flux_e", k_vorticity_flux_e<double>, GRID2(G.nvh, G.split_edge), dim3(TPB), st, G, F, pv, out);
-    LAUNCH("k_vorticity_flux_w", k_vorticity_flux_w<double>, GRID2(G.nsh, G.split_cell), dim3(TPB), st, G, F, pv, out);
+    vorticity_flux_w_t<double>(G, F, pv, out, st);
 }
 
 }  // namespace hor
@@ -2734,14 +2771,21 @@ static void gen_densities_only(const DevGrid &G, const DevState &so, const DevSt
     else LAUNCH_SHM("k_gen_densities", k_gen_densities<0>, g, b, lds, st, G, so, sn, td, K);
 }
 
+/* one thread per column loads each box once, one per box twice; but the
+   columns of a res 6 grid (161 blocks) leave most of the chip idle: 35, 38
+   and 55 us per launch at res 4, 5 and 6 x 26 by column, 7, 14 and 49 by box,
+   and 101 against 242 at res 7 (641 blocks) */
+static bool sed_heat_by_column(const DevGrid &G)
+{ return G.n_cond == 4 && !G.sh_per_box && (G.nsh + TPB - 1)/TPB >= 256; }
+
 void gen_densities(const DevGrid &G, const DevState &so, const DevState &sn, const DevState &td, const double *T,
                    const double *cpc, double *sed_heat, const StepConsts &K, int rk, hipStream_t st)
 {
     if (rk == 0 && G.n_cond > 0) {
-        if (G.n_cond == 4 && G.L == 26 && !G.sh_per_box)
+        if (sed_heat_by_column(G) && G.L == 26)
             LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 26>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
-        else if (G.n_cond == 4 && G.L == 55 && !G.sh_per_box)
+        else if (sed_heat_by_column(G) && G.L == 55)
             LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 55>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
         else if (G.n_cond == 4)
@@ -2755,10 +2799,10 @@ void gen_densities(const DevGrid &G, const DevState &so, const DevState &sn, con
                    const float *cpc, float *sed_heat, const StepConsts &K, int rk, hipStream_t st)
 {
     if (rk == 0 && G.n_cond > 0) {
-        if (G.n_cond == 4 && G.L == 26 && !G.sh_per_box)
+        if (sed_heat_by_column(G) && G.L == 26)
             LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 26>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
-        else if (G.n_cond == 4 && G.L == 55 && !G.sh_per_box)
+        else if (sed_heat_by_column(G) && G.L == 55)
             LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 55>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
         else if (G.n_cond == 4)

@@ -34,6 +34,8 @@ void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const 
 void inner_product(const DevGrid &G, const double *a, const double *b, double *out, hipStream_t st);
 void grad(const DevGrid &G, const double *f, double *out, hipStream_t st);
 void curl_triangles(const DevGrid &G, const double *wind, double *out, hipStream_t st);
+/* fills the grid constant G.vcw (n_oro x 6 x NSH doubles) */
+void vcc_weights(const DevGrid &G, double *vcw, hipStream_t st);
 void vorticity_flux(const DevGrid &G, const double *F, const double *pv, double *out, hipStream_t st);
 }
 

@@ -165,6 +165,54 @@ int game_gpu_init(const game_dims_t *dims, const game_grid_view_t *g, const game
     return rc;
 }
 
+/* How many chunks of layers (gridDim.y) the kernels that walk a column split
+   it into.  A chunk loads its cell's or edge's tables and starts its carried
+   values once, so long chunks do less; but a grid of few columns leaves the
+   chip idle unless its layers are spread over more blocks.  1024 blocks of
+   four waves are about what 256 CUs hold of these kernels.  Results do not
+   depend on the split.  Measured per launch (us), terrain grids of 26
+   layers, FP64, against two edge chunks, one triangle chunk and three layers
+   per cell thread at every size:
+     res 4 (30 edge blocks): pressure gradient 30 -> 8, PV 34 -> 10, TRSK
+       flux 26 -> 10, triangle curl 21 -> 6, kinetic gradient 20 -> 5, moist
+       scalar transport 34 -> 18, vertical corrections 11 -> 9
+     res 5 (120): pressure gradient 36 -> 24, PV 41 -> 29, TRSK flux 31 -> 24,
+       triangle curl 25 -> 13, scalar transport 48 -> 38
+     res 6 (480): PV 93 -> 82, TRSK flux 81 -> 76, triangle curl 39 -> 35; the
+       gradients 70 and 37 with two chunks, 76 and 43 with four
+     res 7 (1920, flat): two edge chunks and one of the triangles (more cost 3
+       to 15 %); scalar transport 406 with three layers per thread, 389 with
+       two, 392 with one; vertical TRSK flux 106, 127 and 145 */
+static void set_layer_splits(DevGrid &G)
+{
+    const int L = G.L, be = (G.nvh + 255)/256, bc = (G.nsh + 255)/256, bt = (G.nt + 255)/256;
+    auto clamp = [](int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); };
+    /* edges: one filled chip; where four chunks or fewer fill it, twice that
+       in at most four chunks for the kernels with long layers, whose last
+       blocks then leave less of it idle */
+    const int fill = 1024/be;
+    G.split_grad = clamp(fill, 2, L);
+    G.split_edge = clamp(fill > 4 ? fill : clamp(2048/be, 1, 4), 2, L);
+    G.split_tri = clamp((1024 + bt - 1)/bt, 1, L);
+    /* cells: two layers per thread, one where two leave the chip idle; the
+       vertical TRSK flux carries more from level to level and takes three
+       levels once three fill the chip */
+    const int run = bc*L <= 512 ? 1 : 2, run_w = bc*L < 3*1024 ? 1 : 3;
+    G.split_cell = (L + run - 1)/run;
+    G.split_cell_w = (L + 1 + run_w - 1)/run_w;
+    /* vertical corrections: about 1280 blocks, two to six terrain levels per thread */
+    const int run_v = bc*G.n_oro <= 512 ? 1 : clamp((bc*G.n_oro + 640)/1280, 2, 6);
+    G.split_vcc = (G.n_oro + run_v - 1)/run_v;
+    if (const char *e = getenv("GAME_GPU_SPLIT_CELL")) {
+        int v = atoi(e);
+        if (v >= 1 && v <= L) G.split_cell = G.split_cell_w = v;
+    }
+    if (const char *e = getenv("GAME_GPU_SPLIT_EDGE")) {
+        int v = atoi(e);
+        if (v >= 1 && v <= L) G.split_edge = G.split_grad = G.split_tri = v;
+    }
+}
+
 static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const game_dualgrid_view_t *dg,
                       const game_config_t *config, int precision)
 {
@@ -206,17 +254,7 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
     G.flat = 1;
     for (size_t k = 0; k < (size_t)d.v && G.flat; ++k) if (g->slope[k] != 0.0) G.flat = 0;
     if (getenv("GAME_GPU_NO_FLAT_SHORTCUT")) G.flat = 0;
-    /* per-cell kernels: one thread per cell and chunk of about three layers
-       -- 163842 columns alone are only 2.5 waves per SIMD at res 7, while a
-       thread that walks a few layers reads the cell's tables once and
-       carries the values its layers share (measured at res 7 x 26: 9 chunks
-       3.80 ms/step, 26 chunks 3.87, 3 chunks 3.89); results do not depend
-       on the split */
-    G.split_cell = (d.n_layers + 2)/3;
-    if (const char *e = getenv("GAME_GPU_SPLIT_CELL")) {
-        int v = atoi(e);
-        if (v >= 1 && v <= d.n_layers) G.split_cell = v;
-    }
+    set_layer_splits(G);
     G.gd_streaming = getenv("GAME_GPU_GD_STREAMING") ? 1 : 0;
     G.gd_per_tracer = getenv("GAME_GPU_GD_PER_TRACER") ? 1 : 0;
     G.round_tendencies = 0;
@@ -230,11 +268,6 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
     G.sh_per_box = getenv("GAME_GPU_SH_PER_BOX") ? 1 : 0;
     G.unfused_phase = getenv("GAME_GPU_UNFUSED_PHASE") ? 1 : 0;
     M->use_graphs = getenv("GAME_GPU_NO_GRAPH") ? 0 : 1;
-    G.split_edge = 2;
-    if (const char *e = getenv("GAME_GPU_SPLIT_EDGE")) {
-        int v = atoi(e);
-        if (v >= 1 && v <= d.n_layers) G.split_edge = v;
-    }
     size_t S = (size_t)d.s, V = (size_t)d.v, NVH = (size_t)d.nvh, NSH = (size_t)d.nsh, NT = (size_t)d.nt;
 #define UP(dst, src, n) do { if ((rc = upload(&(dst), (src), (n)))) return rc; } while (0)
     UP(G.nd, g->normal_distance, V); UP(G.vol, g->volume, S); UP(G.area, g->area, V); UP(G.zs, g->z_scalar, S);
@@ -291,6 +324,14 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
                     t[((size_t)l*8 + j)*NSH + h] = g->inner_product_weights[8*((size_t)l*NSH + h) + j];
         UP(G.ipwT, t.data(), t.size());
         HIP_OK(hipStreamSynchronize(M->stream));
+    }
+    G.vcw = nullptr;
+    if (!G.flat) {
+        double *vcw = nullptr;
+        if ((rc = dalloc((void **)&vcw, sizeof(double)*6*(size_t)G.n_oro*NSH))) return rc;
+        hor::vcc_weights(G, vcw, M->stream);
+        HIP_OK(hipGetLastError());
+        G.vcw = vcw;
     }
     if ((rc = dalloc((void **)&G.idv, sizeof(double)*(size_t)d.s))) return rc;
     M->idv_dt = -1.0;
