@@ -45,6 +45,19 @@ struct DevGrid {
     const double *vcw;
     const double *tw, *drw, *dnd, *dzv, *darea, *fvec;
     const int *from, *to, *adj, *sgn, *ti, *tmc, *dri, *dfrom, *dto, *vit, *vst;
+    /* the tables the step's kernels read, slot-major, so that a wave's lanes
+       read consecutive words (the reference keeps an item's slots together:
+       a wave of edges touches 80 cache lines for one TRSK weight each):
+       per cell the edges c_e[j*nsh + h] and the cells across them c_n, and
+       the bits j where the edge's sign is positive (h is its from-cell),
+       c_from; per edge the TRSK weights, edges and PV indices e_tw, e_ti, e_tm
+       [j*nvh + e] and the rhombus cells and weights e_rc, e_rw; per triangle
+       its edges t_e[j*nt + t], with the top bit set where the sign is
+       negative.  A pentagon's sixth slot holds its first edge and its own
+       cell; the fifth TRSK slot of a pentagon's side holds the side's first
+       entries: valid indices whose terms the kernels leave out */
+    const unsigned *c_e, *c_n, *c_from, *e_ti, *e_tm, *e_rc, *t_e;
+    const double *e_tw, *e_rw;
     /* per-edge differences that calc_pot_vort forms for its density
        extrapolation to the top and the surface, read exactly as the
        reference's struct layout serves them (vorticities.c:48-71) */
@@ -56,10 +69,10 @@ struct DevGrid {
        it when dt changes */
     double *idv;
     /* numbers of layer chunks (gridDim.y) of the kernels that walk a column:
-       per cell (scalar transport, kinetic energy; the vertical TRSK flux's
-       levels), per edge (PV, TRSK flux, mass flux; the gradients), per
-       triangle, and of the terrain levels of the vertical corrections */
-    int split_cell, split_cell_w, split_edge, split_grad, split_tri, split_vcc;
+       per cell the levels of the vertical TRSK flux, per edge (PV and TRSK
+       flux; the gradients), per triangle, and of the terrain levels of the
+       vertical corrections */
+    int split_cell_w, split_edge, split_grad, split_tri, split_vcc;
     /* 1: tracer solver with one (column, tracer) per lane in registers; 0: LDS-staged */
     int gd_streaming;
     /* one tracer per block in the LDS-staged tracer solve instead of all five */
@@ -70,8 +83,6 @@ struct DevGrid {
     int round_tendencies;
     /* 1: sound-wave solver with one column per lane; 0: three phases over LDS */
     int vw_streaming;
-    /* 1 (26 layers): the row-parallel three-phase sound-wave kernel instead of the layer-run one */
-    int vw_rows;
     /* 1: sediment heat with one thread per grid box; 0: one thread per column (26 layers) */
     int sh_per_box;
     /* 1: temperature and phase transitions as two kernels instead of one */
@@ -102,8 +113,9 @@ struct DevWorkT {
     double *vcc;
     /* wind tendency (the FP64 form keeps it in the tendency state) */
     TW *td_wind;
-    /* c_p of every condensate at the step's temperature, n_cond x S: the
-       temperature is fixed for the whole step, so each value is formed once */
+    /* c_p of ice and of liquid water at the step's temperature, 2 x S
+       (condensate k takes c_p k & 1): the temperature is fixed for the whole
+       step, so each value is formed once */
     TW *cpc;
     /* gas density over total density of the step's old state, S (formed with
        the temperature; read by the pressure gradient at the first substep) */
@@ -120,21 +132,6 @@ __device__ __forceinline__ double density_total(const DevGrid &G, const double *
 {   /* derived_quantities.c:83-95: left-to-right sum from 0 */
     double r = 0.0;
     for (int k = 0; k < G.n_const; ++k) r += rho[k*G.s + i];
-    return r;
-}
-
-/* the same sum with the constituent count known at compile time (NC > 0):
-   all loads issue before the first add */
-template <int NC>
-__device__ __forceinline__ double density_total_n(const DevGrid &G, const double *rho, i64 i)
-{
-    if (NC <= 0) return density_total(G, rho, i);
-    double v[NC > 0 ? NC : 1];
-#pragma unroll
-    for (int k = 0; k < NC; ++k) v[k] = rho[k*G.s + i];
-    double r = 0.0;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) r += v[k];
     return r;
 }
 
@@ -166,34 +163,6 @@ __device__ __forceinline__ double c_p_water(double t)
         r = 1.000938 - 2.7052e-3*tc - 2.3235e-5*(tc*tc) + 4.3778e-6*(t2*tc) + 2.7136e-7*(t2*t2);
     }
     return 4186.8*r;
-}
-
-/* even k: ice phases (snow, cloud ice), odd k: liquid (rain, cloud water) */
-__device__ __forceinline__ double c_p_cond(int k, double t)
-{
-    return (k & 1) == 0 ? c_p_ice(t) : c_p_water(t);
-}
-
-/* c_v_mass_weighted_air with the condensates' c_p taken from a table formed
-   at the step's temperature (same terms, same order) */
-template <typename TW>
-__device__ __forceinline__ double c_v_mass_weighted_cp(const DevGrid &G, const double *rho, const TW *cpc, i64 i)
-{
-    double r = 0.0;
-    for (int k = 0; k < G.n_cond; ++k) r += rho[k*G.s + i]*(double)cpc[k*G.s + i];
-    r += rho[(i64)G.n_cond*G.s + i]*GC_C_D_V;
-    if (G.moist == 1) r += rho[(i64)(G.n_cond + 1)*G.s + i]*GC_C_V_V;
-    return r;
-}
-
-/* derived_quantities.c:97-115 */
-__device__ __forceinline__ double c_v_mass_weighted(const DevGrid &G, const double *rho, double T, i64 i)
-{
-    double r = 0.0;
-    for (int k = 0; k < G.n_cond; ++k) r += rho[k*G.s + i]*c_p_cond(k, T);
-    r += rho[(i64)G.n_cond*G.s + i]*GC_C_D_V;
-    if (G.moist == 1) r += rho[(i64)(G.n_cond + 1)*G.s + i]*GC_C_V_V;
-    return r;
 }
 
 /* averaging.c:41-95 */

@@ -16,59 +16,85 @@
 
 #define TPB 256
 #define GRID1(n) dim3((unsigned)(((n) + TPB - 1)/TPB))
-#define GRID2(n, chunks) dim3((unsigned)(((n) + TPB - 1)/TPB), (unsigned)(chunks))
 
 /* Workgroups are dispatched to the eight XCDs round-robin (workgroup i on
    XCD i % 8), each XCD with its own L2.  The gather kernels renumber their
-   workgroups so that each XCD takes one contiguous range of the grid: the
-   neighbour data a workgroup shares with the next one then sits in the same
-   L2 instead of being fetched by several XCDs. */
+   workgroups so that each XCD takes one contiguous range of the grid (x, the
+   horizontal blocks, fastest; then y, the chunks of layers): the neighbour
+   data a workgroup shares with the next one then sits in the same L2 instead
+   of being fetched by several XCDs.  Giving each XCD an eighth of x in every
+   chunk instead, so that the chunks share its tables, was slower (moist
+   scalar transport 389 -> 445 us at res 7 x 26).  Span carries the layers per
+   chunk and the reciprocal of gridDim.x: with divisions in the kernels (this
+   one, and 64-bit ones in the layer split) a wave spent over 300 scalar
+   instructions before its first load. */
 #define N_XCD 8u
+struct Span { int run; unsigned rcp; };
 struct Blk { unsigned x, y; };
-__device__ __forceinline__ Blk xcd_block()
+__device__ __forceinline__ unsigned xcd_linear(unsigned lin, unsigned T)
 {
-    const unsigned T = gridDim.x*gridDim.y, lin = blockIdx.y*gridDim.x + blockIdx.x;
     const unsigned q = T/N_XCD, r = T%N_XCD, x = lin%N_XCD, k = lin/N_XCD;
-    const unsigned m = (x < r) ? x*(q + 1) + k : r*(q + 1) + (x - r)*q + k;
+    return (x < r) ? x*(q + 1) + k : r*(q + 1) + (x - r)*q + k;
+}
+__device__ __forceinline__ Blk xcd_block(Span sp)
+{
+    const unsigned m = xcd_linear(blockIdx.y*gridDim.x + blockIdx.x, gridDim.x*gridDim.y);
+    /* rcp = ceil(2^32/gridDim.x) overestimates the quotient by one at most (m*gridDim.x < 2^32) */
     Blk b;
-    b.x = m%gridDim.x;
-    b.y = m/gridDim.x;
+    b.y = __umulhi(m, sp.rcp);
+    b.x = m - b.y*gridDim.x;
+    if ((int)b.x < 0) { --b.y; b.x += gridDim.x; }
     return b;
 }
-
-/* layers [l0, l1) of chunk `chunk` when n layers are split into gridDim.y chunks */
-__device__ __forceinline__ void layer_chunk(int n, unsigned chunk, int &l0, int &l1)
+/* the same renumbering of a one-dimensional grid */
+__device__ __forceinline__ unsigned xcd_x() { return xcd_linear(blockIdx.x, gridDim.x); }
+/* grid of n horizontal elements in `chunks` chunks, and its Span for `layers` layers or levels */
+static dim3 grid_of(int n, int chunks) { return dim3((unsigned)((n + TPB - 1)/TPB), (unsigned)chunks); }
+static Span span_of(int n, int layers, int chunks)
 {
-    l0 = (int)(((i64)n*chunk)/gridDim.y);
-    l1 = (int)(((i64)n*(chunk + 1))/gridDim.y);
+    const unsigned gx = (unsigned)((n + TPB - 1)/TPB);
+    return Span{(layers + chunks - 1)/chunks, gx > 1 ? (unsigned)(((1ULL << 32) + gx - 1)/gx) : 0xffffffffu};
+}
+
+/* element i of a row whose address is the same for the whole wave: the row's
+   base stays in scalar registers and the lane adds a 32-bit byte offset, so a
+   load costs one instruction and the offset is shared by every row read at
+   the same index (a 64-bit element index takes an address pair per load) */
+template <typename T>
+__device__ __forceinline__ T at(const T *row, unsigned i)
+{
+    return *(const T *)((const char *)row + (size_t)(i*(unsigned)sizeof(T)));
+}
+template <typename T>
+__device__ __forceinline__ void put(T *row, unsigned i, T v)
+{
+    *(T *)((char *)row + (size_t)(i*(unsigned)sizeof(T))) = v;
+}
+
+/* layers [l0, l1) of a chunk when n layers are split into chunks of `run`;
+   the last chunk may be shorter (or empty) */
+__device__ __forceinline__ void layer_chunk(int n, unsigned chunk, int run, int &l0, int &l1)
+{
+    l0 = (int)chunk*run;
+    l1 = l0 + run < n ? l0 + run : n;
 }
 
 /* ------------------------------------------------------------------ */
 /* small device helpers restating reference functions                   */
 /* ------------------------------------------------------------------ */
 
-/* raw vertical covariant gradient at an interior w point (gradient_operators.c:35-54) */
-template <typename TF>
-__device__ __forceinline__ double grad_w_raw(const DevGrid &G, const TF *f, int lev, int h)
+/* the constituent sum of derived_quantities.c:83-95 at element i of a row:
+   rho is constituent 0's row, NC the constituent count, all loads first */
+template <int NC>
+__device__ __forceinline__ double density_total_at(const DevGrid &G, const double *rho, unsigned i)
 {
-    i64 vi = h + (i64)lev*G.vpl;
-    return ((double)f[h + (i64)(lev - 1)*G.nsh] - (double)f[h + (i64)lev*G.nsh])/G.nd[vi];
-}
-
-/* averaging.c:14-39 on a stored vector field.  The weights come from the
-   cell-major copy ipwT: consecutive cells' weights are consecutive words,
-   where ipw holds a cell's eight together (one 64-byte line per lane) */
-__device__ __forceinline__ double remap_verpri2horpri(const DevGrid &G, const double *f, int l, int e)
-{
-    const int fr = G.from[e], to = G.to[e];
-    const double *w6 = G.ipwT + ((i64)l*8 + 6)*G.nsh, *w7 = w6 + G.nsh;
-    double c = w6[fr]*f[(i64)l*G.vpl + fr];
-    c += w6[to]*f[(i64)l*G.vpl + to];
-    if (l < G.L - 1) {
-        c += w7[fr]*f[(i64)(l + 1)*G.vpl + fr];
-        c += w7[to]*f[(i64)(l + 1)*G.vpl + to];
-    }
-    return 0.5*c;
+    double v[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) v[k] = at(rho + (i64)k*G.s, i);
+    double r = 0.0;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) r += v[k];
+    return r;
 }
 
 /* ------------------------------------------------------------------ */
@@ -89,239 +115,243 @@ __global__ void __launch_bounds__(TPB) k_temperature(DevGrid G, DevState s, TO *
         t = t/(1.0 + s.rho[(i64)(G.n_cond + 1)*G.s + i]/s.rho[(i64)G.n_cond*G.s + i]*(GC_M_D/GC_M_V - 1.0));
     T[i] = (TO)t;
     if (cpc) {
+        /* dictionary.c:111-190: snow and cloud ice (even constituents) share
+           the ice formula, rain and cloud water the liquid one */
         const double tt = (double)(TO)t;
-        for (int k = 0; k < G.n_cond; ++k) cpc[(i64)k*G.s + i] = (TO)c_p_cond(k, tt);   /* dictionary.c:111-190 */
+        cpc[i] = (TO)c_p_ice(tt);
+        cpc[G.s + i] = (TO)c_p_water(tt);
     }
+}
+
+/* what the momentum tendency and the wind update read and write beside the
+   pressure gradient (vector_tendencies_expl.c:74-131, manage_rkhevi.c:67-75):
+   the tendency td, the old and new wind, the substep's weight new_w of the
+   new tendency.  friction_acc is zero with momentum diffusion and PBL off:
+   x + 0.0 == x.  The old tendency has weight 1 - new_w = 0 in the first
+   substep, where it is neither read nor added (its product with 0 is a zero,
+   the identity of the sum); IEEE addition commutes, so adding it last changes
+   no bit.  The kernels that form the last missing term take the update along:
+   a kernel of its own read each term again (150 us per substep at res 7 x 26) */
+template <typename TW>
+struct Mom {
+    TW *td;
+    const double *wind_old;
+    double *wind_new;
+    double new_w, dt;
+};
+
+/* derived_quantities.c:15-40 via gas fractions: gas over total density of one
+   box of row l (NC constituents) */
+template <int NC>
+__device__ __forceinline__ double gas_fraction_at(const DevGrid &G, const double *rho, i64 row, unsigned h)
+{
+    constexpr int n_cond = NC == 6 ? 4 : 0;
+    const double total = density_total_at<NC>(G, rho + row, h);
+    return at(rho + n_cond*G.s + row, h)/total;
 }
 
 /* manage_pressure_gradient.c:17-87 at the interior w points (layers 1..L-1),
-   fused with calc_pressure_grad_condensates_v */
-template <typename TW, int NC>
-__global__ void __launch_bounds__(TPB) k_pgrad_w(DevGrid G, DevState s, DevWorkT<TW> W, int first_step, int with_pgrad,
-                                                 const double *gf, double cvw)
+   fused with calc_pressure_grad_condensates_v; gf: the gas fractions of state
+   s, formed with the reference's arithmetic by the temperature kernel.  TEND:
+   with the first substep's tendency, for which the carried momentum advection
+   is there (every step but a first one) */
+template <typename TW, bool TEND>
+__global__ void __launch_bounds__(TPB) k_pgrad_w(DevGrid G, DevState s, DevWorkT<TW> W, int first_step,
+                                                 const double *gf, double cvw, Mom<TW> m, Span sp)
 {
-    i64 n = (i64)(G.L - 1)*G.nsh;
-    i64 t = (i64)xcd_block().x*TPB + threadIdx.x;
-    if (t >= n) return;
-    int lev = (int)(t/G.nsh) + 1, h = (int)(t - (i64)(lev - 1)*G.nsh);
-    i64 w = h + (i64)lev*G.vpl, up = h + (i64)(lev - 1)*G.nsh, lo = h + (i64)lev*G.nsh;
-    i64 gi = (i64)G.n_cond*G.s;
-    /* gf: the gas fractions of state s, formed with this arithmetic by k_temperature */
-    double rt_up = 0.0, rt_lo = 0.0, d_up, d_lo;
-    if (gf) { d_up = gf[up]; d_lo = gf[lo]; }
-    else {
-        rt_up = density_total_n<NC>(G, s.rho, up);
-        rt_lo = density_total_n<NC>(G, s.rho, lo);
-        d_up = s.rho[gi + up]/rt_up;
-        d_lo = s.rho[gi + lo]/rt_lo;
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*TPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
+    const int lev = (int)bk.y + 1;
+    const i64 w = (i64)lev*G.vpl, lo = (i64)lev*G.nsh, up = lo - G.nsh;   /* rows of the level and of the layers around it */
+    const double d_up = at(gf + up, h), d_lo = at(gf + lo, h);
+    const double gm = at(G.gm + w, h);
+    double pvt = 0.0, vg = 0.0;
+    if (TEND) { pvt = (double)at(W.pvt + w, h); vg = (double)at(W.vsq_grad + w, h); }
+    TW old_t = (TW)0;
+    if (!first_step) old_t = (TW)(-(double)at(W.pgrad_nl + w, h) - (double)at(W.pgrad_l + w, h));
+    const double tp_up = at(s.tp + up, h), tp_lo = at(s.tp + lo, h);
+    double raw = (at(s.ep + up, h) - at(s.ep + lo, h))/at(G.nd + w, h);
+    double p1_up = GC_C_D_P*(at(G.thbg + up, h) + tp_up), p1_lo = GC_C_D_P*(at(G.thbg + lo, h) + tp_lo);
+    double nl = (0.5*(p1_up + p1_lo))*raw;
+    double p2_up = GC_C_D_P*tp_up, p2_lo = GC_C_D_P*tp_lo;
+    double ll = (0.5*(p2_up + p2_lo))*at(G.exbg_grad + w, h);
+    nl = (0.5*(d_up + d_lo))*nl;
+    ll = (0.5*(d_up + d_lo))*ll;
+    if (first_step) old_t = (TW)(-nl - ll);
+    /* the momentum tendency's combination of the stored values
+       (vector_tendencies_expl.c), which the second substep reads */
+    const TW comb = (TW)(-cvw*((double)(TW)nl + (double)(TW)ll));
+    double c_up = d_up - 1.0, c_lo = d_lo - 1.0;
+    const TW pgc = (TW)((0.5*(c_up + c_lo))*gm);
+    put(W.pgrad_old + w, h, old_t);
+    put(W.pgrad_nl + w, h, (TW)nl);
+    put(W.pgrad_l + w, h, (TW)ll);
+    put(W.pgrad_comb + w, h, comb);
+    put(W.pgc_v + w, h, pgc);
+    if (TEND) {
+        const double tv = m.new_w*(
+            (double)comb   /* -cvw*(nl + l) */
+            + pvt
+            - 0.5*vg
+            + (double)pgc);
+        put(m.td + w, h, (TW)tv);
     }
-    if (with_pgrad) {
-        if (!first_step) W.pgrad_old[w] = (TW)(-(double)W.pgrad_nl[w] - (double)W.pgrad_l[w]);
-        double raw = (s.ep[up] - s.ep[lo])/G.nd[w];
-        double p1_up = GC_C_D_P*(G.thbg[up] + s.tp[up]), p1_lo = GC_C_D_P*(G.thbg[lo] + s.tp[lo]);
-        double nl = (0.5*(p1_up + p1_lo))*raw;
-        double p2_up = GC_C_D_P*s.tp[up], p2_lo = GC_C_D_P*s.tp[lo];
-        double ll = (0.5*(p2_up + p2_lo))*G.exbg_grad[w];
-        nl = (0.5*(d_up + d_lo))*nl;
-        ll = (0.5*(d_up + d_lo))*ll;
-        W.pgrad_nl[w] = (TW)nl;
-        W.pgrad_l[w] = (TW)ll;
-        if (first_step) W.pgrad_old[w] = (TW)(-nl - ll);
-        /* the momentum tendency's combination of the stored values
-           (vector_tendencies_expl.c) */
-        W.pgrad_comb[w] = (TW)(-cvw*((double)(TW)nl + (double)(TW)ll));
-    }
-    double c_up = d_up - 1.0, c_lo = d_lo - 1.0;   /* s.rho[gi + up]/rt_up - 1.0 */
-    W.pgc_v[w] = (TW)((0.5*(c_up + c_lo))*G.gm[w]);
-}
-
-/* manage_pressure_gradient.c:17-72 at the edges: one thread per edge walks
-   all layers, so the edge's table entries are read once */
-template <bool FLAT, typename TF>
-__device__ __forceinline__ double grad_edge_t(const DevGrid &G, const TF *f, int l, int e, int fr, int to)
-{
-    i64 vi = G.nsh + (i64)l*G.vpl + e;
-    double g = ((double)f[to + (i64)l*G.nsh] - (double)f[fr + (i64)l*G.nsh])/G.nd[vi];
-    if (!FLAT && l >= G.L - G.n_oro) {
-        const double *w6 = G.ipwT + ((i64)l*8 + 6)*G.nsh, *w7 = w6 + G.nsh;
-        double c = w6[fr]*grad_w_raw(G, f, l, fr);
-        c += w6[to]*grad_w_raw(G, f, l, to);
-        if (l < G.L - 1) {
-            c += w7[fr]*grad_w_raw(G, f, l + 1, fr);
-            c += w7[to]*grad_w_raw(G, f, l + 1, to);
-        }
-        c = 0.5*c;
-        g += -G.slope[vi]*c;
-    }
-    return g;
 }
 
 /* grad at the edges (gradient_operators.c:14-33 with the terrain term of
    averaging.c:113-133) for the successive layers l0, l0 + 1, ... of one
    edge, as manage_pressure_gradient.c:17-72 and the kinetic-energy gradient
-   use it.  The two cells' values of layer l + 1 and their vertical
-   gradients at the w level between layers l and l + 1, which layer l's
-   terrain correction reads, are carried to layer l + 1 instead of loaded
+   use it.  Over orography the two cells' values of layer l + 1 and their
+   vertical gradients at the w level between layers l and l + 1, which layer
+   l's terrain correction reads, are carried to layer l + 1 instead of loaded
    and formed again; each quotient is the one the layer-wise formula forms,
    so the results are identical.  The next layer's values are loaded before
-   this layer's are combined.  Used where terrain terms exist: on a flat
-   grid the layer-wise form needs fewer registers (the flat pressure
-   gradient keeps five waves per SIMD). */
+   this layer's are combined.  A flat grid needs none of it and no registers
+   for it.  The weights come from the cell-major copy ipwT: consecutive cells'
+   weights are consecutive words, where ipw holds a cell's eight together (one
+   64-byte line per lane). */
 struct EdgeCarry { double ff, ft, gwf, gwt; };
 
 template <bool FLAT, typename TF>
-__device__ __forceinline__ double grad_edge_walk(const DevGrid &G, const TF *f, int l, int l0, int e, int fr, int to,
-                                                 EdgeCarry &c)
+__device__ __forceinline__ double grad_edge_walk(const DevGrid &G, const TF *f, int l, int l0, unsigned e, unsigned fr,
+                                                 unsigned to, EdgeCarry &c)
 {
     const int nsh = G.nsh, L = G.L, lt = L - G.n_oro;
-    const i64 vi = nsh + (i64)l*G.vpl + e;
-    if (l == l0) { c.ff = (double)f[fr + (i64)l*nsh]; c.ft = (double)f[to + (i64)l*nsh]; }
+    const i64 vi = nsh + (i64)l*G.vpl;
+    const TF *fl = f + (i64)l*nsh;
+    if constexpr (FLAT) return ((double)at(fl, to) - (double)at(fl, fr))/at(G.nd + vi, e);
+    if (l == l0) { c.ff = (double)at(fl, fr); c.ft = (double)at(fl, to); }
     /* layer l + 1 (the last layer reloads itself, unused) */
-    const int ln = l + 1 < L ? l + 1 : l;
-    const double nff = (double)f[fr + (i64)ln*nsh], nft = (double)f[to + (i64)ln*nsh];
-    double g = (c.ft - c.ff)/G.nd[vi];
-    if (!FLAT && l >= lt) {
-        /* grad_w_raw at level l of both cells: carried unless layer l - 1
-           had no terrain term or lies in another chunk */
-        if (l == l0 || l == lt) { c.gwf = grad_w_raw(G, f, l, fr); c.gwt = grad_w_raw(G, f, l, to); }
+    const TF *fn = l + 1 < L ? fl + nsh : fl;
+    const double nff = (double)at(fn, fr), nft = (double)at(fn, to);
+    double g = (c.ft - c.ff)/at(G.nd + vi, e);
+    if (l >= lt) {
         const double *w6 = G.ipwT + ((i64)l*8 + 6)*nsh, *w7 = w6 + nsh;
-        double s = w6[fr]*c.gwf;
-        s += w6[to]*c.gwt;
+        /* the vertical gradient at level l of both cells
+           (gradient_operators.c:35-54): carried unless layer l - 1 had no
+           terrain term or lies in another chunk */
+        if (l == l0 || l == lt) {
+            const double *nw = G.nd + (i64)l*G.vpl;
+            c.gwf = ((double)at(fl - nsh, fr) - c.ff)/at(nw, fr);
+            c.gwt = ((double)at(fl - nsh, to) - c.ft)/at(nw, to);
+        }
+        double s = at(w6, fr)*c.gwf;
+        s += at(w6, to)*c.gwt;
         if (l < L - 1) {
-            /* grad_w_raw at level l + 1 */
-            const double gf1 = (c.ff - nff)/G.nd[fr + (i64)(l + 1)*G.vpl];
-            const double gt1 = (c.ft - nft)/G.nd[to + (i64)(l + 1)*G.vpl];
-            s += w7[fr]*gf1;
-            s += w7[to]*gt1;
+            /* at level l + 1 */
+            const double *nw = G.nd + (i64)(l + 1)*G.vpl;
+            const double gf1 = (c.ff - nff)/at(nw, fr);
+            const double gt1 = (c.ft - nft)/at(nw, to);
+            s += at(w7, fr)*gf1;
+            s += at(w7, to)*gt1;
             c.gwf = gf1;
             c.gwt = gt1;
         }
         s = 0.5*s;
-        g += -G.slope[vi]*s;
+        g += -at(G.slope + vi, e)*s;
     }
     c.ff = nff;
     c.ft = nft;
     return g;
 }
 
-template <bool FLAT, typename TW, int NC>
+/* manage_pressure_gradient.c:17-72 at the edges: one thread per edge walks a
+   chunk of layers, so the edge's table entries are read once.  TEND: with the
+   first substep's tendency and wind update (as k_pgrad_w) */
+template <bool FLAT, typename TW, bool TEND>
 __global__ void __launch_bounds__(TPB) k_pgrad_e(DevGrid G, DevState s, DevWorkT<TW> W, int first_step,
-                                                 const double *gf, double chw, double ohw)
+                                                 const double *gf, double chw, double ohw, Mom<TW> m, Span sp)
 {
-    const Blk bk = xcd_block();
-    int e = bk.x*TPB + threadIdx.x;
-    if (e >= G.nvh) return;
-    const int fr = G.from[e], to = G.to[e];
-    const i64 gi = (i64)G.n_cond*G.s;
+    const Blk bk = xcd_block(sp);
+    const unsigned e = bk.x*TPB + threadIdx.x;
+    if (e >= (unsigned)G.nvh) return;
+    const unsigned fr = G.from[e], to = G.to[e];
     int l0, l1;
-    layer_chunk(G.L, bk.y, l0, l1);
+    layer_chunk(G.L, bk.y, sp.run, l0, l1);
     EdgeCarry carry;
     for (int l = l0; l < l1; ++l) {
-        i64 vi = G.nsh + (i64)l*G.vpl + e;
+        const i64 vi = G.nsh + (i64)l*G.vpl, sl = (i64)l*G.nsh;
         TW old_t = 0;
-        if (!first_step) {
-            old_t = (TW)(-(double)W.pgrad_nl[vi] - (double)W.pgrad_l[vi]);
-            W.pgrad_old[vi] = old_t;
+        if (!first_step) old_t = (TW)(-(double)at(W.pgrad_nl + vi, e) - (double)at(W.pgrad_l + vi, e));
+        double pvt = 0.0, vg = 0.0, wo = 0.0;
+        if (TEND) {
+            pvt = (double)at(W.pvt + vi, e);
+            vg = (double)at(W.vsq_grad + vi, e);
+            wo = at(m.wind_old + vi, e);
         }
-        i64 sf = (i64)l*G.nsh + fr, st = (i64)l*G.nsh + to;
-        double g;
-        if constexpr (FLAT) g = grad_edge_t<FLAT, double>(G, s.ep, l, e, fr, to);
-        else g = grad_edge_walk<FLAT, double>(G, s.ep, l, l0, e, fr, to, carry);
-        double p1_t = GC_C_D_P*(G.thbg[st] + s.tp[st]), p1_f = GC_C_D_P*(G.thbg[sf] + s.tp[sf]);
+        const double g = grad_edge_walk<FLAT, double>(G, s.ep, l, l0, e, fr, to, carry);
+        const double tp_t = at(s.tp + sl, to), tp_f = at(s.tp + sl, fr);
+        double p1_t = GC_C_D_P*(at(G.thbg + sl, to) + tp_t), p1_f = GC_C_D_P*(at(G.thbg + sl, fr) + tp_f);
         double nl = (0.5*(p1_t + p1_f))*g;
-        double p2_t = GC_C_D_P*s.tp[st], p2_f = GC_C_D_P*s.tp[sf];
-        double ll = (0.5*(p2_t + p2_f))*G.exbg_grad[vi];
-        double d_t, d_f;
-        if (gf) { d_t = gf[st]; d_f = gf[sf]; }
-        else {
-            d_t = s.rho[gi + st]/density_total_n<NC>(G, s.rho, st);
-            d_f = s.rho[gi + sf]/density_total_n<NC>(G, s.rho, sf);
-        }
+        double p2_t = GC_C_D_P*tp_t, p2_f = GC_C_D_P*tp_f;
+        double ll = (0.5*(p2_t + p2_f))*at(G.exbg_grad + vi, e);
+        const double d_t = at(gf + sl, to), d_f = at(gf + sl, fr);
         nl = (0.5*(d_t + d_f))*nl;
         ll = (0.5*(d_t + d_f))*ll;
-        W.pgrad_nl[vi] = (TW)nl;
-        W.pgrad_l[vi] = (TW)ll;
-        if (first_step) {
-            old_t = (TW)(-nl - ll);
-            W.pgrad_old[vi] = old_t;
-        }
+        if (first_step) old_t = (TW)(-nl - ll);
         /* the momentum tendency's combination of the stored values
-           (vector_tendencies_expl.c) */
-        W.pgrad_comb[vi] = (TW)(ohw*(double)old_t - chw*((double)(TW)nl + (double)(TW)ll));
-    }
-}
-
-/* scalar_times_vector(rho_gas, wind) into the mass flux density
-   (multiplications.c:35-117).  One thread per edge and chunk of layers (the
-   edge's from/to cells are read once), and one per cell and chunk of w
-   levels, in the same launch. */
-template <typename TW>
-__global__ void __launch_bounds__(TPB) k_mass_flux(DevGrid G, const double *rho_gas, const double *wind, TW *flux)
-{
-    const Blk bk = xcd_block();
-    const int t = bk.x*TPB + threadIdx.x;
-    const int nsh = G.nsh, vpl = G.vpl, L = G.L;
-    int l0, l1;
-    layer_chunk(L, bk.y, l0, l1);
-    if (t < G.nvh) {
-        const int e = t, fr = G.from[e], to = G.to[e];
-        for (int l = l0; l < l1; ++l) {
-            const i64 vi = nsh + (i64)l*vpl + e;
-            const double sv = 0.5*(rho_gas[to + (i64)l*nsh] + rho_gas[fr + (i64)l*nsh]);
-            flux[vi] = (TW)(sv*wind[vi]);
-        }
-    }
-    if (t < nsh) {
-        /* interior w levels 1..L-1: level lev of this chunk's layers [l0, l1) */
-        const int h = t;
-        for (int lev = l0 > 1 ? l0 : 1; lev < l1; ++lev) {
-            const i64 w = (i64)lev*vpl + h;
-            const double sv = 0.5*(rho_gas[h + (i64)(lev - 1)*nsh] + rho_gas[h + (i64)lev*nsh]);
-            flux[w] = (TW)(sv*wind[w]);
+           (vector_tendencies_expl.c), which the second substep reads */
+        const TW comb = (TW)(ohw*(double)old_t - chw*((double)(TW)nl + (double)(TW)ll));
+        put(W.pgrad_old + vi, e, old_t);
+        put(W.pgrad_nl + vi, e, (TW)nl);
+        put(W.pgrad_l + vi, e, (TW)ll);
+        put(W.pgrad_comb + vi, e, comb);
+        if (TEND) {
+            const double tv = m.new_w*(
+                (double)comb   /* ohw*old - chw*(nl + l) */
+                + pvt
+                - 0.5*vg);
+            put(m.td + vi, e, (TW)tv);
+            put(m.wind_new + vi, e, wo + m.dt*tv);
         }
     }
 }
 
-/* vorticities.c:167-222, one thread per triangle walking all layers.
+/* vorticities.c:167-222, one thread per triangle and chunk of layers.
    The loads of the layer below are issued before the current layer is
    formed, and the wind and edge heights of the layers above and below (the
    two candidates of the terrain interpolation) are carried in registers, so
    no load waits on the sign test that selects between them. */
 template <typename TW>
-__global__ void __launch_bounds__(TPB) k_rel_vort_tri(DevGrid G, const double *w, TW *res)
+__global__ void __launch_bounds__(TPB) k_rel_vort_tri(DevGrid G, const double *w, TW *res, Span sp)
 {
-    const Blk bk = xcd_block();
-    const int h = bk.x*TPB + threadIdx.x;
-    if (h >= G.nt) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*TPB + threadIdx.x;
+    if (h >= (unsigned)G.nt) return;
     const int L = G.L, lt = L - G.n_oro, nsh = G.nsh, vpl = G.vpl, nvh = G.nvh;
     const i64 dvpl = G.dvpl;
-    int vit[3];
+    unsigned vit[3];
     double sg[3];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) { vit[j] = G.vit[3*h + j]; sg[j] = (double)G.vst[3*h + j]; }
+    for (int j = 0; j < 3; ++j) {
+        const unsigned q = at(G.t_e + (i64)j*G.nt, h);
+        vit[j] = q & 0x7fffffffu;
+        sg[j] = q >> 31 ? -1.0 : 1.0;
+    }
     struct Lay { double w[3], z[3], nd[3], dz, da; };
     auto load = [&](int l) {
         Lay x;
+        const i64 vi = nsh + (i64)l*vpl, di = nvh + (i64)l*dvpl;
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
-            const i64 vi = nsh + (i64)l*vpl + vit[j];
-            x.w[j] = w[vi];
-            x.z[j] = G.zv[vi];
-            x.nd[j] = G.nd[vi];
+            x.w[j] = at(w + vi, vit[j]);
+            x.z[j] = at(G.zv + vi, vit[j]);
+            x.nd[j] = at(G.nd + vi, vit[j]);
         }
-        const i64 di = nvh + (i64)l*dvpl + h;
-        x.dz = G.dzv[di];
-        x.da = G.darea[di];
+        x.dz = at(G.dzv + di, h);
+        x.da = at(G.darea + di, h);
         return x;
     };
     int l0, l1;
-    layer_chunk(L, bk.y, l0, l1);
+    layer_chunk(L, bk.y, sp.run, l0, l1);
+    if (l0 >= l1) return;
     double wp[3], zp[3];   /* layer l - 1 (layer 0, unused, at the top) */
+    const i64 vp = nsh + (i64)(l0 > 0 ? l0 - 1 : 0)*vpl;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-        const i64 vi = nsh + (i64)(l0 > 0 ? l0 - 1 : 0)*vpl + vit[j];
-        wp[j] = w[vi];
-        zp[j] = G.zv[vi];
+        wp[j] = at(w + vp, vit[j]);
+        zp[j] = at(G.zv + vp, vit[j]);
     }
     Lay cur = load(l0);
     for (int l = l0; l < l1; ++l) {
@@ -341,104 +371,128 @@ __global__ void __launch_bounds__(TPB) k_rel_vort_tri(DevGrid G, const double *w
             }
             r += lrf*cur.nd[j]*sg[j]*vel;
         }
-        res[(i64)l*G.nt + h] = (TW)(r/cur.da);
+        put(res + (i64)l*G.nt, h, (TW)(r/cur.da));
 #pragma unroll
         for (int j = 0; j < 3; ++j) { wp[j] = cur.w[j]; zp[j] = cur.z[j]; }
         cur = nxt;
     }
 }
 
-/* averaging.c:97-111 */
+/* averaging.c:97-111 with averaging.c:14-39: the horizontal covariant
+   component of edge e in layer l; its wind u and the w points wf and wt of
+   level l at its cells are the caller's (it has loaded them) */
 template <bool FLAT>
-__device__ __forceinline__ double horizontal_covariant_t(const DevGrid &G, const double *w, int l, int e)
+__device__ __forceinline__ double horizontal_covariant_t(const DevGrid &G, const double *w, int l, double u,
+                                                         unsigned e, unsigned fr, unsigned to, double wf, double wt)
 {
-    i64 vi = G.nsh + (i64)l*G.vpl + e;
-    double r = w[vi];
+    const i64 vi = G.nsh + (i64)l*G.vpl;
+    double r = u;
     if (!FLAT && l >= G.L - G.n_oro) {
-        double vc = remap_verpri2horpri(G, w, l, e);
-        r += G.slope[vi]*vc;
+        const double *w6 = G.ipwT + ((i64)l*8 + 6)*G.nsh, *w7 = w6 + G.nsh;
+        const double *wn = w + (i64)(l + 1)*G.vpl;
+        /* the lowest layer loads the surface terms and leaves them out */
+        const double slope = at(G.slope + vi, e), a6 = at(w6, fr), b6 = at(w6, to), a7 = at(w7, fr), b7 = at(w7, to);
+        const double nf = at(wn, fr), nt = at(wn, to);
+        double c = a6*wf;
+        c += b6*wt;
+        if (l < G.L - 1) {
+            c += a7*nf;
+            c += b7*nt;
+        }
+        c = 0.5*c;
+        r += slope*c;
     }
     return r;
 }
 
-/* tangential relative vorticity of edge e at level l >= 1 (vorticities.c:131-156) */
-template <bool FLAT>
-__device__ __forceinline__ double rel_vort_tangential(const DevGrid &G, const double *w, int l, int e, int fr, int to)
-{
-    i64 base = (i64)l*G.vpl;
-    const double *nd = G.nd;
-    if (l == G.L) {
-        i64 i2 = base - G.nvh + e;
-        double cv2 = horizontal_covariant_t<FLAT>(G, w, l - 1, e);
-        return 1/G.darea[e + (i64)l*G.dvpl]*nd[i2]*cv2;
-    }
-    i64 i0 = base + G.nsh + e, i1 = base + fr, i2 = base - G.nvh + e, i3 = base + to;
-    double cv0 = horizontal_covariant_t<FLAT>(G, w, l, e);
-    double cv2 = horizontal_covariant_t<FLAT>(G, w, l - 1, e);
-    return 1/G.darea[e + (i64)l*G.dvpl]*(
-        - nd[i0]*cv0
-        + nd[i1]*w[i1]
-        + nd[i2]*cv2
-        - nd[i3]*w[i3]);
-}
-
 /* calc_pot_vort = calc_rel_vort + add_f_to_rel_vort + division by the
-   interpolated density (vorticities.c:18-165).  One thread per edge walks all
-   levels and writes the tangential element of each level and the rhombus
-   element of each layer. */
+   interpolated density (vorticities.c:18-165), and the mass flux density
+   (scalar_times_vector of rho_gas and the wind, multiplications.c:35-117).
+   One thread per edge walks a chunk of levels and writes the tangential
+   element of each level and the rhombus element and mass flux of each layer,
+   whose densities and wind the vorticity reads anyway (a kernel of its own
+   took 92 us at res 7 x 26); the threads that have a cell of their number
+   write the mass flux of its interior w points. */
 template <bool FLAT, typename TW>
 __global__ void __launch_bounds__(TPB) k_pot_vort(DevGrid G, const double *w, const double *rho, const TW *rvt,
-                                                  TW *pv)
+                                                  TW *pv, TW *flux, Span sp)
 {
-    const Blk bk = xcd_block();
-    int e = bk.x*TPB + threadIdx.x;
-    if (e >= G.nvh) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned e = bk.x*TPB + threadIdx.x;
+    if (e >= (unsigned)G.nvh) return;
     const int nvh = G.nvh, nsh = G.nsh, L = G.L, vpl = G.vpl;
-    const int fr = G.from[e], to = G.to[e], fd = G.dfrom[e], td = G.dto[e];
+    const unsigned fr = G.from[e], to = G.to[e], fd = G.dfrom[e], td = G.dto[e];
     const double *nd = G.nd;
-    int dri[4];
+    unsigned dri[4];
     double drw[4];
-    for (int j = 0; j < 4; ++j) { dri[j] = G.dri[4*e + j]; drw[j] = G.drw[4*e + j]; }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { dri[j] = at(G.e_rc + (i64)j*nvh, e); drw[j] = at(G.e_rw + (i64)j*nvh, e); }
     /* the edge's two cells are two of its rhombus cells: their densities come
        with the rhombus loads, and the layer above's are carried from the
        previous level, as are the covariant wind and normal distance of the
        edge in the layer above (each value is the one the reference's
        formula reads, so the arithmetic is unchanged) */
     int pf = 0, pt = 0;
+#pragma unroll
     for (int j = 0; j < 4; ++j) { if (dri[j] == fr) pf = j; if (dri[j] == to) pt = j; }
     const double f_t = G.fvec[e], f_r = G.fvec[nvh + e];
     int l0, l1;
-    layer_chunk(L + 1, bk.y, l0, l1);
-    double rv1 = (l0 <= 1) ? rel_vort_tangential<FLAT>(G, w, 1, e, fr, to) : 0.0;
+    layer_chunk(L + 1, bk.y, sp.run, l0, l1);
+    if (l0 >= l1) return;
+    const bool cell = e < (unsigned)nsh;
+    auto cov = [&](int l, double u, double wf, double wt) {
+        return horizontal_covariant_t<FLAT>(G, w, l, u, e, fr, to, wf, wt);
+    };
+    /* the tangential vorticity of level 1, which the top copies
+       (vorticities.c:158-163); a first chunk that reaches level 1 has it */
+    double rv1 = 0.0;
+    if (l0 <= 1) {
+        const i64 base = vpl;
+        const double wf = at(w + base, fr), wt = at(w + base, to);
+        const double c1 = cov(1, at(w + base + nsh, e), wf, wt), c0 = cov(0, at(w + nsh, e), at(w, fr), at(w, to));
+        rv1 = 1/at(G.darea + G.dvpl, e)*(
+            - at(nd + base + nsh, e)*c1
+            + at(nd + base, fr)*wf
+            + at(nd + nsh, e)*c0
+            - at(nd + base, to)*wt);
+    }
     /* layer l-1 at the edge: density of both cells, covariant wind, normal distance */
     double rf_m = 0.0, rt_m = 0.0, cv_m = 0.0, nd_m = 0.0;
     if (l0 >= 1) {
-        rf_m = rho[(i64)(l0 - 1)*nsh + fr];
-        rt_m = rho[(i64)(l0 - 1)*nsh + to];
-        cv_m = horizontal_covariant_t<FLAT>(G, w, l0 - 1, e);
-        nd_m = nd[nsh + (i64)(l0 - 1)*vpl + e];
+        const double *rm = rho + (i64)(l0 - 1)*nsh, *wm = w + (i64)(l0 - 1)*vpl;
+        rf_m = at(rm, fr);
+        rt_m = at(rm, to);
+        cv_m = cov(l0 - 1, at(wm + nsh, e), FLAT ? 0.0 : at(wm, fr), FLAT ? 0.0 : at(wm, to));
+        nd_m = at(nd + nsh + (i64)(l0 - 1)*vpl, e);
     }
+    double rc_m = (cell && l0 >= 1) ? at(rho + (i64)(l0 - 1)*nsh, e) : 0.0;   /* the cell's density in the layer above */
     for (int l = l0; l < l1; ++l) {
         if (l == L) {
             /* the lowest level (vorticities.c:158-163 and the surface density extrapolation) */
-            const double rv = 1/G.darea[e + (i64)l*G.dvpl]*nd_m*cv_m;
-            const i64 a = (i64)(l - 1)*nsh, b = (i64)(l - 2)*nsh;
-            const double dv = 0.5*(rho[a + fr] + rho[a + to])
-                              + (0.5*(rho[b + fr] + rho[b + to]) - 0.5*(rho[a + fr] + rho[a + to]))
+            const double rv = 1/at(G.darea + (i64)l*G.dvpl, e)*nd_m*cv_m;
+            const double *ra = rho + (i64)(l - 1)*nsh, *rb = ra - nsh;
+            const double af = at(ra, fr), at_ = at(ra, to), bf = at(rb, fr), bt = at(rb, to);
+            const double dv = 0.5*(af + at_)
+                              + (0.5*(bf + bt) - 0.5*(af + at_))
                               /G.pv_sfc_dz1[e]*G.pv_sfc_dz2[e];
-            pv[(i64)l*2*nvh + e] = (TW)((rv + f_t)/dv);
+            put(pv + (i64)l*2*nvh, e, (TW)((rv + f_t)/dv));
             break;
         }
         /* loads of level l */
-        const i64 base = (i64)l*vpl, i0 = base + nsh + e, i1 = base + fr, i3 = base + to;
-        const i64 db = nvh + (i64)l*G.dvpl;
+        const i64 base = (i64)l*vpl, db = nvh + (i64)l*G.dvpl;
+        const double *rl = rho + (i64)l*nsh;
         double r4[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r4[j] = rho[(i64)l*nsh + dri[j]];
-        const double nd0 = nd[i0], nd1 = nd[i1], nd3 = nd[i3], w1 = w[i1], w3 = w[i3];
-        const double da_e = G.darea[e + (i64)l*G.dvpl], af = G.darea[db + fd], at = G.darea[db + td];
-        const double rvf = (double)rvt[(i64)l*G.nt + fd], rvd = (double)rvt[(i64)l*G.nt + td];
-        const double cv0 = horizontal_covariant_t<FLAT>(G, w, l, e);
+        for (int j = 0; j < 4; ++j) r4[j] = at(rl, dri[j]);
+        const double nd0 = at(nd + base + nsh, e), nd1 = at(nd + base, fr), nd3 = at(nd + base, to);
+        const double w1 = at(w + base, fr), w3 = at(w + base, to);
+        const double da_e = at(G.darea + (i64)l*G.dvpl, e), af = at(G.darea + db, fd), at_ = at(G.darea + db, td);
+        const TW *rvl = rvt + (i64)l*G.nt;
+        const double rvf = (double)at(rvl, fd), rvd = (double)at(rvl, td);
+        const double u0 = at(w + base + nsh, e);
+        double rc = 0.0, wc = 0.0;
+        if (cell) { rc = at(rl, e); wc = at(w + base, e); }
+        const double cv0 = cov(l, u0, w1, w3);
         const double rf = pf == 0 ? r4[0] : (pf == 1 ? r4[1] : (pf == 2 ? r4[2] : r4[3]));
         const double rt = pt == 0 ? r4[0] : (pt == 1 ? r4[1] : (pt == 2 ? r4[2] : r4[3]));
         /* tangential element at level l; the top copies level 1 (vorticities.c:158-163) */
@@ -447,55 +501,82 @@ __global__ void __launch_bounds__(TPB) k_pot_vort(DevGrid G, const double *w, co
         else rv = 1/da_e*(- nd0*cv0 + nd1*w1 + nd_m*cv_m - nd3*w3);
         double dv;
         if (l == 0) {
-            const double rf1 = rho[nsh + fr], rt1 = rho[nsh + to];
+            const double rf1 = at(rl + nsh, fr), rt1 = at(rl + nsh, to);
             dv = 0.5*(rf + rt) + (0.5*(rf + rt) - 0.5*(rf1 + rt1))/G.pv_top_dz1[e]*G.pv_top_dz2[e];
         } else dv = 0.25*(rf_m + rt_m + rf + rt);
-        pv[(i64)l*2*nvh + e] = (TW)((rv + f_t)/dv);
+        put(pv + (i64)l*2*nvh, e, (TW)((rv + f_t)/dv));
         /* rhombus element of layer l */
-        const double rr = (af*rvf + at*rvd)/(af + at);
+        const double rr = (af*rvf + at_*rvd)/(af + at_);
         double dr = 0;
 #pragma unroll
         for (int j = 0; j < 4; ++j) dr += drw[j]*r4[j];
-        pv[(i64)l*2*nvh + nvh + e] = (TW)((rr + f_r)/dr);
+        put(pv + (i64)l*2*nvh + nvh, e, (TW)((rr + f_r)/dr));
+        put(flux + base + nsh, e, (TW)((0.5*(rt + rf))*u0));
+        if (cell) {
+            if (l >= 1) put(flux + base, e, (TW)((0.5*(rc_m + rc))*wc));
+            rc_m = rc;
+        }
         rf_m = rf; rt_m = rt; cv_m = cv0; nd_m = nd0;
     }
 }
 
-/* vorticity_flux.c:16-187, horizontal part: one thread per edge, all layers */
-template <typename TW>
+/* vorticity_flux.c:16-187, horizontal part: one thread per edge and chunk of
+   layers.  TEND: with the kinetic-energy gradient (gradient_operators.c:14-33)
+   and the tendency and wind update of vector_tendencies_expl.c:74-131 and
+   manage_rkhevi.c:67-75, whose other terms are there: the flux and the
+   gradient are stored (the next step's first substep reads them) but not read
+   back, and the terrain weights of both are loaded once. */
+template <bool FLAT, typename TW, bool TEND>
 /* at most two waves per SIMD: the register budget lets every gather of a
    layer issue in one batch (measured faster than four waves with the gathers
    issued in pairs) */
 __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_vorticity_flux_e(DevGrid G, const TW *F, const TW *pv, TW *out)
+k_vorticity_flux_e(DevGrid G, const TW *F, const TW *pv, TW *out, DevWorkT<TW> W, Mom<TW> m, Span sp)
 {
-    const Blk bk = xcd_block();
-    int e = bk.x*TPB + threadIdx.x;
-    if (e >= G.nvh) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned e = bk.x*TPB + threadIdx.x;
+    if (e >= (unsigned)G.nvh) return;
     const int nsh = G.nsh, nvh = G.nvh;
     double tw[10];
-    int ti[10], tm[10];
-    for (int j = 0; j < 10; ++j) { tw[j] = G.tw[10*(i64)e + j]; ti[j] = G.ti[10*(i64)e + j]; tm[j] = G.tmc[10*(i64)e + j]; }
-    const int fr = G.from[e], to = G.to[e];
-    const bool pent_f = fr < GAME_N_PENT, pent_t = to < GAME_N_PENT;
+    unsigned ti[10], tm[10];
+#pragma unroll
+    for (int j = 0; j < 10; ++j) {
+        ti[j] = at(G.e_ti + (i64)j*nvh, e);
+        tm[j] = at(G.e_tm + (i64)j*nvh, e);
+        tw[j] = at(G.e_tw + (i64)j*nvh, e);
+    }
+    const unsigned fr = G.from[e], to = G.to[e];
     /* next to a pentagon a side has four terms: its fifth slot reads the
        first slot's (valid) entries and adds -0.0, the exact identity of IEEE
        addition, so every load of a layer issues without a branch */
-    if (pent_f) { ti[4] = ti[0]; tm[4] = tm[0]; }
-    if (pent_t) { ti[9] = ti[5]; tm[9] = tm[5]; }
-    const double *ipwT = G.ipwT;
+    const bool pent_f = fr < GAME_N_PENT, pent_t = to < GAME_N_PENT;
     int l0, l1;
-    layer_chunk(G.L, bk.y, l0, l1);
+    layer_chunk(G.L, bk.y, sp.run, l0, l1);
+    if (l0 >= l1) return;
     /* the w-point terms of layer l+1 are those of layer l+1's upper level:
        carried to the next layer instead of loaded again */
-    double Ff = (double)F[(i64)l0*G.vpl + fr], Ft = (double)F[(i64)l0*G.vpl + to];
-    double q0 = (double)pv[e + (i64)l0*2*nvh];
+    double Ff = (double)at(F + (i64)l0*G.vpl, fr), Ft = (double)at(F + (i64)l0*G.vpl, to);
+    double q0 = (double)at(pv + (i64)l0*2*nvh, e);
+    const double old_w = TEND ? 1.0 - m.new_w : 0.0;
+    EdgeCarry carry;
     for (int l = l0; l < l1; ++l) {
-        i64 fb = nsh + (i64)l*G.vpl, pb = nvh + (i64)l*2*nvh;
+        const i64 vi = nsh + (i64)l*G.vpl;
+        const TW *Fl = F + vi, *pl = pv + nvh + (i64)l*2*nvh;
         double Fv[10], pvv[10];
 #pragma unroll
-        for (int j = 0; j < 10; ++j) { Fv[j] = (double)F[fb + ti[j]]; pvv[j] = (double)pv[pb + tm[j]]; }
-        const double pve = (double)pv[pb + e];
+        for (int j = 0; j < 10; ++j) { Fv[j] = (double)at(Fl, ti[j]); pvv[j] = (double)at(pl, tm[j]); }
+        const double pve = (double)at(pl, e);
+        /* inner-product weights 6 and 7 of the two cells in layer l */
+        const double *w6 = G.ipwT + ((i64)l*8 + 6)*nsh, *w7 = w6 + nsh;
+        const double w6f = at(w6, fr), w6t = at(w6, to), w7f = at(w7, fr), w7t = at(w7, to);
+        const double q1 = (double)at(pl + nvh, e);
+        const double Ff1 = (double)at(F + (i64)(l + 1)*G.vpl, fr), Ft1 = (double)at(F + (i64)(l + 1)*G.vpl, to);
+        double comb = 0.0, wo = 0.0, td_old = 0.0;
+        if (TEND) {
+            comb = (double)at(W.pgrad_comb + vi, e);
+            wo = at(m.wind_old + vi, e);
+            if (old_w != 0.0) td_old = (double)at(m.td + vi, e);
+        }
         double o = 0;
 #pragma unroll
         for (int j = 0; j < 10; ++j) {
@@ -505,54 +586,93 @@ k_vorticity_flux_e(DevGrid G, const TW *F, const TW *pv, TW *out)
             if ((j == 4 || j == 9) && pent) t = -0.0;
             o += t;
         }
-        /* inner-product weights 6 and 7 of the two cells in layer l */
-        const double w6f = ipwT[((i64)l*8 + 6)*nsh + fr], w6t = ipwT[((i64)l*8 + 6)*nsh + to];
-        const double w7f = ipwT[((i64)l*8 + 7)*nsh + fr], w7t = ipwT[((i64)l*8 + 7)*nsh + to];
-        const double q1 = (double)pv[e + (i64)(l + 1)*2*nvh];
-        const double Ff1 = (double)F[(i64)(l + 1)*G.vpl + fr], Ft1 = (double)F[(i64)(l + 1)*G.vpl + to];
         o -= 0.5*w6f*Ff*q0;
         o -= 0.5*w6t*Ft*q0;
         o -= 0.5*w7f*Ff1*q1;
         o -= 0.5*w7t*Ft1*q1;
-        out[nsh + (i64)l*G.vpl + e] = (TW)o;
+        const TW pvt = (TW)o;
+        if (TEND) {
+            const TW vg = (TW)grad_edge_walk<FLAT, TW>(G, W.vsq, l, l0, e, fr, to, carry);
+            double tv = m.new_w*(
+                comb   /* ohw*old - chw*(nl + l) */
+                + (double)pvt
+                - 0.5*(double)vg);
+            if (old_w != 0.0) tv = old_w*td_old + tv;
+            put(W.vsq_grad + vi, e, vg);
+            put(m.td + vi, e, (TW)tv);
+            put(m.wind_new + vi, e, wo + m.dt*tv);
+        }
+        put(out + vi, e, pvt);
         Ff = Ff1; Ft = Ft1; q0 = q1;
     }
 }
 
-/* vorticity_flux.c:373-417, vertical part: one thread per cell, levels 0..L */
-template <typename TW, int RUN>
-__global__ void __launch_bounds__(TPB) k_vorticity_flux_w(DevGrid G, const TW *F, const TW *pv, TW *out)
+/* vorticity_flux.c:373-417, vertical part: one thread per cell and chunk of
+   levels 0..L.  NC > 0: with the kinetic-energy gradient at the interior w
+   points (gradient_operators.c:35-54), the condensates' pressure gradient of
+   the densities rho (calc_pressure_grad_condensates_v; null: it is there) and
+   the tendency (vector_tendencies_expl.c:74-131); NC is the number of
+   constituents */
+template <typename TW, int RUN, int NC>
+__global__ void __launch_bounds__(TPB) k_vorticity_flux_w(DevGrid G, const TW *F, const TW *pv, TW *out, DevWorkT<TW> W,
+                                                          Mom<TW> m, const double *rho, Span sp)
 {
-    const Blk bk = xcd_block();
-    int h = bk.x*TPB + threadIdx.x;
-    if (h >= G.nsh) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*TPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
     const int nsh = G.nsh, nvh = G.nvh;
     const int ne = h < GAME_N_PENT ? 5 : 6;
     /* a fixed six edges: a pentagon's sixth slot reads its first edge and
        adds -0.0, the exact identity of IEEE addition */
-    int adj[6];
+    unsigned adj[6];
 #pragma unroll
-    for (int j = 0; j < 6; ++j) adj[j] = G.adj[6*h + (j < ne ? j : 0)];
+    for (int j = 0; j < 6; ++j) adj[j] = at(G.c_e + (i64)j*G.nsh, h);
     const int L = G.L, vpl = G.vpl;
-    const double *ipwT = G.ipwT;
     /* level l sums the terms of layers l - 1 and l; the flux and weights of
        layer l are carried to level l + 1 instead of loaded again */
     auto load_layer = [&](int l, double *Fx, double *Wx) {
+        const TW *Fl = F + nsh + (i64)l*vpl;
+        const double *wl = G.ipwT + (i64)l*8*nsh;
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            Fx[j] = (double)F[nsh + (i64)l*vpl + adj[j]];
-            Wx[j] = ipwT[((i64)l*8 + j)*nsh + h];
+            Fx[j] = (double)at(Fl, adj[j]);
+            Wx[j] = at(wl + (i64)j*nsh, h);
         }
     };
     int l0, l1;
-    layer_chunk(L + 1, bk.y, l0, l1);
+    layer_chunk(L + 1, bk.y, sp.run, l0, l1);
+    if (l0 >= l1) return;
     double Fm[6], Wm[6];
-    load_layer(l0 >= 1 ? l0 - 1 : 0, Fm, Wm);
+    const int lm = l0 >= 1 ? l0 - 1 : 0;
+    load_layer(lm, Fm, Wm);
+    /* kinetic energy and gas fraction of the layer above, carried */
+    double vs_m = 0.0, d_m = 0.0;
+    const double old_w = NC > 0 ? 1.0 - m.new_w : 0.0;
+    if constexpr (NC > 0) {
+        vs_m = (double)at(W.vsq + (i64)lm*nsh, h);
+        if (rho) d_m = gas_fraction_at<NC>(G, rho, (i64)lm*nsh, h);
+    }
+    /* a level's results: flux, and at interior levels the gradient, the
+       condensates' term and the tendency */
+    struct Out { double flux; TW vg, pgc, td; };
     auto level = [&](int l) {
+        Out r;
         double Fc[6], Wc[6], q[6];
-        load_layer(l <= L - 1 ? l : L - 1, Fc, Wc);
+        const int lc = l <= L - 1 ? l : L - 1;
+        load_layer(lc, Fc, Wc);
+        const TW *pl = pv + (i64)l*2*nvh;
 #pragma unroll
-        for (int j = 0; j < 6; ++j) q[j] = (double)pv[(i64)l*2*nvh + adj[j]];
+        for (int j = 0; j < 6; ++j) q[j] = (double)at(pl, adj[j]);
+        double vs = 0.0, d = 0.0, comb = 0.0, td_old = 0.0, nd = 1.0, gm = 0.0, pgc = 0.0;
+        const i64 row = (i64)l*vpl;
+        if constexpr (NC > 0) {
+            vs = (double)at(W.vsq + (i64)lc*nsh, h);
+            comb = (double)at(W.pgrad_comb + row, h);
+            nd = at(G.nd + row, h);
+            if (old_w != 0.0) td_old = (double)at(m.td + row, h);
+            if (rho) { gm = at(G.gm + row, h); d = gas_fraction_at<NC>(G, rho, (i64)lc*nsh, h); }
+            else pgc = (double)at(W.pgc_v + row, h);
+        }
         double vw = 0.5;
         if (l == 0 || l == L) vw = 1;
         double o = 0;
@@ -574,131 +694,107 @@ __global__ void __launch_bounds__(TPB) k_vorticity_flux_w(DevGrid G, const TW *F
         }
 #pragma unroll
         for (int j = 0; j < 6; ++j) { Fm[j] = Fc[j]; Wm[j] = Wc[j]; }
-        return o;
+        r.flux = o;
+        if constexpr (NC > 0) {
+            r.vg = (TW)((vs_m - vs)/nd);
+            if (rho) {
+                const double c_up = d_m - 1.0, c_lo = d - 1.0;
+                pgc = (double)(TW)((0.5*(c_up + c_lo))*gm);
+            }
+            r.pgc = (TW)pgc;
+            double tv = m.new_w*(
+                comb   /* -cvw*(nl + l) */
+                + (double)(TW)o
+                - 0.5*(double)r.vg
+                + pgc);
+            if (old_w != 0.0) tv = old_w*td_old + tv;
+            r.td = (TW)tv;
+            vs_m = vs;
+            d_m = d;
+        }
+        return r;
+    };
+    auto store = [&](int l, const Out &r) {
+        const i64 row = (i64)l*vpl;
+        put(out + row, h, (TW)r.flux);
+        if constexpr (NC > 0) {
+            const bool inner = l >= 1 && l <= L - 1;
+            if (inner) {
+                put(W.vsq_grad + row, h, r.vg);
+                if (rho) put(W.pgc_v + row, h, r.pgc);
+            }
+            put(m.td + row, h, inner ? r.td : (TW)0.0);
+        }
     };
     if constexpr (RUN > 0) {
         /* chunks of at most RUN levels: every level before any store, so no
            store orders a later level's loads (a step past the chunk repeats
            its last level) */
-        double o[RUN];
+        Out o[RUN];
 #pragma unroll
         for (int t = 0; t < RUN; ++t) o[t] = level(l0 + t < l1 ? l0 + t : l1 - 1);
 #pragma unroll
         for (int t = 0; t < RUN; ++t)
-            if (l0 + t < l1) out[(i64)(l0 + t)*vpl + h] = (TW)o[t];
+            if (l0 + t < l1) store(l0 + t, o[t]);
     } else
-        for (int l = l0; l < l1; ++l) out[(i64)l*vpl + h] = (TW)level(l);
+        for (int l = l0; l < l1; ++l) store(l, level(l));
 }
 
-/* inner_product.c:13-43, one thread per cell, all layers */
-template <typename TW, int RUN>
-__global__ void __launch_bounds__(TPB) k_inner_product(DevGrid G, const double *a, const double *b, TW *out)
+/* inner_product.c:13-43, one thread per box (107 us at res 7 x 26 with two
+   layers per thread, which share the w points between them, 103 with one) */
+template <typename TW>
+__global__ void __launch_bounds__(TPB) k_inner_product(DevGrid G, const double *a, const double *b, TW *out, Span sp)
 {
-    const Blk bk = xcd_block();
-    int h = bk.x*TPB + threadIdx.x;
-    if (h >= G.nsh) return;
-    const int ne = h < GAME_N_PENT ? 5 : 6;
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*TPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
+    const int l = (int)bk.y, ne = h < GAME_N_PENT ? 5 : 6;
     /* a fixed six edges: a pentagon's sixth slot reads its first edge and
        adds -0.0, the exact identity of IEEE addition */
-    int adj[6];
+    unsigned adj[6];
 #pragma unroll
-    for (int j = 0; j < 6; ++j) adj[j] = G.adj[6*h + (j < ne ? j : 0)];
-    int l0, l1;
-    layer_chunk(G.L, bk.y, l0, l1);
-    /* the w point below layer l is the one above layer l + 1: carried */
-    double au = a[h + (i64)l0*G.vpl], bu = b[h + (i64)l0*G.vpl];
-    auto layer = [&](int l) {
-        const double *w = G.ipwT + (i64)l*8*G.nsh + h;   /* weight j at w[j*nsh] */
-        const double al = a[h + (i64)(l + 1)*G.vpl], bl = b[h + (i64)(l + 1)*G.vpl];
-        double o = 0;
+    for (int j = 0; j < 6; ++j) adj[j] = at(G.c_e + (i64)j*G.nsh, h);
+    const double *w = G.ipwT + (i64)l*8*G.nsh;   /* weight j in row w + j*nsh */
+    const i64 up = (i64)l*G.vpl, lo = up + G.vpl, vi = up + G.nsh;
+    const double au = at(a + up, h), bu = at(b + up, h), al = at(a + lo, h), bl = at(b + lo, h);
+    double o = 0;
 #pragma unroll
-        for (int j = 0; j < 6; ++j) {
-            i64 vi = G.nsh + (i64)l*G.vpl + adj[j];
-            double t = w[j*(i64)G.nsh]*a[vi]*b[vi];
-            if (j >= ne) t = -0.0;
-            o += t;
-        }
-        o += w[6*(i64)G.nsh]*au*bu;
-        o += w[7*(i64)G.nsh]*al*bl;
-        au = al;
-        bu = bl;
-        return o;
-    };
-    if constexpr (RUN > 0) {
-        /* chunks of at most RUN layers: every layer before any store, so no
-           store orders a later layer's loads (a step past the chunk repeats
-           its last layer) */
-        double o[RUN];
-#pragma unroll
-        for (int t = 0; t < RUN; ++t) o[t] = layer(l0 + t < l1 ? l0 + t : l1 - 1);
-#pragma unroll
-        for (int t = 0; t < RUN; ++t)
-            if (l0 + t < l1) out[(i64)(l0 + t)*G.nsh + h] = (TW)o[t];
-    } else
-        for (int l = l0; l < l1; ++l) out[(i64)l*G.nsh + h] = (TW)layer(l);
+    for (int j = 0; j < 6; ++j) {
+        double t = at(w + j*(i64)G.nsh, h)*at(a + vi, adj[j])*at(b + vi, adj[j]);
+        if (j >= ne) t = -0.0;
+        o += t;
+    }
+    o += at(w + 6*(i64)G.nsh, h)*au*bu;
+    o += at(w + 7*(i64)G.nsh, h)*al*bl;
+    put(out + (i64)l*G.nsh, h, (TW)o);
 }
 
 /* grad (gradient_operators.c:56-74) of a scalar field: edges (one thread per
-   edge, all layers) */
+   edge and chunk of layers) */
 template <bool FLAT, typename TW>
-__global__ void __launch_bounds__(TPB) k_grad_e(DevGrid G, const TW *f, TW *out)
+__global__ void __launch_bounds__(TPB) k_grad_e(DevGrid G, const TW *f, TW *out, Span sp)
 {
-    const Blk bk = xcd_block();
-    int e = bk.x*TPB + threadIdx.x;
-    if (e >= G.nvh) return;
-    const int fr = G.from[e], to = G.to[e];
+    const Blk bk = xcd_block(sp);
+    const unsigned e = bk.x*TPB + threadIdx.x;
+    if (e >= (unsigned)G.nvh) return;
+    const unsigned fr = G.from[e], to = G.to[e];
     int l0, l1;
-    layer_chunk(G.L, bk.y, l0, l1);
+    layer_chunk(G.L, bk.y, sp.run, l0, l1);
     EdgeCarry carry;
     for (int l = l0; l < l1; ++l)
-        out[G.nsh + (i64)l*G.vpl + e] = FLAT ? (TW)grad_edge_t<FLAT, TW>(G, f, l, e, fr, to)
-                                             : (TW)grad_edge_walk<FLAT, TW>(G, f, l, l0, e, fr, to, carry);
+        put(out + G.nsh + (i64)l*G.vpl, e, (TW)grad_edge_walk<FLAT, TW>(G, f, l, l0, e, fr, to, carry));
 }
 
-/* grad, interior w points */
+/* grad, interior w points (gradient_operators.c:35-54) */
 template <typename TW>
-__global__ void __launch_bounds__(TPB) k_grad_w(DevGrid G, const TW *f, TW *out)
+__global__ void __launch_bounds__(TPB) k_grad_w(DevGrid G, const TW *f, TW *out, Span sp)
 {
-    i64 t = (i64)xcd_block().x*TPB + threadIdx.x;
-    if (t >= (i64)(G.L - 1)*G.nsh) return;
-    int lev = (int)(t/G.nsh) + 1, h = (int)(t - (i64)(lev - 1)*G.nsh);
-    out[h + (i64)lev*G.vpl] = (TW)grad_w_raw(G, f, lev, h);
-}
-
-/* vector_tendencies_expl.c:74-131 fused with the horizontal wind update of
-   manage_rkhevi.c:67-75 */
-template <typename TW>
-__global__ void __launch_bounds__(TPB) k_vector_tend(DevGrid G, DevWorkT<TW> W, TW *tend_w, const double *wind_old,
-                                                     double *wind_new, double new_w, double chw, double ohw,
-                                                     double cvw, double dt)
-{
-    i64 i = (i64)blockIdx.x*TPB + threadIdx.x;
-    if (i >= G.v) return;
-    double old_w = 1.0 - new_w;
-    int l = (int)(i/G.vpl);
-    int h = (int)(i - (i64)l*G.vpl);
-    if (i < G.nsh || i >= G.v - G.nsh) { tend_w[i] = (TW)0.0; return; }
-    /* friction_acc is zero with momentum diffusion and PBL off: x + 0.0 == x.
-       The old tendency has weight 0 in the first substep, where it is neither
-       read nor added (its product with 0 is a zero, the identity of the sum);
-       IEEE addition commutes, so adding it last changes no bit */
-    if (h >= G.nsh) {
-        double tv = new_w*(
-            (double)W.pgrad_comb[i]   /* ohw*old - chw*(nl + l) */
-            + (double)W.pvt[i]
-            - 0.5*(double)W.vsq_grad[i]);
-        if (old_w != 0.0) tv = old_w*(double)tend_w[i] + tv;
-        tend_w[i] = (TW)tv;
-        wind_new[i] = wind_old[i] + dt*tv;
-    } else {
-        double tv = new_w*(
-            (double)W.pgrad_comb[i]   /* -cvw*(nl + l) */
-            + (double)W.pvt[i]
-            - 0.5*(double)W.vsq_grad[i]
-            + (double)W.pgc_v[i]);
-        if (old_w != 0.0) tv = old_w*(double)tend_w[i] + tv;
-        tend_w[i] = (TW)tv;
-    }
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*TPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
+    const int lev = (int)bk.y + 1;
+    const TW *lo = f + (i64)lev*G.nsh;
+    put(out + (i64)lev*G.vpl, h, (TW)(((double)at(lo - G.nsh, h) - (double)at(lo, h))/at(G.nd + (i64)lev*G.vpl, h)));
 }
 
 /* Vertical contravariant corrections (averaging.c:41-95) of the three fields
@@ -706,6 +802,41 @@ __global__ void __launch_bounds__(TPB) k_vector_tend(DevGrid G, DevWorkT<TW> W, 
    the wind (tracers, divergences.c:94-145), the gas mass flux and its
    rhotheta_v flux (divergences.c:41-59); the fluxes are formed on the fly
    exactly as scalar_times_vector_h forms them (multiplications.c:45-67). */
+/* the slot-major tables of DevGrid, one thread per cell, edge and triangle of
+   its number */
+__global__ void __launch_bounds__(TPB) k_tables(DevGrid G, unsigned *c_e, unsigned *c_n, unsigned *c_from, unsigned *e_ti,
+                                                unsigned *e_tm, double *e_tw, unsigned *e_rc, double *e_rw, unsigned *t_e)
+{
+    const int t = (int)(blockIdx.x*TPB + threadIdx.x);
+    if (t < G.nsh) {
+        const int ne = t < GAME_N_PENT ? 5 : 6;
+        unsigned bits = 0;
+        for (int j = 0; j < 6; ++j) {
+            const int e = G.adj[6*t + (j < ne ? j : 0)], f = G.from[e];
+            c_e[(i64)j*G.nsh + t] = (unsigned)e;
+            c_n[(i64)j*G.nsh + t] = (unsigned)(j < ne ? (f == t ? G.to[e] : f) : t);
+            if (j < ne && G.sgn[6*t + j] > 0) bits |= 1u << j;
+        }
+        c_from[t] = bits;
+    }
+    if (t < G.nvh) {
+        for (int j = 0; j < 10; ++j) {
+            const bool pent = (j < 5 ? G.from[t] : G.to[t]) < GAME_N_PENT;
+            const i64 o = 10*(i64)t + (pent && (j == 4 || j == 9) ? j - 4 : j);
+            e_ti[(i64)j*G.nvh + t] = (unsigned)G.ti[o];
+            e_tm[(i64)j*G.nvh + t] = (unsigned)G.tmc[o];
+            e_tw[(i64)j*G.nvh + t] = G.tw[10*(i64)t + j];
+        }
+        for (int j = 0; j < 4; ++j) {
+            e_rc[(i64)j*G.nvh + t] = (unsigned)G.dri[4*(i64)t + j];
+            e_rw[(i64)j*G.nvh + t] = G.drw[4*(i64)t + j];
+        }
+    }
+    if (t < G.nt)
+        for (int j = 0; j < 3; ++j)
+            t_e[(i64)j*G.nt + t] = (unsigned)G.vit[3*t + j] | (G.vst[3*t + j] < 0 ? 0x80000000u : 0u);
+}
+
 /* the weights -0.5*ipw*slope of the corrections, cell-major per terrain level
    and edge slot (a pentagon's sixth slot holds its first edge's, unused):
    grid constants, formed once */
@@ -718,7 +849,7 @@ __global__ void __launch_bounds__(TPB) k_vcc_weights(DevGrid G, double *vcw)
     vcw[t] = -0.5*G.ipwT[((i64)l*8 + jj)*G.nsh + h]*G.slope[G.nsh + (i64)l*G.vpl + G.adj[6*h + jj]];
 }
 
-__global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
+__global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc, Span sp)
 {
     /* one thread per cell walks a chunk of the terrain levels.  The
        correction at level lev sums the cell's edge terms of layer lev - 1 and
@@ -726,9 +857,9 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
        terrain level): the running sum of layer lev - 1's terms is carried to
        the next level, so each layer's edge terms are formed once, and the sums
        are the reference's in the reference's order */
-    const Blk bk = xcd_block();
-    const int h = bk.x*TPB + threadIdx.x;
-    if (h >= G.nsh) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*TPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
     const int nsh = G.nsh, L = G.L, no = G.n_oro, top = L - no;
     const i64 n = (i64)no*nsh;
     const int ne = h < GAME_N_PENT ? 5 : 6;
@@ -737,15 +868,12 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
        are sums of two terms, which IEEE addition forms alike in either
        order, so the cell's own density and theta_v are loaded and divided
        once per layer */
-    int ej[6], nb[6];
+    unsigned ej[6], nb[6];
 #pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        const int e = G.adj[6*h + (j < ne ? j : 0)], f = G.from[e];
-        ej[j] = e;
-        nb[j] = f == h ? G.to[e] : f;
-    }
+    for (int j = 0; j < 6; ++j) { ej[j] = at(G.c_e + (i64)j*nsh, h); nb[j] = at(G.c_n + (i64)j*nsh, h); }
     int c0, c1;
-    layer_chunk(no, bk.y, c0, c1);
+    layer_chunk(no, bk.y, sp.run, c0, c1);
+    if (c0 >= c1) return;
     /* one layer's inputs: the cell's density and rhotheta_v, and per edge
        the wind, the neighbour's density and rhotheta_v and the weight
        -0.5*ipw*slope, a grid constant kept cell-major (coalesced, where the
@@ -753,16 +881,14 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
     struct In { double rh, rt, u[6], rn[6], rtn[6], c[6]; };
     auto load = [&](int l) {
         In x;
-        const i64 si = (i64)l*nsh + h;
-        x.rh = rg[si]; x.rt = s.rt[si];
+        const i64 sl = (i64)l*nsh, vl = nsh + (i64)l*G.vpl, cl = (i64)(l - top)*6*nsh;
+        x.rh = at(rg + sl, h); x.rt = at(s.rt + sl, h);
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            const i64 vi = nsh + (i64)l*G.vpl + ej[j];
-            const i64 sn = (i64)l*nsh + nb[j];
-            x.u[j] = s.wind[vi];
-            x.rn[j] = rg[sn];
-            x.rtn[j] = s.rt[sn];
-            x.c[j] = G.vcw[((i64)(l - top)*6 + j)*nsh + h];
+            x.u[j] = at(s.wind + vl, ej[j]);
+            x.rn[j] = at(rg + sl, nb[j]);
+            x.rtn[j] = at(s.rt + sl, nb[j]);
+            x.c[j] = at(G.vcw + cl + (i64)j*nsh, h);
         }
         return x;
     };
@@ -804,10 +930,10 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
             double rw = pw, r1 = p1, r2 = p2;
             pw = 0.0; p1 = 0.0; p2 = 0.0;
             add_layer(cur, rw, r1, r2, pw, p1, p2);
-            const i64 t = (i64)k*nsh + h;
-            vcc[t] = rw;
-            vcc[n + t] = r1;
-            vcc[2*n + t] = r2;
+            double *row = vcc + (i64)k*nsh;
+            put(row, h, rw);
+            put(row + n, h, r1);
+            put(row + 2*n, h, r2);
         }
         cur = nxt;
     }
@@ -816,19 +942,25 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc)
 /* scalar_tendencies_expl.c:89-177 for every constituent (diffusion off): the
    centred gas mass flux and its rhotheta_v flux, the upstream tracer fluxes,
    their divergences (divergences.c:14-148) and the RK-weighted tendencies.
-   One thread per cell walks all layers; the edge fluxes are formed on the fly
-   from the reference's own formulas, so no flux array is written. */
-template <bool FLAT, typename TW, int NC, int RUN>
+   One thread per box; the edge fluxes are formed on the fly from the
+   reference's own formulas, so no flux array is written.  Bound by how many
+   of its loads are in flight: with the tables slot-major a box of its own per
+   thread costs 13 coalesced table loads, and its 122 registers keep four waves
+   per SIMD with every neighbour load of a constituent in flight, where a
+   thread walking two layers needs 207 (res 7 x 26 moist, us per launch, FP64
+   and mixed: 393 and 366 with the tables read through the edges, 361 and 322
+   with slot-major ones and two layers per thread, 323 and 294 with one) */
+template <bool FLAT, typename TW, int NC>
 __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevWorkT<TW> W, double *td_rho,
-                                                     double *td_rt, int rk)
+                                                     double *td_rt, int rk, Span sp)
 {
-    const Blk bk = xcd_block();
-    int h = bk.x*TPB + threadIdx.x;
-    if (h >= G.nsh) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*TPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
     /* NC: the number of constituents as a compile-time constant (1 dry, 6 moist),
        so the constituent loop unrolls and all neighbour loads can be in flight together */
     const int nsh = G.nsh, vpl = G.vpl, L = G.L, no = G.n_oro;
-    constexpr int ncc = NC > 1 ? NC - 2 : 0, nc = NC;
+    constexpr int ncc = NC > 1 ? NC - 2 : 0;
     const i64 S = G.s, nvcc = (i64)no*nsh;
     const int ne = h < GAME_N_PENT ? 5 : 6;
     /* each edge as (edge, the cell across it, whether h is its from-cell);
@@ -838,27 +970,19 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
        sixth slot reads valid entries (its first edge, its own cell) and adds
        -0.0, the exact identity of IEEE addition, so no branch guards a load
        and the per-edge arrays stay in registers. */
-    int ej[6], nb[6];
-    unsigned from_bits = 0;
+    unsigned ej[6], nb[6];
+    const unsigned from_bits = at(G.c_from, h);
 #pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        const int jj = j < ne ? j : 0;
-        const int e = G.adj[6*h + jj], f = G.from[e], t = G.to[e];
-        ej[j] = e;
-        nb[j] = j < ne ? ((f == h) ? t : f) : h;
-        if (j < ne && G.sgn[6*h + jj] > 0) from_bits |= 1u << j;
-    }
-    int l0, l1;
-    layer_chunk(L, bk.y, l0, l1);
-    /* one layer's tendencies, returned in orho/ort and stored by the caller */
-    auto layer = [&](int l, double *orho, double &ort) {
-        const i64 i = (i64)l*nsh + h;
+    for (int j = 0; j < 6; ++j) { ej[j] = at(G.c_e + (i64)j*nsh, h); nb[j] = at(G.c_n + (i64)j*nsh, h); }
+    const int l = (int)bk.y;
+    double orho[NC], ort;
+    {
+        const i64 sl = (i64)l*nsh, vl = nsh + (i64)l*vpl;
         double a[6], u[6];
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            const i64 vi = nsh + (i64)l*vpl + ej[j];
-            a[j] = G.area[vi];
-            u[j] = s.wind[vi];
+            a[j] = at(G.area + vl, ej[j]);
+            u[j] = at(s.wind + vl, ej[j]);
         }
         /* which faces carry a terrain correction (divergences.c:41-59) */
         int has_u = 0, has_l = 0;
@@ -867,31 +991,39 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
             else if (l == L - 1) has_u = 1;
             else if (l > L - no - 1) { has_u = 1; has_l = 1; }
         }
-        const double vol = G.vol[i];
-        const double area_u = has_u ? G.area[h + (i64)l*vpl] : 0.0;
-        const double area_l = has_l ? G.area[h + (i64)(l + 1)*vpl] : 0.0;
-        const i64 vu = (i64)(l - (L - no))*nsh + h, vl = (i64)(l + 1 - (L - no))*nsh + h;
+        const double vol = at(G.vol + sl, h);
+        const double area_u = has_u ? at(G.area + (i64)l*vpl, h) : 0.0;
+        const double area_l = has_l ? at(G.area + (i64)(l + 1)*vpl, h) : 0.0;
+        /* rows of the corrections at the box's upper and lower faces */
+        const double *vcu = W.vcc + (i64)(l - (L - no))*nsh, *vcl = vcu + nsh;
         /* the new tendencies are kept in registers and stored after every
            load of the layer, so no store orders the loads */
         double out_rt = 0.0;
+        /* moist: c_v_mass_weighted_air (derived_quantities.c:97-115), its
+           condensates' terms added as their densities come by */
+        double cv = 0.0, cp[2] = {0.0, 0.0}, rho_v = 0.0;
+        if constexpr (NC == 6) {
+            cp[0] = (double)at(W.cpc + sl, h);
+            cp[1] = (double)at(W.cpc + S + sl, h);
+            rho_v = at(s.rho + (i64)(NC - 1)*S + sl, h);
+        }
 #pragma unroll
-        for (int k = 0; k < nc; ++k) {
-            const i64 shift = (i64)k*S;
+        for (int k = 0; k < NC; ++k) {
             const double new_w = (rk == 1 && k != ncc) ? 0.5 : 1.0, old_w = 1.0 - new_w;
-            const double *rk_ = s.rho + shift;
-            const double rho_h = rk_[i];
+            const double *rl = s.rho + (i64)k*S + sl;
+            const double rho_h = at(rl, h);
             double res;
             if (k == ncc) {
-                const double th_h = s.rt[i]/rho_h;
+                const double *rtl = s.rt + sl;
+                const double th_h = at(rtl, h)/rho_h;
                 double c1 = 0.0, c2 = 0.0;
 #pragma unroll
                 for (int j = 0; j < 6; ++j) {
-                    const i64 sb = (i64)l*nsh + nb[j];
-                    const double rho_nb = rk_[sb];
+                    const double rho_nb = at(rl, nb[j]);
                     /* times the edge sign +-1: exact, so a sign flip */
                     const bool pos = (from_bits >> j) & 1u;
                     double f1 = (0.5*(rho_h + rho_nb))*u[j];
-                    double f2 = (0.5*(th_h + s.rt[sb]/rho_nb))*f1;
+                    double f2 = (0.5*(th_h + at(rtl, nb[j])/rho_nb))*f1;
                     double t1 = (pos ? f1 : -f1)*a[j], t2 = (pos ? f2 : -f2)*a[j];
                     if (j >= ne) { t1 = -0.0; t2 = -0.0; }
                     c1 += t1;
@@ -900,14 +1032,14 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
                 double v1 = 0.0, v2 = 0.0;
                 if (!FLAT) {
                     if (has_u && has_l) {
-                        v1 = W.vcc[nvcc + vu]*area_u - W.vcc[nvcc + vl]*area_l;
-                        v2 = W.vcc[2*nvcc + vu]*area_u - W.vcc[2*nvcc + vl]*area_l;
+                        v1 = at(vcu + nvcc, h)*area_u - at(vcl + nvcc, h)*area_l;
+                        v2 = at(vcu + 2*nvcc, h)*area_u - at(vcl + 2*nvcc, h)*area_l;
                     } else if (has_l) {
-                        v1 = -W.vcc[nvcc + vl]*area_l;
-                        v2 = -W.vcc[2*nvcc + vl]*area_l;
+                        v1 = -at(vcl + nvcc, h)*area_l;
+                        v2 = -at(vcl + 2*nvcc, h)*area_l;
                     } else if (has_u) {
-                        v1 = W.vcc[nvcc + vu]*area_u;
-                        v2 = W.vcc[2*nvcc + vu]*area_u;
+                        v1 = at(vcu + nvcc, h)*area_u;
+                        v2 = at(vcu + 2*nvcc, h)*area_u;
                     }
                 }
                 double div1 = 1.0/vol*(c1 + v1);
@@ -916,30 +1048,32 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
                 /* the gas weights are 1 and 0 in both substeps: the old
                    tendencies are neither read nor added (their product with 0
                    is a zero, the identity of the sum) */
-                if (!G.moist) {
+                if constexpr (NC == 1) {
                     /* dry: every source term of the reference sum is a zero array */
                     res = new_w*(-div1);
                     out_rt = new_w*(-div2);
                 } else {
                     /* the moist-air gas takes the vapour phase-transition rate
                        (scalar_tendencies_expl.c:94-99, 125-131, 174-176) */
-                    double ptr_v = (double)W.ptr[shift + i];
+                    double ptr_v = (double)at(W.ptr + (i64)k*S + sl, h);
                     const double th = th_h;
                     res = new_w*(-div1 + ptr_v);
-                    double cv = c_v_mass_weighted_cp(G, s.rho, W.cpc, i);
-                    double heat = (double)W.phr[i] + (double)W.sed_heat[i];
+                    cv += rg*GC_C_D_V;
+                    cv += rho_v*GC_C_V_V;
+                    double heat = (double)at(W.phr + sl, h) + (double)at(W.sed_heat + sl, h);
                     out_rt = new_w*(
                         -div2
-                        + GC_C_D_V*rg/cv*heat/(GC_C_D_P*(G.exbg[i] + s.ep[i]))
+                        + GC_C_D_V*rg/cv*heat/(GC_C_D_P*(at(G.exbg + sl, h) + at(s.ep + sl, h)))
                         + ptr_v*th);
                 }
             } else {
+                if (k < ncc) cv += rho_h*cp[k & 1];
                 double c = 0.0;
 #pragma unroll
                 for (int j = 0; j < 6; ++j) {
                     /* upstream density: the from-cell for u >= 0 */
                     const bool is_from = (from_bits >> j) & 1u;
-                    const double rho_nb = rk_[(i64)l*nsh + nb[j]];
+                    const double rho_nb = at(rl, nb[j]);
                     const double sv = ((u[j] >= 0.0) == is_from) ? rho_h : rho_nb;
                     const double f = sv*u[j];
                     double t = (is_from ? f : -f)*a[j];
@@ -949,53 +1083,35 @@ __global__ void __launch_bounds__(TPB) k_scalar_tend(DevGrid G, DevState s, DevW
                 double v = 0.0;
                 if (!FLAT) {
                     if (has_u && has_l) {
-                        double cu = W.vcc[vu], cl = W.vcc[vl];
-                        double du = (cu <= 0.0) ? rk_[i - nsh] : rk_[i];
-                        double dl = (cl <= 0.0) ? rk_[i] : rk_[i + nsh];
+                        double cu = at(vcu, h), cl = at(vcl, h);
+                        double du = (cu <= 0.0) ? at(rl - nsh, h) : rho_h;
+                        double dl = (cl <= 0.0) ? rho_h : at(rl + nsh, h);
                         v = du*cu*area_u - dl*cl*area_l;
                     } else if (has_l) {
-                        double cl = W.vcc[vl];
-                        double dl = (cl <= 0.0) ? rk_[i] : rk_[i + nsh];
+                        double cl = at(vcl, h);
+                        double dl = (cl <= 0.0) ? rho_h : at(rl + nsh, h);
                         v = -dl*cl*area_l;
                     } else if (has_u) {
-                        double cu = W.vcc[vu];
-                        double du = (cu <= 0.0) ? rk_[i - nsh] : rk_[i];
+                        double cu = at(vcu, h);
+                        double du = (cu <= 0.0) ? at(rl - nsh, h) : rho_h;
                         v = du*cu*area_u;
                     }
                 }
                 double div = 1.0/vol*(c + v);
-                i64 shift_pt = (k == ncc + 1) ? shift - S : shift;
+                const int kp = (k == ncc + 1) ? k - 1 : k;
                 /* the old tendency enters with weight 0.5 in the second
                    substep only (a uniform branch); IEEE addition commutes */
-                res = new_w*(-div + (double)W.ptr[shift_pt + i]);
-                if (old_w != 0.0) res = old_w*td_rho[shift + i] + res;
+                res = new_w*(-div + (double)at(W.ptr + (i64)kp*S + sl, h));
+                if (old_w != 0.0) res = old_w*at(td_rho + (i64)k*S + sl, h) + res;
             }
             orho[k] = res;
         }
         ort = out_rt;
-    };
-    auto store = [&](int l, const double *orho, double ort) {
-        const i64 i = (i64)l*nsh + h;
+    }
+    const i64 sl = (i64)l*nsh;
 #pragma unroll
-        for (int k = 0; k < NC; ++k) td_rho[(i64)k*S + i] = orho[k];
-        td_rt[i] = ort;
-    };
-    if constexpr (RUN > 0) {
-        /* chunks of at most RUN layers: the loads and arithmetic of all its layers come
-           before any store, so no store orders a later layer's loads (a step
-           past the chunk repeats its last layer and stores nothing) */
-        double orho[RUN][NC], ort[RUN];
-#pragma unroll
-        for (int t = 0; t < RUN; ++t) layer(l0 + t < l1 ? l0 + t : l1 - 1, orho[t], ort[t]);
-#pragma unroll
-        for (int t = 0; t < RUN; ++t)
-            if (l0 + t < l1) store(l0 + t, orho[t], ort[t]);
-    } else
-        for (int l = l0; l < l1; ++l) {
-            double orho[NC], ort = 0.0;
-            layer(l, orho, ort);
-            store(l, orho, ort);
-        }
+    for (int k = 0; k < NC; ++k) put(td_rho + (i64)k*S + sl, h, orho[k]);
+    put(td_rt + sl, h, ort);
 }
 
 /* three_band_solver_ver_waves (column_solvers.c:19-383), one column per lane.
@@ -1153,24 +1269,11 @@ __global__ void __launch_bounds__(128) k_ver_waves(DevGrid G, DevState so, DevSt
     }
 }
 
-/* The same solve in three phases over a block of VW_NCOL columns, for
-   parallelism: the streaming kernel above gives each column one lane for
-   all of its work, 2.5 waves per SIMD at res 7, and its recurrence arrays
-   live in scratch.  Here
-     1. every thread builds rows (column, interface) of the tridiagonal
-        system into LDS, each from the two layers around the interface;
-     2. one lane per column runs the Thomas elimination and back
-        substitution on LDS, then all threads apply the damping;
-     3. every thread forms the new state of (column, layer) boxes into
-        registers; after a barrier (the reads of state snr may be of the
-        state being written) they are stored.
-   Every quantity is formed with the arithmetic of the streaming kernel, so
-   the two kernels agree bit for bit. */
 /* Thomas algorithm (column_solvers.c:641-667) on rows j*NCOL + col of LDS
    arrays c, d, e, r (n rows): the multipliers overwrite e, the solution r.
    The next row is read before the current one is written, so each step
    waits on its division chain only, not on an LDS round trip. */
-template <int NCOL, int NMAX>
+template <int NCOL>
 __device__ __forceinline__ void thomas_lds(const double *cc, const double *dd, double *ee, double *rr, int n, int col)
 {
     double ep = 0.0, x;
@@ -1180,9 +1283,8 @@ __device__ __forceinline__ void thomas_lds(const double *cc, const double *dd, d
     ee[col] = ep; rr[col] = x;
     double cp = cc[col], dn = 0.0, en = 0.0, rn = 0.0;
     if (n > 1) { dn = dd[NCOL + col]; en = ee[NCOL + col]; rn = rr[NCOL + col]; }
-#pragma unroll
-    for (int j = 1; j < NMAX; ++j) {
-        if (j >= n) break;
+#pragma unroll 4
+    for (int j = 1; j < n; ++j) {
         const int o = j*NCOL + col, on = (j + 1 < n ? j + 1 : j)*NCOL + col;
         const double cpn = cc[o], dnn = dd[on], enn = ee[on], rnn = rr[on];
         const double den = dn - ep*cp;
@@ -1194,10 +1296,8 @@ __device__ __forceinline__ void thomas_lds(const double *cc, const double *dd, d
     /* back substitution, upwards */
     double eb = 0.0, rb = 0.0;
     if (n > 1) { eb = ee[(n - 2)*NCOL + col]; rb = rr[(n - 2)*NCOL + col]; }
-#pragma unroll
-    for (int t = 0; t < NMAX - 1; ++t) {
-        const int j = n - 2 - t;
-        if (j < 0) break;
+#pragma unroll 4
+    for (int j = n - 2; j >= 0; --j) {
         const int o = j*NCOL + col, om = (j > 0 ? j - 1 : 0)*NCOL + col;
         const double ebn = ee[om], rbn = rr[om];
         x = rb - eb*x;
@@ -1252,9 +1352,6 @@ __device__ __forceinline__ void thomas_lds_ce(double *ce, const unsigned char *f
     }
 }
 
-#define VW_NCOL 32
-#define VW_THREADS 256
-
 /* the state of box (i, j) the solver reads, loaded in one batch: old state,
    tendencies, the state snr (the new state before this substep writes it),
    volume and background exner */
@@ -1262,15 +1359,16 @@ struct VwBox {
     double vol, exbg, rho_o, rt_o, ep_o, tp_o, trho, trt, rho_n, rt_n, ep_n;
 };
 
+/* box at element o of the rows jb*nsh (wave-uniform) of the S fields */
 __device__ __forceinline__ VwBox vw_box(const DevGrid &G, const DevState &so, const DevState &snr,
-                                        const DevState &td, int i, int j)
+                                        const DevState &td, i64 jb, unsigned o)
 {
-    const i64 b = i + (i64)j*G.nsh, gi = (i64)G.n_cond*G.s;
+    const i64 gi = (i64)G.n_cond*G.s + jb;
     VwBox x;
-    x.vol = G.vol[b]; x.exbg = G.exbg[b];
-    x.rho_o = so.rho[gi + b]; x.rt_o = so.rt[b]; x.ep_o = so.ep[b]; x.tp_o = so.tp[b];
-    x.trho = td.rho[gi + b]; x.trt = td.rt[b];
-    x.rho_n = snr.rho[gi + b]; x.rt_n = snr.rt[b]; x.ep_n = snr.ep[b];
+    x.vol = at(G.vol + jb, o); x.exbg = at(G.exbg + jb, o);
+    x.rho_o = at(so.rho + gi, o); x.rt_o = at(so.rt + jb, o); x.ep_o = at(so.ep + jb, o); x.tp_o = at(so.tp + jb, o);
+    x.trho = at(td.rho + gi, o); x.trt = at(td.rt + jb, o);
+    x.rho_n = at(snr.rho + gi, o); x.rt_n = at(snr.rt + jb, o); x.ep_n = at(snr.ep + jb, o);
     return x;
 }
 
@@ -1301,217 +1399,88 @@ __device__ __forceinline__ ColumnLayer vw_layer(const VwBox &x, double dt, int r
     return c;
 }
 
-/* The same solve in three phases over a block of VW_NCOL columns, for
-   parallelism: the streaming kernel above gives each column one lane for
-   all of its work, 2.5 waves per SIMD at res 7, and its recurrence arrays
-   live in scratch.  Here
-     1. every thread builds rows (column, interface) of the tridiagonal
-        system into LDS, each from the two layers around the interface;
-     2. one lane per column runs the Thomas elimination and back
-        substitution on LDS, then all threads apply the damping;
-     3. every thread forms the new state of (column, layer) boxes into
-        registers; after a barrier (the reads of state snr may be of the
-        state being written) they are stored.
-   Each row and box loads all of its inputs in one unconditional batch
-   (indices clamped in range, unused values discarded), so a thread waits on
-   memory once per row, not once per branch.  Every quantity is formed with
-   the arithmetic of the streaming kernel, so the two agree bit for bit. */
-template <int LT, typename TWIND>
-__global__ void __launch_bounds__(VW_THREADS) k_ver_waves_3p(DevGrid G, DevState so, DevState snr, DevState sn,
-                                                             DevState td, const TWIND *td_wind, StepConsts K, int rk)
+/* The same solve with NCOL columns per block and a group of NCOL lanes for
+   every VR_PER boxes of them, in three phases:
+     1. each group walks its boxes and builds their rows of the three-band
+        system (row j couples interfaces j - 1, j, j + 1) into LDS, forming
+        each box's linearisation (column_layer, nine divisions at rk 1) once;
+     2. one lane per column eliminates and substitutes back in LDS, then every
+        group damps its own rows' solution;
+     3. each group forms the new state of its boxes.
+   The kernel is bound by its loads and by the divisions (about 26 per box,
+   half its time at res 7), so a box is linearised once: its explicit density,
+   rhotheta_v and gamma wait for phase 3 in LDS, the interface theta and
+   density in registers, and only what those do not hold (volume, old exner
+   and rhotheta_v, area, old wind, background) is loaded again, during the
+   elimination.  Four boxes per group keep three waves per SIMD (166
+   registers; all of it in registers needs 206 and spills below that) and make
+   a block 144 to 256 threads at any depth; the columns per block (64 up to 16
+   layers, 32 up to 32, 16 beyond) keep its LDS under 56 KiB, three blocks per
+   CU.  A lane's loads take its column and the distance of its group from the
+   wave's first row as one offset to rows that are the same for the wave.
+   Against the kernels for 26 and 55 layers (runs of seven boxes, the state
+   read and linearised again in phase 3) and the one for other depths, us per
+   launch: res 7 x 26 206 -> 195, res 6 x 26 72 -> 65, res 4 x 26 23 -> 17,
+   res 5 x 41 41 -> 33, res 6 x 55 141 -> 144.  Every quantity keeps the
+   arithmetic of k_ver_waves, so the two agree bit for bit. */
+#define VR_PER 4
+__host__ __device__ constexpr int vr_ncol(int layers) { return layers <= 16 ? 64 : (layers <= 32 ? 32 : 16); }
+static int vr_threads(int layers) { return (layers + VR_PER - 1)/VR_PER*vr_ncol(layers); }
+
+template <int NCOL, typename TWIND>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) k_ver_waves_run(DevGrid G, DevState so, DevState snr, DevState sn,
+                                                       DevState td, const TWIND *td_wind, StepConsts K, int rk)
 {
     extern __shared__ double lds[];
-    const int L = LT > 0 ? LT : G.L, NI = L - 1;
-    const int nsh = G.nsh, vpl = G.vpl;
-    const i64 gi = (i64)G.n_cond*G.s;
+    const int L = G.L, NI = L - 1, nsh = G.nsh, vpl = G.vpl;
     const double dt = K.dt, iw = K.impl_weight;
     const double dt2 = dt*dt;
-    const double *zs = G.zs, *area = G.area;
-    const int i0 = xcd_block().x*VW_NCOL;
-    double *cc = lds, *dd = lds + NI*VW_NCOL, *ee = lds + 2*NI*VW_NCOL, *rr = lds + 3*NI*VW_NCOL;
-
-    /* phase 1: row j couples interfaces j-1, j, j+1 (column_solvers.c:141-189) */
-    constexpr int MAXIT1 = ((LT > 0 ? LT : GAME_MAX_LAYERS) - 1)*VW_NCOL/VW_THREADS + 1;
-#pragma unroll
-    for (int it = 0; it < MAXIT1; ++it) {
-        const int idx = threadIdx.x + it*VW_THREADS;
-        if (idx >= NI*VW_NCOL) break;
-        const int j = idx/VW_NCOL, ic = i0 + (idx - j*VW_NCOL);
-        const int i = ic < nsh ? ic : nsh - 1;
-        const int j2 = j + 2 < L ? j + 2 : L - 1;   /* layer j+2, clamped */
-        const i64 b = i + (i64)j*nsh, lo = b + nsh, l2 = i + (i64)j2*nsh;
-        const i64 wi = i + (i64)(j + 1)*vpl;
-        /* one batch of loads */
-        const VwBox A = vw_box(G, so, snr, td, i, j), B = vw_box(G, so, snr, td, i, j + 1);
-        const double rt_n2 = snr.rt[l2], rho_n2 = snr.rho[gi + l2], rho_o2 = so.rho[gi + l2], exbg2 = G.exbg[l2];
-        const double zb = zs[b], zl = zs[lo], z2 = zs[l2];
-        const double w_old = so.wind[wi], tdw = (double)td_wind[wi], a_w = area[wi];
-        const double w_old2 = so.wind[i + (i64)j2*vpl];   /* w at level j+2 (interface j+1) */
-        const ColumnLayer ca = vw_layer(A, dt, rk), cb = vw_layer(B, dt, rk);
-        const double tin = 0.5*(A.rt_n/A.rho_n + B.rt_n/B.rho_n), rio = 0.5*(A.rho_o + B.rho_o);
-        const double rie = 0.5*(ca.re + cb.re);
-        const double d = -(tin*tin)*(ca.ga + cb.ga)
-                         + 0.5*(A.exbg - B.exbg)*(cb.al - ca.al + tin*(cb.be - ca.be))
-                         - (zb - zl)/(iw*dt2*GC_C_D_P*rio)
-                           *(2.0/a_w + dt*w_old*0.5*(-1.0/A.vol + 1.0/B.vol));
-        const double r = -(w_old + dt*tdw)*(zb - zl)/(iw*dt2*GC_C_D_P)
-                         + tin*(ca.epe - cb.epe)/dt
-                         + 0.5/dt*(ca.tpe + cb.tpe)*(A.exbg - B.exbg)
-                         - (zb - zl)/(iw*dt2*GC_C_D_P)*w_old*rie/rio;
-        double e = 0.0, c = 0.0;
-        if (j < L - 2) {
-            /* theta_int_new and rho_int_old of interface j+1 */
-            const double tin_n = 0.5*(B.rt_n/B.rho_n + rt_n2/rho_n2), rio_n = 0.5*(B.rho_o + rho_o2);
-            c = tin_n*cb.ga*tin
-                + 0.5*(B.exbg - exbg2)*(cb.al + cb.be*tin)
-                - (zl - z2)/(iw*dt*GC_C_D_P)*0.5*w_old2/(B.vol*rio_n);
-            e = tin*cb.ga*tin_n
-                - 0.5*(A.exbg - B.exbg)*(cb.al + cb.be*tin_n)
-                + (zb - zl)/(iw*dt*GC_C_D_P)*0.5*w_old/(B.vol*rio);
-        }
-        cc[idx] = c; dd[idx] = d; ee[idx] = e; rr[idx] = r;
-    }
-    __syncthreads();
-    /* phase 2: Thomas algorithm (column_solvers.c:641-667), one lane per column;
-       the multipliers overwrite e, the solution overwrites r */
-    if (threadIdx.x < VW_NCOL && i0 + (int)threadIdx.x < nsh)
-        thomas_lds<VW_NCOL, (LT > 0 ? LT : GAME_MAX_LAYERS) - 1>(cc, dd, ee, rr, NI, threadIdx.x);
-    __syncthreads();
-    /* Klemp (2008) damping of the solved fluxes (column_solvers.c:284-298) */
-#pragma unroll
-    for (int it = 0; it < MAXIT1; ++it) {
-        const int idx = threadIdx.x + it*VW_THREADS;
-        if (idx >= NI*VW_NCOL) break;
-        const int j = idx/VW_NCOL, ic = i0 + (idx - j*VW_NCOL);
-        const int i = ic < nsh ? ic : nsh - 1;
-        rr[idx] = rr[idx]/(1.0 + dt*G.damp[(i64)j*nsh + i]);
-    }
-    __syncthreads();
-    /* phase 3: new state of box (column, layer j) (column_solvers.c:300-370) */
-    constexpr int MAXIT3 = (LT > 0 ? LT : GAME_MAX_LAYERS)*VW_NCOL/VW_THREADS + 1;
-    double o_rho[MAXIT3], o_rt[MAXIT3], o_tp[MAXIT3], o_ep[MAXIT3], o_w[MAXIT3];
-#pragma unroll
-    for (int it = 0; it < MAXIT3; ++it) {
-        o_rho[it] = 0.0; o_rt[it] = 0.0; o_tp[it] = 0.0; o_ep[it] = 0.0; o_w[it] = 0.0;
-        const int idx = threadIdx.x + it*VW_THREADS;
-        if (idx >= L*VW_NCOL) break;
-        const int j = idx/VW_NCOL, col = idx - j*VW_NCOL, ic = i0 + col;
-        const int i = ic < nsh ? ic : nsh - 1;
-        const int jm = j >= 1 ? j - 1 : 0, jp = j < L - 1 ? j + 1 : L - 1;
-        const i64 b = i + (i64)j*nsh, bm = i + (i64)jm*nsh, bp = i + (i64)jp*nsh;
-        const i64 wi = i + (i64)(j >= 1 ? j : 1)*vpl;
-        /* one batch of loads */
-        const VwBox A = vw_box(G, so, snr, td, i, j);
-        const double rt_np = snr.rt[bp], rho_np = snr.rho[gi + bp];
-        const double rt_nm = snr.rt[bm], rho_nm = snr.rho[gi + bm], rho_om = so.rho[gi + bm];
-        const double trho_m = td.rho[gi + bm], vm = G.vol[bm];
-        const double thbg = G.thbg[b], a_w = area[wi], w_o = so.wind[wi];
-        const double x_j = (j < L - 1) ? rr[j*VW_NCOL + col] : 0.0;
-        const double x_m = (j >= 1) ? rr[(j - 1)*VW_NCOL + col] : 0.0;
-        const double x_mm = (j >= 2) ? rr[(j - 2)*VW_NCOL + col] : 0.0;
-        const ColumnLayer cl = vw_layer(A, dt, rk);
-        /* theta_int_new of the interfaces below (j) and above (j-1) the box */
-        const double tin_j = (j < L - 1) ? 0.5*(A.rt_n/A.rho_n + rt_np/rho_np) : 0.0;
-        const double tin_m = (j >= 1) ? 0.5*(rt_nm/rho_nm + A.rt_n/A.rho_n) : 0.0;
-        const double v = A.vol;
-        double rho_n, rt_n;
-        if (j == 0) {
-            rho_n = cl.re + dt*(x_j)/v;
-            rt_n = cl.rte + dt*(tin_j*x_j)/v;
-        } else if (j == L - 1) {
-            rho_n = cl.re + dt*(-x_m)/v;
-            rt_n = cl.rte + dt*(-tin_m*x_m)/v;
-        } else {
-            rho_n = cl.re + dt*(-x_m + x_j)/v;
-            rt_n = cl.rte + dt*(-tin_m*x_m + tin_j*x_j)/v;
-        }
-        o_rho[it] = rho_n;
-        o_rt[it] = rt_n;
-        o_tp[it] = rt_n/rho_n - thbg;
-        o_ep[it] = A.ep_o + v*cl.ga*(rt_n - A.rt_o);
-        if (j >= 1) {
-            /* the new density of the box above, with the arithmetic of its own thread */
-            const double re_m = rho_om + dt*trho_m;
-            double rho_m;
-            if (j - 1 == 0) rho_m = re_m + dt*(x_m)/vm;
-            else rho_m = re_m + dt*(-x_mm + x_m)/vm;
-            const double rio_m = 0.5*(rho_om + A.rho_o);   /* rho_int_old(j - 1) */
-            const double din = 0.5*(rho_m + rho_n);
-            o_w[it] = (2.0*x_m/a_w - din*w_o)/rio_m;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < MAXIT3; ++it) {
-        const int idx = threadIdx.x + it*VW_THREADS;
-        if (idx >= L*VW_NCOL) break;
-        const int j = idx/VW_NCOL, i = i0 + (idx - j*VW_NCOL);
-        if (i >= nsh) continue;
-        const i64 b = i + (i64)j*nsh;
-        sn.rho[gi + b] = o_rho[it];
-        sn.rt[b] = o_rt[it];
-        sn.tp[b] = o_tp[it];
-        sn.ep[b] = o_ep[it];
-        if (j >= 1) sn.wind[i + (i64)j*vpl] = o_w[it];
-    }
-}
-
-/* The 26- and 55-layer sound-wave solve with each wave walking a run of
-   layers of a block of vr_ncol(L) columns (lane = column): a row of the three-band system
-   needs the layers above and below its interface, so walking down a run
-   forms each layer's linearisation (column_layer, nine divisions at rk 1)
-   once instead of twice and loads each box once; the inputs of the next
-   layer are loaded before the current row is formed.  Phase 2 is the same
-   one-lane-per-column elimination (a full wave per block), phase 3 walks
-   runs of boxes the same way, carrying the box above's values (its new
-   density is the one its own step formed).  Every quantity keeps the
-   arithmetic of k_ver_waves. */
-#define VR_THREADS 256
-/* columns per block: 64 at 26 layers (50 KiB of LDS, three blocks per CU),
-   32 at 55 layers (55 KiB, two blocks per CU; the lanes of a column group
-   are half a wave) */
-__host__ __device__ constexpr int vr_ncol(int lt) { return lt == 26 ? 64 : 32; }
-
-template <int LT, typename TWIND>
-__global__ void __launch_bounds__(VR_THREADS) k_ver_waves_run(DevGrid G, DevState so, DevState snr, DevState sn,
-                                                              DevState td, const TWIND *td_wind, StepConsts K, int rk)
-{
-    extern __shared__ double lds[];
-    constexpr int VR_NCOL = vr_ncol(LT);
-    constexpr int L = LT, NI = LT - 1;
-    constexpr int NW = VR_THREADS/VR_NCOL;
-    constexpr int PER1 = (NI + NW - 1)/NW, PER3 = (L + NW - 1)/NW;
-    /* every wave's run of rows and of boxes starts inside the column, so
-       each of its first loads is in range */
-    static_assert((NW - 1)*PER1 < NI && (NW - 1)*PER3 < L, "a wave of the block would have an empty run");
-    const int nsh = G.nsh, vpl = G.vpl;
-    const i64 gi = (i64)G.n_cond*G.s;
-    const double dt = K.dt, iw = K.impl_weight;
-    const double dt2 = dt*dt;
-    const double *zs = G.zs, *area = G.area;
-    const int i0 = xcd_block().x*VR_NCOL;
-    const int w = threadIdx.x/VR_NCOL, col = threadIdx.x - w*VR_NCOL;
+    const int i0 = (int)xcd_x()*NCOL;
+    if (i0 >= nsh) return;
+    /* the row above the wave's first (uniform; the first itself at the top),
+       and this lane's group's first row */
+    const int jf = __builtin_amdgcn_readfirstlane((int)threadIdx.x/64)*(64/NCOL)*VR_PER, jw = jf > 0 ? jf - 1 : 0;
+    const int j0 = (int)threadIdx.x/NCOL*VR_PER, col = (int)threadIdx.x%NCOL;
     const bool live = i0 + col < nsh;
     const int i = live ? i0 + col : nsh - 1;
-    double *cc = lds, *dd = lds + NI*VR_NCOL, *ee = lds + 2*NI*VR_NCOL, *rr = lds + 3*NI*VR_NCOL;
+    const i64 jb = (i64)jw*nsh, wb = (i64)jw*vpl, gi = (i64)G.n_cond*G.s + jb;
+    /* offsets from row jw to row or level j >= jw of column i, clamped to the last */
+    auto os = [&](int j) { return (unsigned)((j < L ? j : L - 1) - jw)*(unsigned)nsh + (unsigned)i; };
+    auto ow = [&](int lev) { return (unsigned)((lev < L ? lev : L) - jw)*(unsigned)vpl + (unsigned)i; };
+    double *cc = lds, *dd = lds + NI*NCOL, *ee = lds + 2*NI*NCOL, *rr = lds + 3*NI*NCOL;
 
-    /* phase 1: rows j0..j1-1 of this wave (column_solvers.c:141-189) */
+    /* what phase 3 needs of the group's boxes (LDS) and, at index t + 1, of the
+       interface below box j0 + t; index 0 and k_re0 are the box above the group */
+    double k_re0, k_tin[VR_PER + 1], k_rio[VR_PER + 1];
+    double *p_re = lds + 4*NI*NCOL, *p_rte = p_re + L*NCOL, *p_vga = p_rte + L*NCOL;
+    /* phase 1: rows j0 .. j0 + VR_PER - 1 (column_solvers.c:141-189) */
     {
-        const int j0 = w*PER1, j1 = j0 + PER1 < NI ? j0 + PER1 : NI;
-        VwBox A = vw_box(G, so, snr, td, i, j0), B = vw_box(G, so, snr, td, i, j0 + 1);
-        double za = zs[i + (i64)j0*nsh], zb = zs[i + (i64)(j0 + 1)*nsh];
+        VwBox A = vw_box(G, so, snr, td, jb, os(j0)), B = vw_box(G, so, snr, td, jb, os(j0 + 1));
+        double za = at(G.zs + jb, os(j0)), zb = at(G.zs + jb, os(j0 + 1));
+        /* the box above (the group's own first box at the top, unused) */
+        const unsigned om = os(j0 > 0 ? j0 - 1 : 0);
+        const double rho_om = at(so.rho + gi, om), trho_m = at(td.rho + gi, om);
+        const double rt_nm = at(snr.rt + jb, om), rho_nm = at(snr.rho + gi, om);
+        k_re0 = rho_om + dt*trho_m;
         ColumnLayer ca = vw_layer(A, dt, rk), cb = vw_layer(B, dt, rk);
+        auto keep = [&](int j, const VwBox &x, const ColumnLayer &c) {
+            if (j < L) { const int ix = j*NCOL + col; p_re[ix] = c.re; p_rte[ix] = c.rte; p_vga[ix] = x.vol*c.ga; }
+        };
+        keep(j0, A, ca);
+        keep(j0 + 1, B, cb);
+        double th_a = A.rt_n/A.rho_n, th_b = B.rt_n/B.rho_n;
+        k_tin[0] = 0.5*(rt_nm/rho_nm + th_a);
+        k_rio[0] = 0.5*(rho_om + A.rho_o);
 #pragma unroll
-        for (int t = 0; t < PER1; ++t) {
+        for (int t = 0; t < VR_PER; ++t) {
             const int j = j0 + t;
-            if (j >= j1) break;
-            const int j2 = j + 2 < L ? j + 2 : L - 1;   /* layer j+2, clamped */
-            const VwBox C = vw_box(G, so, snr, td, i, j2);
-            const double zc = zs[i + (i64)j2*nsh];
-            const i64 wi = i + (i64)(j + 1)*vpl;
-            const double w_old = so.wind[wi], tdw = (double)td_wind[wi], a_w = area[wi];
-            const double w_old2 = so.wind[i + (i64)j2*vpl];   /* w at level j+2 (interface j+1) */
-            const double tin = 0.5*(A.rt_n/A.rho_n + B.rt_n/B.rho_n), rio = 0.5*(A.rho_o + B.rho_o);
+            const unsigned o2 = os(j + 2), wi = ow(j + 1);
+            const VwBox C = vw_box(G, so, snr, td, jb, o2);
+            const double zc = at(G.zs + jb, o2);
+            const double w_old = at(so.wind + wb, wi), tdw = (double)at(td_wind + wb, wi), a_w = at(G.area + wb, wi);
+            const double w_old2 = at(so.wind + wb, ow(j + 2 < L ? j + 2 : L - 1));   /* w at level j+2 (interface j+1) */
+            const double th_c = C.rt_n/C.rho_n;
+            const double tin = 0.5*(th_a + th_b), rio = 0.5*(A.rho_o + B.rho_o);
             const double rie = 0.5*(ca.re + cb.re);
             const double d = -(tin*tin)*(ca.ga + cb.ga)
                              + 0.5*(A.exbg - B.exbg)*(cb.al - ca.al + tin*(cb.be - ca.be))
@@ -1523,7 +1492,7 @@ __global__ void __launch_bounds__(VR_THREADS) k_ver_waves_run(DevGrid G, DevStat
                              - (za - zb)/(iw*dt2*GC_C_D_P)*w_old*rie/rio;
             double e = 0.0, c = 0.0;
             if (j < L - 2) {
-                const double tin_n = 0.5*(B.rt_n/B.rho_n + C.rt_n/C.rho_n), rio_n = 0.5*(B.rho_o + C.rho_o);
+                const double tin_n = 0.5*(th_b + th_c), rio_n = 0.5*(B.rho_o + C.rho_o);
                 c = tin_n*cb.ga*tin
                     + 0.5*(B.exbg - C.exbg)*(cb.al + cb.be*tin)
                     - (zb - zc)/(iw*dt*GC_C_D_P)*0.5*w_old2/(B.vol*rio_n);
@@ -1531,91 +1500,69 @@ __global__ void __launch_bounds__(VR_THREADS) k_ver_waves_run(DevGrid G, DevStat
                     - 0.5*(A.exbg - B.exbg)*(cb.al + cb.be*tin_n)
                     + (za - zb)/(iw*dt*GC_C_D_P)*0.5*w_old/(B.vol*rio);
             }
-            const int idx = j*VR_NCOL + col;
-            cc[idx] = c; dd[idx] = d; ee[idx] = e; rr[idx] = r;
-            A = B; ca = cb; za = zb;
-            B = C; cb = vw_layer(C, dt, rk); zb = zc;
+            if (j < NI) {
+                const int idx = j*NCOL + col;
+                cc[idx] = c; dd[idx] = d; ee[idx] = e; rr[idx] = r;
+            }
+            k_tin[t + 1] = tin; k_rio[t + 1] = rio;
+            A = B; ca = cb; za = zb; th_a = th_b;
+            B = C; cb = vw_layer(C, dt, rk); zb = zc; th_b = th_c;
+            if (t + 2 < VR_PER) keep(j + 2, C, cb);
         }
     }
+    /* what else phases 2 and 3 need, in flight during the elimination: these
+       reads of the state come before the barriers, its writes after them */
+    __builtin_amdgcn_sched_barrier(0);
+    double k_vol[VR_PER + 1], k_epo[VR_PER], k_rto[VR_PER], k_aw[VR_PER], k_wo[VR_PER], k_thbg[VR_PER], k_damp[VR_PER];
+    k_vol[0] = at(G.vol + jb, os(j0 > 0 ? j0 - 1 : 0));
+#pragma unroll
+    for (int t = 0; t < VR_PER; ++t) {
+        const unsigned o = os(j0 + t), wi = ow(j0 + t);
+        k_vol[t + 1] = at(G.vol + jb, o); k_epo[t] = at(so.ep + jb, o); k_rto[t] = at(so.rt + jb, o);
+        k_aw[t] = at(G.area + wb, wi); k_wo[t] = at(so.wind + wb, wi);
+        k_thbg[t] = at(G.thbg + jb, o);
+        k_damp[t] = at(G.damp + jb, os(j0 + t < NI ? j0 + t : NI - 1));
+    }
     __syncthreads();
-    if (threadIdx.x < VR_NCOL && live) thomas_lds<VR_NCOL, NI>(cc, dd, ee, rr, NI, col);
+    /* phase 2: Thomas algorithm (column_solvers.c:641-667), one lane per column */
+    if ((int)threadIdx.x < NCOL && live) thomas_lds<NCOL>(cc, dd, ee, rr, NI, col);
     __syncthreads();
     /* Klemp (2008) damping of the solved fluxes (column_solvers.c:284-298) */
 #pragma unroll
-    for (int it = 0; it < (NI*VR_NCOL + VR_THREADS - 1)/VR_THREADS; ++it) {
-        const int idx = threadIdx.x + it*VR_THREADS;
-        if (idx >= NI*VR_NCOL) break;
-        const int j = idx/VR_NCOL, ic = i0 + (idx - j*VR_NCOL);
-        const int ii = ic < nsh ? ic : nsh - 1;
-        rr[idx] = rr[idx]/(1.0 + dt*G.damp[(i64)j*nsh + ii]);
+    for (int t = 0; t < VR_PER; ++t) {
+        const int idx = (j0 + t)*NCOL + col;
+        if (j0 + t < NI) rr[idx] = rr[idx]/(1.0 + dt*k_damp[t]);
     }
     __syncthreads();
-    /* phase 3: new state of boxes k0..k1-1 of this wave (column_solvers.c:300-370) */
-    const int k0 = w*PER3, k1 = k0 + PER3 < L ? k0 + PER3 : L;
-    double o_rho[PER3], o_rt[PER3], o_tp[PER3], o_ep[PER3], o_w[PER3];
-    {
-        VwBox A = vw_box(G, so, snr, td, i, k0);
-        /* the box above the run: theta, old density and new density */
-        double rt_nm = 0.0, rho_nm = 1.0, rho_om = 0.0, rho_prev = 0.0;
-        if (k0 >= 1) {
-            const i64 bm = i + (i64)(k0 - 1)*nsh;
-            rt_nm = snr.rt[bm]; rho_nm = snr.rho[gi + bm]; rho_om = so.rho[gi + bm];
-            const double re_m = rho_om + dt*td.rho[gi + bm], vm = G.vol[bm];
-            const double x_m = rr[(k0 - 1)*VR_NCOL + col];
-            if (k0 - 1 == 0) rho_prev = re_m + dt*(x_m)/vm;
-            else rho_prev = re_m + dt*(-rr[(k0 - 2)*VR_NCOL + col] + x_m)/vm;
-        }
+    /* phase 3: the new state of boxes j0 .. j0 + VR_PER - 1 (column_solvers.c:300-370);
+       every read of the state, which may be the one written, came before the barriers */
+    double x_m = j0 >= 1 ? rr[(j0 - 1)*NCOL + col] : 0.0;
+    const double x_mm = j0 >= 2 ? rr[(j0 - 2)*NCOL + col] : 0.0;
+    /* the new density of the box above, with the arithmetic of its own group */
+    double rho_prev = k_re0 + dt*(j0 == 1 ? x_m : -x_mm + x_m)/k_vol[0];
 #pragma unroll
-        for (int t = 0; t < PER3; ++t) {
-            o_rho[t] = 0.0; o_rt[t] = 0.0; o_tp[t] = 0.0; o_ep[t] = 0.0; o_w[t] = 0.0;
-            const int j = k0 + t;
-            if (j >= k1) break;
-            const int jp = j + 1 < L ? j + 1 : L - 1;
-            const VwBox P = vw_box(G, so, snr, td, i, jp);
-            const i64 b = i + (i64)j*nsh, wi = i + (i64)(j >= 1 ? j : 1)*vpl;
-            const double thbg = G.thbg[b], a_w = area[wi], w_o = so.wind[wi];
-            const double x_j = (j < L - 1) ? rr[j*VR_NCOL + col] : 0.0;
-            const double x_m = (j >= 1) ? rr[(j - 1)*VR_NCOL + col] : 0.0;
-            const ColumnLayer cl = vw_layer(A, dt, rk);
-            const double tin_j = (j < L - 1) ? 0.5*(A.rt_n/A.rho_n + P.rt_n/P.rho_n) : 0.0;
-            const double tin_m = (j >= 1) ? 0.5*(rt_nm/rho_nm + A.rt_n/A.rho_n) : 0.0;
-            const double v = A.vol;
-            double rho_n, rt_n;
-            if (j == 0) {
-                rho_n = cl.re + dt*(x_j)/v;
-                rt_n = cl.rte + dt*(tin_j*x_j)/v;
-            } else if (j == L - 1) {
-                rho_n = cl.re + dt*(-x_m)/v;
-                rt_n = cl.rte + dt*(-tin_m*x_m)/v;
-            } else {
-                rho_n = cl.re + dt*(-x_m + x_j)/v;
-                rt_n = cl.rte + dt*(-tin_m*x_m + tin_j*x_j)/v;
-            }
-            o_rho[t] = rho_n;
-            o_rt[t] = rt_n;
-            o_tp[t] = rt_n/rho_n - thbg;
-            o_ep[t] = A.ep_o + v*cl.ga*(rt_n - A.rt_o);
+    for (int t = 0; t < VR_PER; ++t) {
+        const int j = j0 + t;
+        const double x_j = j < NI ? rr[j*NCOL + col] : 0.0;
+        const double tin_m = k_tin[t], tin_j = k_tin[t + 1], v = k_vol[t + 1];
+        const double sr = j == 0 ? x_j : (j == L - 1 ? -x_m : -x_m + x_j);
+        const double st = j == 0 ? tin_j*x_j : (j == L - 1 ? -tin_m*x_m : -tin_m*x_m + tin_j*x_j);
+        const int ix = (j < L ? j : L - 1)*NCOL + col;
+        const double rho_n = p_re[ix] + dt*sr/v;
+        const double rt_n = p_rte[ix] + dt*st/v;
+        if (live && j < L) {
+            const unsigned o = os(j);
+            put(sn.rho + gi, o, rho_n);
+            put(sn.rt + jb, o, rt_n);
+            put(sn.tp + jb, o, rt_n/rho_n - k_thbg[t]);
+            put(sn.ep + jb, o, k_epo[t] + p_vga[ix]*(rt_n - k_rto[t]));
             if (j >= 1) {
-                const double rio_m = 0.5*(rho_om + A.rho_o);   /* rho_int_old(j - 1) */
                 const double din = 0.5*(rho_prev + rho_n);
-                o_w[t] = (2.0*x_m/a_w - din*w_o)/rio_m;
+                put(sn.wind + wb, ow(j), (2.0*x_m/k_aw[t] - din*k_wo[t])/k_rio[t]);
             }
-            rt_nm = A.rt_n; rho_nm = A.rho_n; rho_om = A.rho_o; rho_prev = rho_n;
-            A = P;
         }
-    }
-    __syncthreads();
-    if (!live) return;
-#pragma unroll
-    for (int t = 0; t < PER3; ++t) {
-        const int j = k0 + t;
-        if (j >= k1) break;
-        const i64 b = i + (i64)j*nsh;
-        sn.rho[gi + b] = o_rho[t];
-        sn.rt[b] = o_rt[t];
-        sn.tp[b] = o_tp[t];
-        sn.ep[b] = o_ep[t];
-        if (j >= 1) sn.wind[i + (i64)j*vpl] = o_w[t];
+        x_m = x_j;
+        rho_prev = rho_n;
     }
 }
 
@@ -1670,10 +1617,11 @@ __global__ void __launch_bounds__(GD_THREADS) k_gen_densities(DevGrid G, DevStat
     const int L = LT > 0 ? LT : G.L, nsh = G.nsh, ncc = G.n_cond;
     /* the tracer is the fast block index: the blocks of one group of columns
        run side by side on one XCD and share the wind, area and volume columns in L2 */
-    const unsigned ntr = (unsigned)G.n_const - 1, blk = xcd_block().x;
+    const unsigned ntr = (unsigned)G.n_const - 1, blk = xcd_x();
     const int tr = (int)(blk%ntr);
     const int k = tr < ncc ? tr : tr + 1;   /* skip the gas */
     const int i0 = (int)(blk/ntr)*GD_NCOL;
+    if (i0 >= nsh) return;
     const double iw = 0.5, ew = 1.0 - iw, dt = K.dt;
     const double *vol = G.vol, *area = G.area;
     const double *rho_o = so.rho + (i64)k*G.s;
@@ -1845,7 +1793,8 @@ __global__ void __launch_bounds__(NT) k_gen_densities_all(DevGrid G, DevState so
     static_assert(NSYS <= NT, "one lane per system in phase 2");
     const int nsh = G.nsh, vpl = G.vpl;
     const i64 S = G.s;
-    const int i0 = (int)xcd_block().x*NCOLS;
+    const int i0 = (int)xcd_x()*NCOLS;
+    if (i0 >= nsh) return;
     const double iw = 0.5, ew = 1.0 - iw, dt = K.dt;
     double *ce = lds, *dd = lds + L*NSYS, *rr = lds + 2*L*NSYS;
     unsigned char *fl = (unsigned char *)(lds + 3*L*NSYS);
@@ -1981,7 +1930,7 @@ template <int LT>
 __global__ void __launch_bounds__(128) k_gen_densities_stream(DevGrid G, DevState so, DevState sn, DevState td,
                                                               StepConsts K)
 {
-    const unsigned ntr = (unsigned)G.n_const - 1, blk = xcd_block().x;
+    const unsigned ntr = (unsigned)G.n_const - 1, blk = xcd_x();
     const int tr = (int)(blk%ntr);
     const int ncc = G.n_cond;
     const int k = tr < ncc ? tr : tr + 1;
@@ -2052,13 +2001,16 @@ __global__ void __launch_bounds__(128) k_gen_densities_stream(DevGrid G, DevStat
    the condensates in the reference's constituent order, starting from 0 */
 template <typename TW, int NCC>
 __global__ void __launch_bounds__(TPB) k_sed_heat(DevGrid G, DevState so, DevState sn, const TW *T, const TW *cpc,
-                                                  TW *sed_heat, StepConsts K)
+                                                  TW *sed_heat, StepConsts K, Span sp)
 {
-    const i64 b = (i64)xcd_block().x*TPB + threadIdx.x;
-    if (b >= G.s) return;
-    /* NCC > 0: the condensate count at compile time, so both loops unroll */
-    const int nsh = G.nsh, vpl = G.vpl, L = G.L, ncc = NCC > 0 ? NCC : G.n_cond;
-    const int j = (int)(b/nsh), i = (int)(b - (i64)j*nsh);
+    const Blk bk = xcd_block(sp);
+    const int i = (int)(bk.x*TPB + threadIdx.x);
+    if (i >= G.nsh) return;
+    /* NCC: the condensate count at compile time, so both loops unroll */
+    const int nsh = G.nsh, vpl = G.vpl, L = G.L;
+    constexpr int ncc = NCC;
+    const int j = (int)bk.y;
+    const i64 b = (i64)j*nsh + i;
     const double *vol = G.vol, *area = G.area;
     double sh = 0.0;
 #pragma unroll
@@ -2081,7 +2033,7 @@ __global__ void __launch_bounds__(TPB) k_sed_heat(DevGrid G, DevState so, DevSta
             const bool lo = fr >= 0.0;
             const double d0 = rho_o[bb + nsh], d1 = rho_o[bb];
             const double t0 = (double)T[bb + nsh], t1 = (double)T[bb];
-            const double c0 = (double)cpc[(i64)k*G.s + bb + nsh], c1 = (double)cpc[(i64)k*G.s + bb];
+            const double c0 = (double)cpc[(i64)(k & 1)*G.s + bb + nsh], c1 = (double)cpc[(i64)(k & 1)*G.s + bb];
             const double doi = lo ? d0 : d1, toi = lo ? t0 : t1, cpi = lo ? c0 : c1;
             fr = doi*fr;
             const double f = cpi*toi*fr;
@@ -2092,7 +2044,7 @@ __global__ void __launch_bounds__(TPB) k_sed_heat(DevGrid G, DevState so, DevSta
             const i64 low = i + G.s - nsh, sfc = i + G.v - nsh;
             sh += -fe_m/vol[b];
             const double tl = (double)T[low];
-            sh += -vsink*tl*(double)cpc[(i64)k*G.s + low]*rho_o[low]*area[sfc]/vol[b];
+            sh += -vsink*tl*(double)cpc[(i64)(k & 1)*G.s + low]*rho_o[low]*area[sfc]/vol[b];
         } else sh += (-fe_m + fe)/vol[b];
     }
     sed_heat[b] = (TW)sh;
@@ -2119,7 +2071,7 @@ __device__ __forceinline__ void sed_heat_column(const DevGrid &G, const StepCons
     /* values of the box above the current interface */
     double d_up[NCC], c_up[NCC], t_up = (double)T[i];
 #pragma unroll
-    for (int k = 0; k < NCC; ++k) { d_up[k] = rho_o[k*S + i]; c_up[k] = (double)cpc[k*S + i]; }
+    for (int k = 0; k < NCC; ++k) { d_up[k] = rho_o[k*S + i]; c_up[k] = (double)cpc[(k & 1)*S + i]; }
     double fe_m[NCC];
 #pragma unroll
     for (int k = 0; k < NCC; ++k) fe_m[k] = 0.0;
@@ -2137,7 +2089,7 @@ __device__ __forceinline__ void sed_heat_column(const DevGrid &G, const StepCons
 #pragma unroll
             for (int k = 0; k < NCC; ++k) {
                 d_lo[k] = rho_o[k*S + b + nsh];
-                c_lo[k] = (double)cpc[k*S + b + nsh];
+                c_lo[k] = (double)cpc[(k & 1)*S + b + nsh];
                 double fr = wn;
                 fr -= vsink[k];
                 fr = a*fr;
@@ -2170,7 +2122,7 @@ template <typename TW, int NCC, int LT>
 __global__ void __launch_bounds__(TPB) k_sed_heat_col(DevGrid G, DevState so, DevState sn, const TW *T, const TW *cpc,
                                                       TW *sed_heat, StepConsts K)
 {
-    const int i = xcd_block().x*TPB + threadIdx.x;
+    const int i = (int)(xcd_x()*TPB + threadIdx.x);
     if (i >= G.nsh) return;
     sed_heat_column<TW, NCC, LT>(G, K, i, so.rho, sn.wind, G.area, G.vol, T, cpc, sed_heat);
 }
@@ -2350,7 +2302,7 @@ __global__ void __launch_bounds__(TPB) k_phase_trans(DevGrid G, DevState s, cons
     const i64 S = G.s;
     double r[6], cp[4], out[5], heat;
     for (int k = 0; k < 6; ++k) r[k] = s.rho[k*S + i];
-    for (int k = 0; k < 4; ++k) cp[k] = (double)cpc[k*S + i];
+    for (int k = 0; k < 4; ++k) cp[k] = (double)cpc[(k & 1)*S + i];
     phase_trans_point(r, (double)temp[i], cp, dt, out, heat);
     for (int k = 0; k < 5; ++k) ptr[k*S + i] = (TW)out[k];
     phr[i] = (TW)heat;
@@ -2385,11 +2337,9 @@ __global__ void __launch_bounds__(TPB) k_temp_phase(DevGrid G, DevState s, TW *T
        cloud water the liquid one; each is evaluated once */
     const TW c_ice = (TW)c_p_ice(tt), c_liq = (TW)c_p_water(tt);
     double cp[4];
-    for (int k = 0; k < 4; ++k) {
-        const TW c = (k & 1) == 0 ? c_ice : c_liq;
-        cpc[k*S + i] = c;
-        cp[k] = (double)c;
-    }
+    for (int k = 0; k < 4; ++k) cp[k] = (double)((k & 1) == 0 ? c_ice : c_liq);
+    cpc[i] = c_ice;
+    cpc[S + i] = c_liq;
     double out[5], heat;
     phase_trans_point(r, tt, cp, dt, out, heat);
     for (int k = 0; k < 5; ++k) ptr[k*S + i] = (TW)out[k];
@@ -2473,11 +2423,6 @@ namespace hor {
         if (G.flat) LAUNCH(NAME, (KERNEL<true, TW>), GRIDDIM, dim3(TPB), st, __VA_ARGS__);    \
         else LAUNCH(NAME, (KERNEL<false, TW>), GRIDDIM, dim3(TPB), st, __VA_ARGS__);          \
     } while (0)
-#define FLAT_DISPATCH_NC(NAME, KERNEL, NC, GRIDDIM, ...)                                          \
-    do {                                                                                      \
-        if (G.flat) LAUNCH(NAME, (KERNEL<true, TW, NC>), GRIDDIM, dim3(TPB), st, __VA_ARGS__);\
-        else LAUNCH(NAME, (KERNEL<false, TW, NC>), GRIDDIM, dim3(TPB), st, __VA_ARGS__);      \
-    } while (0)
 
 /* launches f for the longest chunk of n layers or levels in `chunks` chunks:
    1, 2 or 3 (the kernel holds a chunk's results until its last load), or 0
@@ -2493,71 +2438,90 @@ static void run_dispatch(int n, int chunks, F f)
 }
 
 template <typename TW>
-static void pgrad_t(const DevGrid &G, const DevState &s, const DevWorkT<TW> &W, int first, double itw, hipStream_t st)
+static void pgrad_t(const DevGrid &G, const DevState &s, const DevWorkT<TW> &W, int first, double itw, const Mom<TW> &m,
+                    hipStream_t st)
 {
-    /* the weights of the momentum tendency, as vector_tend_t forms them */
+    /* the weights of the momentum tendency */
     const double chw = 0.5 + itw, ohw = 1.0 - chw, cvw = 1.0 - itw;
-    if (G.n_const == 6) {
-        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 6>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, first, 1,
-               (const double *)W.gas_frac, cvw);
-        FLAT_DISPATCH_NC("k_pgrad_e", k_pgrad_e, 6, GRID2(G.nvh, G.split_grad), G, s, W, first,
-                         (const double *)W.gas_frac, chw, ohw);
+    const double *gf = W.gas_frac;
+    const dim3 gw = grid_of(G.nsh, G.L - 1), ge = grid_of(G.nvh, G.split_grad), b(TPB);
+    const Span sw = span_of(G.nsh, 1, 1), se = span_of(G.nvh, G.L, G.split_grad);
+    if (first) {
+        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, false>), gw, b, st, G, s, W, first, gf, cvw, m, sw);
+        if (G.flat) LAUNCH("k_pgrad_e", (k_pgrad_e<true, TW, false>), ge, b, st, G, s, W, first, gf, chw, ohw, m, se);
+        else LAUNCH("k_pgrad_e", (k_pgrad_e<false, TW, false>), ge, b, st, G, s, W, first, gf, chw, ohw, m, se);
     } else {
-        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 1>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, first, 1,
-               (const double *)W.gas_frac, cvw);
-        FLAT_DISPATCH_NC("k_pgrad_e", k_pgrad_e, 1, GRID2(G.nvh, G.split_grad), G, s, W, first,
-                         (const double *)W.gas_frac, chw, ohw);
+        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, true>), gw, b, st, G, s, W, first, gf, cvw, m, sw);
+        if (G.flat) LAUNCH("k_pgrad_e", (k_pgrad_e<true, TW, true>), ge, b, st, G, s, W, first, gf, chw, ohw, m, se);
+        else LAUNCH("k_pgrad_e", (k_pgrad_e<false, TW, true>), ge, b, st, G, s, W, first, gf, chw, ohw, m, se);
     }
 }
 
 template <typename TW>
-static void pgc_v_t(const DevGrid &G, const DevState &s, const DevWorkT<TW> &W, hipStream_t st)
+static void vorticity_flux_t(const DevGrid &G, const TW *F, const TW *pv, TW *out, hipStream_t st)
 {
-    /* the constituent count (6 or 1) as a compile-time constant, so the
-       density sums unroll and their loads issue together */
-    if (G.n_const == 6)
-        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 6>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, 0, 0, nullptr, 0.0);
-    else
-        LAUNCH("k_pgrad_w", (k_pgrad_w<TW, 1>), GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, s, W, 0, 0, nullptr, 0.0);
+    const DevWorkT<TW> W{};
+    const Mom<TW> m{};
+    LAUNCH("k_vorticity_flux_e", (k_vorticity_flux_e<true, TW, false>), grid_of(G.nvh, G.split_edge), dim3(TPB), st, G, F, pv,
+           out, W, m, span_of(G.nvh, G.L, G.split_edge));
+    run_dispatch(G.L + 1, G.split_cell_w, [&](auto r) {
+        LAUNCH("k_vorticity_flux_w", (k_vorticity_flux_w<TW, decltype(r)::value, 0>), grid_of(G.nsh, G.split_cell_w),
+               dim3(TPB), st, G, F, pv, out, W, m, (const double *)nullptr, span_of(G.nsh, G.L + 1, G.split_cell_w));
+    });
 }
 
 template <typename TW>
-static void vorticity_flux_w_t(const DevGrid &G, const TW *F, const TW *pv, TW *out, hipStream_t st)
+static void momentum_e_t(const DevGrid &G, const DevWorkT<TW> &W, const Mom<TW> &m, hipStream_t st)
 {
+    const dim3 g = grid_of(G.nvh, G.split_edge), b(TPB);
+    const Span sp = span_of(G.nvh, G.L, G.split_edge);
+    const TW *F = W.flux, *pv = W.pv;
+    if (G.flat) LAUNCH("k_vorticity_flux_e", (k_vorticity_flux_e<true, TW, true>), g, b, st, G, F, pv, W.pvt, W, m, sp);
+    else LAUNCH("k_vorticity_flux_e", (k_vorticity_flux_e<false, TW, true>), g, b, st, G, F, pv, W.pvt, W, m, sp);
+}
+
+template <typename TW>
+static void momentum_w_t(const DevGrid &G, const DevWorkT<TW> &W, const Mom<TW> &m, const double *rho, hipStream_t st)
+{
+    const dim3 g = grid_of(G.nsh, G.split_cell_w), b(TPB);
+    const Span sp = span_of(G.nsh, G.L + 1, G.split_cell_w);
+    const TW *F = W.flux, *pv = W.pv;
     run_dispatch(G.L + 1, G.split_cell_w, [&](auto r) {
-        LAUNCH("k_vorticity_flux_w", (k_vorticity_flux_w<TW, decltype(r)::value>), GRID2(G.nsh, G.split_cell_w), dim3(TPB),
-               st, G, F, pv, out);
+        constexpr int RUN = decltype(r)::value;
+        if (G.n_const == 6)
+            LAUNCH("k_vorticity_flux_w", (k_vorticity_flux_w<TW, RUN, 6>), g, b, st, G, F, pv, W.pvt, W, m, rho, sp);
+        else LAUNCH("k_vorticity_flux_w", (k_vorticity_flux_w<TW, RUN, 1>), g, b, st, G, F, pv, W.pvt, W, m, rho, sp);
     });
 }
 
 template <typename TW>
 static void inner_product_t(const DevGrid &G, const double *a, const double *b, TW *out, hipStream_t st)
 {
-    run_dispatch(G.L, G.split_cell, [&](auto r) {
-        LAUNCH("k_inner_product", (k_inner_product<TW, decltype(r)::value>), GRID2(G.nsh, G.split_cell), dim3(TPB), st, G,
-               a, b, out);
-    });
+    LAUNCH("k_inner_product", k_inner_product<TW>, grid_of(G.nsh, G.L), dim3(TPB), st, G, a, b, out, span_of(G.nsh, 1, 1));
+}
+
+template <typename TW>
+static void grad_t(const DevGrid &G, const TW *f, TW *out, hipStream_t st)
+{
+    FLAT_DISPATCH("k_grad_e", k_grad_e, grid_of(G.nvh, G.split_grad), G, f, out, span_of(G.nvh, G.L, G.split_grad));
+    LAUNCH("k_grad_w", k_grad_w<TW>, grid_of(G.nsh, G.L - 1), dim3(TPB), st, G, f, out,
+           span_of(G.nsh, 1, 1));
+}
+
+template <typename TW>
+static void rel_vort_tri_t(const DevGrid &G, const double *wind, TW *out, hipStream_t st)
+{
+    LAUNCH("k_rel_vort_tri", k_rel_vort_tri<TW>, grid_of(G.nt, G.split_tri), dim3(TPB), st, G, wind, out,
+           span_of(G.nt, G.L, G.split_tri));
 }
 
 template <typename TW>
 static void advection_pv_t(const DevGrid &G, const double *wind, const double *rho_gas, const DevWorkT<TW> &W,
                            hipStream_t st)
 {
-    LAUNCH("k_mass_flux", k_mass_flux<TW>, GRID2(G.nvh > G.nsh ? G.nvh : G.nsh, G.split_edge), dim3(TPB), st, G,
-           rho_gas, wind, W.flux);
-    LAUNCH("k_rel_vort_tri", k_rel_vort_tri<TW>, GRID2(G.nt, G.split_tri), dim3(TPB), st, G, wind, W.rvt);
-    FLAT_DISPATCH("k_pot_vort", k_pot_vort, GRID2(G.nvh, G.split_edge), G, wind, rho_gas, (const TW *)W.rvt, W.pv);
-    LAUNCH("k_vorticity_flux_e", k_vorticity_flux_e<TW>, GRID2(G.nvh, G.split_edge), dim3(TPB), st, G, (const TW *)W.flux,
-           (const TW *)W.pv, W.pvt);
-    vorticity_flux_w_t<TW>(G, W.flux, W.pv, W.pvt, st);
-}
-
-template <typename TW>
-static void advection_kinetic_t(const DevGrid &G, const double *wind, const DevWorkT<TW> &W, hipStream_t st)
-{
-    inner_product_t<TW>(G, wind, wind, W.vsq, st);
-    FLAT_DISPATCH("k_grad_e", k_grad_e, GRID2(G.nvh, G.split_grad), G, (const TW *)W.vsq, W.vsq_grad);
-    LAUNCH("k_grad_w", k_grad_w<TW>, GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, (const TW *)W.vsq, W.vsq_grad);
+    rel_vort_tri_t<TW>(G, wind, W.rvt, st);
+    FLAT_DISPATCH("k_pot_vort", k_pot_vort, grid_of(G.nvh, G.split_edge), G, wind, rho_gas, (const TW *)W.rvt, W.pv, W.flux,
+                  span_of(G.nvh, G.L + 1, G.split_edge));
 }
 
 template <typename TW>
@@ -2565,16 +2529,9 @@ static void advection_t(const DevGrid &G, const double *wind, const double *rho_
                         hipStream_t st)
 {
     advection_pv_t<TW>(G, wind, rho_gas, W, st);
-    advection_kinetic_t<TW>(G, wind, W, st);
-}
-
-template <typename TW>
-static void vector_tend_t(const DevGrid &G, const DevWorkT<TW> &W, TW *tend_w, const double *w_old, double *w_new,
-                          double new_w, double itw, double dt, hipStream_t st)
-{
-    double chw = 0.5 + itw, ohw = 1.0 - chw, cvw = 1.0 - itw;
-    LAUNCH("k_vector_tend", k_vector_tend<TW>, GRID1(G.v), dim3(TPB), st, G, W, tend_w, w_old, w_new, new_w, chw, ohw,
-           cvw, dt);
+    vorticity_flux_t<TW>(G, W.flux, W.pv, W.pvt, st);
+    inner_product_t<TW>(G, wind, wind, W.vsq, st);
+    grad_t<TW>(G, W.vsq, W.vsq_grad, st);
 }
 
 /* the precision of FP32 storage on an FP64 array (a probe of the mixed form) */
@@ -2608,45 +2565,39 @@ static void scalar_tend_t(const DevGrid &G, const DevState &s, const DevState &t
            -0.5*ipw*slope as a grid constant (one coalesced load for a
            coalesced load and a gather) it takes 49.6 us per launch at
            res 6 x 26 where it took 58.9 */
-        LAUNCH("k_vcc", k_vcc, GRID2(G.nsh, G.split_vcc), dim3(TPB), st, G, s, W.vcc);
-    run_dispatch(G.L, G.split_cell, [&](auto r) {
-        constexpr int RUN = decltype(r)::value;
-        const dim3 g = GRID2(G.nsh, G.split_cell), b(TPB);
-        if (G.n_const == 6) {
-            if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 6, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
-            else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 6, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
-        } else {
-            if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 1, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
-            else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 1, RUN>), g, b, st, G, s, W, td.rho, td.rt, rk);
-        }
-    });
+        LAUNCH("k_vcc", k_vcc, grid_of(G.nsh, G.split_vcc), dim3(TPB), st, G, s, W.vcc,
+               span_of(G.nsh, G.n_oro, G.split_vcc));
+    const dim3 g = grid_of(G.nsh, G.L), b(TPB);
+    const Span sp = span_of(G.nsh, 1, 1);
+    if (G.n_const == 6) {
+        if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 6>), g, b, st, G, s, W, td.rho, td.rt, rk, sp);
+        else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 6>), g, b, st, G, s, W, td.rho, td.rt, rk, sp);
+    } else {
+        if (G.flat) LAUNCH("k_scalar_tend", (k_scalar_tend<true, TW, 1>), g, b, st, G, s, W, td.rho, td.rt, rk, sp);
+        else LAUNCH("k_scalar_tend", (k_scalar_tend<false, TW, 1>), g, b, st, G, s, W, td.rho, td.rt, rk, sp);
+    }
     scalar_tend_probe<TW>(G, td, st);
 }
 
-void pgrad(const DevGrid &G, const DevState &s, const DevWork &W, int first, double itw, hipStream_t st)
-{ pgrad_t<double>(G, s, W, first, itw, st); }
-void pgrad(const DevGrid &G, const DevState &s, const DevWorkF &W, int first, double itw, hipStream_t st)
-{ pgrad_t<float>(G, s, W, first, itw, st); }
-void pgc_v(const DevGrid &G, const DevState &s, const DevWork &W, hipStream_t st) { pgc_v_t<double>(G, s, W, st); }
-void pgc_v(const DevGrid &G, const DevState &s, const DevWorkF &W, hipStream_t st) { pgc_v_t<float>(G, s, W, st); }
-void advection(const DevGrid &G, const double *wind, const double *rho_gas, const DevWork &W, hipStream_t st)
-{ advection_t<double>(G, wind, rho_gas, W, st); }
-void advection(const DevGrid &G, const double *wind, const double *rho_gas, const DevWorkF &W, hipStream_t st)
-{ advection_t<float>(G, wind, rho_gas, W, st); }
-void advection_pv(const DevGrid &G, const double *wind, const double *rho_gas, const DevWork &W, hipStream_t st)
-{ advection_pv_t<double>(G, wind, rho_gas, W, st); }
-void advection_pv(const DevGrid &G, const double *wind, const double *rho_gas, const DevWorkF &W, hipStream_t st)
-{ advection_pv_t<float>(G, wind, rho_gas, W, st); }
-void advection_kinetic(const DevGrid &G, const double *wind, const DevWork &W, hipStream_t st)
-{ advection_kinetic_t<double>(G, wind, W, st); }
-void advection_kinetic(const DevGrid &G, const double *wind, const DevWorkF &W, hipStream_t st)
-{ advection_kinetic_t<float>(G, wind, W, st); }
-void vector_tend(const DevGrid &G, const DevWork &W, double *tend_w, const double *w_old, double *w_new,
-                 double new_w, double itw, double dt, hipStream_t st)
-{ vector_tend_t<double>(G, W, tend_w, w_old, w_new, new_w, itw, dt, st); }
-void vector_tend(const DevGrid &G, const DevWorkF &W, float *tend_w, const double *w_old, double *w_new,
-                 double new_w, double itw, double dt, hipStream_t st)
-{ vector_tend_t<float>(G, W, tend_w, w_old, w_new, new_w, itw, dt, st); }
+/* the entry points of both forms */
+#define BOTH_FORMS(T, WORK)                                                                                         \
+    void pgrad(const DevGrid &G, const DevState &s, const WORK &W, int first, double itw, T *td, const double *w_old,   \
+               double *w_new, double dt, hipStream_t st)                                                            \
+    { pgrad_t<T>(G, s, W, first, itw, Mom<T>{td, w_old, w_new, 1.0, dt}, st); }                                     \
+    void advection(const DevGrid &G, const double *wind, const double *rho_gas, const WORK &W, hipStream_t st)      \
+    { advection_t<T>(G, wind, rho_gas, W, st); }                                                                    \
+    void advection_pv(const DevGrid &G, const double *wind, const double *rho_gas, const WORK &W, hipStream_t st)   \
+    { advection_pv_t<T>(G, wind, rho_gas, W, st); }                                                                 \
+    void kinetic_energy(const DevGrid &G, const double *wind, const WORK &W, hipStream_t st)                        \
+    { inner_product_t<T>(G, wind, wind, W.vsq, st); }                                                               \
+    void momentum_e(const DevGrid &G, const WORK &W, T *td, const double *w_old, double *w_new, double new_w,       \
+                    double dt, hipStream_t st)                                                                      \
+    { momentum_e_t<T>(G, W, Mom<T>{td, w_old, w_new, new_w, dt}, st); }                                             \
+    void momentum_w(const DevGrid &G, const WORK &W, T *td, double new_w, const double *rho, hipStream_t st)        \
+    { momentum_w_t<T>(G, W, Mom<T>{td, nullptr, nullptr, new_w, 0.0}, rho, st); }
+BOTH_FORMS(double, DevWork)
+BOTH_FORMS(float, DevWorkF)
+#undef BOTH_FORMS
 void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const DevWork &W, int rk, hipStream_t st)
 { scalar_tend_t<double>(G, s, td, W, rk, st); }
 void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const DevWorkF &W, int rk, hipStream_t st)
@@ -2656,24 +2607,22 @@ void inner_product(const DevGrid &G, const double *a, const double *b, double *o
 { inner_product_t<double>(G, a, b, out, st); }
 
 /* single operators (FP64), for the operator-level interface and its adjoints */
-void grad(const DevGrid &G, const double *f, double *out, hipStream_t st)
-{
-    typedef double TW;
-    FLAT_DISPATCH("k_grad_e", k_grad_e, GRID2(G.nvh, G.split_grad), G, f, out);
-    LAUNCH("k_grad_w", k_grad_w<double>, GRID1((i64)(G.L - 1)*G.nsh), dim3(TPB), st, G, f, out);
-}
-
+void grad(const DevGrid &G, const double *f, double *out, hipStream_t st) { grad_t<double>(G, f, out, st); }
 void curl_triangles(const DevGrid &G, const double *wind, double *out, hipStream_t st)
-{ LAUNCH("k_rel_vort_tri", k_rel_vort_tri<double>, GRID2(G.nt, G.split_tri), dim3(TPB), st, G, wind, out); }
+{ rel_vort_tri_t<double>(G, wind, out, st); }
+
+void tables(const DevGrid &G, unsigned *c_e, unsigned *c_n, unsigned *c_from, unsigned *e_ti, unsigned *e_tm, double *e_tw,
+            unsigned *e_rc, double *e_rw, unsigned *t_e, hipStream_t st)
+{
+    const int n = G.nvh > G.nt ? G.nvh : G.nt;   /* more than nsh */
+    LAUNCH("k_tables", k_tables, GRID1(n), dim3(TPB), st, G, c_e, c_n, c_from, e_ti, e_tm, e_tw, e_rc, e_rw, t_e);
+}
 
 void vcc_weights(const DevGrid &G, double *vcw, hipStream_t st)
 { LAUNCH("k_vcc_weights", k_vcc_weights, GRID1((i64)G.n_oro*6*G.nsh), dim3(TPB), st, G, vcw); }
 
 void vorticity_flux(const DevGrid &G, const double *F, const double *pv, double *out, hipStream_t st)
-{
-    LAUNCH("k_vorticity_flux_e", k_vorticity_flux_e<double>, GRID2(G.nvh, G.split_edge), dim3(TPB), st, G, F, pv, out);
-    vorticity_flux_w_t<double>(G, F, pv, out, st);
-}
+{ vorticity_flux_t<double>(G, F, pv, out, st); }
 
 }  // namespace hor
 
@@ -2712,23 +2661,16 @@ static void ver_waves_t(const DevGrid &G, const DevState &so, const DevState &sn
         else LAUNCH("k_ver_waves", (k_ver_waves<0, TWIND>), g, b, st, G, so, snr, sn, td, td_wind, K, rk);
         return;
     }
-    if ((G.L == 26 || G.L == 55) && !G.vw_rows) {
-        const int ncol = vr_ncol(G.L);
-        dim3 g((G.nsh + ncol - 1)/ncol), b(VR_THREADS);
-        size_t lds = (size_t)4*(G.L - 1)*ncol*sizeof(double);   /* 50 KiB at 26 layers, 55 KiB at 55 */
-        if (G.L == 26)
-            LAUNCH_SHM("k_ver_waves", (k_ver_waves_run<26, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
-        else
-            LAUNCH_SHM("k_ver_waves", (k_ver_waves_run<55, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
-        return;
-    }
-    dim3 g((G.nsh + VW_NCOL - 1)/VW_NCOL), b(VW_THREADS);
-    size_t lds = (size_t)4*(G.L - 1)*VW_NCOL*sizeof(double);   /* 25 KiB at 26 layers, 63 KiB at 64 */
-    if (G.L == 26)
-        LAUNCH_SHM("k_ver_waves", (k_ver_waves_3p<26, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
-    else if (G.L == 55)
-        LAUNCH_SHM("k_ver_waves", (k_ver_waves_3p<55, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
-    else LAUNCH_SHM("k_ver_waves", (k_ver_waves_3p<0, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
+    const int ncol = vr_ncol(G.L);
+    const dim3 g((unsigned)((G.nsh + ncol - 1)/ncol)), b((unsigned)vr_threads(G.L));
+    /* four rows of the system and three values per box: 45 KiB at 26 layers, 55 KiB at 63 */
+    const size_t lds = (size_t)(4*(G.L - 1) + 3*G.L)*ncol*sizeof(double);
+    if (ncol == 64)
+        LAUNCH_SHM("k_ver_waves", (k_ver_waves_run<64, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
+    else if (ncol == 32)
+        LAUNCH_SHM("k_ver_waves", (k_ver_waves_run<32, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
+    else
+        LAUNCH_SHM("k_ver_waves", (k_ver_waves_run<16, TWIND>), g, b, lds, st, G, so, snr, sn, td, td_wind, K, rk);
 }
 
 void ver_waves(const DevGrid &G, const DevState &so, const DevState &snr, const DevState &sn, const DevState &td,
@@ -2743,7 +2685,7 @@ static void gen_densities_only(const DevGrid &G, const DevState &so, const DevSt
                                const StepConsts &K, hipStream_t st)
 {
     if (G.gd_streaming) {
-        dim3 g(((G.nsh + 127)/128)*(G.n_const - 1)), b(128);
+        const dim3 g((unsigned)(((G.nsh + 127)/128)*(G.n_const - 1))), b(128);
         if (G.L == 26) LAUNCH("k_gen_densities", k_gen_densities_stream<26>, g, b, st, G, so, sn, td, K);
         else if (G.L == 55) LAUNCH("k_gen_densities", k_gen_densities_stream<55>, g, b, st, G, so, sn, td, K);
         else LAUNCH("k_gen_densities", k_gen_densities_stream<0>, g, b, st, G, so, sn, td, K);
@@ -2757,13 +2699,13 @@ static void gen_densities_only(const DevGrid &G, const DevState &so, const DevSt
            columns (54 KiB, two blocks per CU) took 701 us against 516:
            fewer systems in flight for the longer serial elimination */
         constexpr int NCOLS = 16, NT = 256;
-        dim3 g((G.nsh + NCOLS - 1)/NCOLS), b(NT);
+        const dim3 g((unsigned)((G.nsh + NCOLS - 1)/NCOLS)), b(NT);
         size_t lds = (size_t)3*26*5*NCOLS*sizeof(double) + (((size_t)26*5*NCOLS + 7) & ~(size_t)7);
         LAUNCH_SHM("k_gen_densities", (k_gen_densities_all<26, NCOLS, NT>), g, b, lds, st, G, so, sn, td, K);
         return;
     }
     const int ncol = gd_ncol(G.L == 26 ? 26 : (G.L == 55 ? 55 : 0));
-    dim3 g(((G.nsh + ncol - 1)/ncol)*(G.n_const - 1)), b(GD_THREADS);
+    const dim3 g((unsigned)(((G.nsh + ncol - 1)/ncol)*(G.n_const - 1))), b(GD_THREADS);
     /* 41 KiB at 26 layers, 43 KiB at 55, 50 KiB at 64 */
     size_t lds = (size_t)3*G.L*ncol*sizeof(double) + (((size_t)G.L*ncol + 7) & ~(size_t)7);
     if (G.L == 26) LAUNCH_SHM("k_gen_densities", k_gen_densities<26>, g, b, lds, st, G, so, sn, td, K);
@@ -2783,14 +2725,13 @@ void gen_densities(const DevGrid &G, const DevState &so, const DevState &sn, con
 {
     if (rk == 0 && G.n_cond > 0) {
         if (sed_heat_by_column(G) && G.L == 26)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 26>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
+            LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 26>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
         else if (sed_heat_by_column(G) && G.L == 55)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 55>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
+            LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 55>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
-        else if (G.n_cond == 4)
-            LAUNCH("k_sed_heat", (k_sed_heat<double, 4>), GRID1(G.s), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K);
-        else LAUNCH("k_sed_heat", (k_sed_heat<double, 0>), GRID1(G.s), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K);
+        else LAUNCH("k_sed_heat", (k_sed_heat<double, 4>), grid_of(G.nsh, G.L), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K,
+                    span_of(G.nsh, 1, 1));
     }
     gen_densities_only(G, so, sn, td, K, st);
 }
@@ -2800,14 +2741,13 @@ void gen_densities(const DevGrid &G, const DevState &so, const DevState &sn, con
 {
     if (rk == 0 && G.n_cond > 0) {
         if (sed_heat_by_column(G) && G.L == 26)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 26>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
+            LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 26>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
         else if (sed_heat_by_column(G) && G.L == 55)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 55>), GRID1(G.nsh), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
+            LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 55>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
                    K);
-        else if (G.n_cond == 4)
-            LAUNCH("k_sed_heat", (k_sed_heat<float, 4>), GRID1(G.s), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K);
-        else LAUNCH("k_sed_heat", (k_sed_heat<float, 0>), GRID1(G.s), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K);
+        else LAUNCH("k_sed_heat", (k_sed_heat<float, 4>), grid_of(G.nsh, G.L), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K,
+                    span_of(G.nsh, 1, 1));
     }
     gen_densities_only(G, so, sn, td, K, st);
 }

@@ -10,30 +10,42 @@
 /* horizontal operators and tendencies: work arrays double (FP64 form) or
    float (mixed form), register arithmetic FP64 in both */
 namespace hor {
-/* the gas fractions come from W.gas_frac: s must be the state the last
-   col::temperature(..., W.gas_frac, ...) was formed from */
-/* itw: the implicit weight of the momentum tendency (W.pgrad_comb) */
-void pgrad(const DevGrid &G, const DevState &s, const DevWork &W, int first, double itw, hipStream_t st);
-void pgrad(const DevGrid &G, const DevState &s, const DevWorkF &W, int first, double itw, hipStream_t st);
-void pgc_v(const DevGrid &G, const DevState &s, const DevWork &W, hipStream_t st);
-void pgc_v(const DevGrid &G, const DevState &s, const DevWorkF &W, hipStream_t st);
+/* the pressure gradient of s (nl, l, old, their combination W.pgrad_comb for
+   the implicit weight itw, and the condensates' term), and in every step but
+   a first one the first substep's momentum tendency td and wind update
+   (w_new = w_old + dt td at the edges), which read the carried W.pvt and
+   W.vsq_grad.  The gas fractions come from W.gas_frac: s must be the state
+   the last col::temperature(..., W.gas_frac, ...) was formed from */
+void pgrad(const DevGrid &G, const DevState &s, const DevWork &W, int first, double itw, double *td,
+           const double *w_old, double *w_new, double dt, hipStream_t st);
+void pgrad(const DevGrid &G, const DevState &s, const DevWorkF &W, int first, double itw, float *td,
+           const double *w_old, double *w_new, double dt, hipStream_t st);
+/* mass flux, PV, TRSK flux, kinetic energy and its gradient */
 void advection(const DevGrid &G, const double *wind, const double *rho_gas, const DevWork &W, hipStream_t st);
 void advection(const DevGrid &G, const double *wind, const double *rho_gas, const DevWorkF &W, hipStream_t st);
-/* the two independent parts of advection: mass flux, PV and the TRSK flux
-   (pot_vort_tend); kinetic energy and its gradient (v_squared_grad) */
+/* the step's parts of it: mass flux, triangle vorticity and PV; kinetic energy */
 void advection_pv(const DevGrid &G, const double *wind, const double *rho_gas, const DevWork &W, hipStream_t st);
 void advection_pv(const DevGrid &G, const double *wind, const double *rho_gas, const DevWorkF &W, hipStream_t st);
-void advection_kinetic(const DevGrid &G, const double *wind, const DevWork &W, hipStream_t st);
-void advection_kinetic(const DevGrid &G, const double *wind, const DevWorkF &W, hipStream_t st);
-void vector_tend(const DevGrid &G, const DevWork &W, double *tend_w, const double *w_old, double *w_new,
-                 double new_w, double itw, double dt, hipStream_t st);
-void vector_tend(const DevGrid &G, const DevWorkF &W, float *tend_w, const double *w_old, double *w_new,
-                 double new_w, double itw, double dt, hipStream_t st);
+void kinetic_energy(const DevGrid &G, const double *wind, const DevWork &W, hipStream_t st);
+void kinetic_energy(const DevGrid &G, const double *wind, const DevWorkF &W, hipStream_t st);
+/* and, from W.flux, W.pv and W.vsq: TRSK flux, kinetic-energy gradient and the
+   tendency td = (1 - new_w) td + new_w (...) -- at the edges with the wind
+   update; at the w points with the condensates' term of the densities rho
+   (null: W.pgc_v as it is) */
+void momentum_e(const DevGrid &G, const DevWork &W, double *td, const double *w_old, double *w_new, double new_w,
+                double dt, hipStream_t st);
+void momentum_e(const DevGrid &G, const DevWorkF &W, float *td, const double *w_old, double *w_new, double new_w,
+                double dt, hipStream_t st);
+void momentum_w(const DevGrid &G, const DevWork &W, double *td, double new_w, const double *rho, hipStream_t st);
+void momentum_w(const DevGrid &G, const DevWorkF &W, float *td, double new_w, const double *rho, hipStream_t st);
 void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const DevWork &W, int rk, hipStream_t st);
 void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const DevWorkF &W, int rk, hipStream_t st);
 void inner_product(const DevGrid &G, const double *a, const double *b, double *out, hipStream_t st);
 void grad(const DevGrid &G, const double *f, double *out, hipStream_t st);
 void curl_triangles(const DevGrid &G, const double *wind, double *out, hipStream_t st);
+/* fills the slot-major tables of DevGrid from the others */
+void tables(const DevGrid &G, unsigned *c_e, unsigned *c_n, unsigned *c_from, unsigned *e_ti, unsigned *e_tm, double *e_tw,
+            unsigned *e_rc, double *e_rw, unsigned *t_e, hipStream_t st);
 /* fills the grid constant G.vcw (n_oro x 6 x NSH doubles) */
 void vcc_weights(const DevGrid &G, double *vcw, hipStream_t st);
 void vorticity_flux(const DevGrid &G, const double *F, const double *pv, double *out, hipStream_t st);
@@ -42,7 +54,7 @@ void vorticity_flux(const DevGrid &G, const double *F, const double *pv, double 
 /* column solvers, point physics and state arithmetic shared by both forms:
    FP64 arithmetic; the work arrays are double (FP64 form) or float (mixed) */
 namespace col {
-/* cpc (may be null): c_p of every condensate at the temperature, n_cond x S;
+/* cpc (may be null): c_p of ice and of liquid water at the temperature, 2 x S;
    gf (may be null): gas density over total density, S */
 void temperature(const DevGrid &G, const DevState &s, double *T, double *cpc, double *gf, hipStream_t st);
 void temperature(const DevGrid &G, const DevState &s, float *T, float *cpc, double *gf, hipStream_t st);

@@ -171,41 +171,42 @@ int game_gpu_init(const game_dims_t *dims, const game_grid_view_t *g, const game
    chip idle unless its layers are spread over more blocks.  1024 blocks of
    four waves are about what 256 CUs hold of these kernels.  Results do not
    depend on the split.  Measured per launch (us), terrain grids of 26
-   layers, FP64, against two edge chunks, one triangle chunk and three layers
-   per cell thread at every size:
+   layers, FP64, against two edge chunks and one of the triangles at every size:
      res 4 (30 edge blocks): pressure gradient 30 -> 8, PV 34 -> 10, TRSK
-       flux 26 -> 10, triangle curl 21 -> 6, kinetic gradient 20 -> 5, moist
-       scalar transport 34 -> 18, vertical corrections 11 -> 9
+       flux 26 -> 10, triangle curl 21 -> 6, kinetic gradient 20 -> 5
      res 5 (120): pressure gradient 36 -> 24, PV 41 -> 29, TRSK flux 31 -> 24,
-       triangle curl 25 -> 13, scalar transport 48 -> 38
+       triangle curl 25 -> 13
      res 6 (480): PV 93 -> 82, TRSK flux 81 -> 76, triangle curl 39 -> 35; the
        gradients 70 and 37 with two chunks, 76 and 43 with four
-     res 7 (1920, flat): two edge chunks and one of the triangles (more cost 3
-       to 15 %); scalar transport 406 with three layers per thread, 389 with
-       two, 392 with one; vertical TRSK flux 106, 127 and 145 */
+     res 7 (1920, flat): more than two edge chunks and one of the triangles
+       cost 3 to 15 % */
 static void set_layer_splits(DevGrid &G)
 {
     const int L = G.L, be = (G.nvh + 255)/256, bc = (G.nsh + 255)/256, bt = (G.nt + 255)/256;
     auto clamp = [](int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); };
     /* edges: one filled chip; where four chunks or fewer fill it, twice that
        in at most four chunks for the kernels with long layers, whose last
-       blocks then leave less of it idle */
+       blocks then leave less of it idle.  The flat gradients carry nothing
+       between layers: one layer per thread (pressure gradient with the wind
+       update at res 7 x 26: 328 us with two chunks, 317 with 13, 313 with 26) */
     const int fill = 1024/be;
-    G.split_grad = clamp(fill, 2, L);
+    G.split_grad = G.flat ? L : clamp(fill, 2, L);
     G.split_edge = clamp(fill > 4 ? fill : clamp(2048/be, 1, 4), 2, L);
     G.split_tri = clamp((1024 + bt - 1)/bt, 1, L);
-    /* cells: two layers per thread, one where two leave the chip idle; the
-       vertical TRSK flux carries more from level to level and takes three
-       levels once three fill the chip */
-    const int run = bc*L <= 512 ? 1 : 2, run_w = bc*L < 3*1024 ? 1 : 3;
-    G.split_cell = (L + run - 1)/run;
+    /* cells: the vertical TRSK flux carries a layer's fluxes and weights from
+       level to level and takes three levels per thread once three fill the
+       chip (with the tendency at res 7 x 26: 215 us with three, 325 with two;
+       res 5: 17 with one, 23 with two) */
+    const int run_w = bc*L < 3*1024 ? 1 : 3;
     G.split_cell_w = (L + 1 + run_w - 1)/run_w;
-    /* vertical corrections: about 1280 blocks, two to six terrain levels per thread */
+    /* vertical corrections: about 1280 blocks, two to six terrain levels per
+       thread (res 4: one level 9 us, two 11; res 5: two 19, one 22, three 21;
+       res 6: three 50, four 51, six 64) */
     const int run_v = bc*G.n_oro <= 512 ? 1 : clamp((bc*G.n_oro + 640)/1280, 2, 6);
     G.split_vcc = (G.n_oro + run_v - 1)/run_v;
     if (const char *e = getenv("GAME_GPU_SPLIT_CELL")) {
         int v = atoi(e);
-        if (v >= 1 && v <= L) G.split_cell = G.split_cell_w = v;
+        if (v >= 1 && v <= L) G.split_cell_w = v;
     }
     if (const char *e = getenv("GAME_GPU_SPLIT_EDGE")) {
         int v = atoi(e);
@@ -264,7 +265,6 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
         else if (!strcmp(e, "both")) G.round_tendencies = 3;
     }
     G.vw_streaming = getenv("GAME_GPU_VW_STREAMING") ? 1 : 0;
-    G.vw_rows = getenv("GAME_GPU_VW_ROWS") ? 1 : 0;
     G.sh_per_box = getenv("GAME_GPU_SH_PER_BOX") ? 1 : 0;
     G.unfused_phase = getenv("GAME_GPU_UNFUSED_PHASE") ? 1 : 0;
     M->use_graphs = getenv("GAME_GPU_NO_GRAPH") ? 0 : 1;
@@ -325,6 +325,18 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
         UP(G.ipwT, t.data(), t.size());
         HIP_OK(hipStreamSynchronize(M->stream));
     }
+    {
+        unsigned *c_e, *c_n, *c_from, *e_ti, *e_tm, *e_rc, *t_e;
+        double *e_tw, *e_rw;
+        struct { unsigned **p; size_t n; } ut[] = {{&c_e, 6*NSH}, {&c_n, 6*NSH}, {&c_from, NSH}, {&e_ti, 10*NVH},
+                                                   {&e_tm, 10*NVH}, {&e_rc, 4*NVH}, {&t_e, 3*NT}};
+        for (auto &x : ut) if ((rc = dalloc((void **)x.p, x.n*sizeof(unsigned)))) return rc;
+        if ((rc = dzeros(&e_tw, 10*NVH)) || (rc = dzeros(&e_rw, 4*NVH))) return rc;
+        hor::tables(G, c_e, c_n, c_from, e_ti, e_tm, e_tw, e_rc, e_rw, t_e, M->stream);
+        HIP_OK(hipGetLastError());
+        G.c_e = c_e; G.c_n = c_n; G.c_from = c_from; G.e_ti = e_ti; G.e_tm = e_tm; G.e_rc = e_rc; G.t_e = t_e;
+        G.e_tw = e_tw; G.e_rw = e_rw;
+    }
     G.vcw = nullptr;
     if (!G.flat) {
         double *vcw = nullptr;
@@ -357,7 +369,7 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
         if ((rc = dzeros(&W.gas_frac, S))) return rc;
         if ((rc = dzeros(&W.pv, (size_t)d.curl))) return rc;
         if ((rc = dzeros(&W.ptr, (size_t)(d.n_cond + 1)*S))) return rc;
-        if ((rc = dzeros(&W.cpc, (size_t)(d.n_cond > 0 ? d.n_cond : 1)*S))) return rc;
+        if ((rc = dzeros(&W.cpc, (size_t)(d.n_cond > 0 ? 2 : 1)*S))) return rc;
         W.td_wind = M->s[GAME_STATE_TENDENCY].wind;
     } else {
         /* mixed: every work array FP32; the tendency state keeps FP64 densities
@@ -371,7 +383,7 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
         if ((rc = fzeros(&W.rvt, (size_t)d.dual_v_vectors))) return rc;
         if ((rc = fzeros(&W.pv, (size_t)d.curl))) return rc;
         if ((rc = fzeros(&W.ptr, (size_t)(d.n_cond + 1)*S))) return rc;
-        if ((rc = fzeros(&W.cpc, (size_t)(d.n_cond > 0 ? d.n_cond : 1)*S))) return rc;
+        if ((rc = fzeros(&W.cpc, (size_t)(d.n_cond > 0 ? 2 : 1)*S))) return rc;
         if ((rc = dzeros(&W.vcc, 3*(size_t)G.n_oro*NSH))) return rc;
         if ((rc = dzeros(&W.gas_frac, S))) return rc;
         if ((rc = dzeros(&W.flux2, 8))) return rc;
@@ -544,29 +556,42 @@ static int step_t(const WK &W, TW *td_wind, double dt, int first, const StepTape
         DevState sns = snr;                                 /* ... with the horizontal wind just updated */
         sns.wind = sn.wind;
         const double *rho_gas = snr.rho + (i64)G.n_cond*G.s;
-        if ((rk == 1 || first) && conc) {
-            /* the pressure gradient and the kinetic energy on the side
-               stream, the PV and TRSK flux on this one: they read the same
-               state and write different arrays */
-            HIP_OK(hipEventRecord(M->ev_fork, st));
-            HIP_OK(hipStreamWaitEvent(M->side, M->ev_fork, 0));
-            if (rk == 0) hor::pgrad(G, snr, W, first, M->cfg.impl_thermo_weight, M->side);
-            else hor::pgc_v(G, snr, W, M->side);
-            hor::advection_kinetic(G, snr.wind, W, M->side);
-            hor::advection_pv(G, snr.wind, rho_gas, W, st);
-            HIP_OK(hipEventRecord(M->ev_join, M->side));
-            HIP_OK(hipStreamWaitEvent(st, M->ev_join, 0));
-        } else {
-            if (rk == 0) hor::pgrad(G, snr, W, first, M->cfg.impl_thermo_weight, st);
-            else hor::pgc_v(G, snr, W, st);
-            if (rk == 1 || first) hor::advection(G, snr.wind, rho_gas, W, st);
+        /* rk 0 of every step but a first one: the pressure gradient with the
+           tendency from the carried advection */
+        if (rk == 0) hor::pgrad(G, snr, W, first, M->cfg.impl_thermo_weight, td_wind, so.wind, sn.wind, dt, st);
+        if (rk == 1 || first) {
+            const double new_w = rk == 1 ? 0.5 : 1.0;
+            /* the condensates' term of the first substep's densities; at rk 0 the pressure gradient has it */
+            const double *pgc_rho = rk == 1 ? snr.rho : nullptr;
+            if (conc) {
+                /* the kinetic energy on the side stream (where the first
+                   substep's tracer solve may still run) beside the PV on this
+                   one: they read the same state and write different arrays;
+                   then the two parts of the tendency, which read both */
+                HIP_OK(hipEventRecord(M->ev_fork, st));
+                HIP_OK(hipStreamWaitEvent(M->side, M->ev_fork, 0));
+                hor::kinetic_energy(G, snr.wind, W, M->side);
+                hor::advection_pv(G, snr.wind, rho_gas, W, st);
+                HIP_OK(hipEventRecord(M->ev_join, M->side));
+                HIP_OK(hipEventRecord(M->ev_fork, st));
+                HIP_OK(hipStreamWaitEvent(st, M->ev_join, 0));
+                HIP_OK(hipStreamWaitEvent(M->side, M->ev_fork, 0));
+                hor::momentum_w(G, W, td_wind, new_w, pgc_rho, M->side);
+                hor::momentum_e(G, W, td_wind, so.wind, sn.wind, new_w, dt, st);
+                HIP_OK(hipEventRecord(M->ev_join, M->side));
+                HIP_OK(hipStreamWaitEvent(st, M->ev_join, 0));
+            } else {
+                hor::kinetic_energy(G, snr.wind, W, st);
+                hor::advection_pv(G, snr.wind, rho_gas, W, st);
+                hor::momentum_w(G, W, td_wind, new_w, pgc_rho, st);
+                hor::momentum_e(G, W, td_wind, so.wind, sn.wind, new_w, dt, st);
+            }
         }
         if constexpr (std::is_same<WK, DevWork>::value)
             if (tape && rk == 1) {
                 HIP_OK(hipMemcpyAsync(tape->flux, W.flux, (size_t)M->d.v*sizeof(double), hipMemcpyDeviceToDevice, st));
                 HIP_OK(hipMemcpyAsync(tape->pv, W.pv, (size_t)M->d.curl*sizeof(double), hipMemcpyDeviceToDevice, st));
             }
-        hor::vector_tend(G, W, td_wind, so.wind, sn.wind, rk == 1 ? 0.5 : 1.0, M->cfg.impl_thermo_weight, dt, st);
         hor::scalar_tend(G, sns, td, W, rk, st);
         if (sizeof(TW) == sizeof(double)) col::ver_waves(G, so, snr, sn, td, M->K, rk, st);
         else col::ver_waves(G, so, snr, sn, td, (const float *)td_wind, M->K, rk, st);
@@ -575,7 +600,7 @@ static int step_t(const WK &W, TW *td_wind, double dt, int first, const StepTape
                 /* the first substep's tracer solve (and sediment heat) on the
                    side stream: it writes only the tracer densities and the
                    sediment heat, which the second substep's PV chain does not
-                   read; its pressure-gradient kernel, which reads all the
+                   read; the tendency at the w points, which reads all the
                    densities, follows on the side stream */
                 HIP_OK(hipEventRecord(M->ev_fork, st));
                 HIP_OK(hipStreamWaitEvent(M->side, M->ev_fork, 0));
