@@ -398,9 +398,132 @@ __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const d
 }
 
 /* ------------------------------------------------------------------ */
-/* batched three-band solve and its adjoint (one column per lane;        */
-/* element j of column k at j*ncol + k, so lanes read consecutive words) */
+/* batched three-band solve and its adjoint (element j of column k at    */
+/* j*ncol + k, so lanes read consecutive words)                          */
 /* ------------------------------------------------------------------ */
+/* One column per lane with its quotients and solution in LDS (systems of at
+   most TL_ROWS rows): the rows of the next batch are loaded while the lane
+   eliminates the current ones, so a wave has 32 row loads in flight where the
+   walking kernel below waits for four at every row, and the quotients and the
+   intermediate solution cost no traffic.  Each block is one wave of `lanes`
+   columns, 64 up to 64 rows and 32 beyond, which keeps its LDS within 64 KiB.
+   Bound by memory for many columns and by the recurrence's divisions for few
+   (batches of 16 rows gain nothing, and staging a block's rows in LDS for one
+   lane per column, 67 and 114 us at 163,842 columns, less).  us per solve and
+   per adjoint, walking and here: 26 rows of 163,842 columns 183 together -> 39
+   and 58 (4.3 and 5.3 TB/s), 55 rows of 10,243 columns 77 and 105 -> 17 and
+   20.  All rows of a column are read before
+   any output of it is written, and each value is formed as the walking kernel
+   forms it. */
+#define TL_ROWS 128
+#define TL_B 8
+static int tl_lanes(int n) { return n <= 64 ? 64 : 32; }
+/* rows j0 .. j0 + TL_B - 1 of column k: lo[j - 1], d[j], up[j], r[j]; rows that
+   the system does not have repeat its last, and a single row has no bands */
+struct TlRows { double lo[TL_B], d[TL_B], up[TL_B], r[TL_B]; };
+__device__ __forceinline__ TlRows tl_load(const double *lo, const double *d, const double *up, const double *r, int n,
+                                          int ncol, int j0, unsigned k)
+{
+    TlRows x;
+#pragma unroll
+    for (int t = 0; t < TL_B; ++t) {
+        const int j = j0 + t < n ? j0 + t : n - 1, jl = j > 0 ? j - 1 : 0, ju = j < n - 1 ? j : jl;
+        x.lo[t] = n > 1 ? at(lo + (i64)jl*ncol, k) : 0.0;
+        x.up[t] = n > 1 ? at(up + (i64)ju*ncol, k) : 0.0;
+        x.d[t] = at(d + (i64)j*ncol, k);
+        x.r[t] = at(r + (i64)j*ncol, k);
+    }
+    return x;
+}
+
+/* column_solvers.c:641-667 downwards; quotients and solution to this lane's
+   LDS columns q and s (stride lanes) */
+__device__ __forceinline__ void tl_down(const double *lo, const double *d, const double *up, const double *r, int n,
+                                        int ncol, unsigned k, double *q, double *s, int lanes)
+{
+    TlRows cur = tl_load(lo, d, up, r, n, ncol, 0, k);
+    double ep = 0.0, x = 0.0;
+    for (int j0 = 0; j0 < n; j0 += TL_B) {
+        const TlRows nxt = tl_load(lo, d, up, r, n, ncol, j0 + TL_B < n ? j0 + TL_B : j0, k);
+#pragma unroll
+        for (int t = 0; t < TL_B; ++t) {
+            const int j = j0 + t;
+            if (j < n) {
+                if (j == 0) {
+                    if (n > 1) ep = cur.up[t]/cur.d[t];
+                    x = cur.r[t]/cur.d[t];
+                } else {
+                    const double den = cur.d[t] - ep*cur.lo[t];
+                    x = (cur.r[t] - x*cur.lo[t])/den;
+                    if (j < n - 1) ep = cur.up[t]/den;
+                }
+                q[j*lanes] = ep;
+                s[j*lanes] = x;
+            }
+        }
+        cur = nxt;
+    }
+}
+
+__global__ void __launch_bounds__(64) k_thomas_lds(int n, int ncol, const double *c, const double *d, const double *e,
+                                                   const double *r, double *x)
+{
+    extern __shared__ double lds[];
+    const int lanes = (int)blockDim.x;
+    const unsigned k = xcd_x()*blockDim.x + threadIdx.x;
+    if (k >= (unsigned)ncol) return;
+    double *q = lds + threadIdx.x, *s = q + n*lanes;
+    tl_down(c, d, e, r, n, ncol, k, q, s, lanes);
+    double xj = 0.0;
+#pragma unroll 4
+    for (int j = n - 1; j >= 0; --j) {
+        xj = j == n - 1 ? s[j*lanes] : s[j*lanes] - q[j*lanes]*xj;
+        put(x + (i64)j*ncol, k, xj);
+    }
+}
+
+/* the transposed solve A^T rb = xb (sub-diagonal e, super-diagonal c) and the
+   band cotangents -rb x^T */
+__global__ void __launch_bounds__(64) k_thomas_adj_lds(int n, int ncol, const double *c, const double *d, const double *e,
+                                                       const double *x, const double *xb, double *rb, double *cb,
+                                                       double *db, double *eb)
+{
+    extern __shared__ double lds[];
+    const int lanes = (int)blockDim.x;
+    const unsigned k = xcd_x()*blockDim.x + threadIdx.x;
+    if (k >= (unsigned)ncol) return;
+    double *q = lds + threadIdx.x, *s = q + n*lanes;
+    tl_down(e, d, c, xb, n, ncol, k, q, s, lanes);
+    /* upwards, the solution's rows loaded TL_B ahead */
+    auto load = [&](int j1, double *y) {
+#pragma unroll
+        for (int t = 0; t < TL_B; ++t) y[t] = at(x + (i64)(j1 - t > 0 ? j1 - t : 0)*ncol, k);
+    };
+    double cur[TL_B], nxt[TL_B], rj = 0.0, xj = 0.0;
+    load(n - 1, cur);
+    for (int j1 = n - 1; j1 >= 0; j1 -= TL_B) {
+        load(j1 - TL_B > 0 ? j1 - TL_B : 0, nxt);
+#pragma unroll
+        for (int t = 0; t < TL_B; ++t) {
+            const int j = j1 - t;
+            if (j >= 0) {
+                const double r1 = rj, x1 = xj;   /* row j + 1 */
+                rj = j == n - 1 ? s[j*lanes] : s[j*lanes] - q[j*lanes]*rj;
+                xj = cur[t];
+                put(rb + (i64)j*ncol, k, rj);
+                put(db + (i64)j*ncol, k, -rj*xj);
+                if (j < n - 1) {
+                    put(cb + (i64)j*ncol, k, -r1*xj);
+                    put(eb + (i64)j*ncol, k, -rj*x1);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TL_B; ++t) cur[t] = nxt[t];
+    }
+}
+
+/* one column per lane, for systems of more rows */
 __global__ void __launch_bounds__(ATPB) k_thomas(int n, int ncol, const double *c, const double *d, const double *e,
                                                  const double *r, double *x, double *ep)
 {
@@ -495,11 +618,29 @@ void inner_product_adjoint(const DevGrid &G, const AdjTables &A, const double *b
 
 void thomas(int n, int ncol, const double *c, const double *d, const double *e, const double *r, double *x,
             double *work, hipStream_t st)
-{ LAUNCH("k_thomas", k_thomas, AGRID(ncol), dim3(ATPB), st, n, ncol, c, d, e, r, x, work); }
+{
+    if (n > TL_ROWS) {
+        LAUNCH("k_thomas", k_thomas, AGRID(ncol), dim3(ATPB), st, n, ncol, c, d, e, r, x, work);
+        return;
+    }
+    const int lanes = tl_lanes(n);
+    const dim3 g((unsigned)((ncol + lanes - 1)/lanes)), b((unsigned)lanes);
+    const size_t lds = (size_t)2*n*lanes*sizeof(double);
+    LAUNCH_SHM("k_thomas", k_thomas_lds, g, b, lds, st, n, ncol, c, d, e, r, x);
+}
 
 void thomas_adjoint(int n, int ncol, const double *c, const double *d, const double *e, const double *x,
                     const double *xb, double *rb, double *cb, double *db, double *eb, double *work, hipStream_t st)
-{ LAUNCH("k_thomas_adj", k_thomas_adj, AGRID(ncol), dim3(ATPB), st, n, ncol, c, d, e, x, xb, rb, cb, db, eb, work); }
+{
+    if (n > TL_ROWS) {
+        LAUNCH("k_thomas_adj", k_thomas_adj, AGRID(ncol), dim3(ATPB), st, n, ncol, c, d, e, x, xb, rb, cb, db, eb, work);
+        return;
+    }
+    const int lanes = tl_lanes(n);
+    const dim3 g((unsigned)((ncol + lanes - 1)/lanes)), b((unsigned)lanes);
+    const size_t lds = (size_t)2*n*lanes*sizeof(double);
+    LAUNCH_SHM("k_thomas_adj", k_thomas_adj_lds, g, b, lds, st, n, ncol, c, d, e, x, xb, rb, cb, db, eb);
+}
 
 }  // namespace adj
 

@@ -17,58 +17,12 @@
 #define TPB 256
 #define GRID1(n) dim3((unsigned)(((n) + TPB - 1)/TPB))
 
-/* Workgroups are dispatched to the eight XCDs round-robin (workgroup i on
-   XCD i % 8), each XCD with its own L2.  The gather kernels renumber their
-   workgroups so that each XCD takes one contiguous range of the grid (x, the
-   horizontal blocks, fastest; then y, the chunks of layers): the neighbour
-   data a workgroup shares with the next one then sits in the same L2 instead
-   of being fetched by several XCDs.  Giving each XCD an eighth of x in every
-   chunk instead, so that the chunks share its tables, was slower (moist
-   scalar transport 389 -> 445 us at res 7 x 26).  Span carries the layers per
-   chunk and the reciprocal of gridDim.x: with divisions in the kernels (this
-   one, and 64-bit ones in the layer split) a wave spent over 300 scalar
-   instructions before its first load. */
-#define N_XCD 8u
-struct Span { int run; unsigned rcp; };
-struct Blk { unsigned x, y; };
-__device__ __forceinline__ unsigned xcd_linear(unsigned lin, unsigned T)
-{
-    const unsigned q = T/N_XCD, r = T%N_XCD, x = lin%N_XCD, k = lin/N_XCD;
-    return (x < r) ? x*(q + 1) + k : r*(q + 1) + (x - r)*q + k;
-}
-__device__ __forceinline__ Blk xcd_block(Span sp)
-{
-    const unsigned m = xcd_linear(blockIdx.y*gridDim.x + blockIdx.x, gridDim.x*gridDim.y);
-    /* rcp = ceil(2^32/gridDim.x) overestimates the quotient by one at most (m*gridDim.x < 2^32) */
-    Blk b;
-    b.y = __umulhi(m, sp.rcp);
-    b.x = m - b.y*gridDim.x;
-    if ((int)b.x < 0) { --b.y; b.x += gridDim.x; }
-    return b;
-}
-/* the same renumbering of a one-dimensional grid */
-__device__ __forceinline__ unsigned xcd_x() { return xcd_linear(blockIdx.x, gridDim.x); }
 /* grid of n horizontal elements in `chunks` chunks, and its Span for `layers` layers or levels */
 static dim3 grid_of(int n, int chunks) { return dim3((unsigned)((n + TPB - 1)/TPB), (unsigned)chunks); }
 static Span span_of(int n, int layers, int chunks)
 {
     const unsigned gx = (unsigned)((n + TPB - 1)/TPB);
     return Span{(layers + chunks - 1)/chunks, gx > 1 ? (unsigned)(((1ULL << 32) + gx - 1)/gx) : 0xffffffffu};
-}
-
-/* element i of a row whose address is the same for the whole wave: the row's
-   base stays in scalar registers and the lane adds a 32-bit byte offset, so a
-   load costs one instruction and the offset is shared by every row read at
-   the same index (a 64-bit element index takes an address pair per load) */
-template <typename T>
-__device__ __forceinline__ T at(const T *row, unsigned i)
-{
-    return *(const T *)((const char *)row + (size_t)(i*(unsigned)sizeof(T)));
-}
-template <typename T>
-__device__ __forceinline__ void put(T *row, unsigned i, T v)
-{
-    *(T *)((char *)row + (size_t)(i*(unsigned)sizeof(T))) = v;
 }
 
 /* layers [l0, l1) of a chunk when n layers are split into chunks of `run`;
@@ -1266,43 +1220,6 @@ __global__ void __launch_bounds__(128) k_ver_waves(DevGrid G, DevState so, DevSt
         tin_m = tin_j;
         rho_new_m = rho_n;
         rio_m = rio_j;
-    }
-}
-
-/* Thomas algorithm (column_solvers.c:641-667) on rows j*NCOL + col of LDS
-   arrays c, d, e, r (n rows): the multipliers overwrite e, the solution r.
-   The next row is read before the current one is written, so each step
-   waits on its division chain only, not on an LDS round trip. */
-template <int NCOL>
-__device__ __forceinline__ void thomas_lds(const double *cc, const double *dd, double *ee, double *rr, int n, int col)
-{
-    double ep = 0.0, x;
-    const double d0 = dd[col];
-    if (n > 1) ep = ee[col]/d0;
-    x = rr[col]/d0;
-    ee[col] = ep; rr[col] = x;
-    double cp = cc[col], dn = 0.0, en = 0.0, rn = 0.0;
-    if (n > 1) { dn = dd[NCOL + col]; en = ee[NCOL + col]; rn = rr[NCOL + col]; }
-#pragma unroll 4
-    for (int j = 1; j < n; ++j) {
-        const int o = j*NCOL + col, on = (j + 1 < n ? j + 1 : j)*NCOL + col;
-        const double cpn = cc[o], dnn = dd[on], enn = ee[on], rnn = rr[on];
-        const double den = dn - ep*cp;
-        if (j < n - 1) ep = en/den;
-        x = (rn - x*cp)/den;
-        ee[o] = ep; rr[o] = x;
-        cp = cpn; dn = dnn; en = enn; rn = rnn;
-    }
-    /* back substitution, upwards */
-    double eb = 0.0, rb = 0.0;
-    if (n > 1) { eb = ee[(n - 2)*NCOL + col]; rb = rr[(n - 2)*NCOL + col]; }
-#pragma unroll 4
-    for (int j = n - 2; j >= 0; --j) {
-        const int o = j*NCOL + col, om = (j > 0 ? j - 1 : 0)*NCOL + col;
-        const double ebn = ee[om], rbn = rr[om];
-        x = rb - eb*x;
-        rr[o] = x;
-        eb = ebn; rb = rbn;
     }
 }
 

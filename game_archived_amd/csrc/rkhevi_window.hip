@@ -461,10 +461,14 @@ static void ver_waves_adjoint(const sadj::VwArgs &a, hipStream_t st)
     const i64 ni = (i64)(G.L - 1)*G.nsh;
     launch("k_vw_layer_fwd", sadj::VwLayerFwd{a}, G.s, st);
     launch("k_vw_iface_fwd", sadj::VwIfaceFwd{a}, ni, st);
-    launch("k_vw_solve", sadj::VwSolve{a, 0}, G.nsh, st);
+    auto band = [&](int k) { return a.ws + (i64)k*G.L*G.nsh; };
+    adj::thomas(G.L - 1, G.nsh, band(sadj::VW_C), band(sadj::VW_D), band(sadj::VW_E), band(sadj::VW_R), band(sadj::VW_X),
+                nullptr, st);   /* at most 62 rows: no work array */
     launch("k_vw_layer_new", sadj::VwLayerNew{a}, G.s, st);
     launch("k_vw_iface_sol_bar", sadj::VwIfaceSolBar{a}, ni, st);
-    launch("k_vw_solve_t", sadj::VwSolve{a, 1}, G.nsh, st);
+    /* the transposed system: e below the diagonal, c above it */
+    adj::thomas(G.L - 1, G.nsh, band(sadj::VW_E), band(sadj::VW_D), band(sadj::VW_C), band(sadj::VW_BX), band(sadj::VW_BR),
+                nullptr, st);
     launch("k_vw_iface_bar", sadj::VwIfaceBar{a}, ni, st);
     launch("k_vw_layer_bar", sadj::VwLayerBar{a}, G.s, st);
 }

@@ -57,8 +57,8 @@ GAME_HD inline void split_index(i64 t, int n, int &q, int &r)
 /*   then rho, rt, w, tp, ep of the new state.                          */
 /* The reverse runs as seven launches: the per-layer coefficients       */
 /* (VwLayerFwd), the per-interface bands (VwIfaceFwd), the solve        */
-/* (VwSolve, one thread per column), the cotangent of the solution      */
-/* (VwIfaceSolBar), the transposed solve (VwSolveT), the interface      */
+/* (adj::thomas), the cotangent of the solution                          */
+/* (VwIfaceSolBar), the transposed solve (adj::thomas), the interface    */
 /* cotangents (VwIfaceBar) and the per-layer cotangents (VwLayerBar).   */
 /* Every launch but the two solves has one thread per (layer, column)   */
 /* or (interface, column), and every contribution an interface makes to */
@@ -66,7 +66,7 @@ GAME_HD inline void split_index(i64 t, int n, int &q, int &r)
 /* writers.  The workspace holds VW_N arrays of L doubles per column,   */
 /* array k of column c element j at (k*L + j)*ncol + c.                 */
 /* ------------------------------------------------------------------ */
-enum { VW_AL, VW_BE, VW_GA, VW_TIN, VW_C, VW_D, VW_E, VW_R, VW_X, VW_EP, VW_BX, VW_BR, VW_BTIN, VW_BRIO,
+enum { VW_AL, VW_BE, VW_GA, VW_TIN, VW_C, VW_D, VW_E, VW_R, VW_X, VW_BX, VW_BR, VW_BTIN, VW_BRIO,
        VW_RN, VW_RTN, VW_BRE, VW_BRTE, VW_N };
 
 struct VwArgs {
@@ -235,37 +235,6 @@ struct VwLayerNew {
         a.W(VW_RTN, j, c) = rtn;
         a.W(VW_BRE, j, c) = bre;
         a.W(VW_BRTE, j, c) = brte;
-    }
-};
-
-/* Thomas algorithm of column_solvers.c:641-667: A x = r (bands c below,
-   d, e above) or, with transpose, A^T x = r (e below, c above); the
-   quotients go to VW_EP */
-struct VwSolve {
-    VwArgs a;
-    int transpose;
-    GAME_HD void operator()(i64 t) const
-    {
-        if (t >= a.G.nsh) return;
-        const int c = (int)t, n = a.G.L - 1;
-        const int lo_b = transpose ? VW_E : VW_C, up_b = transpose ? VW_C : VW_E;
-        const int rhs = transpose ? VW_BX : VW_R, out = transpose ? VW_BR : VW_X;
-        double ep = n > 1 ? a.W(up_b, 0, c)/a.W(VW_D, 0, c) : 0.0, rp = a.W(rhs, 0, c)/a.W(VW_D, 0, c);
-        a.W(VW_EP, 0, c) = ep;
-        a.W(out, 0, c) = rp;
-        for (int j = 1; j < n; ++j) {
-            const double lo = a.W(lo_b, j - 1, c);
-            const double den = a.W(VW_D, j, c) - ep*lo;
-            rp = (a.W(rhs, j, c) - rp*lo)/den;
-            if (j < n - 1) ep = a.W(up_b, j, c)/den;
-            a.W(VW_EP, j, c) = ep;
-            a.W(out, j, c) = rp;
-        }
-        double x = rp;
-        for (int j = n - 2; j >= 0; --j) {
-            x = a.W(out, j, c) - a.W(VW_EP, j, c)*x;
-            a.W(out, j, c) = x;
-        }
     }
 };
 
