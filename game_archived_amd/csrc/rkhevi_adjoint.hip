@@ -22,58 +22,52 @@
 #include "rkhevi_dev.h"
 #include "rkhevi_adjoint.h"
 
-#define ATPB 256
+#define ATPB TPB
 #define AGRID(n) dim3((unsigned)(((n) + ATPB - 1)/ATPB))
-/* kernels that walk layers: one thread per (cell or edge, chunk of layers) */
-#define ACHUNKS 4
-#define AGRID2(n) dim3((unsigned)(((n) + ATPB - 1)/ATPB), ACHUNKS)
-
-__device__ __forceinline__ void adj_chunk(int n, int &l0, int &l1)
-{
-    l0 = (int)(((i64)n*blockIdx.y)/gridDim.y);
-    l1 = (int)(((i64)n*(blockIdx.y + 1))/gridDim.y);
-}
 
 /* ------------------------------------------------------------------ */
 /* grad^T: fbar(c, l) from gbar at the cell's edges and w points        */
 /* ------------------------------------------------------------------ */
-__global__ void __launch_bounds__(ATPB) k_grad_adj(DevGrid G, AdjTables A, const double *gb, double *fb, double gs,
-                                                   int acc)
+__global__ void __launch_bounds__(ATPB) k_grad_adj(DevGrid G, const double *gb, double *fb, double gs, int acc, Span sp)
 {
     /* the input is gs*gb, formed as it is loaded; acc adds the result to fb */
     /* one thread per (cell, chunk of layers): layer l's edge cotangents feed
        the horizontal term of layer l and the terrain terms of the w points
        l (ipw slot 6) and l + 1 (slot 7); each w point's cotangent is formed
        once and carried to the next layer */
-    const int h = blockIdx.x*ATPB + threadIdx.x;
-    if (h >= G.nsh) return;
+    const Blk bk = linear_block();
+    const unsigned h = bk.x*ATPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
     const int nsh = G.nsh, vpl = G.vpl, L = G.L, top = G.flat ? L : L - G.n_oro;
     const int ne = h < GAME_N_PENT ? 5 : 6;
-    int ej[6];
-    double sg[6];
+    unsigned ej[6];
+    const unsigned from = at(G.c_from, h);
 #pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        const int jj = j < ne ? j : 0;
-        ej[j] = G.adj[6*h + jj];
-        sg[j] = j < ne ? (double)G.sgn[6*h + jj] : 0.0;
-    }
+    for (int j = 0; j < 6; ++j) ej[j] = at(G.c_e + (i64)j*nsh, h);
     int l0, l1;
-    adj_chunk(L, l0, l1);
+    layer_chunk(L, bk.y, sp.run, l0, l1);
+    if (l0 >= l1) return;
     /* layer l: the horizontal sum and the two terrain sums */
     auto layer = [&](int l, double &hs, double &s6, double &s7) {
-        double g[6], sl[6];
+        double g[6], sl[6], nd[6];
+        const i64 vi = nsh + (i64)l*vpl;
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            const i64 vi = nsh + (i64)l*vpl + ej[j];
-            g[j] = gs*gb[vi];
-            sl[j] = (l >= top) ? G.slope[vi] : 0.0;
-            /* g_e = (f_to - f_from)/d_e: the from-cell (sign +1) gets -1/d_e */
-            if (j == 0) hs = 0.0;
-            hs += -sg[j]*g[j]/G.nd[vi];
+            g[j] = gs*at(gb + vi, ej[j]);
+            sl[j] = (l >= top) ? at(G.slope + vi, ej[j]) : 0.0;
+            nd[j] = at(G.nd + vi, ej[j]);
+        }
+        hs = 0.0;
+        /* g_e = (f_to - f_from)/d_e: the from-cell (sign +1) gets -1/d_e */
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            const double sg = j < ne ? ((from >> j) & 1u ? 1.0 : -1.0) : 0.0;
+            hs += -sg*g[j]/nd[j];
         }
         s6 = 0.0; s7 = 0.0;
         if (l >= top) {
-            const double w6 = G.ipw[8*((i64)l*nsh + h) + 6], w7 = G.ipw[8*((i64)l*nsh + h) + 7];
+            const double *wl = G.ipwT + ((i64)l*8 + 6)*nsh;
+            const double w6 = at(wl, h), w7 = at(wl + nsh, h);
 #pragma unroll
             for (int j = 0; j < 6; ++j) {
                 if (j < ne) {
@@ -85,8 +79,8 @@ __global__ void __launch_bounds__(ATPB) k_grad_adj(DevGrid G, AdjTables A, const
     };
     /* the cotangent of the vertical gradient at w point lev over its normal distance */
     auto wcot = [&](int lev, double s6, double s7_above) {
-        double r = gs*gb[h + (i64)lev*vpl] + s6 + s7_above;
-        return r/G.nd[h + (i64)lev*vpl];
+        double r = gs*at(gb + (i64)lev*vpl, h) + s6 + s7_above;
+        return r/at(G.nd + (i64)lev*vpl, h);
     };
     double hs, s6, s7, s7p = 0.0, unused_h, unused_s6;
     if (l0 >= 1) layer(l0 - 1, unused_h, unused_s6, s7p);
@@ -99,8 +93,8 @@ __global__ void __launch_bounds__(ATPB) k_grad_adj(DevGrid G, AdjTables A, const
             wn = wcot(l + 1, s6n, s7);
         }
         const double v = hs + wn - wc;
-        const i64 o = (i64)l*nsh + h;
-        fb[o] = acc ? fb[o] + v : v;
+        double *row = fb + (i64)l*nsh;
+        put(row, h, acc ? at(row, h) + v : v);
         hs = hn; s7 = s7n; wc = wn;
     }
 }
@@ -108,60 +102,137 @@ __global__ void __launch_bounds__(ATPB) k_grad_adj(DevGrid G, AdjTables A, const
 /* ------------------------------------------------------------------ */
 /* divv_h and divv_h^T                                                   */
 /* ------------------------------------------------------------------ */
-__global__ void __launch_bounds__(ATPB) k_divv(DevGrid G, const double *in, double *out)
+/* divergences.c:14-64 with averaging.c:41-95, one thread per cell and chunk of
+   layers.  The correction at terrain level lev sums the cell's edge terms of
+   layer lev - 1 and then of layer lev, from zero (from layer lev alone at the
+   top one): layer lev - 1's running sum is carried, so each layer's edges are
+   read once (170 -> 63 us at res 6 x 26 over the mountain against forming
+   both corrections of every box from ipw and slope) */
+template <bool FLAT>
+__global__ void __launch_bounds__(ATPB) k_divv(DevGrid G, const double *in, double *out, Span sp)
 {
-    i64 t = (i64)blockIdx.x*ATPB + threadIdx.x;
-    if (t >= G.s) return;
-    const int l = (int)(t/G.nsh), h = (int)(t - (i64)l*G.nsh);
-    if (!G.flat) { out[t] = divv_h_cell(G, in, l, h); return; }
-    /* flat surface: the terrain terms are zero; the six edges load in one batch
-       (a pentagon's sixth slot reads its first edge and adds -0.0) */
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*ATPB + threadIdx.x;
+    if (h >= (unsigned)G.nsh) return;
+    const int nsh = G.nsh, vpl = G.vpl, L = G.L, top = FLAT ? L : L - G.n_oro;
     const int ne = h < GAME_N_PENT ? 5 : 6;
-    double v[6], a[6], sg[6];
+    /* a fixed six edges: a pentagon's sixth slot reads its first edge and adds
+       -0.0, the exact identity of IEEE addition */
+    unsigned ej[6];
+    const unsigned from = at(G.c_from, h);
 #pragma unroll
-    for (int j = 0; j < 6; ++j) {
-        const int jj = j < ne ? j : 0;
-        const i64 vi = G.nsh + (i64)l*G.vpl + G.adj[6*h + jj];
-        v[j] = in[vi]; a[j] = G.area[vi]; sg[j] = (double)G.sgn[6*h + jj];
-    }
-    double comp_h = 0.0;
+    for (int j = 0; j < 6; ++j) ej[j] = at(G.c_e + (i64)j*nsh, h);
+    int l0, l1;
+    layer_chunk(L, bk.y, sp.run, l0, l1);
+    if (l0 >= l1) return;
+    /* layer l's edges; its horizontal sum, and its terrain terms added to both
+       the correction at level l (cu) and the start of that at level l + 1 (cn) */
+    auto layer = [&](int l, double &cu, double &cn) {
+        const i64 vi = nsh + (i64)l*vpl;
+        double v[6], a[6], c[6];
 #pragma unroll
-    for (int j = 0; j < 6; ++j) comp_h += j < ne ? v[j]*sg[j]*a[j] : -0.0;
-    out[t] = 1.0/G.vol[t]*comp_h;
-}
-
-/* cotangent of the vertical contravariant correction vcc(c, lev), lev in
-   [L - n_oro, L - 1]: it enters layer lev with +area_w(lev) and layer lev - 1
-   with -area_w(lev) (divergences.c:41-59) */
-__device__ __forceinline__ double vcc_cot(const DevGrid &G, const double *db, int c, int lev)
-{
-    i64 s0 = (i64)lev*G.nsh + c, s1 = s0 - G.nsh;
-    double a = G.area[c + (i64)lev*G.vpl];
-    return db[s0]/G.vol[s0]*a - db[s1]/G.vol[s1]*a;
-}
-
-__global__ void __launch_bounds__(ATPB) k_divv_adj(DevGrid G, AdjTables A, const double *db, double *Fb)
-{
-    i64 t = (i64)blockIdx.x*ATPB + threadIdx.x;
-    if (t >= G.v) return;
-    const int nsh = G.nsh, vpl = G.vpl, L = G.L, no = G.n_oro;
-    const int l = (int)(t/vpl), h = (int)(t - (i64)l*vpl);
-    if (h < nsh) { Fb[t] = 0.0; return; }   /* divv_h reads horizontal components only */
-    const int e = h - nsh;
-    const int fr = G.from[e], to = G.to[e];
-    const i64 sf = (i64)l*nsh + fr, st = (i64)l*nsh + to;
-    double r = G.area[t]*(db[sf]/G.vol[sf] - db[st]/G.vol[st]);
-    if (!G.flat && l >= L - no) {
-        const int cell[2] = {fr, to}, slot[2] = {A.slot_from[e], A.slot_to[e]};
-        for (int p = 0; p < 2; ++p) {
-            const int c = cell[p];
-            double k = -0.5*G.ipw[8*((i64)l*nsh + c) + slot[p]]*G.slope[t];
-            double v = vcc_cot(G, db, c, l);
-            if (l + 1 <= L - 1) v += vcc_cot(G, db, c, l + 1);
-            r += k*v;
+        for (int j = 0; j < 6; ++j) {
+            v[j] = at(in + vi, ej[j]);
+            a[j] = at(G.area + vi, ej[j]);
+            c[j] = 0.0;
+            if (!FLAT && l >= top) c[j] = at(G.vcw + ((i64)(l - top)*6 + j)*nsh, h);
         }
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            const double t = ((from >> j) & 1u ? v[j] : -v[j])*a[j];
+            s += j < ne ? t : -0.0;
+        }
+        if (!FLAT && l >= top) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j)
+                if (j < ne) {
+                    const double t = c[j]*v[j];
+                    cu += t;
+                    cn += t;
+                }
+        }
+        return s;
+    };
+    /* cu: the correction at the layer's upper level; cn: the next one's start */
+    double cu = 0.0, cn = 0.0;
+    if (!FLAT && l0 > top) { double unused = 0.0; layer(l0 - 1, unused, cu); }
+    double s = layer(l0, cu, cn);
+    for (int l = l0; l < l1; ++l) {
+        double cl = cn, cnn = 0.0, sn = 0.0;
+        if (l + 1 < L && (l + 1 < l1 || (!FLAT && l + 1 >= top))) sn = layer(l + 1, cl, cnn);
+        double comp = s;
+        if constexpr (!FLAT) {
+            double comp_v = 0.0;
+            if (l == top - 1) comp_v = -cl*at(G.area + (i64)(l + 1)*vpl, h);
+            else if (l == L - 1) comp_v = cu*at(G.area + (i64)l*vpl, h);
+            else if (l > top - 1) comp_v = cu*at(G.area + (i64)l*vpl, h) - cl*at(G.area + (i64)(l + 1)*vpl, h);
+            comp = s + comp_v;
+        }
+        put(out + (i64)l*nsh, h, 1.0/at(G.vol + (i64)l*nsh, h)*comp);
+        s = sn; cu = cl; cn = cnn;
     }
-    Fb[t] = r;
+}
+
+/* one thread per edge and chunk of layers; the cotangent of the vertical
+   contravariant correction vcc(c, lev), lev in [L - n_oro, L - 1], enters layer
+   lev with +area_w(lev) and layer lev - 1 with -area_w(lev)
+   (divergences.c:41-59): formed once per level and carried, as is each cell's
+   quotient by its volume */
+__global__ void __launch_bounds__(ATPB) k_divv_adj(DevGrid G, AdjTables A, const double *db, double *Fb, Span sp)
+{
+    const Blk bk = xcd_block(sp);
+    const unsigned t = bk.x*ATPB + threadIdx.x;
+    const int nsh = G.nsh, vpl = G.vpl, L = G.L, top = G.flat ? L : L - G.n_oro;
+    int l0, l1;
+    layer_chunk(L, bk.y, sp.run, l0, l1);
+    /* divv_h reads horizontal components only */
+    if (t < (unsigned)nsh) {
+        for (int l = l0; l < l1; ++l) put(Fb + (i64)l*vpl, t, 0.0);
+        if (l0 < l1 && l1 == L) put(Fb + (i64)L*vpl, t, 0.0);
+    }
+    if (t >= (unsigned)G.nvh || l0 >= l1) return;
+    const unsigned e = t, cell[2] = {(unsigned)G.from[e], (unsigned)G.to[e]};
+    const unsigned slot[2] = {(unsigned)G.flat ? 0u : (unsigned)A.slot_from[e], (unsigned)G.flat ? 0u : (unsigned)A.slot_to[e]};
+    double q[2], qm[2] = {0.0, 0.0}, vc[2] = {0.0, 0.0};   /* db/vol of this layer and the one above; vcc_cot at this layer's level */
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        q[p] = at(db + (i64)l0*nsh, cell[p])/at(G.vol + (i64)l0*nsh, cell[p]);
+        if (l0 >= 1) qm[p] = at(db + (i64)(l0 - 1)*nsh, cell[p])/at(G.vol + (i64)(l0 - 1)*nsh, cell[p]);
+    }
+    auto cot = [&](int lev, int p, double lo, double up) {
+        const double a = at(G.area + (i64)lev*vpl, cell[p]);
+        return lo*a - up*a;
+    };
+    if (l0 >= top) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) vc[p] = cot(l0, p, q[p], qm[p]);
+    }
+    for (int l = l0; l < l1; ++l) {
+        const i64 vi = nsh + (i64)l*vpl;
+        const int ln = l + 1 < L ? l + 1 : l;
+        double qn[2], vn[2] = {0.0, 0.0};
+#pragma unroll
+        for (int p = 0; p < 2; ++p) qn[p] = at(db + (i64)ln*nsh, cell[p])/at(G.vol + (i64)ln*nsh, cell[p]);
+        double r = at(G.area + vi, e)*(q[0] - q[1]);
+        if (l + 1 >= top && l + 1 <= L - 1) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p) vn[p] = cot(l + 1, p, qn[p], q[p]);
+        }
+        if (l >= top) {
+            const double *wl = G.vcw + (i64)(l - top)*6*nsh;
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const double k = at(wl, slot[p]*(unsigned)nsh + cell[p]);
+                double v = vc[p];
+                if (l + 1 <= L - 1) v += vn[p];
+                r += k*v;
+            }
+        }
+        put(Fb + vi, e, r);
+#pragma unroll
+        for (int p = 0; p < 2; ++p) { q[p] = qn[p]; vc[p] = vn[p]; }
+    }
 }
 
 /* ------------------------------------------------------------------ */
@@ -178,20 +249,20 @@ struct CurlAdjTerm {
     int d[2];            /* -1: the other term goes to l-1, +1: to l+1, 0: none */
 };
 
-__device__ __forceinline__ CurlAdjTerm curl_adj_term(const DevGrid &G, const double *zb, int e, const int *tri,
+__device__ __forceinline__ CurlAdjTerm curl_adj_term(const DevGrid &G, const double *zb, unsigned e, const unsigned *tri,
                                                      const double *sg, int l)
 {
     const int nsh = G.nsh, vpl = G.vpl, L = G.L;
-    const i64 vi = nsh + (i64)l*vpl + e;
+    const i64 vi = nsh + (i64)l*vpl;
     const i64 vu = l > 0 ? vi - vpl : vi, vd = l < L - 1 ? vi + vpl : vu;
-    const double nd = G.nd[vi], zv = G.zv[vi], zu = G.zv[vu], zd = G.zv[vd];
+    const double nd = at(G.nd + vi, e), zv = at(G.zv + vi, e), zu = at(G.zv + vu, e), zd = at(G.zv + vd, e);
     double z[2], da[2], dzv[2];
+    const i64 di = G.nvh + (i64)l*G.dvpl;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-        const i64 di = G.nvh + (i64)l*G.dvpl + tri[p];
-        z[p] = zb[(i64)l*G.nt + tri[p]];
-        da[p] = G.darea[di];
-        dzv[p] = G.dzv[di];
+        z[p] = at(zb + (i64)l*G.nt, tri[p]);
+        da[p] = at(G.darea + di, tri[p]);
+        dzv[p] = at(G.dzv + di, tri[p]);
     }
     CurlAdjTerm c;
 #pragma unroll
@@ -215,26 +286,27 @@ __device__ __forceinline__ CurlAdjTerm curl_adj_term(const DevGrid &G, const dou
     return c;
 }
 
-__global__ void __launch_bounds__(ATPB) k_curl_adj(DevGrid G, AdjTables A, const double *zb, double *wb, int acc)
+__global__ void __launch_bounds__(ATPB) k_curl_adj(DevGrid G, AdjTables A, const double *zb, double *wb, int acc, Span sp)
 {
     /* acc adds the edge cotangents to wb and leaves its w points; otherwise
        the w points are set to zero */
-    const int t = blockIdx.x*ATPB + threadIdx.x;
+    const Blk bk = xcd_block(sp);
+    const unsigned t = bk.x*ATPB + threadIdx.x;
     const int nsh = G.nsh, vpl = G.vpl, L = G.L;
     int l0, l1;
-    adj_chunk(L, l0, l1);
-    if (!acc && t < nsh) {
-        for (int l = l0; l < l1; ++l) wb[(i64)l*vpl + t] = 0.0;
-        if (l1 == L) wb[(i64)L*vpl + t] = 0.0;
+    layer_chunk(L, bk.y, sp.run, l0, l1);
+    if (!acc && t < (unsigned)nsh) {
+        for (int l = l0; l < l1; ++l) put(wb + (i64)l*vpl, t, 0.0);
+        if (l0 < l1 && l1 == L) put(wb + (i64)L*vpl, t, 0.0);
     }
-    if (t >= G.nvh) return;
-    const int e = t;
-    int tri[2];
+    if (t >= (unsigned)G.nvh || l0 >= l1) return;
+    const unsigned e = t;
+    unsigned tri[2];
     double sg[2];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-        tri[p] = A.tri_of_edge[2*e + p];
-        sg[p] = (double)G.vst[3*tri[p] + A.tri_slot[2*e + p]];
+        tri[p] = (unsigned)A.tri_of_edge[2*(i64)e + p];
+        sg[p] = at(G.t_e + (i64)A.tri_slot[2*(i64)e + p]*G.nt, tri[p]) >> 31 ? -1.0 : 1.0;
     }
     CurlAdjTerm prev = {}, cur = curl_adj_term(G, zb, e, tri, sg, l0), nxt = {};
     if (l0 >= 1) prev = curl_adj_term(G, zb, e, tri, sg, l0 - 1);
@@ -247,8 +319,8 @@ __global__ void __launch_bounds__(ATPB) k_curl_adj(DevGrid G, AdjTables A, const
             r += cur.s[p];
             if (lp + 1 <= L - 1 && nxt.d[p] == -1) r += nxt.o[p];
         }
-        const i64 o = nsh + (i64)lp*vpl + e;
-        wb[o] = acc ? wb[o] + r : r;
+        double *row = wb + nsh + (i64)lp*vpl;
+        put(row, e, acc ? at(row, e) + r : r);
         prev = cur;
         cur = nxt;
         if (lp + 2 <= L - 1 && lp + 1 < l1) nxt = curl_adj_term(G, zb, e, tri, sg, lp + 2);
@@ -258,34 +330,46 @@ __global__ void __launch_bounds__(ATPB) k_curl_adj(DevGrid G, AdjTables A, const
 /* ------------------------------------------------------------------ */
 /* rhombus density and its adjoint                                      */
 /* ------------------------------------------------------------------ */
-__global__ void __launch_bounds__(ATPB) k_rhombus(DevGrid G, const double *rho, double *out)
+__global__ void __launch_bounds__(ATPB) k_rhombus(DevGrid G, const double *rho, double *out, Span sp)
 {
-    i64 t = (i64)blockIdx.x*ATPB + threadIdx.x;
-    if (t >= (i64)G.L*G.nvh) return;
-    const int l = (int)(t/G.nvh), e = (int)(t - (i64)l*G.nvh);
-    double dr = 0.0;
-    for (int j = 0; j < 4; ++j) dr += G.drw[4*e + j]*rho[(i64)l*G.nsh + G.dri[4*e + j]];
-    out[t] = dr;
+    const Blk bk = xcd_block(sp);
+    const unsigned e = bk.x*ATPB + threadIdx.x;
+    if (e >= (unsigned)G.nvh) return;
+    unsigned c[4];
+    double w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { c[j] = at(G.e_rc + (i64)j*G.nvh, e); w[j] = at(G.e_rw + (i64)j*G.nvh, e); }
+    int l0, l1;
+    layer_chunk(G.L, bk.y, sp.run, l0, l1);
+    for (int l = l0; l < l1; ++l) {
+        const double *row = rho + (i64)l*G.nsh;
+        double dr = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) dr += w[j]*at(row, c[j]);
+        put(out + (i64)l*G.nvh, e, dr);
+    }
 }
 
-__global__ void __launch_bounds__(ATPB) k_rhombus_adj(DevGrid G, AdjTables A, const double *db, double *rb)
+__global__ void __launch_bounds__(ATPB) k_rhombus_adj(DevGrid G, AdjTables A, const double *db, double *rb, Span sp)
 {
     /* one thread per (cell, chunk of layers): the cell's rhombus entries are
        loaded once, in ascending (edge, slot) order, padding weighted 0 */
-    const int c = blockIdx.x*ATPB + threadIdx.x;
-    if (c >= G.nsh) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned c = bk.x*ATPB + threadIdx.x;
+    if (c >= (unsigned)G.nsh) return;
     const int nsh = G.nsh, nvh = G.nvh;
-    int e[ADJ_RH_MAX];
+    unsigned e[ADJ_RH_MAX];
     double w[ADJ_RH_MAX];
 #pragma unroll
-    for (int k = 0; k < ADJ_RH_MAX; ++k) { e[k] = A.rhp_e[(i64)k*nsh + c]; w[k] = A.rhp_w[(i64)k*nsh + c]; }
+    for (int k = 0; k < ADJ_RH_MAX; ++k) { e[k] = (unsigned)at(A.rhp_e + (i64)k*nsh, c); w[k] = at(A.rhp_w + (i64)k*nsh, c); }
     int l0, l1;
-    adj_chunk(G.L, l0, l1);
+    layer_chunk(G.L, bk.y, sp.run, l0, l1);
     for (int l = l0; l < l1; ++l) {
+        const double *row = db + (i64)l*nvh;
         double r = 0.0;
 #pragma unroll
-        for (int k = 0; k < ADJ_RH_MAX; ++k) r += w[k]*db[(i64)l*nvh + e[k]];
-        rb[(i64)l*nsh + c] = r;
+        for (int k = 0; k < ADJ_RH_MAX; ++k) r += w[k]*at(row, e[k]);
+        put(rb + (i64)l*nsh, c, r);
     }
 }
 
@@ -298,68 +382,82 @@ __device__ __forceinline__ double vflux_w_weight(const DevGrid &G, int lev)
 }
 
 __global__ void __launch_bounds__(ATPB) k_vflux_adj_e(DevGrid G, AdjTables A, const double *pv, const double *ob,
-                                                      double *Fb)
+                                                      double *Fb, Span sp)
 {
     /* horizontal F of edge e' at layer l, one thread per (edge, chunk of
        layers): its TRSK reverse entries are loaded once */
-    const int ep = blockIdx.x*ATPB + threadIdx.x;
-    if (ep >= G.nvh) return;
+    const Blk bk = xcd_block(sp);
+    const unsigned ep = bk.x*ATPB + threadIdx.x;
+    if (ep >= (unsigned)G.nvh) return;
     const int nsh = G.nsh, nvh = G.nvh, vpl = G.vpl;
-    int e[ADJ_TR_MAX], m[ADJ_TR_MAX];
+    unsigned e[ADJ_TR_MAX], m[ADJ_TR_MAX];
     bool hf[ADJ_TR_MAX];
     double w[ADJ_TR_MAX];
 #pragma unroll
     for (int k = 0; k < ADJ_TR_MAX; ++k) {
-        e[k] = A.trp_e[(i64)k*nvh + ep];
-        const int mm = A.trp_m[(i64)k*nvh + ep];
+        e[k] = (unsigned)at(A.trp_e + (i64)k*nvh, ep);
+        const int mm = at(A.trp_m + (i64)k*nvh, ep);
         hf[k] = mm < 0;
-        m[k] = mm < 0 ? -mm - 1 : mm;
-        w[k] = A.trp_w[(i64)k*nvh + ep];
+        m[k] = (unsigned)(mm < 0 ? -mm - 1 : mm);
+        w[k] = at(A.trp_w + (i64)k*nvh, ep);
     }
-    const int cell[2] = {G.from[ep], G.to[ep]}, slot[2] = {A.slot_from[ep], A.slot_to[ep]};
+    const unsigned cell[2] = {(unsigned)G.from[ep], (unsigned)G.to[ep]};
+    const unsigned sc[2] = {(unsigned)A.slot_from[ep]*(unsigned)nsh + cell[0], (unsigned)A.slot_to[ep]*(unsigned)nsh + cell[1]};
     int l0, l1;
-    adj_chunk(G.L, l0, l1);
+    layer_chunk(G.L, bk.y, sp.run, l0, l1);
+    if (l0 >= l1) return;
+    /* the vertical outputs of the edge's two cells and its own PV at level l, carried */
+    double q0 = at(pv + (i64)l0*2*nvh, ep), o0[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) o0[p] = at(ob + (i64)l0*vpl, cell[p]);
     for (int l = l0; l < l1; ++l) {
-        const i64 pb = nvh + (i64)l*2*nvh;
+        const double *pl = pv + nvh + (i64)l*2*nvh, *ol = ob + nsh + (i64)l*vpl;
+        double pm[ADJ_TR_MAX], pe[ADJ_TR_MAX], oe[ADJ_TR_MAX];
+#pragma unroll
+        for (int k = 0; k < ADJ_TR_MAX; ++k) { pm[k] = at(pl, m[k]); pe[k] = at(pl, e[k]); oe[k] = at(ol, e[k]); }
+        const double q1 = at(pl + nvh, ep);
+        double wt[2], o1[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            wt[p] = at(G.ipwT + (i64)l*8*nsh, sc[p]);
+            o1[p] = at(ob + (i64)(l + 1)*vpl, cell[p]);
+        }
         double r = 0.0;
 #pragma unroll
         for (int k = 0; k < ADJ_TR_MAX; ++k) {
-            const double pm = pv[pb + m[k]], pe = pv[pb + e[k]];
-            const double q = hf[k] ? 0.5*(pm + pe) : pm;
-            r += w[k]*q*ob[nsh + (i64)l*vpl + e[k]];
+            const double q = hf[k] ? 0.5*(pm[k] + pe[k]) : pm[k];
+            r += w[k]*q*oe[k];
         }
-        /* the vertical outputs of the edge's two cells at levels l and l + 1 */
-        const double q1 = pv[(i64)(l + 1)*2*nvh + ep], q0 = pv[(i64)l*2*nvh + ep];
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-            const int c = cell[p];
-            const double wt = G.ipwT[((i64)l*8 + slot[p])*nsh + c];
-            r += vflux_w_weight(G, l + 1)*wt*q1*ob[(i64)(l + 1)*vpl + c];
-            r += vflux_w_weight(G, l)*wt*q0*ob[(i64)l*vpl + c];
+            r += vflux_w_weight(G, l + 1)*wt[p]*q1*o1[p];
+            r += vflux_w_weight(G, l)*wt[p]*q0*o0[p];
         }
-        Fb[nsh + (i64)l*vpl + ep] = r;
+        put(Fb + nsh + (i64)l*vpl, ep, r);
+        q0 = q1; o0[0] = o1[0]; o0[1] = o1[1];
     }
 }
 
-__global__ void __launch_bounds__(ATPB) k_vflux_adj_w(DevGrid G, const double *pv, const double *ob, double *Fb)
+__global__ void __launch_bounds__(ATPB) k_vflux_adj_w(DevGrid G, const double *pv, const double *ob, double *Fb, Span sp)
 {
     /* vertical F of cell h at level l: the w terms of the cell's edges at
        layers l (ipw slot 6) and l - 1 (slot 7) (vorticity_flux.c:110-187);
        all loads first, layer indices clamped, out-of-range terms masked */
-    const i64 t = (i64)blockIdx.x*ATPB + threadIdx.x;
+    const Blk bk = xcd_block(sp);
+    const unsigned h = bk.x*ATPB + threadIdx.x;
     const int nsh = G.nsh, nvh = G.nvh, vpl = G.vpl, L = G.L;
-    if (t >= (i64)(L + 1)*nsh) return;
-    const int l = (int)(t/nsh), h = (int)(t - (i64)l*nsh);
+    if (h >= (unsigned)nsh) return;
+    const int l = (int)bk.y;
     const int ne = h < GAME_N_PENT ? 5 : 6;
     const int la = l <= L - 1 ? l : L - 1, lb = l >= 1 ? l - 1 : 0;
-    const double w6 = G.ipwT[((i64)la*8 + 6)*nsh + h], w7 = G.ipwT[((i64)lb*8 + 7)*nsh + h];
+    const double w6 = at(G.ipwT + ((i64)la*8 + 6)*nsh, h), w7 = at(G.ipwT + ((i64)lb*8 + 7)*nsh, h);
     double q[6], oa[6], obb[6];
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
-        const int e = G.adj[6*h + (j < ne ? j : 0)];
-        q[j] = pv[e + (i64)l*2*nvh];
-        oa[j] = ob[nsh + (i64)la*vpl + e];
-        obb[j] = ob[nsh + (i64)lb*vpl + e];
+        const unsigned e = at(G.c_e + (i64)j*nsh, h);
+        q[j] = at(pv + (i64)l*2*nvh, e);
+        oa[j] = at(ob + nsh + (i64)la*vpl, e);
+        obb[j] = at(ob + nsh + (i64)lb*vpl, e);
     }
     double r = 0.0;
 #pragma unroll
@@ -368,7 +466,7 @@ __global__ void __launch_bounds__(ATPB) k_vflux_adj_w(DevGrid G, const double *p
         if (l <= L - 1) r += -0.5*w6*q[j]*oa[j];
         if (l >= 1) r += -0.5*w7*q[j]*obb[j];
     }
-    Fb[(i64)l*vpl + h] = r;
+    put(Fb + (i64)l*vpl, h, r);
 }
 
 /* ------------------------------------------------------------------ */
@@ -377,24 +475,28 @@ __global__ void __launch_bounds__(ATPB) k_vflux_adj_w(DevGrid G, const double *p
 __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const double *b, const double *ib,
                                                  double *ab, double scale, int acc)
 {
-    /* acc: ab += scale*result; otherwise ab = result */
-    i64 t = (i64)blockIdx.x*ATPB + threadIdx.x;
-    if (t >= G.v) return;
-    const int nsh = G.nsh, vpl = G.vpl, L = G.L;
-    const int l = (int)(t/vpl), h = (int)(t - (i64)l*vpl);
-    double r = 0.0;
-    if (h >= nsh) {
-        const int e = h - nsh;
-        const int fr = G.from[e], to = G.to[e];
-        const i64 sf = (i64)l*nsh + fr, st = (i64)l*nsh + to;
-        r = b[t]*(G.ipw[8*sf + A.slot_from[e]]*ib[sf] + G.ipw[8*st + A.slot_to[e]]*ib[st]);
-    } else {
-        double s = 0.0;
-        if (l >= 1) s += G.ipw[8*((i64)(l - 1)*nsh + h) + 7]*ib[(i64)(l - 1)*nsh + h];
-        if (l <= L - 1) s += G.ipw[8*((i64)l*nsh + h) + 6]*ib[(i64)l*nsh + h];
-        r = b[t]*s;
+    /* acc: ab += scale*result; otherwise ab = result.  One thread per edge and
+       level, which does the cell of its number too */
+    const Blk bk = linear_block();
+    const unsigned t = bk.x*ATPB + threadIdx.x;
+    const int nsh = G.nsh, L = G.L, l = (int)bk.y;
+    const i64 row = (i64)l*G.vpl;
+    if (t < (unsigned)G.nvh && l < L) {
+        const unsigned fr = G.from[t], to = G.to[t];
+        const unsigned sf = (unsigned)A.slot_from[t]*(unsigned)nsh + fr, st = (unsigned)A.slot_to[t]*(unsigned)nsh + to;
+        const double *wl = G.ipwT + (i64)l*8*nsh, *il = ib + (i64)l*nsh;
+        const double old = acc ? at(ab + row + nsh, t) : 0.0;
+        const double r = at(b + row + nsh, t)*(at(wl, sf)*at(il, fr) + at(wl, st)*at(il, to));
+        put(ab + row + nsh, t, acc ? old + scale*r : r);
     }
-    ab[t] = acc ? ab[t] + scale*r : r;
+    if (t < (unsigned)nsh) {
+        const double old = acc ? at(ab + row, t) : 0.0;
+        double s = 0.0;
+        if (l >= 1) s += at(G.ipwT + ((i64)(l - 1)*8 + 7)*nsh, t)*at(ib + (i64)(l - 1)*nsh, t);
+        if (l <= L - 1) s += at(G.ipwT + ((i64)l*8 + 6)*nsh, t)*at(ib + (i64)l*nsh, t);
+        const double r = at(b + row, t)*s;
+        put(ab + row, t, acc ? old + scale*r : r);
+    }
 }
 
 /* ------------------------------------------------------------------ */
@@ -585,36 +687,45 @@ __global__ void __launch_bounds__(ATPB) k_thomas_adj(int n, int ncol, const doub
 /* ------------------------------------------------------------------ */
 namespace adj {
 
-void grad_adjoint(const DevGrid &G, const AdjTables &A, const double *gb, double *fb, hipStream_t st, double gs,
+/* the edge kernels also do the cells of their numbers, fewer than the edges (nvh = 3 nsh - 6) */
+#define CELL_GRID grid_of(G.nsh, G.split_adj_c)
+#define EDGE_GRID grid_of(G.nvh, G.split_adj_e)
+#define CELL_SPAN span_of(G.nsh, G.L, G.split_adj_c)
+#define EDGE_SPAN span_of(G.nvh, G.L, G.split_adj_e)
+
+void grad_adjoint(const DevGrid &G, const AdjTables &, const double *gb, double *fb, hipStream_t st, double gs,
                   int acc)
-{ LAUNCH("k_grad_adj", k_grad_adj, AGRID2(G.nsh), dim3(ATPB), st, G, A, gb, fb, gs, acc); }
+{ LAUNCH("k_grad_adj", k_grad_adj, CELL_GRID, dim3(ATPB), st, G, gb, fb, gs, acc, CELL_SPAN); }
 
 void divv_h(const DevGrid &G, const double *in, double *out, hipStream_t st)
-{ LAUNCH("k_divv", k_divv, AGRID(G.s), dim3(ATPB), st, G, in, out); }
+{
+    if (G.flat) LAUNCH("k_divv", k_divv<true>, CELL_GRID, dim3(ATPB), st, G, in, out, CELL_SPAN);
+    else LAUNCH("k_divv", k_divv<false>, CELL_GRID, dim3(ATPB), st, G, in, out, CELL_SPAN);
+}
 
 void divv_h_adjoint(const DevGrid &G, const AdjTables &A, const double *db, double *Fb, hipStream_t st)
-{ LAUNCH("k_divv_adj", k_divv_adj, AGRID(G.v), dim3(ATPB), st, G, A, db, Fb); }
+{ LAUNCH("k_divv_adj", k_divv_adj, EDGE_GRID, dim3(ATPB), st, G, A, db, Fb, EDGE_SPAN); }
 
 void curl_triangles_adjoint(const DevGrid &G, const AdjTables &A, const double *zb, double *wb, hipStream_t st,
                             int acc)
-{ LAUNCH("k_curl_adj", k_curl_adj, AGRID2(G.nvh > G.nsh ? G.nvh : G.nsh), dim3(ATPB), st, G, A, zb, wb, acc); }
+{ LAUNCH("k_curl_adj", k_curl_adj, EDGE_GRID, dim3(ATPB), st, G, A, zb, wb, acc, EDGE_SPAN); }
 
 void rhombus_density(const DevGrid &G, const double *rho, double *out, hipStream_t st)
-{ LAUNCH("k_rhombus", k_rhombus, AGRID((i64)G.L*G.nvh), dim3(ATPB), st, G, rho, out); }
+{ LAUNCH("k_rhombus", k_rhombus, EDGE_GRID, dim3(ATPB), st, G, rho, out, EDGE_SPAN); }
 
 void rhombus_density_adjoint(const DevGrid &G, const AdjTables &A, const double *db, double *rb, hipStream_t st)
-{ LAUNCH("k_rhombus_adj", k_rhombus_adj, AGRID2(G.nsh), dim3(ATPB), st, G, A, db, rb); }
+{ LAUNCH("k_rhombus_adj", k_rhombus_adj, CELL_GRID, dim3(ATPB), st, G, A, db, rb, CELL_SPAN); }
 
 void vorticity_flux_adjoint(const DevGrid &G, const AdjTables &A, const double *pv, const double *ob, double *Fb,
                             hipStream_t st)
 {
-    LAUNCH("k_vflux_adj_e", k_vflux_adj_e, AGRID2(G.nvh), dim3(ATPB), st, G, A, pv, ob, Fb);
-    LAUNCH("k_vflux_adj_w", k_vflux_adj_w, AGRID((i64)(G.L + 1)*G.nsh), dim3(ATPB), st, G, pv, ob, Fb);
+    LAUNCH("k_vflux_adj_e", k_vflux_adj_e, EDGE_GRID, dim3(ATPB), st, G, A, pv, ob, Fb, EDGE_SPAN);
+    LAUNCH("k_vflux_adj_w", k_vflux_adj_w, grid_of(G.nsh, G.L + 1), dim3(ATPB), st, G, pv, ob, Fb, span_of(G.nsh, 1, 1));
 }
 
 void inner_product_adjoint(const DevGrid &G, const AdjTables &A, const double *b, const double *ib, double *ab,
                            hipStream_t st, double scale, int acc)
-{ LAUNCH("k_ip_adj", k_ip_adj, AGRID(G.v), dim3(ATPB), st, G, A, b, ib, ab, scale, acc); }
+{ LAUNCH("k_ip_adj", k_ip_adj, grid_of(G.nvh, G.L + 1), dim3(ATPB), st, G, A, b, ib, ab, scale, acc); }
 
 void thomas(int n, int ncol, const double *c, const double *d, const double *e, const double *r, double *x,
             double *work, hipStream_t st)

@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 
 #define GAME_N_PENT 12
+/* threads per block of the kernels with one thread per element of a row */
+#define TPB 256
 #define GAME_MAX_LAYERS 64
 
 /* src/game_constants.h */
@@ -34,10 +36,10 @@ struct DevGrid {
     int flat;   /* slope == 0 everywhere: every terrain-correction term is an exact zero */
     i64 s, v, curl;
     double radius, toa;
-    const double *nd, *vol, *area, *zs, *zv, *phi, *gm, *slope, *thbg, *exbg, *exbg_grad, *ipw;
+    const double *nd, *vol, *area, *zs, *zv, *phi, *gm, *slope, *thbg, *exbg, *exbg_grad;
     /* the inner-product weights in layer-major, slot-major order, so that
        lanes of consecutive cells read consecutive addresses:
-       ipwT[(l*8 + j)*nsh + h] = ipw[8*(l*nsh + h) + j] */
+       ipwT[(l*8 + j)*nsh + h] is weight j of cell h in layer l */
     const double *ipwT;
     /* terrain grids: -0.5*ipw*slope of every cell's edges in the terrain
        layers, vcw[(k*6 + j)*nsh + h] for layer L - n_oro + k and slot j (the
@@ -73,6 +75,8 @@ struct DevGrid {
        flux; the gradients), per triangle, and of the terrain levels of the
        vertical corrections */
     int split_cell_w, split_edge, split_grad, split_tri, split_vcc;
+    /* the same of the operator adjoints' kernels, per cell and per edge */
+    int split_adj_c, split_adj_e;
     /* 1: tracer solver with one (column, tracer) per lane in registers; 0: LDS-staged */
     int gd_streaming;
     /* one tracer per block in the LDS-staged tracer solve instead of all five */
@@ -157,8 +161,30 @@ __device__ __forceinline__ Blk xcd_block(Span sp)
     if ((int)b.x < 0) { --b.y; b.x += gridDim.x; }
     return b;
 }
+/* the blocks as they are dispatched: for kernels that mostly stream, where eight
+   ranges far apart cost more than neighbours in one L2 give (us per launch,
+   renumbered and as dispatched: flat PV with the mass flux at res 7 x 26 270
+   and 240, mixed 226 and 202; but kinetic energy at res 6 31 and 34, vertical
+   corrections over the res 6 mountain 44 and 56, sound waves 198 and 228) */
+__device__ __forceinline__ Blk linear_block() { return Blk{blockIdx.x, blockIdx.y}; }
 /* the same renumbering of a one-dimensional grid */
 __device__ __forceinline__ unsigned xcd_x() { return xcd_linear(blockIdx.x, gridDim.x); }
+/* grid of n horizontal elements in `chunks` chunks, and its Span for `layers` layers or levels */
+static dim3 grid_of(int n, int chunks) { return dim3((unsigned)((n + TPB - 1)/TPB), (unsigned)chunks); }
+static Span span_of(int n, int layers, int chunks)
+{
+    const unsigned gx = (unsigned)((n + TPB - 1)/TPB);
+    return Span{(layers + chunks - 1)/chunks, gx > 1 ? (unsigned)(((1ULL << 32) + gx - 1)/gx) : 0xffffffffu};
+}
+
+/* layers [l0, l1) of a chunk when n layers are split into chunks of `run`;
+   the last chunk may be shorter (or empty) */
+__device__ __forceinline__ void layer_chunk(int n, unsigned chunk, int run, int &l0, int &l1)
+{
+    l0 = (int)chunk*run;
+    l1 = l0 + run < n ? l0 + run : n;
+}
+
 /* element i of a row whose address is the same for the whole wave: the row's
    base stays in scalar registers and the lane adds a 32-bit byte offset, so a
    load costs one instruction and the offset is shared by every row read at
@@ -246,57 +272,6 @@ __device__ __forceinline__ double c_p_water(double t)
         r = 1.000938 - 2.7052e-3*tc - 2.3235e-5*(tc*tc) + 4.3778e-6*(t2*tc) + 2.7136e-7*(t2*t2);
     }
     return 4186.8*r;
-}
-
-/* averaging.c:41-95 */
-__device__ __forceinline__ double vertical_contravariant_corr(const DevGrid &G, const double *f, int l, int h)
-{
-    double r = 0;
-    int ne = h < GAME_N_PENT ? 5 : 6;
-    if (l >= G.L - G.n_oro) {
-        if (l == G.L - G.n_oro) {
-            for (int i = 0; i < ne; ++i) {
-                i64 si = (i64)l*G.nsh + h, vi = G.nsh + (i64)l*G.vpl + G.adj[6*h + i];
-                r += -0.5*G.ipw[8*si + i]*G.slope[vi]*f[vi];
-            }
-        } else {
-            for (int i = 0; i < ne; ++i) {
-                i64 si = (i64)(l - 1)*G.nsh + h, vi = G.nsh + (i64)(l - 1)*G.vpl + G.adj[6*h + i];
-                r += -0.5*G.ipw[8*si + i]*G.slope[vi]*f[vi];
-            }
-            for (int i = 0; i < ne; ++i) {
-                i64 si = (i64)l*G.nsh + h, vi = G.nsh + (i64)l*G.vpl + G.adj[6*h + i];
-                r += -0.5*G.ipw[8*si + i]*G.slope[vi]*f[vi];
-            }
-        }
-    }
-    return r;
-}
-
-/* divergences.c:14-64 for cell h of layer l */
-__device__ __forceinline__ double divv_h_cell(const DevGrid &G, const double *in, int l, int h)
-{
-    int ne = h < GAME_N_PENT ? 5 : 6;
-    i64 i = (i64)l*G.nsh + h;
-    double comp_h = 0.0;
-    for (int j = 0; j < ne; ++j) {
-        i64 vi = G.nsh + (i64)l*G.vpl + G.adj[6*h + j];
-        comp_h += in[vi]*G.sgn[6*h + j]*G.area[vi];
-    }
-    double comp_v = 0.0;
-    int L = G.L, no = G.n_oro;
-    if (l == L - no - 1) {
-        double cl = vertical_contravariant_corr(G, in, l + 1, h);
-        comp_v = -cl*G.area[h + (i64)(l + 1)*G.vpl];
-    } else if (l == L - 1) {
-        double cu = vertical_contravariant_corr(G, in, l, h);
-        comp_v = cu*G.area[h + (i64)l*G.vpl];
-    } else if (l > L - no - 1) {
-        double cu = vertical_contravariant_corr(G, in, l, h);
-        double cl = vertical_contravariant_corr(G, in, l + 1, h);
-        comp_v = cu*G.area[h + (i64)l*G.vpl] - cl*G.area[h + (i64)(l + 1)*G.vpl];
-    }
-    return 1.0/G.vol[i]*(comp_h + comp_v);
 }
 
 /* per-kernel timing with HIP events on the launch stream (off unless enabled) */

@@ -14,24 +14,7 @@
 #include "rkhevi_dev.h"
 #include "rkhevi_kernels.h"
 
-#define TPB 256
 #define GRID1(n) dim3((unsigned)(((n) + TPB - 1)/TPB))
-
-/* grid of n horizontal elements in `chunks` chunks, and its Span for `layers` layers or levels */
-static dim3 grid_of(int n, int chunks) { return dim3((unsigned)((n + TPB - 1)/TPB), (unsigned)chunks); }
-static Span span_of(int n, int layers, int chunks)
-{
-    const unsigned gx = (unsigned)((n + TPB - 1)/TPB);
-    return Span{(layers + chunks - 1)/chunks, gx > 1 ? (unsigned)(((1ULL << 32) + gx - 1)/gx) : 0xffffffffu};
-}
-
-/* layers [l0, l1) of a chunk when n layers are split into chunks of `run`;
-   the last chunk may be shorter (or empty) */
-__device__ __forceinline__ void layer_chunk(int n, unsigned chunk, int run, int &l0, int &l1)
-{
-    l0 = (int)chunk*run;
-    l1 = l0 + run < n ? l0 + run : n;
-}
 
 /* ------------------------------------------------------------------ */
 /* small device helpers restating reference functions                   */
@@ -270,7 +253,7 @@ __global__ void __launch_bounds__(TPB) k_pgrad_e(DevGrid G, DevState s, DevWorkT
 template <typename TW>
 __global__ void __launch_bounds__(TPB) k_rel_vort_tri(DevGrid G, const double *w, TW *res, Span sp)
 {
-    const Blk bk = xcd_block(sp);
+    const Blk bk = linear_block();
     const unsigned h = bk.x*TPB + threadIdx.x;
     if (h >= (unsigned)G.nt) return;
     const int L = G.L, lt = L - G.n_oro, nsh = G.nsh, vpl = G.vpl, nvh = G.nvh;
@@ -371,7 +354,7 @@ template <bool FLAT, typename TW>
 __global__ void __launch_bounds__(TPB) k_pot_vort(DevGrid G, const double *w, const double *rho, const TW *rvt,
                                                   TW *pv, TW *flux, Span sp)
 {
-    const Blk bk = xcd_block(sp);
+    const Blk bk = FLAT ? linear_block() : xcd_block(sp);
     const unsigned e = bk.x*TPB + threadIdx.x;
     if (e >= (unsigned)G.nvh) return;
     const int nvh = G.nvh, nsh = G.nsh, L = G.L, vpl = G.vpl;

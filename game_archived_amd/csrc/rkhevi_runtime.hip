@@ -183,7 +183,7 @@ int game_gpu_init(const game_dims_t *dims, const game_grid_view_t *g, const game
 static void set_layer_splits(DevGrid &G)
 {
     const int L = G.L, be = (G.nvh + 255)/256, bc = (G.nsh + 255)/256, bt = (G.nt + 255)/256;
-    auto clamp = [](int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); };
+    auto clamp = [](int v, int lo, int hi) { return v > hi ? hi : (v < lo ? lo : v); };
     /* edges: one filled chip; where four chunks or fewer fill it, twice that
        in at most four chunks for the kernels with long layers, whose last
        blocks then leave less of it idle.  The flat gradients carry nothing
@@ -204,13 +204,17 @@ static void set_layer_splits(DevGrid &G)
        res 6: three 50, four 51, six 64) */
     const int run_v = bc*G.n_oro <= 512 ? 1 : clamp((bc*G.n_oro + 640)/1280, 2, 6);
     G.split_vcc = (G.n_oro + run_v - 1)/run_v;
+    /* the adjoints: a filled chip, at least four chunks; a cell's chunk forms
+       a layer above and below it again, so it has two layers or more */
+    G.split_adj_c = clamp(1024/bc, 4, (L + 1)/2);
+    G.split_adj_e = clamp(fill, 4, L);
     if (const char *e = getenv("GAME_GPU_SPLIT_CELL")) {
         int v = atoi(e);
-        if (v >= 1 && v <= L) G.split_cell_w = v;
+        if (v >= 1 && v <= L) G.split_cell_w = G.split_adj_c = v;
     }
     if (const char *e = getenv("GAME_GPU_SPLIT_EDGE")) {
         int v = atoi(e);
-        if (v >= 1 && v <= L) G.split_edge = G.split_grad = G.split_tri = v;
+        if (v >= 1 && v <= L) G.split_edge = G.split_grad = G.split_tri = G.split_adj_e = v;
     }
 }
 
@@ -273,7 +277,7 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
     UP(G.nd, g->normal_distance, V); UP(G.vol, g->volume, S); UP(G.area, g->area, V); UP(G.zs, g->z_scalar, S);
     UP(G.zv, g->z_vector, V); UP(G.phi, g->gravity_potential, S); UP(G.gm, g->gravity_m, V);
     UP(G.slope, g->slope, V); UP(G.thbg, g->theta_v_bg, S); UP(G.exbg, g->exner_bg, S);
-    UP(G.exbg_grad, g->exner_bg_grad, V); UP(G.ipw, g->inner_product_weights, 8*S);
+    UP(G.exbg_grad, g->exner_bg_grad, V);
     UP(G.tw, g->trsk_weights, 10*NVH); UP(G.drw, g->density_to_rhombi_weights, 4*NVH);
     UP(G.dnd, dg->normal_distance, (size_t)d.dual_v); UP(G.dzv, dg->z_vector, (size_t)d.dual_v);
     UP(G.darea, dg->area, (size_t)d.curl); UP(G.fvec, dg->f_vec, 2*NVH);

@@ -36,6 +36,9 @@ namespace sadj {
 GAME_HD inline i64 eidx(const DevGrid &G, int l, int e) { return G.nsh + (i64)l*G.vpl + e; }
 GAME_HD inline i64 widx(const DevGrid &G, int lev, int h) { return (i64)lev*G.vpl + h; }
 GAME_HD inline i64 sidx(const DevGrid &G, int l, int h) { return (i64)l*G.nsh + h; }
+/* inner-product weight j of cell h in layer l: from the cell-major copy, whose
+   consecutive cells are consecutive words */
+GAME_HD inline double ipw(const DevGrid &G, int l, int h, int j) { return G.ipwT[((i64)l*8 + j)*G.nsh + h]; }
 /* (q, r) = (t / n, t % n) for a flat index below 2^32 (every array here) */
 GAME_HD inline void split_index(i64 t, int n, int &q, int &r)
 {
@@ -526,7 +529,7 @@ GAME_HD inline double divv_adj_edge(const DevGrid &G, const AdjTables &A, const 
         const int cell[2] = {fr, to}, slot[2] = {A.slot_from[e], A.slot_to[e]};
         for (int p = 0; p < 2; ++p) {
             const int c = cell[p];
-            const double k = -0.5*G.ipw[8*sidx(G, l, c) + slot[p]]*G.slope[vi];
+            const double k = G.vcw[((i64)(l - top)*6 + slot[p])*G.nsh + c];   /* -0.5*ipw*slope */
             double v = vc[(i64)(l - top)*G.nsh + c];
             if (l + 1 <= G.L - 1) v += vc[(i64)(l + 1 - top)*G.nsh + c];
             r += k*v;
@@ -583,7 +586,7 @@ struct ScalarTendAdjC {
            sixth reads its first edge and adds nothing (same sums) */
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            const i64 k = (i64)l*G.nvh + G.adj[6*c + (j < ne ? j : 0)];
+            const i64 k = (i64)l*G.nvh + G.c_e[(i64)j*G.nsh + c];
             const double p1 = P1[k], p2 = P2[k];
             if (j < ne) {
                 thvb += p1;
@@ -623,7 +626,7 @@ struct StvAdjS {
         double a[6], f[6];
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            vi[j] = eidx(G, l, G.adj[6*c + (j < ne ? j : 0)]);
+            vi[j] = eidx(G, l, (int)G.c_e[(i64)j*G.nsh + c]);
             a[j] = v1[vi[j]];
             f[j] = Fb[vi[j]];
         }
@@ -773,19 +776,19 @@ struct VFluxPvAdjTan {
         /* the non-standard term of the edge in layer lev (ipw slot 6, w at
            level lev) and in layer lev - 1 (slot 7, w at level lev) */
         if (lev <= L - 1)
-            r += -0.5*ob[eidx(G, lev, e)]*(G.ipw[8*sidx(G, lev, fr) + 6]*F[widx(G, lev, fr)]
-                                           + G.ipw[8*sidx(G, lev, to) + 6]*F[widx(G, lev, to)]);
+            r += -0.5*ob[eidx(G, lev, e)]*(ipw(G, lev, fr, 6)*F[widx(G, lev, fr)]
+                                           + ipw(G, lev, to, 6)*F[widx(G, lev, to)]);
         if (lev >= 1)
-            r += -0.5*ob[eidx(G, lev - 1, e)]*(G.ipw[8*sidx(G, lev - 1, fr) + 7]*F[widx(G, lev, fr)]
-                                               + G.ipw[8*sidx(G, lev - 1, to) + 7]*F[widx(G, lev, to)]);
+            r += -0.5*ob[eidx(G, lev - 1, e)]*(ipw(G, lev - 1, fr, 7)*F[widx(G, lev, fr)]
+                                               + ipw(G, lev - 1, to, 7)*F[widx(G, lev, to)]);
         /* the vertical outputs of the edge's two cells at level lev */
         const double vw = vflux_vert_weight(G, lev);
         const int cell[2] = {fr, to}, slot[2] = {A.slot_from[e], A.slot_to[e]};
         for (int p = 0; p < 2; ++p) {
             const int c = cell[p];
             double s = 0.0;
-            if (lev >= 1) s += G.ipw[8*sidx(G, lev - 1, c) + slot[p]]*F[eidx(G, lev - 1, e)];
-            if (lev <= L - 1) s += G.ipw[8*sidx(G, lev, c) + slot[p]]*F[eidx(G, lev, e)];
+            if (lev >= 1) s += ipw(G, lev - 1, c, slot[p])*F[eidx(G, lev - 1, e)];
+            if (lev <= L - 1) s += ipw(G, lev, c, slot[p])*F[eidx(G, lev, e)];
             r += vw*s*ob[widx(G, lev, c)];
         }
         pvb[(i64)lev*2*nvh + e] = r;
@@ -901,19 +904,34 @@ struct TanVortAdjC {
         const bool rows = lev >= 1 && lev <= L - 1;
         const bool t6 = !G.flat && lev >= o0 && lev <= L - 1, t7 = !G.flat && lev - 1 >= o0 && lev - 1 < L - 1;
         const double ndw = rows ? G.nd[wi] : 0.0;
-        const double w6 = t6 ? G.ipw[8*sidx(G, lev, c) + 6] : 0.0, w7 = t7 ? G.ipw[8*sidx(G, lev - 1, c) + 7] : 0.0;
+        const double w6 = t6 ? ipw(G, lev, c, 6) : 0.0, w7 = t7 ? ipw(G, lev - 1, c, 7) : 0.0;
+        const unsigned from = G.c_from[c];
+        /* the cell's edges, a fixed six so that every load issues at once (a
+           pentagon's sixth slot reads its first edge and adds nothing); rows
+           out of range are clamped and left out */
+        const int lr = rows ? lev : 1, l6 = t6 ? lev : L - 1, l7 = t7 ? lev - 1 : L - 1;
+        double da[6], tc[6], s6[6], c6[6], s7[6], c7[6];
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            const int e = (int)G.c_e[(i64)j*G.nsh + c];
+            da[j] = G.darea[(i64)lr*G.dvpl + e];
+            tc[j] = tan_row_cot(G, rvb, lr, e);
+            s6[j] = 0.0; c6[j] = 0.0; s7[j] = 0.0; c7[j] = 0.0;
+            if (!G.flat) {
+                s6[j] = G.slope[eidx(G, l6, e)];
+                c6[j] = cvb[(i64)l6*G.nvh + e];
+                s7[j] = G.slope[eidx(G, l7, e)];
+                c7[j] = cvb[(i64)l7*G.nvh + e];
+            }
+        }
         double r = 0.0;
-        /* the cell's edges; the sign is +1 where the cell is the edge's from-cell */
+        /* the sign is +1 where the cell is the edge's from-cell */
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
             if (j < ne) {
-                const int e = G.adj[6*c + j];
-                if (rows) {
-                    const double s = (double)G.sgn[6*c + j];
-                    r += s*ndw/G.darea[(i64)lev*G.dvpl + e]*tan_row_cot(G, rvb, lev, e);
-                }
-                if (t6) r += 0.5*G.slope[eidx(G, lev, e)]*w6*cvb[(i64)lev*G.nvh + e];
-                if (t7) r += 0.5*G.slope[eidx(G, lev - 1, e)]*w7*cvb[(i64)(lev - 1)*G.nvh + e];
+                if (rows) r += ((from >> j) & 1u ? ndw : -ndw)/da[j]*tc[j];
+                if (t6) r += 0.5*s6[j]*w6*c6[j];
+                if (t7) r += 0.5*s7[j]*w7*c7[j];
             }
         }
         b_wind[wi] += r;
@@ -938,7 +956,7 @@ struct HalfDensAdj {
            sixth slot reads its first edge (same sum) */
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            const int e = G.adj[6*c + (j < ne ? j : 0)];
+            const int e = (int)G.c_e[(i64)j*G.nsh + c];
             const double da = dvb[(i64)l*nv2 + e], db = dvb[(i64)(l + 1)*nv2 + e];
             /* a pentagon's sixth slot adds -0.0, the exact identity of IEEE
                addition */
