@@ -72,6 +72,7 @@ __global__ void __launch_bounds__(TPB) k_temperature(DevGrid G, DevState s, TO *
 template <typename TW>
 struct Mom {
     TW *td;
+    const TW *td_old;       /* the first substep's, read with weight 1 - new_w: td, or the tape's */
     const double *wind_old;
     double *wind_new;
     double new_w, dt;
@@ -512,7 +513,7 @@ k_vorticity_flux_e(DevGrid G, const TW *F, const TW *pv, TW *out, DevWorkT<TW> W
         if (TEND) {
             comb = (double)at(W.pgrad_comb + vi, e);
             wo = at(m.wind_old + vi, e);
-            if (old_w != 0.0) td_old = (double)at(m.td + vi, e);
+            if (old_w != 0.0) td_old = (double)at(m.td_old + vi, e);
         }
         double o = 0;
 #pragma unroll
@@ -606,7 +607,7 @@ __global__ void __launch_bounds__(TPB) k_vorticity_flux_w(DevGrid G, const TW *F
             vs = (double)at(W.vsq + (i64)lc*nsh, h);
             comb = (double)at(W.pgrad_comb + row, h);
             nd = at(G.nd + row, h);
-            if (old_w != 0.0) td_old = (double)at(m.td + row, h);
+            if (old_w != 0.0) td_old = (double)at(m.td_old + row, h);
             if (rho) { gm = at(G.gm + row, h); d = gas_fraction_at<NC>(G, rho, (i64)lc*nsh, h); }
             else pgc = (double)at(W.pgc_v + row, h);
         }
@@ -2483,18 +2484,19 @@ static void scalar_tend_t(const DevGrid &G, const DevState &s, const DevState &t
 #define BOTH_FORMS(T, WORK)                                                                                         \
     void pgrad(const DevGrid &G, const DevState &s, const WORK &W, int first, double itw, T *td, const double *w_old,   \
                double *w_new, double dt, hipStream_t st)                                                            \
-    { pgrad_t<T>(G, s, W, first, itw, Mom<T>{td, w_old, w_new, 1.0, dt}, st); }                                     \
+    { pgrad_t<T>(G, s, W, first, itw, Mom<T>{td, td, w_old, w_new, 1.0, dt}, st); }                                     \
     void advection(const DevGrid &G, const double *wind, const double *rho_gas, const WORK &W, hipStream_t st)      \
     { advection_t<T>(G, wind, rho_gas, W, st); }                                                                    \
     void advection_pv(const DevGrid &G, const double *wind, const double *rho_gas, const WORK &W, hipStream_t st)   \
     { advection_pv_t<T>(G, wind, rho_gas, W, st); }                                                                 \
     void kinetic_energy(const DevGrid &G, const double *wind, const WORK &W, hipStream_t st)                        \
     { inner_product_t<T>(G, wind, wind, W.vsq, st); }                                                               \
-    void momentum_e(const DevGrid &G, const WORK &W, T *td, const double *w_old, double *w_new, double new_w,       \
-                    double dt, hipStream_t st)                                                                      \
-    { momentum_e_t<T>(G, W, Mom<T>{td, w_old, w_new, new_w, dt}, st); }                                             \
-    void momentum_w(const DevGrid &G, const WORK &W, T *td, double new_w, const double *rho, hipStream_t st)        \
-    { momentum_w_t<T>(G, W, Mom<T>{td, nullptr, nullptr, new_w, 0.0}, rho, st); }
+    void momentum_e(const DevGrid &G, const WORK &W, T *td, const T *td_old, const double *w_old, double *w_new,    \
+                    double new_w, double dt, hipStream_t st)                                                        \
+    { momentum_e_t<T>(G, W, Mom<T>{td, td_old, w_old, w_new, new_w, dt}, st); }                                     \
+    void momentum_w(const DevGrid &G, const WORK &W, T *td, const T *td_old, double new_w, const double *rho,       \
+                    hipStream_t st)                                                                                 \
+    { momentum_w_t<T>(G, W, Mom<T>{td, td_old, nullptr, nullptr, new_w, 0.0}, rho, st); }
 BOTH_FORMS(double, DevWork)
 BOTH_FORMS(float, DevWorkF)
 #undef BOTH_FORMS

@@ -29,15 +29,17 @@ void advection_pv(const DevGrid &G, const double *wind, const double *rho_gas, c
 void kinetic_energy(const DevGrid &G, const double *wind, const DevWork &W, hipStream_t st);
 void kinetic_energy(const DevGrid &G, const double *wind, const DevWorkF &W, hipStream_t st);
 /* and, from W.flux, W.pv and W.vsq: TRSK flux, kinetic-energy gradient and the
-   tendency td = (1 - new_w) td + new_w (...) -- at the edges with the wind
+   tendency td = (1 - new_w) td_old + new_w (...) -- at the edges with the wind
    update; at the w points with the condensates' term of the densities rho
    (null: W.pgc_v as it is) */
-void momentum_e(const DevGrid &G, const DevWork &W, double *td, const double *w_old, double *w_new, double new_w,
-                double dt, hipStream_t st);
-void momentum_e(const DevGrid &G, const DevWorkF &W, float *td, const double *w_old, double *w_new, double new_w,
-                double dt, hipStream_t st);
-void momentum_w(const DevGrid &G, const DevWork &W, double *td, double new_w, const double *rho, hipStream_t st);
-void momentum_w(const DevGrid &G, const DevWorkF &W, float *td, double new_w, const double *rho, hipStream_t st);
+void momentum_e(const DevGrid &G, const DevWork &W, double *td, const double *td_old, const double *w_old, double *w_new,
+                double new_w, double dt, hipStream_t st);
+void momentum_e(const DevGrid &G, const DevWorkF &W, float *td, const float *td_old, const double *w_old, double *w_new,
+                double new_w, double dt, hipStream_t st);
+void momentum_w(const DevGrid &G, const DevWork &W, double *td, const double *td_old, double new_w, const double *rho,
+                hipStream_t st);
+void momentum_w(const DevGrid &G, const DevWorkF &W, float *td, const float *td_old, double new_w, const double *rho,
+                hipStream_t st);
 void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const DevWork &W, int rk, hipStream_t st);
 void scalar_tend(const DevGrid &G, const DevState &s, const DevState &td, const DevWorkF &W, int rk, hipStream_t st);
 void inner_product(const DevGrid &G, const double *a, const double *b, double *out, hipStream_t st);

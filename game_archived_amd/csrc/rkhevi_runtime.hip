@@ -513,36 +513,14 @@ static int get_irrev_t(const WK &W, game_irrev_view_t *h)
    state_old: the step then also runs on a state_new buffer that holds an
    older state, which lets game_gpu_run_steps swap the two buffers instead of
    copying. */
-/* the five fields of a state, device to device */
-static int copy_state_d2d(const DevState &dst, const DevState &src, hipStream_t st)
-{
-    const size_t S = (size_t)M->d.s*sizeof(double), V = (size_t)M->d.v*sizeof(double);
-    HIP_OK(hipMemcpyAsync(dst.rho, src.rho, S*(size_t)M->d.n_const, hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(dst.rt, src.rt, S, hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(dst.tp, src.tp, S, hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(dst.ep, src.ep, S, hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(dst.wind, src.wind, V, hipMemcpyDeviceToDevice, st));
-    return 0;
-}
-
-static int copy_tendency(double *rho, double *rt_, double *wind, const DevState &td, hipStream_t st)
-{
-    const size_t S = (size_t)M->d.s*sizeof(double), V = (size_t)M->d.v*sizeof(double);
-    HIP_OK(hipMemcpyAsync(rho, td.rho, S, hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(rt_, td.rt, S, hipMemcpyDeviceToDevice, st));
-    HIP_OK(hipMemcpyAsync(wind, td.wind, V, hipMemcpyDeviceToDevice, st));
-    return 0;
-}
-
 template <class WK, typename TW>
-static int step_t(const WK &W, TW *td_wind, double dt, int first, const StepTape *tape = nullptr)
+static int step_t(const WK &work, TW *td_wind, double dt, int first, const StepTape *tape = nullptr)
 {
     hipStream_t st = M->stream;
     const DevGrid &G = M->G;
-    DevState &so = M->s[GAME_STATE_OLD], &sn = M->s[GAME_STATE_NEW], &td = M->s[GAME_STATE_TENDENCY];
+    const DevState &so = tape ? tape->s : M->s[GAME_STATE_OLD];
+    WK W = work;
     M->K.dt = dt;
-    int rc;
-    if (tape && (rc = copy_state_d2d(tape->s, so, st))) return rc;
     if (G.n_const > 1 && dt != M->idv_dt) {
         col::tracer_quotients(G, dt, st);
         M->idv_dt = dt;
@@ -556,13 +534,24 @@ static int step_t(const WK &W, TW *td_wind, double dt, int first, const StepTape
     /* per-kernel events time each kernel alone: with them on, one stream */
     const bool conc = M->concurrent && !g_kernel_timer;
     for (int rk = 0; rk < 2; ++rk) {
-        const DevState &snr = rk == 0 ? so : sn;           /* state_new before this substep writes it */
+        /* the new state; the tape keeps the first substep's beside the second's */
+        const DevState &sn = !tape ? M->s[GAME_STATE_NEW] : rk == 0 ? tape->s1 : tape->out;
+        const DevState &td = !tape ? M->s[GAME_STATE_TENDENCY] : rk == 0 ? tape->td0 : tape->td1;
+        TW *tdw = td_wind;
+        const TW *tdw_old = td_wind;
+        if constexpr (std::is_same<WK, DevWork>::value)
+            if (tape) {
+                tdw = td.wind;
+                tdw_old = tape->td0.wind;
+                if (rk == 1) { W.flux = tape->flux; W.pv = tape->pv; }
+            }
+        const DevState &snr = rk == 0 ? so : tape ? tape->s1 : sn;   /* state_new before this substep writes it */
         DevState sns = snr;                                 /* ... with the horizontal wind just updated */
         sns.wind = sn.wind;
         const double *rho_gas = snr.rho + (i64)G.n_cond*G.s;
         /* rk 0 of every step but a first one: the pressure gradient with the
            tendency from the carried advection */
-        if (rk == 0) hor::pgrad(G, snr, W, first, M->cfg.impl_thermo_weight, td_wind, so.wind, sn.wind, dt, st);
+        if (rk == 0) hor::pgrad(G, snr, W, first, M->cfg.impl_thermo_weight, tdw, so.wind, sn.wind, dt, st);
         if (rk == 1 || first) {
             const double new_w = rk == 1 ? 0.5 : 1.0;
             /* the condensates' term of the first substep's densities; at rk 0 the pressure gradient has it */
@@ -580,27 +569,22 @@ static int step_t(const WK &W, TW *td_wind, double dt, int first, const StepTape
                 HIP_OK(hipEventRecord(M->ev_fork, st));
                 HIP_OK(hipStreamWaitEvent(st, M->ev_join, 0));
                 HIP_OK(hipStreamWaitEvent(M->side, M->ev_fork, 0));
-                hor::momentum_w(G, W, td_wind, new_w, pgc_rho, M->side);
-                hor::momentum_e(G, W, td_wind, so.wind, sn.wind, new_w, dt, st);
+                hor::momentum_w(G, W, tdw, tdw_old, new_w, pgc_rho, M->side);
+                hor::momentum_e(G, W, tdw, tdw_old, so.wind, sn.wind, new_w, dt, st);
                 HIP_OK(hipEventRecord(M->ev_join, M->side));
                 HIP_OK(hipStreamWaitEvent(st, M->ev_join, 0));
             } else {
                 hor::kinetic_energy(G, snr.wind, W, st);
                 hor::advection_pv(G, snr.wind, rho_gas, W, st);
-                hor::momentum_w(G, W, td_wind, new_w, pgc_rho, st);
-                hor::momentum_e(G, W, td_wind, so.wind, sn.wind, new_w, dt, st);
+                hor::momentum_w(G, W, tdw, tdw_old, new_w, pgc_rho, st);
+                hor::momentum_e(G, W, tdw, tdw_old, so.wind, sn.wind, new_w, dt, st);
             }
         }
-        if constexpr (std::is_same<WK, DevWork>::value)
-            if (tape && rk == 1) {
-                HIP_OK(hipMemcpyAsync(tape->flux, W.flux, (size_t)M->d.v*sizeof(double), hipMemcpyDeviceToDevice, st));
-                HIP_OK(hipMemcpyAsync(tape->pv, W.pv, (size_t)M->d.curl*sizeof(double), hipMemcpyDeviceToDevice, st));
-            }
         hor::scalar_tend(G, sns, td, W, rk, st);
         if (sizeof(TW) == sizeof(double)) col::ver_waves(G, so, snr, sn, td, M->K, rk, st);
-        else col::ver_waves(G, so, snr, sn, td, (const float *)td_wind, M->K, rk, st);
+        else col::ver_waves(G, so, snr, sn, td, (const float *)tdw, M->K, rk, st);
         if (G.n_const > 1) {
-            if (conc && rk == 0 && !tape) {
+            if (conc && rk == 0) {
                 /* the first substep's tracer solve (and sediment heat) on the
                    side stream: it writes only the tracer densities and the
                    sediment heat, which the second substep's PV chain does not
@@ -611,19 +595,14 @@ static int step_t(const WK &W, TW *td_wind, double dt, int first, const StepTape
                 col::gen_densities(G, so, sn, td, W.temp, W.cpc, W.sed_heat, M->K, rk, M->side);
             } else col::gen_densities(G, so, sn, td, W.temp, W.cpc, W.sed_heat, M->K, rk, st);
         }
-        if (tape && rk == 0) {
-            if ((rc = copy_state_d2d(tape->s1, sn, st))) return rc;
-            if ((rc = copy_tendency(tape->td0_rho, tape->td0_rt, tape->td0_wind, td, st))) return rc;
-        }
-        if (tape && rk == 1 && (rc = copy_tendency(tape->td1_rho, tape->td1_rt, tape->td1_wind, td, st))) return rc;
     }
     HIP_OK(hipGetLastError());
     return 0;
 }
 
-int rt::step_fp64(double dt, int first, const StepTape *tape)
+int rt::step_fp64(double dt, int first, const StepTape &tape)
 {
-    return step_t(M->W, M->s[GAME_STATE_TENDENCY].wind, dt, first, tape);
+    return step_t(M->W, tape.td0.wind, dt, first, &tape);
 }
 
 extern "C" {

@@ -7,10 +7,11 @@
  * Checkpointing: the forward sweep stores the state and the carried forcings
  * (the previous step's pressure gradient nl + l and momentum advection) every
  * `checkpoint_every` steps.  The reverse sweep visits the segments last to
- * first; each segment is run forward once more from its checkpoint with every
- * step's inputs and substep results copied to a tape (StepTape), then its steps
- * are reversed last to first.  Memory: one checkpoint per segment plus one
- * segment of tapes.
+ * first; each segment is run forward once more from its checkpoint on a tape
+ * (StepTape: every step's input, substep results and tendencies, which the
+ * step's kernels write there instead of into the resident buffers), then its
+ * steps are reversed last to first.  Memory: one checkpoint per segment plus
+ * one segment of tapes.
  *
  * Reverse of one step (manage_rkhevi.c:20-100 backwards; see step_adjoint.h
  * for the functors):
@@ -199,6 +200,15 @@ int alloc_state(DevState &s)
     return 0;
 }
 
+int alloc_tendency(DevState &s)
+{
+    const size_t S = (size_t)M->d.s, V = (size_t)M->d.v;
+    int rc;
+    s.tp = s.ep = nullptr;
+    if ((rc = zeros(&s.rho, S)) || (rc = zeros(&s.rt, S)) || (rc = zeros(&s.wind, V))) return rc;
+    return 0;
+}
+
 int alloc_cot(Cot &c)
 {
     const size_t S = (size_t)M->d.s, V = (size_t)M->d.v;
@@ -248,10 +258,9 @@ int window_alloc(Window &w, int k, int n_ckpt)
     w.tape.resize(k);
     for (int j = 0; j < k; ++j) {
         StepTape &t = w.tape[j];
-        if ((rc = alloc_state(t.s)) || (rc = alloc_state(t.s1)) || (rc = zeros(&t.td0_rho, S))
-            || (rc = zeros(&t.td0_rt, S)) || (rc = zeros(&t.td0_wind, V)) || (rc = zeros(&t.td1_rho, S))
-            || (rc = zeros(&t.td1_rt, S)) || (rc = zeros(&t.td1_wind, V)) || (rc = zeros(&t.flux, V))
-            || (rc = zeros(&t.pv, CURL)))
+        /* the first step of a segment starts from the checkpoint itself */
+        if ((j > 0 && (rc = alloc_state(t.s))) || (rc = alloc_state(t.s1)) || (rc = alloc_tendency(t.td0))
+            || (rc = alloc_tendency(t.td1)) || (rc = zeros(&t.flux, V)) || (rc = zeros(&t.pv, CURL)))
             return rc;
     }
     if ((rc = alloc_state(w.seg_end)) || (rc = alloc_cot(w.bS)) || (rc = alloc_cot(w.bSn)) || (rc = alloc_cot(w.bS1)))
@@ -284,21 +293,62 @@ int copy(double *dst, const double *src, size_t n)
     return 0;
 }
 
-int copy_state(const DevState &dst, const DevState &src)
+/* copies up to COPY_MAX arrays in one launch: grid.y the array, COPY_PER loads
+   of a thread in flight before its stores.  A copy call per array costs 4 us
+   at res 4, most of it the launch, and 9 us at res 6 x 26; with the tapes
+   copied too they were 1200 of the calls of a 24-step gradient and 6 % of its
+   time.  For the library's own arrays only: a caller's pointer goes through
+   the copy call, which also takes host memory */
+#define COPY_MAX 32
+#define COPY_PER 4
+struct CopyMany {
+    double *dst[COPY_MAX];
+    const double *src[COPY_MAX];
+    i64 n[COPY_MAX];
+};
+
+__global__ void __launch_bounds__(WTPB) k_copy_many(CopyMany c)
 {
-    const size_t S = (size_t)M->d.s, V = (size_t)M->d.v;
-    int rc;
-    if ((rc = copy(dst.rho, src.rho, S)) || (rc = copy(dst.rt, src.rt, S)) || (rc = copy(dst.tp, src.tp, S))
-        || (rc = copy(dst.ep, src.ep, S)) || (rc = copy(dst.wind, src.wind, V)))
-        return rc;
-    return 0;
+    const int a = (int)blockIdx.y;
+    const i64 n = c.n[a], t = (i64)blockIdx.x*(WTPB*COPY_PER) + threadIdx.x;
+    const double *src = c.src[a];
+    double *dst = c.dst[a];
+    double v[COPY_PER];
+#pragma unroll
+    for (int k = 0; k < COPY_PER; ++k) if (t + k*WTPB < n) v[k] = src[t + k*WTPB];
+#pragma unroll
+    for (int k = 0; k < COPY_PER; ++k) if (t + k*WTPB < n) dst[t + k*WTPB] = v[k];
 }
 
-int zero(double *p, size_t n)
-{
-    HIP_OK(hipMemsetAsync(p, 0, n*sizeof(double), M->stream));
-    return 0;
-}
+struct CopyList {
+    CopyMany c{};
+    int cnt = 0;
+    i64 longest = 0;
+    hipStream_t st;
+    explicit CopyList(hipStream_t stream) : st(stream) {}
+    void add(double *dst, const double *src, size_t n)
+    {
+        if (cnt == COPY_MAX) run();
+        c.dst[cnt] = dst;
+        c.src[cnt] = src;
+        c.n[cnt++] = (i64)n;
+        if ((i64)n > longest) longest = (i64)n;
+    }
+    void add_state(const DevState &dst, const DevState &src)
+    {
+        const size_t S = (size_t)M->d.s, V = (size_t)M->d.v;
+        add(dst.rho, src.rho, S); add(dst.rt, src.rt, S); add(dst.tp, src.tp, S); add(dst.ep, src.ep, S);
+        add(dst.wind, src.wind, V);
+    }
+    void run()
+    {
+        if (cnt > 0)
+            LAUNCH("k_copy_many", k_copy_many, dim3((unsigned)((longest + WTPB*COPY_PER - 1)/(WTPB*COPY_PER)), (unsigned)cnt),
+                   dim3(WTPB), st, c);
+        cnt = 0;
+        longest = 0;
+    }
+};
 
 /* zeroes up to ZERO_MAX arrays in one launch */
 #define ZERO_MAX 20
@@ -330,16 +380,6 @@ struct ZeroList {
     void run(hipStream_t st) const { launch("k_zero_many", z, longest, st); }
 };
 
-int zero_cot(const Cot &c)
-{
-    const size_t S = (size_t)M->d.s, V = (size_t)M->d.v;
-    int rc;
-    if ((rc = zero(c.rho, S)) || (rc = zero(c.rt, S)) || (rc = zero(c.tp, S)) || (rc = zero(c.ep, S))
-        || (rc = zero(c.wind, V)))
-        return rc;
-    return 0;
-}
-
 int check_window_model(void)
 {
     if (!M) return GAME_ERR_NOT_INIT;
@@ -359,41 +399,79 @@ int load_controls(const double *rho0, const double *rt0, const double *wind0)
     if ((rc = copy(n.rho, rho0, S)) || (rc = copy(n.rt, rt0, S)) || (rc = copy(n.wind, wind0, V))) return rc;
     EosState f{M->G, n.rho, n.rt, n.tp, n.ep};
     launch("k_eos_state", f, M->G.s, M->stream);
-    return copy_state(M->s[GAME_STATE_OLD], n);
-}
-
-/* one step as game_gpu_run_steps takes it: the state buffers exchanged, then
-   manage_rkhevi, eagerly when taped */
-int window_step(double dt, int first, const StepTape *tape)
-{
-    DevState t = M->s[GAME_STATE_OLD];
-    M->s[GAME_STATE_OLD] = M->s[GAME_STATE_NEW];
-    M->s[GAME_STATE_NEW] = t;
-    return step_fp64(dt, first, tape);
-}
-
-int save_checkpoint(int c)
-{
-    Window &w = *Wn;
-    const size_t V = (size_t)M->d.v;
-    int rc;
-    if ((rc = copy_state(w.ck_state[c], M->s[GAME_STATE_NEW])) || (rc = copy(w.ck_nl[c], M->W.pgrad_nl, V))
-        || (rc = copy(w.ck_l[c], M->W.pgrad_l, V)) || (rc = copy(w.ck_pvt[c], M->W.pvt, V))
-        || (rc = copy(w.ck_vsqg[c], M->W.vsq_grad, V)))
-        return rc;
+    CopyList cl(M->stream);
+    cl.add_state(M->s[GAME_STATE_OLD], n);
+    cl.run();
     return 0;
 }
 
-int restore_checkpoint(int c)
+void save_checkpoint(int c)
 {
     Window &w = *Wn;
     const size_t V = (size_t)M->d.v;
-    int rc;
-    if ((rc = copy_state(M->s[GAME_STATE_NEW], w.ck_state[c])) || (rc = copy_state(M->s[GAME_STATE_OLD], w.ck_state[c]))
-        || (rc = copy(M->W.pgrad_nl, w.ck_nl[c], V)) || (rc = copy(M->W.pgrad_l, w.ck_l[c], V))
-        || (rc = copy(M->W.pvt, w.ck_pvt[c], V)) || (rc = copy(M->W.vsq_grad, w.ck_vsqg[c], V)))
-        return rc;
+    CopyList cl(M->stream);
+    cl.add_state(w.ck_state[c], M->s[GAME_STATE_NEW]);
+    cl.add(w.ck_nl[c], M->W.pgrad_nl, V); cl.add(w.ck_l[c], M->W.pgrad_l, V);
+    cl.add(w.ck_pvt[c], M->W.pvt, V); cl.add(w.ck_vsqg[c], M->W.vsq_grad, V);
+    cl.run();
+}
+
+/* the carried forcings; the state is read in the checkpoint */
+void restore_forcings(int c)
+{
+    Window &w = *Wn;
+    const size_t V = (size_t)M->d.v;
+    CopyList cl(M->stream);
+    cl.add(M->W.pgrad_nl, w.ck_nl[c], V); cl.add(M->W.pgrad_l, w.ck_l[c], V);
+    cl.add(M->W.pvt, w.ck_pvt[c], V); cl.add(M->W.vsq_grad, w.ck_vsqg[c], V);
+    cl.run();
+}
+
+/* the winds the taped steps write get the top and surface w, which no step
+   writes (the resident states hold them both) */
+void tape_fixed_w()
+{
+    Window &w = *Wn;
+    const size_t n = (size_t)M->G.nsh, low = (size_t)M->G.L*(size_t)M->G.vpl;
+    const double *src = M->s[GAME_STATE_NEW].wind;
+    CopyList cl(M->stream);
+    auto rows = [&](double *dst) { cl.add(dst, src, n); cl.add(dst + low, src + low, n); };
+    for (size_t j = 0; j < w.tape.size(); ++j) {
+        if (j > 0) rows(w.tape[j].s.wind);
+        rows(w.tape[j].s1.wind);
+    }
+    rows(w.seg_end.wind);
+    cl.run();
+}
+
+/* m steps from state s on the tape, the last one's result in seg_end */
+int taped_segment(const DevState &s, int m, double dt, int first)
+{
+    Window &w = *Wn;
+    w.tape[0].s = s;
+    for (int j = 0; j < m; ++j) {
+        w.tape[j].out = j == m - 1 ? w.seg_end : w.tape[j + 1].s;
+        int rc = step_fp64(dt, first && j == 0, w.tape[j]);
+        if (rc) return rc;
+    }
     return 0;
+}
+
+/* the resident states, tendency, mass flux and potential vorticity as m steps
+   of the first segment leave them; OLD first, which may be a copy of NEW */
+void resident_from_tape(int m)
+{
+    Window &w = *Wn;
+    const StepTape &t = w.tape[m - 1];
+    const size_t S = (size_t)M->d.s, V = (size_t)M->d.v;
+    const DevState &td = M->s[GAME_STATE_TENDENCY];
+    CopyList cl(M->stream);
+    cl.add_state(M->s[GAME_STATE_OLD], t.s);
+    cl.add(td.rho, t.td1.rho, S); cl.add(td.rt, t.td1.rt, S); cl.add(td.wind, t.td1.wind, V);
+    cl.add(M->W.flux, t.flux, V); cl.add(M->W.pv, t.pv, (size_t)M->d.curl);
+    cl.run();
+    cl.add_state(M->s[GAME_STATE_NEW], w.seg_end);
+    cl.run();
 }
 
 /* reverse of the momentum advection of (wind, rho) for the cotangent advb of
@@ -454,7 +532,7 @@ int advection_adjoint(const double *wind, const double *rho, const double *flux,
 }
 
 /* reverse of step n from its tape; w.bS holds the cotangent of the state the
-   step produced (whose wind edges are next->wind), w.bP the cotangent of the
+   step produced (T.out), w.bP the cotangent of the
    step's pressure gradient nl + l, w.bA that of its second-substep advection;
    on return w.bS, w.bP, w.bA hold the same for the step before */
 /* the reverse of the gas's scalar tendencies (scalar_tendencies_expl.c:107-176)
@@ -491,7 +569,7 @@ static void ver_waves_adjoint(const sadj::VwArgs &a, hipStream_t st)
     launch("k_vw_layer_bar", sadj::VwLayerBar{a}, G.s, st);
 }
 
-int step_adjoint(const StepTape &T, const DevState &next, double dt, int first)
+int step_adjoint(const StepTape &T, double dt, int first)
 {
     Window &w = *Wn;
     const DevGrid &G = M->G;
@@ -525,13 +603,13 @@ int step_adjoint(const StepTape &T, const DevState &next, double dt, int first)
     /* ---- second substep ---- */
     {
         sadj::VwArgs a{G, 1, dt, iw, T.s.rho, T.s.rt, T.s.tp, T.s.ep, T.s.wind, T.s1.rho, T.s1.rt, T.s1.ep,
-                       T.td1_rho, T.td1_rt, T.td1_wind, w.bS.rho, w.bS.rt, w.bS.wind, w.bS.tp, w.bS.ep,
+                       T.td1.rho, T.td1.rt, T.td1.wind, w.bS.rho, w.bS.rt, w.bS.wind, w.bS.tp, w.bS.ep,
                        w.bSn.rho, w.bSn.rt, w.bSn.tp, w.bSn.ep, w.bSn.wind, w.bS1.rho, w.bS1.rt, w.bS1.ep,
                        w.bt1_rho, w.bt1_rt, w.bt1_wind, w.ws};
         ver_waves_adjoint(a, st);
     }
     launch("k_pass_adj", PassThroughAdj{G, w.bS.wind, w.bU, w.bSn.wind}, G.v, st);
-    scalar_tend_adjoint(T.s1.rho, T.s1.rt, next.wind, w.bt1_rho, w.bt1_rt, w.bS1.rho, w.bS1.rt);
+    scalar_tend_adjoint(T.s1.rho, T.s1.rt, T.out.wind, w.bt1_rho, w.bt1_rt, w.bS1.rho, w.bS1.rt);
     launch("k_wind_update_adj", sadj::WindUpdateAdj{G, dt, w.bU, w.bSn.wind, w.bt1_wind, 0}, G.v, st);
     launch("k_tend_adj_rk1", sadj::TendAdjRk1{G, ohw, chw, cvw, w.bt1_wind, w.bA, w.bt0_wind, w.bPold, w.bP, w.bA1},
            G.v, st);
@@ -539,7 +617,7 @@ int step_adjoint(const StepTape &T, const DevState &next, double dt, int first)
     /* ---- first substep ---- */
     {
         sadj::VwArgs a{G, 0, dt, iw, T.s.rho, T.s.rt, T.s.tp, T.s.ep, T.s.wind, T.s.rho, T.s.rt, T.s.ep,
-                       T.td0_rho, T.td0_rt, T.td0_wind, w.bS1.rho, w.bS1.rt, w.bS1.wind, w.bS1.tp, w.bS1.ep,
+                       T.td0.rho, T.td0.rt, T.td0.wind, w.bS1.rho, w.bS1.rt, w.bS1.wind, w.bS1.tp, w.bS1.ep,
                        w.bSn.rho, w.bSn.rt, w.bSn.tp, w.bSn.ep, w.bSn.wind, w.bSn.rho, w.bSn.rt, w.bSn.ep,
                        w.bt0_rho, w.bt0_rt, w.bt0_wind, w.ws};
         ver_waves_adjoint(a, st);
@@ -594,30 +672,31 @@ int window_run(int n_steps, double dt, int k, const double *rho0, const double *
     w.n_ev = 0;
     w.mark(PH_FORWARD, st);
     if ((rc = load_controls(rho0, rt0, wind0))) return rc;
-    for (int n = 0; n < n_steps; ++n) {
-        if (n % k == 0 && n < last0 && (rc = save_checkpoint(n/k))) return rc;
-        if (n >= last0) rc = window_step(dt, n == 0, &w.tape[n - last0]);
-        else rc = game_gpu_run_steps(1, dt, n == 0);               /* graph replays after the first */
-        if (rc) return rc;
+    tape_fixed_w();
+    for (int n = 0; n < last0; ++n) {
+        if (n % k == 0) save_checkpoint(n/k);
+        if ((rc = game_gpu_run_steps(1, dt, n == 0))) return rc;   /* graph replays after the first */
     }
+    if ((rc = taped_segment(M->s[GAME_STATE_NEW], n_steps - last0, dt, last0 == 0))) return rc;
     /* the terminal cotangent from the final state */
-    if ((rc = zero_cot(w.bS)) || (rc = zero(w.bP, V)) || (rc = zero(w.bA, V))) return rc;
-    if ((rc = terminal(M->s[GAME_STATE_NEW], w.bS))) return rc;
+    {
+        ZeroList zl;
+        zl.add_cot(w.bS);
+        zl.add(w.bP, V); zl.add(w.bA, V);
+        zl.run(st);
+    }
+    if ((rc = terminal(w.seg_end, w.bS))) return rc;
     /* reverse sweep by segments */
     for (int c = n_ckpt - 1; c >= 0; --c) {
-        const int n0 = c*k, n1 = (n0 + k < n_steps) ? n0 + k : n_steps;
+        const int n0 = c*k, m = (n0 + k < n_steps) ? k : n_steps - n0;
         w.mark(c == n_ckpt - 1 ? PH_FORWARD : PH_REVERSE, st);
         if (c < n_ckpt - 1) {
-            if ((rc = restore_checkpoint(c))) return rc;
-            for (int n = n0; n < n1; ++n)
-                if ((rc = window_step(dt, n == 0, &w.tape[n - n0]))) return rc;
+            restore_forcings(c);
+            if ((rc = taped_segment(w.ck_state[c], m, dt, n0 == 0))) return rc;
         }
-        if ((rc = copy_state(w.seg_end, M->s[GAME_STATE_NEW]))) return rc;
         w.mark(PH_RECOMPUTE, st);
-        for (int n = n1 - 1; n >= n0; --n) {
-            const DevState &next = (n == n1 - 1) ? w.seg_end : w.tape[n - n0 + 1].s;
-            if ((rc = step_adjoint(w.tape[n - n0], next, dt, n == 0))) return rc;
-        }
+        for (int j = m - 1; j >= 0; --j)
+            if ((rc = step_adjoint(w.tape[j], dt, n0 + j == 0))) return rc;
     }
     w.mark(PH_REVERSE, st);
     /* the control variables: rho, rhotheta_v, wind */
@@ -628,6 +707,7 @@ int window_run(int n_steps, double dt, int k, const double *rho0, const double *
     }
     if ((rc = copy(rho_bar, w.bS.rho, S)) || (rc = copy(rt_bar, w.bS.rt, S)) || (rc = copy(wind_bar, w.bS.wind, V)))
         return rc;
+    resident_from_tape(n_ckpt > 1 ? k : n_steps);
     w.mark(PH_FINISH, st);
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(st));

@@ -125,8 +125,10 @@ struct Model {
    (FP64 form): the state the step starts from, the state after the first
    substep, and the tendencies of both substeps (rho, rhotheta_v, wind) */
 struct StepTape {
-    DevState s, s1;
-    double *td0_rho, *td0_rt, *td0_wind, *td1_rho, *td1_rt, *td1_wind;
+    /* the step's input, the state after the first substep, the step's result */
+    DevState s, s1, out;
+    /* the two substeps' tendencies (rho, rt and wind) */
+    DevState td0, td1;
     /* the second substep's mass flux and potential vorticity (FP64 form) */
     double *flux, *pv;
 };
@@ -137,9 +139,10 @@ int dalloc(void **p, size_t n);
 void dfree(void *p);
 int dzeros(double **dst, size_t count);
 int build_adjoint_tables(void);
-/* one step of the FP64 form on the resident states, eager launches; with a
-   tape, the step's inputs and substep results are copied into it */
-int step_fp64(double dt, int first, const StepTape *tape);
+/* one step of the FP64 form, eager launches, from tape->s: what it leaves on
+   the tape its kernels write there, so nothing is copied and the resident
+   states stay as they are (dry models) */
+int step_fp64(double dt, int first, const StepTape &tape);
 
 }  // namespace rt
 
