@@ -77,17 +77,15 @@ struct DevGrid {
     int split_cell_w, split_edge, split_grad, split_tri, split_vcc;
     /* the same of the operator adjoints' kernels, per cell and per edge */
     int split_adj_c, split_adj_e;
-    /* 1: tracer solver with one (column, tracer) per lane in registers; 0: LDS-staged */
+    /* 1: tracer solver with one (column, tracer) per lane; 0: a column over the waves of a block */
     int gd_streaming;
-    /* one tracer per block in the LDS-staged tracer solve instead of all five */
-    int gd_per_tracer;
     /* mixed form, a precision probe: bit 0 rounds the density tendencies,
        bit 1 the rhotheta_v tendency, to FP32 after the scalar tendencies
        (the precision of FP32 storage, not its bytes) */
     int round_tendencies;
     /* 1: sound-wave solver with one column per lane; 0: three phases over LDS */
     int vw_streaming;
-    /* 1: sediment heat with one thread per grid box; 0: one thread per column (26 layers) */
+    /* 1: sediment heat with one thread per grid box; 0: per chunk of layers */
     int sh_per_box;
     /* 1: temperature and phase transitions as two kernels instead of one */
     int unfused_phase;

@@ -1207,52 +1207,6 @@ __global__ void __launch_bounds__(128) k_ver_waves(DevGrid G, DevState so, DevSt
     }
 }
 
-/* thomas_lds for systems whose every row has one off-diagonal entry at
-   most: interface j (between rows j and j + 1) stores that entry in ce[j]
-   and in fl[j] whether it is the upper one (e_j, fl 1) or the lower one
-   (c_j, row j + 1's, fl 0); the other is 0.0, as the reference leaves it.
-   The arithmetic is thomas_lds's; the multipliers overwrite ce. */
-template <int NCOL, int NMAX>
-__device__ __forceinline__ void thomas_lds_ce(double *ce, const unsigned char *fl, const double *dd, double *rr,
-                                              int n, int col)
-{
-    const double d0 = dd[col], q0 = ce[col];
-    const bool f0 = fl[col];
-    double ep = 0.0, x;
-    if (n > 1) ep = (f0 ? q0 : 0.0)/d0;
-    x = rr[col]/d0;
-    ce[col] = ep; rr[col] = x;
-    double cp = f0 ? 0.0 : q0, dn = 0.0, rn = 0.0, qn = 0.0;
-    bool fn = false;
-    if (n > 1) { dn = dd[NCOL + col]; rn = rr[NCOL + col]; qn = ce[NCOL + col]; fn = fl[NCOL + col]; }
-#pragma unroll
-    for (int j = 1; j < NMAX; ++j) {
-        if (j >= n) break;
-        const int o = j*NCOL + col, on = (j + 1 < n ? j + 1 : j)*NCOL + col;
-        const double dnn = dd[on], rnn = rr[on], qnn = ce[on];
-        const bool fnn = fl[on];
-        const double en = fn ? qn : 0.0, cpn = fn ? 0.0 : qn;
-        const double den = dn - ep*cp;
-        if (j < n - 1) ep = en/den;
-        x = (rn - x*cp)/den;
-        ce[o] = ep; rr[o] = x;
-        cp = cpn; dn = dnn; rn = rnn; qn = qnn; fn = fnn;
-    }
-    /* back substitution, upwards */
-    double eb = 0.0, rb = 0.0;
-    if (n > 1) { eb = ce[(n - 2)*NCOL + col]; rb = rr[(n - 2)*NCOL + col]; }
-#pragma unroll
-    for (int t = 0; t < NMAX - 1; ++t) {
-        const int j = n - 2 - t;
-        if (j < 0) break;
-        const int o = j*NCOL + col, om = (j > 0 ? j - 1 : 0)*NCOL + col;
-        const double ebn = ce[om], rbn = rr[om];
-        x = rb - eb*x;
-        rr[o] = x;
-        eb = ebn; rb = rbn;
-    }
-}
-
 /* the state of box (i, j) the solver reads, loaded in one batch: old state,
    tendencies, the state snr (the new state before this substep writes it),
    volume and background exner */
@@ -1316,8 +1270,8 @@ __device__ __forceinline__ ColumnLayer vw_layer(const VwBox &x, double dt, int r
    elimination.  Four boxes per group keep three waves per SIMD (166
    registers; all of it in registers needs 206 and spills below that) and make
    a block 144 to 256 threads at any depth; the columns per block (64 up to 16
-   layers, 32 up to 32, 16 beyond) keep its LDS under 56 KiB, three blocks per
-   CU.  A lane's loads take its column and the distance of its group from the
+   layers, 32 up to 32, 16 beyond) keep its LDS under 56 KiB: three blocks per
+   CU (46 KiB at 26 layers) or two (55 KiB at 16, 32 and 63).  A lane's loads take its column and the distance of its group from the
    wave's first row as one offset to rows that are the same for the wave.
    Against the kernels for 26 and 55 layers (runs of seven boxes, the state
    read and linearised again in phase 3) and the one for other depths, us per
@@ -1467,25 +1421,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))
     }
 }
 
-/* three_band_solver_gen_densities (column_solvers.c:385-639).
-
-   The tracers of a column are independent of each other except through the
-   sediment heat, which k_sed_heat forms separately, so one block solves NCOL
-   columns of one tracer in three phases:
-     1. every thread builds rows (column, layer) of the tridiagonal system
-        into LDS -- all loads independent, fully coalesced; an interface has
-        one nonzero off-diagonal (the upstream side of its flux), stored
-        once with a flag, so a column takes three doubles and a byte per row;
-     2. one lane per column runs the Thomas elimination on LDS;
-     3. every thread writes the clipped solution back, coalesced.
-   Each coefficient is formed with the reference's arithmetic. */
-#define GD_THREADS 256
-/* columns per block: 64 at 26 layers (41 KiB of LDS, three blocks per CU;
-   60 columns and four blocks measured no faster); 32 for deeper columns
-   (43 KiB at 55 layers: three blocks per CU where four-array rows allowed
-   two, 50 KiB at 64) -- the lanes of a 32-column group are half a wave */
-__host__ __device__ constexpr int gd_ncol(int lt) { return lt == 26 ? 64 : 32; }
-
 /* vertical fluxes of tracer k through interface jj of column i
    (column_solvers.c:414-465): fi with the old wind, fr with the new wind
    times the upstream density */
@@ -1509,324 +1444,137 @@ __device__ __forceinline__ void tracer_iface_flux(const DevGrid &G, const DevSta
     fr = doi*fr;
 }
 
-template <int LT>
-__global__ void __launch_bounds__(GD_THREADS) k_gen_densities(DevGrid G, DevState so, DevState sn, DevState td,
-                                                              StepConsts K)
+/* three_band_solver_gen_densities (column_solvers.c:385-639): a block solves
+   64 columns of one tracer, wave w the rows w*GD_PER .. of each, one column
+   per lane, all of it in registers.
+     1. every wave loads its rows at once and forms them (column_solvers.c:466-615).
+        An interface has one nonzero off-diagonal, the upstream side of its
+        flux: above a row that the row above depends on (e) the row's own lower
+        entry c is 0.0, so the pivot d - (e/d)*c of the elimination
+        (column_solvers.c:641-660) is d exactly and the quotients e/d of all
+        rows are formed here, in parallel;
+     2. the waves take turns downwards with x = (r - x*c)/d, the last row's x
+        handed on in LDS, and upwards with x - (e/d)*x;
+     3. each wave writes its clipped rows (column_solvers.c:616-637).
+   What the rows' loads and the turns leave idle other blocks fill, so the
+   columns in flight count: nine rows per wave take 148 registers and three
+   waves at 26 layers (four blocks per CU), seven rows 120 registers and eight
+   waves at 55 layers (two).  us per launch, against rows staged in LDS for one
+   lane per system (five tracers per block at 26 layers, one otherwise) and
+   here with 5, 7 and 9 rows:
+     res 7 x 26   187 -> 229, 174, 168 (680 MB: 4.0 TB/s)
+     res 5 x 26    19 -> 19.1, 15.3, 14.8
+     res 5 x 41    47 -> 39.6, 30.6, 37.9
+     res 6 x 55   139 -> 168, 102, 175 (360 MB: 3.5 TB/s)
+   One lane per system with its column in LDS took 175, 33 and 166 us at
+   res 7 x 26, 5 x 41 and 6 x 55: six waves per CU at 26 layers, two at 55. */
+template <int GD_PER, int NT>
+__global__ void __launch_bounds__(NT) k_gen_densities(DevGrid G, DevState so, DevState sn, DevState td, StepConsts K)
 {
-    extern __shared__ double lds[];
-    constexpr int GD_NCOL = gd_ncol(LT);
-    const int L = LT > 0 ? LT : G.L, nsh = G.nsh, ncc = G.n_cond;
+    __shared__ double hand[64];
+    const int L = G.L, nsh = G.nsh, ncc = G.n_cond, vpl = G.vpl;
     /* the tracer is the fast block index: the blocks of one group of columns
        run side by side on one XCD and share the wind, area and volume columns in L2 */
-    const unsigned ntr = (unsigned)G.n_const - 1, blk = xcd_x();
-    const int tr = (int)(blk%ntr);
+    const unsigned ntr = (unsigned)G.n_const - 1, blk = xcd_x(), grp = blk/ntr;
+    const int tr = (int)(blk - grp*ntr);
     const int k = tr < ncc ? tr : tr + 1;   /* skip the gas */
-    const int i0 = (int)(blk/ntr)*GD_NCOL;
-    if (i0 >= nsh) return;
+    const unsigned lane = threadIdx.x & 63u;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nw = (int)(blockDim.x >> 6);
+    /* lanes past the last column solve the last one again and write nothing */
+    const bool mine = grp*64 + lane < (unsigned)nsh;
+    const unsigned i = mine ? grp*64 + lane : (unsigned)nsh - 1;
     const double iw = 0.5, ew = 1.0 - iw, dt = K.dt;
-    const double *vol = G.vol, *area = G.area;
-    const double *rho_o = so.rho + (i64)k*G.s;
-    const double *trho = td.rho + (i64)k*G.s;
-    double vsink = 0.0;
-    if (k < ncc/4) vsink = K.snow_v;
-    else if (k < ncc/2) vsink = K.rain_v;
-    else if (k < ncc) vsink = K.cloud_v;
-    /* one off-diagonal per interface (the flux's sign picks c or e), so three
-       arrays of doubles and one of flags */
-    double *ce = lds, *dd = lds + L*GD_NCOL, *rr = lds + 2*L*GD_NCOL;
-    unsigned char *fl = (unsigned char *)(lds + 3*L*GD_NCOL);
-
-    /* phase 1: rows (column_solvers.c:466-615).  Each wave takes a run of
-       layers of the block's columns (lane = column, so every load is
-       coalesced) and walks down it: the flux through the interface below
-       row j is the flux above row j+1, formed once.  (iw dt)/vol comes from
-       the per-box table the runtime keeps for the current dt: the same
-       quotient, formed once instead of once per tracer and row.  The inputs
-       of every row of the run are loaded before the first row is formed
-       (indices clamped in range; a step past the run repeats its last row
-       and writes nothing), so the walk waits on memory once, not once per
-       row: about fifty loads in flight per wave, within the registers the
-       LDS-bound occupancy leaves (206 -> 200 us at 26 layers, res 7, and
-       524 -> 516 us at 55, against one row ahead).  Lanes past the last
-       column compute the last column's rows; phases 2 and 3 skip them. */
+    const double *rho_o = so.rho + (i64)k*G.s, *trho = td.rho + (i64)k*G.s;
+    const bool cond = k < ncc;
+    const double sv = k < ncc/4 ? K.snow_v : (k < ncc/2 ? K.rain_v : (cond ? K.cloud_v : 0.0));
+    /* rows j0 .. j0 + GD_PER - 1 < L; rows past the last are loaded as the last
+       and not used (every wave has at least one row) */
+    const int j0 = w*GD_PER;
+    double r[GD_PER], d[GD_PER], c[GD_PER], ep[GD_PER];
     {
-        constexpr int NW = GD_THREADS/GD_NCOL;
-        constexpr int PER_MAX = ((LT > 0 ? LT : GAME_MAX_LAYERS) + NW - 1)/NW;
-        const int per = (L + NW - 1)/NW;
-        const int w = threadIdx.x/GD_NCOL, col = threadIdx.x - w*GD_NCOL;
-        const int i = i0 + col < nsh ? i0 + col : nsh - 1;
-        const int j0 = w*per, j1 = j0 + per < L ? j0 + per : L;
-        const double *idv = G.idv;
-        const int vpl = G.vpl;
-        const double sv = k < ncc/4 ? K.snow_v : (k < ncc/2 ? K.rain_v : (k < ncc ? K.cloud_v : 0.0));
-        /* the bottom row's sedimentation terms: surface area and lowest density */
-        const double a_sfc = area[i + G.v - nsh], r_low = rho_o[i + G.s - nsh];
-        struct In { double wo, wn, a, dlo, dup, q, qlo, v, rb, tb; };
-        /* the loads of row j and of the interface below it */
-        auto load = [&](int j) {
-            In x;
-            const int jc = j < L - 1 ? j : L - 2;
-            const i64 wi = i + (i64)(jc + 1)*vpl, bc = i + (i64)jc*nsh, b = i + (i64)j*nsh;
-            x.wo = so.wind[wi]; x.wn = sn.wind[wi]; x.a = area[wi];
-            x.dlo = rho_o[bc + nsh]; x.dup = rho_o[bc];
-            x.q = idv[b]; x.qlo = idv[j < L - 1 ? b + nsh : b];
-            x.v = vol[b]; x.rb = rho_o[b]; x.tb = trho[b];
-            return x;
-        };
-        /* the same for row j + 1 of the walk, given row j: its density above
-           the interface, its own density and its quotient are row j's
-           density below and quotient below (for the last row the first is
-           not used), so three of the ten values come from registers */
-        auto load_next = [&](int j, const In &prev) {
-            In x;
-            const int jc = j < L - 1 ? j : L - 2;
-            const i64 wi = i + (i64)(jc + 1)*vpl, bc = i + (i64)jc*nsh, b = i + (i64)j*nsh;
-            x.wo = so.wind[wi]; x.wn = sn.wind[wi]; x.a = area[wi];
-            x.dlo = rho_o[bc + nsh]; x.dup = prev.dlo;
-            x.q = prev.qlo; x.qlo = idv[j < L - 1 ? b + nsh : b];
-            x.v = vol[b]; x.rb = prev.dlo; x.tb = trho[b];
-            return x;
-        };
-        /* interface fluxes (column_solvers.c:414-465) */
-        auto iface = [&](const In &x, int jj, double &fi, double &fr) {
-            double wo = x.wo, wn = x.wn;
-            if (k < ncc) { wo -= sv; wn -= sv; }
-            wo = x.a*wo;
-            wn = x.a*wn;
-            const double doi = (wn >= 0.0) ? x.dlo : x.dup;
-            fi = jj < L - 1 ? wo : 0.0;
-            fr = jj < L - 1 ? doi*wn : 0.0;
-        };
-        /* a wave whose run starts past the last layer (more waves than runs
-           when L is small against the waves of the block) has no row: it
-           loads nothing */
-        if (j0 < j1) {
-            double fi_m = 0.0, fr_m = 0.0;
-            /* every load of the run is issued before the first row is formed:
-               the interface above the run (its flux enters the first row;
-               interface 0 stands in, unused, for the top run), then the rows
-               (a step past the run's end repeats its last row, unused) */
-            In xm;
-            {
-                const int jm = j0 > 0 ? j0 - 1 : 0;
-                const i64 wi = i + (i64)(jm + 1)*vpl, bc = i + (i64)jm*nsh;
-                xm.wo = so.wind[wi]; xm.wn = sn.wind[wi]; xm.a = area[wi];
-                xm.dlo = rho_o[bc + nsh]; xm.dup = rho_o[bc];
-            }
-            In xs[PER_MAX];
-            xs[0] = load(j0);
+        const int jm = j0 > 0 ? j0 - 1 : 0;
+        const i64 wm = (i64)(jm + 1)*vpl;
+        const double wo_m = at(so.wind + wm, i), wn_m = at(sn.wind + wm, i), a_m = at(G.area + wm, i);
+        const double up_m = at(rho_o + (i64)jm*nsh, i), r_low = at(rho_o + (i64)(L - 1)*nsh, i);
+        const double a_sfc = at(G.area + (i64)L*vpl, i);
+        double rb = at(rho_o + (i64)j0*nsh, i), q = at(G.idv + (i64)j0*nsh, i);   /* q = iw*dt/vol, kept for the current dt */
+        double wo[GD_PER], wn[GD_PER], a[GD_PER], dlo[GD_PER], qlo[GD_PER], v[GD_PER], tb[GD_PER];
 #pragma unroll
-            for (int t = 1; t < PER_MAX; ++t) xs[t] = load_next(j0 + t < j1 ? j0 + t : j1 - 1, xs[t - 1]);
-            if (j0 > 0) iface(xm, j0 - 1, fi_m, fr_m);
+        for (int t = 0; t < GD_PER; ++t) {
+            const int j = j0 + t < L ? j0 + t : L - 1, jc = j < L - 1 ? j : L - 2;
+            const i64 wi = (i64)(jc + 1)*vpl, b = (i64)j*nsh, lo = (i64)(jc + 1)*nsh;
+            wo[t] = at(so.wind + wi, i); wn[t] = at(sn.wind + wi, i); a[t] = at(G.area + wi, i);
+            dlo[t] = at(rho_o + lo, i); qlo[t] = at(G.idv + lo, i);
+            v[t] = at(G.vol + b, i); tb[t] = at(trho + b, i);
+        }
+        /* the interface above the first row (column_solvers.c:414-465): fi with
+           the old wind, fr with the new one times the upstream density; the
+           top row has none: no fi, and an fr and a c of zero */
+        double fi_m = -1.0, fr_m = 0.0, c_m = 0.0;
+        if (j0 > 0) {
+            const double fn = a_m*(wn_m - sv);
+            fi_m = a_m*(wo_m - sv);
+            fr_m = (fn >= 0.0 ? rb : up_m)*fn;
+            c_m = fi_m >= 0.0 ? 0.0 : q*fi_m;
+        }
 #pragma unroll
-            for (int t = 0; t < PER_MAX; ++t) {
-                const bool valid = j0 + t < j1;
-                const int j = valid ? j0 + t : j1 - 1;
-                const In &cur = xs[t];
-                const int idx = j*GD_NCOL + col;
-                double fi, fr;
-                iface(cur, j, fi, fr);
-                const double q = cur.q, v = cur.v;   /* q = iw*dt/vol[b] */
-                double d;
-                if (j == 0) d = (fi >= 0.0) ? 1.0 : 1.0 - q*fi;
-                else if (j == L - 1) {
-                    d = (fi_m >= 0.0) ? 1.0 + q*fi_m : 1.0;
-                    if (k < ncc) d += iw*vsink*dt*a_sfc/v;
-                } else {
-                    d = 1.0;
-                    if (fi_m >= 0.0) d += q*fi_m;
-                    if (fi < 0.0) d -= q*fi;
-                }
-                double r = cur.rb + dt*cur.tb;
-                if (j == 0) r += ew*dt*fr/v;
-                else if (j == L - 1) {
-                    r += -ew*dt*fr_m/v;
-                    if (k < ncc) r += -ew*vsink*dt*r_low*a_sfc/v;
-                } else r += ew*dt*(-fr_m + fr)/v;
-                /* off-diagonals of interface j (column_solvers.c:475-488);
-                   -iw*dt/vol*fi is (-(iw*dt/vol))*fi exactly; the other one
-                   stays 0.0 */
-                double o = 0.0;
-                const bool up = fi >= 0.0;
-                if (j < L - 1) o = up ? (-q)*fi : cur.qlo*fi;
-                if (valid) { ce[idx] = o; fl[idx] = up; dd[idx] = d; rr[idx] = r; }
-                fi_m = fi;
-                fr_m = fr;
+        for (int t = 0; t < GD_PER; ++t) {
+            const bool last = j0 + t >= L - 1;
+            const double fn = a[t]*(wn[t] - sv);
+            const double doi = fn >= 0.0 ? dlo[t] : rb;
+            const double fi = last ? 0.0 : a[t]*(wo[t] - sv), fr = last ? -0.0 : doi*fn;
+            double dj = 1.0, rj = rb + dt*tb[t];
+            if (fi_m >= 0.0) dj += q*fi_m;
+            if (fi < 0.0) dj -= q*fi;
+            rj += ew*dt*(-fr_m + fr)/v[t];
+            if (last && cond) {
+                dj += iw*sv*dt*a_sfc/v[t];
+                rj += -ew*sv*dt*r_low*a_sfc/v[t];
             }
+            const bool up = fi >= 0.0;
+            r[t] = rj;
+            d[t] = dj;
+            c[t] = c_m;
+            ep[t] = up && !last ? (-q)*fi/dj : 0.0;
+            c_m = up ? 0.0 : qlo[t]*fi;
+            fi_m = fi;
+            fr_m = fr;
+            rb = dlo[t];
+            q = qlo[t];
         }
     }
-    __syncthreads();
-    /* phase 2: Thomas algorithm (column_solvers.c:641-667), one lane per column;
-       the multipliers overwrite e, the solution overwrites r */
-    if (threadIdx.x < GD_NCOL && i0 + (int)threadIdx.x < nsh)
-        thomas_lds_ce<GD_NCOL, (LT > 0 ? LT : GAME_MAX_LAYERS)>(ce, fl, dd, rr, L, threadIdx.x);
-    __syncthreads();
-    /* phase 3: clipped solution (column_solvers.c:616-637) */
+    double x = 0.0;
+    for (int s = 0; s < nw; ++s) {
+        if (w == s) {
+            if (s > 0) x = hand[lane];
+#pragma unroll
+            for (int t = 0; t < GD_PER; ++t)
+                if (j0 + t < L) { x = (r[t] - x*c[t])/d[t]; r[t] = x; }
+            if (s < nw - 1) hand[lane] = x;
+        }
+        __syncthreads();
+    }
     double *rho_n = sn.rho + (i64)k*G.s;
-    for (int idx = threadIdx.x; idx < L*GD_NCOL; idx += GD_THREADS) {
-        const int j = idx/GD_NCOL, col = idx - j*GD_NCOL, i = i0 + col;
-        if (i >= nsh) continue;
-        double v = rr[idx];
-        if (v < 0.0) v = 0.0;
-        rho_n[i + (i64)j*nsh] = v;
-    }
-}
-
-/* The moist tracer solve with the five tracers of a group of NCOLS columns in
-   one block (the default at 26 layers; k_gen_densities above is the
-   one-tracer-per-block form, the default otherwise).  A row's inputs that every tracer shares --
-   the old and new vertical wind and the area of the interface below it, the
-   volume and (iw dt)/volume -- are loaded once for the five tracers, and a
-   tracer's density above an interface is the one below the interface
-   above, carried down the run, so phase 1 issues 16 loads per row instead
-   of 35.  Tracer t is constituent t for the four condensates (snow, rain,
-   cloud ice, cloud water: t < 4) and constituent 5 for the vapour; the gas
-   (constituent 4) has no tracer solve.  Each coefficient is formed with
-   the arithmetic of k_gen_densities, phase 2 runs one lane per (tracer,
-   column) system and phase 3 writes the five tracers back, coalesced along
-   the columns. */
-template <int LT, int NCOLS, int NT>
-__global__ void __launch_bounds__(NT) k_gen_densities_all(DevGrid G, DevState so, DevState sn, DevState td,
-                                                          StepConsts K)
-{
-    extern __shared__ double lds[];
-    constexpr int NTR = 5, NSYS = NTR*NCOLS, NW = NT/NCOLS, L = LT, PER = (L + NW - 1)/NW;
-    static_assert(NSYS <= NT, "one lane per system in phase 2");
-    const int nsh = G.nsh, vpl = G.vpl;
-    const i64 S = G.s;
-    const int i0 = (int)xcd_x()*NCOLS;
-    if (i0 >= nsh) return;
-    const double iw = 0.5, ew = 1.0 - iw, dt = K.dt;
-    double *ce = lds, *dd = lds + L*NSYS, *rr = lds + 2*L*NSYS;
-    unsigned char *fl = (unsigned char *)(lds + 3*L*NSYS);
-    /* tracer t's constituent and sinking speed (column_solvers.c:414-465) */
-    auto kof = [](int t) { return t < 4 ? t : 5; };
-    auto vs = [&](int t) { return t < 1 ? K.snow_v : (t < 2 ? K.rain_v : (t < 4 ? K.cloud_v : 0.0)); };
-
-    /* phase 1: rows j0..j1-1 of the five tracers of column col
-       (column_solvers.c:466-615).  Every load of the run is issued before
-       the first row is formed (a step past the run's end repeats its last
-       row and writes nothing); a run starting past the last layer loads
-       nothing.  Lanes past the last column compute the last column's rows;
-       phases 2 and 3 skip them. */
-    {
-        const int w = threadIdx.x/NCOLS, col = threadIdx.x - w*NCOLS;
-        const int i = i0 + col < nsh ? i0 + col : nsh - 1;
-        const int j0 = w*PER, j1 = j0 + PER < L ? j0 + PER : L;
-        if (j0 < j1) {
-            const double a_sfc = G.area[i + G.v - nsh];
-            /* the interface above the run (its fluxes enter the first row;
-               interface 0 stands in, unused, for the top run) */
-            const int jm = j0 > 0 ? j0 - 1 : 0;
-            const i64 wim = i + (i64)(jm + 1)*vpl;
-            const double wo_m = so.wind[wim], wn_m = sn.wind[wim], a_m = G.area[wim];
-            /* per tracer: the density of the run's first row, of the row
-               above it and of the lowest layer */
-            double r0[NTR], dup_m[NTR], r_low[NTR];
+    for (int s = nw - 1; s >= 0; --s) {
+        if (w == s) {
+            if (s < nw - 1) x = hand[lane];
 #pragma unroll
-            for (int t = 0; t < NTR; ++t) {
-                const double *ro = so.rho + (i64)kof(t)*S;
-                r0[t] = ro[i + (i64)j0*nsh];
-                dup_m[t] = ro[i + (i64)jm*nsh];
-                r_low[t] = ro[i + S - nsh];
-            }
-            /* per row j: the interface below it (jc, clamped to the lowest
-               interface for the last row, whose fluxes are zero) */
-            double wo[PER], wn[PER], ar[PER], q[PER], qlo[PER], v[PER], dlo[PER][NTR], tb[PER][NTR];
-#pragma unroll
-            for (int u = 0; u < PER; ++u) {
-                const int j = j0 + u < j1 ? j0 + u : j1 - 1;
-                const int jc = j < L - 1 ? j : L - 2;
-                const i64 wi = i + (i64)(jc + 1)*vpl, b = i + (i64)j*nsh;
-                wo[u] = so.wind[wi]; wn[u] = sn.wind[wi]; ar[u] = G.area[wi];
-                q[u] = G.idv[b]; qlo[u] = G.idv[j < L - 1 ? b + nsh : b]; v[u] = G.vol[b];
-#pragma unroll
-                for (int t = 0; t < NTR; ++t) {
-                    const i64 kS = (i64)kof(t)*S;
-                    dlo[u][t] = so.rho[kS + i + (i64)(jc + 1)*nsh];
-                    tb[u][t] = td.rho[kS + b];
-                }
-            }
-            double fi_m[NTR], fr_m[NTR];
-#pragma unroll
-            for (int t = 0; t < NTR; ++t) {
-                fi_m[t] = 0.0;
-                fr_m[t] = 0.0;
-                if (j0 > 0) {
-                    double o_ = wo_m, n_ = wn_m;
-                    if (t < 4) { o_ -= vs(t); n_ -= vs(t); }
-                    o_ = a_m*o_;
-                    n_ = a_m*n_;
-                    const double doi = (n_ >= 0.0) ? r0[t] : dup_m[t];
-                    fi_m[t] = o_;
-                    fr_m[t] = doi*n_;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < PER; ++u) {
-                const bool valid = j0 + u < j1;
-                const int j = valid ? j0 + u : j1 - 1;
-                const double qq = q[u], vv = v[u];
-#pragma unroll
-                for (int t = 0; t < NTR; ++t) {
-                    const double sv = vs(t);
-                    /* the row's own density, which is also the density above
-                       its interface below (fluxes of the last row are zero) */
-                    const double rb = u == 0 ? r0[t] : dlo[u - 1][t];
-                    double wo_ = wo[u], wn_ = wn[u];
-                    if (t < 4) { wo_ -= sv; wn_ -= sv; }
-                    wo_ = ar[u]*wo_;
-                    wn_ = ar[u]*wn_;
-                    const double doi = (wn_ >= 0.0) ? dlo[u][t] : rb;
-                    const double fi = j < L - 1 ? wo_ : 0.0;
-                    const double fr = j < L - 1 ? doi*wn_ : 0.0;
-                    double d;
-                    if (j == 0) d = (fi >= 0.0) ? 1.0 : 1.0 - qq*fi;
-                    else if (j == L - 1) {
-                        d = (fi_m[t] >= 0.0) ? 1.0 + qq*fi_m[t] : 1.0;
-                        if (t < 4) d += iw*sv*dt*a_sfc/vv;
-                    } else {
-                        d = 1.0;
-                        if (fi_m[t] >= 0.0) d += qq*fi_m[t];
-                        if (fi < 0.0) d -= qq*fi;
-                    }
-                    double r = rb + dt*tb[u][t];
-                    if (j == 0) r += ew*dt*fr/vv;
-                    else if (j == L - 1) {
-                        r += -ew*dt*fr_m[t]/vv;
-                        if (t < 4) r += -ew*sv*dt*r_low[t]*a_sfc/vv;
-                    } else r += ew*dt*(-fr_m[t] + fr)/vv;
-                    /* off-diagonals of interface j (column_solvers.c:475-488) */
-                    double o = 0.0;
-                    const bool up = fi >= 0.0;
-                    if (j < L - 1) o = up ? (-qq)*fi : qlo[u]*fi;
-                    const int idx = j*NSYS + t*NCOLS + col;
-                    if (valid) { ce[idx] = o; fl[idx] = up; dd[idx] = d; rr[idx] = r; }
-                    fi_m[t] = fi;
-                    fr_m[t] = fr;
-                }
-            }
+            for (int t = GD_PER - 1; t >= 0; --t)
+                if (j0 + t < L) { x = j0 + t < L - 1 ? r[t] - ep[t]*x : r[t]; r[t] = x; }
+            if (s > 0) hand[lane] = x;
         }
+        if (s > 0) __syncthreads();
     }
-    __syncthreads();
-    /* phase 2: Thomas algorithm (column_solvers.c:641-667), lane = system */
-    if (threadIdx.x < NSYS && i0 + (int)(threadIdx.x%NCOLS) < nsh)
-        thomas_lds_ce<NSYS, L>(ce, fl, dd, rr, L, threadIdx.x);
-    __syncthreads();
-    /* phase 3: clipped solution (column_solvers.c:616-637) */
-    for (int idx = threadIdx.x; idx < L*NSYS; idx += NT) {
-        const int j = idx/NSYS, sys = idx - j*NSYS, t = sys/NCOLS, col = sys - t*NCOLS, i = i0 + col;
-        if (i >= nsh) continue;
-        double x = rr[idx];
-        if (x < 0.0) x = 0.0;
-        sn.rho[(i64)kof(t)*S + i + (i64)j*nsh] = x;
-    }
+    if (!mine) return;
+#pragma unroll
+    for (int t = 0; t < GD_PER; ++t)
+        if (j0 + t < L) put(rho_n + (i64)(j0 + t)*nsh, i, r[t] < 0.0 ? 0.0 : r[t]);
 }
 
 /* The same tracer solve with one (column, tracer) per lane, the rows
    generated and eliminated in one downward sweep through registers (the
    layout k_ver_waves uses); selected with GAME_GPU_GD_STREAMING for
-   measurement against the LDS-staged kernel above. */
+   measurement against the kernel above. */
 template <int LT>
 __global__ void __launch_bounds__(128) k_gen_densities_stream(DevGrid G, DevState so, DevState sn, DevState td,
                                                               StepConsts K)
@@ -1898,57 +1646,73 @@ __global__ void __launch_bounds__(128) k_gen_densities_stream(DevGrid G, DevStat
 }
 
 /* sediment heat of the condensates at rk 0 (column_solvers.c:414-465 and the
-   sh updates of :500-611): one thread per grid box adds the contributions of
-   the condensates in the reference's constituent order, starting from 0 */
-template <typename TW, int NCC>
+   sh updates of :500-611), a chunk of RUN boxes of a column per thread: the
+   flux of each condensate through each interface is formed once, the
+   contributions are added in the reference's constituent order, starting
+   from 0, and every load of the chunk is issued before its first store */
+template <typename TW, int NCC, int RUN>
 __global__ void __launch_bounds__(TPB) k_sed_heat(DevGrid G, DevState so, DevState sn, const TW *T, const TW *cpc,
                                                   TW *sed_heat, StepConsts K, Span sp)
 {
     const Blk bk = xcd_block(sp);
-    const int i = (int)(bk.x*TPB + threadIdx.x);
-    if (i >= G.nsh) return;
-    /* NCC: the condensate count at compile time, so both loops unroll */
+    const unsigned i = bk.x*TPB + threadIdx.x;
+    if (i >= (unsigned)G.nsh) return;
     const int nsh = G.nsh, vpl = G.vpl, L = G.L;
-    constexpr int ncc = NCC;
-    const int j = (int)bk.y;
-    const i64 b = (i64)j*nsh + i;
-    const double *vol = G.vol, *area = G.area;
-    double sh = 0.0;
+    const i64 S = G.s;
+    int l0, l1;
+    layer_chunk(L, bk.y, RUN, l0, l1);
+    if (l0 >= l1) return;
+    /* box l0 - 1 + t, and the interface above box l0 + t; a step past the
+       chunk or the column repeats the nearest row and is not used */
+    double d[RUN + 2][NCC], c[RUN + 2][2], tt[RUN + 2], wn[RUN + 1], a[RUN + 1], v[RUN];
 #pragma unroll
-    for (int k = 0; k < ncc; ++k) {
-        const double *rho_o = so.rho + (i64)k*G.s;
-        double vsink;
-        if (k < ncc/4) vsink = K.snow_v;
-        else if (k < ncc/2) vsink = K.rain_v;
-        else vsink = K.cloud_v;
-        double fe = 0.0, fe_m = 0.0;
+    for (int t = 0; t < RUN + 2; ++t) {
+        const int j = l0 - 1 + t < 0 ? 0 : (l0 - 1 + t < L ? l0 - 1 + t : L - 1);
+        const i64 b = (i64)j*nsh;
 #pragma unroll
-        for (int pass = 0; pass < 2; ++pass) {
-            const int jj = pass == 0 ? j : j - 1;
-            if (jj < 0 || jj > L - 2) continue;
-            double fr = sn.wind[i + (i64)(jj + 1)*vpl];
-            fr -= vsink;
-            fr = area[i + (i64)(jj + 1)*vpl]*fr;
-            const i64 bb = i + (i64)jj*nsh;
-            /* the upstream box is chosen after both are loaded */
-            const bool lo = fr >= 0.0;
-            const double d0 = rho_o[bb + nsh], d1 = rho_o[bb];
-            const double t0 = (double)T[bb + nsh], t1 = (double)T[bb];
-            const double c0 = (double)cpc[(i64)(k & 1)*G.s + bb + nsh], c1 = (double)cpc[(i64)(k & 1)*G.s + bb];
-            const double doi = lo ? d0 : d1, toi = lo ? t0 : t1, cpi = lo ? c0 : c1;
-            fr = doi*fr;
-            const double f = cpi*toi*fr;
-            if (pass == 0) fe = f; else fe_m = f;
-        }
-        if (j == 0) sh += fe/vol[b];
-        else if (j == L - 1) {
-            const i64 low = i + G.s - nsh, sfc = i + G.v - nsh;
-            sh += -fe_m/vol[b];
-            const double tl = (double)T[low];
-            sh += -vsink*tl*(double)cpc[(i64)(k & 1)*G.s + low]*rho_o[low]*area[sfc]/vol[b];
-        } else sh += (-fe_m + fe)/vol[b];
+        for (int k = 0; k < NCC; ++k) d[t][k] = at(so.rho + k*S + b, i);
+        c[t][0] = (double)at(cpc + b, i);
+        c[t][1] = (double)at(cpc + S + b, i);
+        tt[t] = (double)at(T + b, i);
     }
-    sed_heat[b] = (TW)sh;
+#pragma unroll
+    for (int t = 0; t < RUN + 1; ++t) {
+        const int j = l0 + t < L ? l0 + t : L;
+        wn[t] = at(sn.wind + (i64)j*vpl, i);
+        a[t] = at(G.area + (i64)j*vpl, i);
+    }
+#pragma unroll
+    for (int t = 0; t < RUN; ++t) v[t] = at(G.vol + (i64)(l0 + t < L ? l0 + t : L - 1)*nsh, i);
+    double sh[RUN];
+#pragma unroll
+    for (int t = 0; t < RUN; ++t) sh[t] = 0.0;
+#pragma unroll
+    for (int k = 0; k < NCC; ++k) {
+        const double sv = k < NCC/4 ? K.snow_v : (k < NCC/2 ? K.rain_v : K.cloud_v);
+        /* through the interface above box l0 + t (column_solvers.c:414-465) */
+        auto flux = [&](int t) {
+            double fr = a[t]*(wn[t] - sv);
+            const bool lo = fr >= 0.0;
+            const double doi = lo ? d[t + 1][k] : d[t][k], toi = lo ? tt[t + 1] : tt[t], cpi = lo ? c[t + 1][k & 1] : c[t][k & 1];
+            fr = doi*fr;
+            return cpi*toi*fr;
+        };
+        double f = flux(0);
+#pragma unroll
+        for (int t = 0; t < RUN; ++t) {
+            const int j = l0 + t;
+            const double fl = flux(t + 1);
+            if (j == 0) sh[t] += fl/v[t];
+            else if (j == L - 1) {
+                sh[t] += -f/v[t];
+                /* a[t + 1] is the surface's area */
+                sh[t] += -sv*tt[t + 1]*c[t + 1][k & 1]*d[t + 1][k]*a[t + 1]/v[t];
+            } else sh[t] += (-f + fl)/v[t];
+            f = fl;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < RUN; ++t) if (l0 + t < l1) put(sed_heat + (i64)(l0 + t)*nsh, i, (TW)sh[t]);
 }
 
 /* The same sums with one thread per column walking down its layers: the flux
@@ -2593,64 +2357,49 @@ static void gen_densities_only(const DevGrid &G, const DevState &so, const DevSt
         else LAUNCH("k_gen_densities", k_gen_densities_stream<0>, g, b, st, G, so, sn, td, K);
         return;
     }
-    if (G.n_const == 6 && G.n_cond == 4 && !G.gd_per_tracer && G.L == 26) {
-        /* five tracers per block at 26 layers: 16 columns and 256 threads
-           (51 KiB of LDS, three blocks per CU), res 7: 190 us against 200
-           for one tracer per block; 8 columns and 128 threads 224 us, 12
-           columns 196 us (256 threads) and 204 us (192).  At 55 layers 8
-           columns (54 KiB, two blocks per CU) took 701 us against 516:
-           fewer systems in flight for the longer serial elimination */
-        constexpr int NCOLS = 16, NT = 256;
-        const dim3 g((unsigned)((G.nsh + NCOLS - 1)/NCOLS)), b(NT);
-        size_t lds = (size_t)3*26*5*NCOLS*sizeof(double) + (((size_t)26*5*NCOLS + 7) & ~(size_t)7);
-        LAUNCH_SHM("k_gen_densities", (k_gen_densities_all<26, NCOLS, NT>), g, b, lds, st, G, so, sn, td, K);
-        return;
-    }
-    const int ncol = gd_ncol(G.L == 26 ? 26 : (G.L == 55 ? 55 : 0));
-    const dim3 g((unsigned)(((G.nsh + ncol - 1)/ncol)*(G.n_const - 1))), b(GD_THREADS);
-    /* 41 KiB at 26 layers, 43 KiB at 55, 50 KiB at 64 */
-    size_t lds = (size_t)3*G.L*ncol*sizeof(double) + (((size_t)G.L*ncol + 7) & ~(size_t)7);
-    if (G.L == 26) LAUNCH_SHM("k_gen_densities", k_gen_densities<26>, g, b, lds, st, G, so, sn, td, K);
-    else if (G.L == 55) LAUNCH_SHM("k_gen_densities", k_gen_densities<55>, g, b, lds, st, G, so, sn, td, K);
-    else LAUNCH_SHM("k_gen_densities", k_gen_densities<0>, g, b, lds, st, G, so, sn, td, K);
+    /* nine rows per wave up to 27 layers, seven beyond (k_gen_densities) */
+    const int per = G.L <= 27 ? 9 : 7, nw = (G.L + per - 1)/per;
+    const dim3 g((unsigned)(((G.nsh + 63)/64)*(G.n_const - 1))), b((unsigned)(64*nw));
+    static_assert(64*((27 + 8)/9) <= 192 && 64*((GAME_MAX_LAYERS + 6)/7) <= 640, "the blocks' threads");
+    if (per == 9) LAUNCH("k_gen_densities", (k_gen_densities<9, 192>), g, b, st, G, so, sn, td, K);
+    else LAUNCH("k_gen_densities", (k_gen_densities<7, 640>), g, b, st, G, so, sn, td, K);
 }
 
-/* one thread per column loads each box once, one per box twice; but the
-   columns of a res 6 grid (161 blocks) leave most of the chip idle: 35, 38
-   and 55 us per launch at res 4, 5 and 6 x 26 by column, 7, 14 and 49 by box,
-   and 101 against 242 at res 7 (641 blocks) */
-static bool sed_heat_by_column(const DevGrid &G)
-{ return G.n_cond == 4 && !G.sh_per_box && (G.nsh + TPB - 1)/TPB >= 256; }
+/* A chunk of five layers loads 13 values per box where one of one layer loads
+   26, at 146 registers and three waves per SIMD; a grid that chunks of five
+   leave short of blocks takes two.  us per launch with one, two, five and
+   seven layers: res 5 x 41 9.2, 9.1, 10.5, 10.6; res 6 x 55 57, 43, 34, 35
+   (71 by column); res 7 x 26 FP64 146, 113, 88, 83 and mixed 117, 86, 72, 69.
+   Above 256 blocks of columns one thread per column loads each box once: 77
+   and 64 at res 7 x 26 (38 at res 5, where the 41 blocks leave the chip idle) */
+template <typename TW>
+static void sed_heat_t(const DevGrid &G, const DevState &so, const DevState &sn, const TW *T, const TW *cpc, TW *sed_heat,
+                       const StepConsts &K, hipStream_t st)
+{
+    const int bc = (G.nsh + TPB - 1)/TPB;
+    if (G.L == 26 && bc >= 256 && !G.sh_per_box) {
+        LAUNCH("k_sed_heat", (k_sed_heat_col<TW, 4, 26>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K);
+        return;
+    }
+    const int run = G.sh_per_box ? 1 : (bc*G.L < 4096 ? 2 : 5);
+    const dim3 g = grid_of(G.nsh, (G.L + run - 1)/run), b(TPB);
+    const Span sp = span_of(G.nsh, 1, 1);
+    if (run == 1) LAUNCH("k_sed_heat", (k_sed_heat<TW, 4, 1>), g, b, st, G, so, sn, T, cpc, sed_heat, K, sp);
+    else if (run == 2) LAUNCH("k_sed_heat", (k_sed_heat<TW, 4, 2>), g, b, st, G, so, sn, T, cpc, sed_heat, K, sp);
+    else LAUNCH("k_sed_heat", (k_sed_heat<TW, 4, 5>), g, b, st, G, so, sn, T, cpc, sed_heat, K, sp);
+}
 
 void gen_densities(const DevGrid &G, const DevState &so, const DevState &sn, const DevState &td, const double *T,
                    const double *cpc, double *sed_heat, const StepConsts &K, int rk, hipStream_t st)
 {
-    if (rk == 0 && G.n_cond > 0) {
-        if (sed_heat_by_column(G) && G.L == 26)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 26>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
-                   K);
-        else if (sed_heat_by_column(G) && G.L == 55)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<double, 4, 55>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
-                   K);
-        else LAUNCH("k_sed_heat", (k_sed_heat<double, 4>), grid_of(G.nsh, G.L), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K,
-                    span_of(G.nsh, 1, 1));
-    }
+    if (rk == 0 && G.n_cond > 0) sed_heat_t(G, so, sn, T, cpc, sed_heat, K, st);
     gen_densities_only(G, so, sn, td, K, st);
 }
 
 void gen_densities(const DevGrid &G, const DevState &so, const DevState &sn, const DevState &td, const float *T,
                    const float *cpc, float *sed_heat, const StepConsts &K, int rk, hipStream_t st)
 {
-    if (rk == 0 && G.n_cond > 0) {
-        if (sed_heat_by_column(G) && G.L == 26)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 26>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
-                   K);
-        else if (sed_heat_by_column(G) && G.L == 55)
-            LAUNCH("k_sed_heat", (k_sed_heat_col<float, 4, 55>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat,
-                   K);
-        else LAUNCH("k_sed_heat", (k_sed_heat<float, 4>), grid_of(G.nsh, G.L), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K,
-                    span_of(G.nsh, 1, 1));
-    }
+    if (rk == 0 && G.n_cond > 0) sed_heat_t(G, so, sn, T, cpc, sed_heat, K, st);
     gen_densities_only(G, so, sn, td, K, st);
 }
 

@@ -261,7 +261,6 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
     if (getenv("GAME_GPU_NO_FLAT_SHORTCUT")) G.flat = 0;
     set_layer_splits(G);
     G.gd_streaming = getenv("GAME_GPU_GD_STREAMING") ? 1 : 0;
-    G.gd_per_tracer = getenv("GAME_GPU_GD_PER_TRACER") ? 1 : 0;
     G.round_tendencies = 0;
     if (const char *e = getenv("GAME_GPU_ROUND_TENDENCIES")) {
         if (!strcmp(e, "rho")) G.round_tendencies = 1;
