@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(ATPB) k_vflux_adj_w(DevGrid G, const double *p
 __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const double *b, const double *ib,
                                                  double *ab, double scale, int acc)
 {
-    /* acc: ab += scale*result; otherwise ab = result.  One thread per edge and
+    /* acc 1: ab += scale*result, 2: ab = scale*result, 0: ab = result.  One thread per edge and
        level, which does the cell of its number too */
     const Blk bk = linear_block();
     const unsigned t = bk.x*ATPB + threadIdx.x;
@@ -485,12 +485,12 @@ __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const d
         const unsigned fr = G.from[t], to = G.to[t];
         const unsigned sf = (unsigned)A.slot_from[t]*(unsigned)nsh + fr, st = (unsigned)A.slot_to[t]*(unsigned)nsh + to;
         const double *wl = G.ipwT + (i64)l*8*nsh, *il = ib + (i64)l*nsh;
-        const double old = acc ? at(ab + row + nsh, t) : 0.0;
+        const double old = acc == 1 ? at(ab + row + nsh, t) : 0.0;
         const double r = at(b + row + nsh, t)*(at(wl, sf)*at(il, fr) + at(wl, st)*at(il, to));
         put(ab + row + nsh, t, acc ? old + scale*r : r);
     }
     if (t < (unsigned)nsh) {
-        const double old = acc ? at(ab + row, t) : 0.0;
+        const double old = acc == 1 ? at(ab + row, t) : 0.0;
         double s = 0.0;
         if (l >= 1) s += at(G.ipwT + ((i64)(l - 1)*8 + 7)*nsh, t)*at(ib + (i64)(l - 1)*nsh, t);
         if (l <= L - 1) s += at(G.ipwT + ((i64)l*8 + 6)*nsh, t)*at(ib + (i64)l*nsh, t);

@@ -98,24 +98,6 @@ struct EosStateAdj {
     }
 };
 
-/* edges and interior w of a wind cotangent: edges to ub (written), the top
-   and surface w (passed through unchanged by the step) added to b_in */
-struct PassThroughAdj {
-    DevGrid G;
-    const double *b_out;
-    double *ub, *b_in;
-    GAME_HD void operator()(i64 t) const
-    {
-        if (t >= G.v) return;
-        const int lev = (int)(t/G.vpl), h = (int)(t - (i64)lev*G.vpl);
-        if (h >= G.nsh) ub[t] = b_out[t];
-        else {
-            ub[t] = 0.0;
-            if (lev == 0 || lev == G.L) b_in[t] += b_out[t];
-        }
-    }
-};
-
 struct DiffToCot {
     i64 n;
     const double *x, *y;
@@ -137,7 +119,7 @@ struct Window {
     DevState seg_end;
     Cot bS, bSn, bS1;
     double *bt0_rho, *bt0_rt, *bt0_wind, *bt1_rho, *bt1_rt, *bt1_wind;
-    double *bP, *bPold, *bA, *bA1, *bAprev, *bU;
+    double *bP, *bPold, *bA, *bA1, *bAprev;
     double *Fb, *Fthb, *cvb, *vsqb, *tmpV1, *tmpV2, *fluxb, *pvb, *rvb, *dvb, *zb, *ws, *ones, *vcb;
     DevWork AW;
     /* phase clock of the last gradient: events and the phase each closes */
@@ -267,7 +249,7 @@ int window_alloc(Window &w, int k, int n_ckpt)
         return rc;
     double **sv[] = {&w.bt0_rho, &w.bt0_rt, &w.bt1_rho, &w.bt1_rt, &w.vsqb, &w.ones};
     for (double **p : sv) if ((rc = zeros(p, S))) return rc;
-    double **vv[] = {&w.bt0_wind, &w.bt1_wind, &w.bP, &w.bPold, &w.bA, &w.bA1, &w.bAprev, &w.bU, &w.tmpV1, &w.tmpV2,
+    double **vv[] = {&w.bt0_wind, &w.bt1_wind, &w.bP, &w.bPold, &w.bA, &w.bA1, &w.bAprev, &w.tmpV1, &w.tmpV2,
                      &w.fluxb};
     for (double **p : vv) if ((rc = zeros(p, V))) return rc;
     double **ev[] = {&w.Fb, &w.Fthb, &w.cvb};
@@ -479,9 +461,9 @@ void resident_from_tape(int m)
    accumulated into b_wind and b_rho */
 /* the reverse of the momentum advection of (wind, rho); flux and pv are the
    forward's mass flux and potential vorticity if taped, else null (they are
-   then recomputed) */
+   then recomputed).  new_b_wind: b_wind is written, not added to */
 int advection_adjoint(const double *wind, const double *rho, const double *flux, const double *pv,
-                      const double *advb, double *b_wind, double *b_rho)
+                      const double *advb, double *b_wind, double *b_rho, int new_b_wind = 0)
 {
     Window &w = *Wn;
     const DevGrid &G = M->G;
@@ -501,7 +483,7 @@ int advection_adjoint(const double *wind, const double *rho, const double *flux,
         HIP_OK(hipStreamWaitEvent(side, M->ev_fork, 0));
     }
     adj::grad_adjoint(G, A, advb, w.vsqb, side ? side : st, -0.5);
-    adj::inner_product_adjoint(G, A, wind, w.vsqb, b_wind, side ? side : st, 2.0, 1);
+    adj::inner_product_adjoint(G, A, wind, w.vsqb, b_wind, side ? side : st, 2.0, new_b_wind ? 2 : 1);
     /* TRSK flux: in the mass flux (with two streams on the side stream too: its
        cotangent is read only by the mass flux's reverse after the join) and
        in the PV */
@@ -536,17 +518,20 @@ int advection_adjoint(const double *wind, const double *rho, const double *flux,
    step's pressure gradient nl + l, w.bA that of its second-substep advection;
    on return w.bS, w.bP, w.bA hold the same for the step before */
 /* the reverse of the gas's scalar tendencies (scalar_tendencies_expl.c:107-176)
-   of densities (rho, rt) with the updated wind: the wind's cotangent goes to
-   w.bU, the densities' are added to (b_rho, b_rt) */
+   of densities (rho, rt) with the updated wind, with the momentum tendency's
+   reverse m (tb: the cotangent of its w tendency); the densities' cotangents
+   are added to (b_rho, b_rt) */
 static void scalar_tend_adjoint(const double *rho, const double *rt, const double *wind, const double *b_trho,
-                                const double *b_trt, double *b_rho, double *b_rt)
+                                const double *b_trt, double *b_rho, double *b_rt, const sadj::MomAdj &m,
+                                const double *tb)
 {
     Window &w = *Wn;
     const DevGrid &G = M->G;
     hipStream_t st = M->stream;
     if (!G.flat) launch("k_vcc_cot", sadj::VccCot{G, b_trho, b_trt, w.vcb}, (i64)G.n_oro*G.nsh, st);
     launch("k_scalar_tend_adj_e", sadj::ScalarTendAdjE{G, M->A, rho, rt, wind, b_trho, b_trt, w.vcb, w.Fb, w.Fthb,
-                                                       w.bU}, (i64)G.L*G.nvh, st);
+                                                       m}, (i64)G.L*G.nvh, st);
+    launch("k_tend_adj_w", sadj::TendAdjW{m, tb}, (i64)(G.L + 1)*G.nsh, st);
     launch_gather("k_scalar_tend_adj_c", sadj::ScalarTendAdjC{G, rho, rt, w.Fb, w.Fthb, b_rho, b_rt}, G.s, st);
 }
 
@@ -577,17 +562,7 @@ int step_adjoint(const StepTape &T, double dt, int first)
     hipStream_t st = M->stream;
     const double iw = M->cfg.impl_thermo_weight;
     const double chw = 0.5 + iw, ohw = 1.0 - chw, cvw = 1.0 - iw;
-    const size_t S = (size_t)G.s, V = (size_t)G.v;
     int rc;
-    {
-        ZeroList zl;
-        zl.add_cot(w.bSn);
-        zl.add_cot(w.bS1);
-        zl.add(w.bt0_rho, S); zl.add(w.bt0_rt, S); zl.add(w.bt0_wind, V);
-        zl.add(w.bt1_rho, S); zl.add(w.bt1_rt, S); zl.add(w.bt1_wind, V);
-        zl.add(w.bPold, V);
-        zl.run(st);
-    }
     /* the gradient of the step's exner_pert, which the pressure gradient's
        reverse below needs, depends on the tape alone: with two streams it is
        formed on the side stream now (joined by the advection reverse's join
@@ -608,12 +583,12 @@ int step_adjoint(const StepTape &T, double dt, int first)
                        w.bt1_rho, w.bt1_rt, w.bt1_wind, w.ws};
         ver_waves_adjoint(a, st);
     }
-    launch("k_pass_adj", PassThroughAdj{G, w.bS.wind, w.bU, w.bSn.wind}, G.v, st);
-    scalar_tend_adjoint(T.s1.rho, T.s1.rt, T.out.wind, w.bt1_rho, w.bt1_rt, w.bS1.rho, w.bS1.rt);
-    launch("k_wind_update_adj", sadj::WindUpdateAdj{G, dt, w.bU, w.bSn.wind, w.bt1_wind, 0}, G.v, st);
-    launch("k_tend_adj_rk1", sadj::TendAdjRk1{G, ohw, chw, cvw, w.bt1_wind, w.bA, w.bt0_wind, w.bPold, w.bP, w.bA1},
-           G.v, st);
-    if ((rc = advection_adjoint(T.s1.wind, T.s1.rho, T.flux, T.pv, w.bA1, w.bS1.wind, w.bS1.rho))) return rc;
+    {
+        const sadj::MomAdj m{G, 1, dt, ohw, chw, cvw, w.bS.wind, w.bSn.wind, w.bt0_wind, w.bPold, w.bP, w.bA, w.bA1};
+        scalar_tend_adjoint(T.s1.rho, T.s1.rt, T.out.wind, w.bt1_rho, w.bt1_rt, w.bS1.rho, w.bS1.rt, m, w.bt1_wind);
+    }
+    if ((rc = advection_adjoint(T.s1.wind, T.s1.rho, T.flux, T.pv, w.bA1, w.bS1.wind, w.bS1.rho, 1)))
+        return rc;
     /* ---- first substep ---- */
     {
         sadj::VwArgs a{G, 0, dt, iw, T.s.rho, T.s.rt, T.s.tp, T.s.ep, T.s.wind, T.s.rho, T.s.rt, T.s.ep,
@@ -622,14 +597,14 @@ int step_adjoint(const StepTape &T, double dt, int first)
                        w.bt0_rho, w.bt0_rt, w.bt0_wind, w.ws};
         ver_waves_adjoint(a, st);
     }
-    launch("k_pass_adj", PassThroughAdj{G, w.bS1.wind, w.bU, w.bSn.wind}, G.v, st);
-    scalar_tend_adjoint(T.s.rho, T.s.rt, T.s1.wind, w.bt0_rho, w.bt0_rt, w.bSn.rho, w.bSn.rt);
-    launch("k_wind_update_adj", sadj::WindUpdateAdj{G, dt, w.bU, w.bSn.wind, w.bt0_wind, 1}, G.v, st);
-    launch("k_tend_adj_rk0", sadj::TendAdjRk0{G, ohw, chw, cvw, w.bt0_wind, w.bPold, w.bP, w.bAprev}, G.v, st);
+    {
+        const sadj::MomAdj m{G, 0, dt, ohw, chw, cvw, w.bS1.wind, w.bSn.wind, w.bt0_wind, w.bPold, w.bP, nullptr, w.bAprev};
+        scalar_tend_adjoint(T.s.rho, T.s.rt, T.s1.wind, w.bt0_rho, w.bt0_rt, w.bSn.rho, w.bSn.rt, m, w.bt0_wind);
+    }
     if (first) {
         /* pgrad_old = -(nl + l) of this step; the advection of the first
            substep computed from this step's state */
-        launch("k_axpy", sadj::Axpy{G.v, -1.0, w.bPold, w.bP, 1}, G.v, st);
+        launch("k_axpy", sadj::Axpy{G.v, 1.0, w.bPold, w.bP, 1}, G.v, st);
         if ((rc = advection_adjoint(T.s.wind, T.s.rho, nullptr, nullptr, w.bAprev, w.bSn.wind, w.bSn.rho)))
             return rc;
     }
@@ -645,7 +620,7 @@ int step_adjoint(const StepTape &T, double dt, int first)
     launch("k_theta_adj", sadj::ThetaBoundaryAdj{G, T.s.rho, T.s.rt, w.bSn.rho, w.bSn.rt, w.bSn.tp}, G.s, st);
     /* hand over to the step before */
     std::swap(w.bS, w.bSn);
-    if (!first) launch("k_axpy", sadj::Axpy{G.v, -1.0, w.bPold, w.bP, 0}, G.v, st);
+    if (!first) std::swap(w.bP, w.bPold);
     std::swap(w.bA, w.bAprev);
     HIP_OK(hipGetLastError());
     return 0;
