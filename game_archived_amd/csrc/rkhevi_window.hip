@@ -540,8 +540,8 @@ static void ver_waves_adjoint(const sadj::VwArgs &a, hipStream_t st)
 {
     const DevGrid &G = a.G;
     const i64 ni = (i64)(G.L - 1)*G.nsh;
-    launch("k_vw_layer_fwd", sadj::VwLayerFwd{a}, G.s, st);
-    launch("k_vw_iface_fwd", sadj::VwIfaceFwd{a}, ni, st);
+    const int chunks = (G.L + VW_RUN - 1)/VW_RUN;
+    launch("k_vw_rows_fwd", sadj::VwRowsFwd{a, chunks}, (i64)chunks*G.nsh, st);
     auto band = [&](int k) { return a.ws + (i64)k*G.L*G.nsh; };
     adj::thomas(G.L - 1, G.nsh, band(sadj::VW_C), band(sadj::VW_D), band(sadj::VW_E), band(sadj::VW_R), band(sadj::VW_X),
                 nullptr, st);   /* at most 62 rows: no work array */

@@ -58,13 +58,14 @@ GAME_HD inline void split_index(i64 t, int n, int &q, int &r)
 /*   rho_ie = mean of re, theta_i = mean of rt_n/rho_n,                 */
 /*   the bands c, d, e and right-hand side r, x = A^-1 r, damping,      */
 /*   then rho, rt, w, tp, ep of the new state.                          */
-/* The reverse runs as seven launches: the per-layer coefficients       */
-/* (VwLayerFwd), the per-interface bands (VwIfaceFwd), the solve        */
-/* (adj::thomas), the cotangent of the solution                          */
-/* (VwIfaceSolBar), the transposed solve (adj::thomas), the interface    */
-/* cotangents (VwIfaceBar) and the per-layer cotangents (VwLayerBar).   */
-/* Every launch but the two solves has one thread per (layer, column)   */
-/* or (interface, column), and every contribution an interface makes to */
+/* The reverse runs as seven launches: the per-layer coefficients and    */
+/* the per-interface bands (VwRowsFwd), the solve (adj::thomas), the    */
+/* new state and its cotangents (VwLayerNew), the cotangent of the      */
+/* solution (VwIfaceSolBar), the transposed solve (adj::thomas), the    */
+/* interface cotangents (VwIfaceBar) and the per-layer cotangents       */
+/* (VwLayerBar).                                                        */
+/* The launches after the first solve have one thread per (layer,       */
+/* column) or (interface, column), and every contribution an interface makes to */
 /* its neighbours is gathered by the neighbour, so no element has two  */
 /* writers.  The workspace holds VW_N arrays of L doubles per column,   */
 /* array k of column c element j at (k*L + j)*ncol + c.                 */
@@ -153,75 +154,96 @@ struct VwArgs {
     }
 };
 
-/* alpha, beta, gamma of layer j (column_solvers.c:99-121) */
-struct VwLayerFwd {
+/* alpha, beta, gamma of the layers (column_solvers.c:99-121) and the bands of
+   the interfaces below them (:141-189), VW_RUN layers of a column per thread:
+   every load of the chunk is issued before its first store and a value that
+   several rows use is loaded and formed once.  As two kernels, one thread per
+   layer and one per interface, they took 65 us at res 6 x 26, here 39
+   (41 with one layer, 39 with three; 134 registers) */
+#define VW_RUN 2
+struct VwRowsFwd {
     VwArgs a;
+    int chunks;
     GAME_HD void operator()(i64 t) const
     {
         const DevGrid &G = a.G;
-        if (t >= G.s) return;
-        int j, c;
-        a.split(t, j, c);
-        const i64 b = sidx(G, j, c);
-        const double ro = a.rho_o[b], rto = a.rt_o[b], vol = G.vol[b], exbg = G.exbg[b];
-        double al, be, ga;
-        if (a.rk == 0) {
-            al = -rto/(ro*ro)/vol;
-            be = 1.0/ro/vol;
-            ga = GC_R_D/(GC_C_D_V*rto)*(exbg + a.ep_o[b])/vol;
-        } else {
-            const double pdw = 0.5;
-            const double rn = a.rho_n[b], rtn = a.rt_n[b];
-            const double ao = -rto/(ro*ro), bo = 1.0/ro, go = GC_R_D/(GC_C_D_V*rto)*(exbg + a.ep_o[b]);
-            const double an = -rtn/(rn*rn), bn = 1.0/rn, gn = GC_R_D/(GC_C_D_V*rtn)*(exbg + a.ep_n[b]);
-            al = ((1.0 - pdw)*ao + pdw*an)/vol;
-            be = ((1.0 - pdw)*bo + pdw*bn)/vol;
-            ga = ((1.0 - pdw)*go + pdw*gn)/vol;
+        const int L = G.L, n = L - 1;
+        if (t >= (i64)chunks*G.nsh) return;
+        int q, c;
+        a.split(t, q, c);
+        const int j0 = q*VW_RUN;
+        const double dt = a.dt, iw = a.iw, *rnp = a.rn_(), *rtnp = a.rtn_();
+        /* layer j0 + k and the interface below it; rows past the column repeat
+           its last and are not used */
+        double ro[VW_RUN + 2], rn[VW_RUN + 2], rtn[VW_RUN + 2], zs[VW_RUN + 2], ex[VW_RUN + 2];
+        double rto[VW_RUN + 1], ep[VW_RUN + 1], tp[VW_RUN + 1], vol[VW_RUN + 1], tr[VW_RUN + 1], tt[VW_RUN + 1],
+            epn[VW_RUN + 1], wo[VW_RUN + 1];
+        double ar[VW_RUN], tw[VW_RUN];
+#pragma unroll
+        for (int k = 0; k < VW_RUN + 2; ++k) {
+            const i64 b = sidx(G, j0 + k < L ? j0 + k : L - 1, c);
+            ro[k] = a.rho_o[b]; rn[k] = rnp[b]; rtn[k] = rtnp[b]; zs[k] = G.zs[b]; ex[k] = G.exbg[b];
         }
-        a.W(VW_AL, j, c) = al;
-        a.W(VW_BE, j, c) = be;
-        a.W(VW_GA, j, c) = ga;
-    }
-};
-
-/* theta_i, the bands and the right-hand side of interface j
-   (column_solvers.c:123-190) */
-struct VwIfaceFwd {
-    VwArgs a;
-    GAME_HD double tin(int j, int c) const
-    {
-        const double *rn = a.rn_(), *rtn = a.rtn_();
-        const i64 b = sidx(a.G, j, c), lo = sidx(a.G, j + 1, c);
-        return 0.5*(rtn[b]/rn[b] + rtn[lo]/rn[lo]);
-    }
-    GAME_HD void operator()(i64 t) const
-    {
-        const DevGrid &G = a.G;
-        const int n = G.L - 1;
-        if (t >= (i64)n*G.nsh) return;
-        int j, c;
-        a.split(t, j, c);
-        const double dt = a.dt, iw = a.iw;
-        const i64 b = sidx(G, j, c), lo = sidx(G, j + 1, c), wi = widx(G, j + 1, c);
-        const double ti = tin(j, c), rio = a.rio(j, c), wo = a.wind_o[wi];
-        const double rie = 0.5*(a.re(j, c) + a.re(j + 1, c));
-        const double dz = G.zs[b] - G.zs[lo], dex = G.exbg[b] - G.exbg[lo];
-        const double q = dz/(iw*(dt*dt)*GC_C_D_P);
-        const double ga0 = a.W(VW_GA, j, c), ga1 = a.W(VW_GA, j + 1, c);
-        const double al0 = a.W(VW_AL, j, c), al1 = a.W(VW_AL, j + 1, c);
-        const double be0 = a.W(VW_BE, j, c), be1 = a.W(VW_BE, j + 1, c);
-        a.W(VW_TIN, j, c) = ti;
-        a.W(VW_D, j, c) = -(ti*ti)*(ga0 + ga1) + 0.5*dex*(al1 - al0 + ti*(be1 - be0))
-                          - dz/(iw*(dt*dt)*GC_C_D_P*rio)*(2.0/G.area[wi] + dt*wo*0.5*(-1.0/G.vol[b] + 1.0/G.vol[lo]));
-        a.W(VW_R, j, c) = -(wo + dt*a.t_wind[wi])*q + ti*(a.epe(j, c) - a.epe(j + 1, c))/dt
-                          + 0.5/dt*(a.tpe(j, c) + a.tpe(j + 1, c))*dex - q*wo*rie/rio;
-        if (j < n - 1) {
-            const i64 l2 = sidx(G, j + 2, c);
-            const double dz1 = G.zs[lo] - G.zs[l2], dex1 = G.exbg[lo] - G.exbg[l2];
-            const double ti1 = tin(j + 1, c), rio1 = a.rio(j + 1, c);
-            a.W(VW_C, j, c) = ti1*ga1*ti + 0.5*dex1*(al1 + be1*ti)
-                              - dz1/(iw*dt*GC_C_D_P)*0.5*a.wind_o[widx(G, j + 2, c)]/(G.vol[lo]*rio1);
-            a.W(VW_E, j, c) = ti*ga1*ti1 - 0.5*dex*(al1 + be1*ti1) + dz/(iw*dt*GC_C_D_P)*0.5*wo/(G.vol[lo]*rio);
+#pragma unroll
+        for (int k = 0; k < VW_RUN + 1; ++k) {
+            const int j = j0 + k < L ? j0 + k : L - 1;
+            const i64 b = sidx(G, j, c);
+            rto[k] = a.rt_o[b]; ep[k] = a.ep_o[b]; tp[k] = a.tp_o[b]; vol[k] = G.vol[b]; tr[k] = a.t_rho[b];
+            tt[k] = a.t_rt[b]; epn[k] = a.rk == 0 ? 0.0 : a.ep_n[b];
+            wo[k] = a.wind_o[widx(G, j + 1, c)];
+        }
+#pragma unroll
+        for (int k = 0; k < VW_RUN; ++k) {
+            const i64 wi = widx(G, j0 + k < L ? j0 + k + 1 : L, c);
+            ar[k] = G.area[wi];
+            tw[k] = a.t_wind[wi];
+        }
+        double al[VW_RUN + 1], be[VW_RUN + 1], ga[VW_RUN + 1], th[VW_RUN + 2];
+#pragma unroll
+        for (int k = 0; k < VW_RUN + 1; ++k) {
+            if (a.rk == 0) {
+                al[k] = -rto[k]/(ro[k]*ro[k])/vol[k];
+                be[k] = 1.0/ro[k]/vol[k];
+                ga[k] = GC_R_D/(GC_C_D_V*rto[k])*(ex[k] + ep[k])/vol[k];
+            } else {
+                const double pdw = 0.5;
+                const double ao = -rto[k]/(ro[k]*ro[k]), bo = 1.0/ro[k], go = GC_R_D/(GC_C_D_V*rto[k])*(ex[k] + ep[k]);
+                const double an = -rtn[k]/(rn[k]*rn[k]), bn = 1.0/rn[k], gn = GC_R_D/(GC_C_D_V*rtn[k])*(ex[k] + epn[k]);
+                al[k] = ((1.0 - pdw)*ao + pdw*an)/vol[k];
+                be[k] = ((1.0 - pdw)*bo + pdw*bn)/vol[k];
+                ga[k] = ((1.0 - pdw)*go + pdw*gn)/vol[k];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < VW_RUN + 2; ++k) th[k] = rtn[k]/rn[k];
+        auto re = [&](int k) { return ro[k] + dt*tr[k]; };
+        auto tpe = [&](int k) { return tp[k] + dt*vol[k]*(al[k]*tr[k] + be[k]*tt[k]); };
+        auto epe = [&](int k) { return ep[k] + dt*vol[k]*ga[k]*tt[k]; };
+        auto rio = [&](int k) { return 0.5*(ro[k] + ro[k + 1]); };
+        auto tin = [&](int k) { return 0.5*(th[k] + th[k + 1]); };
+#pragma unroll
+        for (int k = 0; k < VW_RUN; ++k) {
+            const int j = j0 + k;
+            if (j >= L) break;
+            a.W(VW_AL, j, c) = al[k];
+            a.W(VW_BE, j, c) = be[k];
+            a.W(VW_GA, j, c) = ga[k];
+            if (j >= n) break;
+            const double ti = tin(k), rie = 0.5*(re(k) + re(k + 1));
+            const double dz = zs[k] - zs[k + 1], dex = ex[k] - ex[k + 1];
+            const double qz = dz/(iw*(dt*dt)*GC_C_D_P);
+            a.W(VW_TIN, j, c) = ti;
+            a.W(VW_D, j, c) = -(ti*ti)*(ga[k] + ga[k + 1]) + 0.5*dex*(al[k + 1] - al[k] + ti*(be[k + 1] - be[k]))
+                              - dz/(iw*(dt*dt)*GC_C_D_P*rio(k))*(2.0/ar[k] + dt*wo[k]*0.5*(-1.0/vol[k] + 1.0/vol[k + 1]));
+            a.W(VW_R, j, c) = -(wo[k] + dt*tw[k])*qz + ti*(epe(k) - epe(k + 1))/dt
+                              + 0.5/dt*(tpe(k) + tpe(k + 1))*dex - qz*wo[k]*rie/rio(k);
+            if (j < n - 1) {
+                const double dz1 = zs[k + 1] - zs[k + 2], dex1 = ex[k + 1] - ex[k + 2], ti1 = tin(k + 1);
+                a.W(VW_C, j, c) = ti1*ga[k + 1]*ti + 0.5*dex1*(al[k + 1] + be[k + 1]*ti)
+                                  - dz1/(iw*dt*GC_C_D_P)*0.5*wo[k + 1]/(vol[k + 1]*rio(k + 1));
+                a.W(VW_E, j, c) = ti*ga[k + 1]*ti1 - 0.5*dex*(al[k + 1] + be[k + 1]*ti1)
+                                  + dz/(iw*dt*GC_C_D_P)*0.5*wo[k]/(vol[k + 1]*rio(k));
+            }
         }
     }
 };
