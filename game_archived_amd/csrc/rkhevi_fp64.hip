@@ -787,6 +787,8 @@ __global__ void __launch_bounds__(TPB) k_vcc_weights(DevGrid G, double *vcw)
     vcw[t] = -0.5*G.ipwT[((i64)l*8 + jj)*G.nsh + h]*G.slope[G.nsh + (i64)l*G.vpl + G.adj[6*h + jj]];
 }
 
+/* MOIST: with the correction of the wind itself, which the tracers take */
+template <bool MOIST>
 __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc, Span sp)
 {
     /* one thread per cell walks a chunk of the terrain levels.  The
@@ -848,19 +850,21 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc,
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
             if (j < ne) {
-                aw += tw[j]; a1 += t1[j]; a2 += t2[j];
-                pw += tw[j]; p1 += t1[j]; p2 += t2[j];
+                if (MOIST) { aw += tw[j]; pw += tw[j]; }
+                a1 += t1[j]; a2 += t2[j];
+                p1 += t1[j]; p2 += t2[j];
             }
         }
     };
     double pw = 0.0, p1 = 0.0, p2 = 0.0;
     /* the layer above the chunk (its terms start the first level's sum),
        then the chunk's layers, each loaded before the one before it is
-       summed (a step past the chunk reloads its last layer, unused) */
+       summed */
     const int k_first = c0 > 0 ? c0 - 1 : c0;
     In cur = load(top + k_first);
     for (int k = k_first; k < c1; ++k) {
-        const In nxt = load(top + (k + 1 < c1 ? k + 1 : k));
+        In nxt = cur;
+        if (k + 1 < c1) nxt = load(top + k + 1);
         if (k < c0) {
             double dw = 0.0, d1 = 0.0, d2 = 0.0;
             add_layer(cur, pw, p1, p2, dw, d1, d2);
@@ -869,7 +873,7 @@ __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc,
             pw = 0.0; p1 = 0.0; p2 = 0.0;
             add_layer(cur, rw, r1, r2, pw, p1, p2);
             double *row = vcc + (i64)k*nsh;
-            put(row, h, rw);
+            if (MOIST) put(row, h, rw);
             put(row + n, h, r1);
             put(row + 2*n, h, r2);
         }
@@ -2223,15 +2227,18 @@ template <typename TW>
 static void scalar_tend_t(const DevGrid &G, const DevState &s, const DevState &td, const DevWorkT<TW> &W, int rk,
                           hipStream_t st)
 {
-    if (!G.flat)
-        /* the chunks of terrain levels: set_layer_splits.  Loading each layer
-           before the one above it is summed took the kernel's time in the
-           mountain window's gradient from 5.98 to 5.46 ms; with the weights
-           -0.5*ipw*slope as a grid constant (one coalesced load for a
-           coalesced load and a gather) it takes 49.6 us per launch at
-           res 6 x 26 where it took 58.9 */
-        LAUNCH("k_vcc", k_vcc, grid_of(G.nsh, G.split_vcc), dim3(TPB), st, G, s, W.vcc,
-               span_of(G.nsh, G.n_oro, G.split_vcc));
+    /* the chunks of terrain levels: set_layer_splits.  Bound by the gathers of
+       six neighbours' densities and winds (107 MB that it cannot do without at
+       res 6 x 26, 22 us at a copy's rate): each layer loaded before the one above
+       it is summed, the weights -0.5*ipw*slope a grid constant (59 -> 43 us per
+       launch), no load past the chunk's end and, for a dry model, no correction
+       of the wind itself, which only the tracers take (43 -> 35) */
+    if (!G.flat) {
+        const dim3 g = grid_of(G.nsh, G.split_vcc);
+        const Span sp = span_of(G.nsh, G.n_oro, G.split_vcc);
+        if (G.n_const > 1) LAUNCH("k_vcc", k_vcc<true>, g, dim3(TPB), st, G, s, W.vcc, sp);
+        else LAUNCH("k_vcc", k_vcc<false>, g, dim3(TPB), st, G, s, W.vcc, sp);
+    }
     const dim3 g = grid_of(G.nsh, G.L), b(TPB);
     const Span sp = span_of(G.nsh, 1, 1);
     if (G.n_const == 6) {

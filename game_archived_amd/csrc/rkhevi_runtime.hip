@@ -199,10 +199,12 @@ static void set_layer_splits(DevGrid &G)
        res 5: 17 with one, 23 with two) */
     const int run_w = bc*L < 3*1024 ? 1 : 3;
     G.split_cell_w = (L + 1 + run_w - 1)/run_w;
-    /* vertical corrections: about 1280 blocks, two to six terrain levels per
-       thread (res 4: one level 9 us, two 11; res 5: two 19, one 22, three 21;
-       res 6: three 50, four 51, six 64) */
-    const int run_v = bc*G.n_oro <= 512 ? 1 : clamp((bc*G.n_oro + 640)/1280, 2, 6);
+    /* vertical corrections: a chunk loads the layer above it too, so three
+       terrain levels per thread where they leave enough blocks and one where
+       not (one, two, three, four and six levels, us per launch: res 4 x 26 6.2,
+       7.3, 8.4, 9.9, 12.7; res 5 x 26 15.2, 16.1, 20.9, 18.3, 23.8; res 6 x 26
+       44, 41, 35, 41, 48; res 6 x 55 92, 81, 80, 84, 86) */
+    const int run_v = bc*G.n_oro <= 1024 ? 1 : 3;
     G.split_vcc = (G.n_oro + run_v - 1)/run_v;
     /* the adjoints: a filled chip, at least four chunks; a cell's chunk forms
        a layer above and below it again, so it has two layers or more */
