@@ -1475,7 +1475,7 @@ __device__ __forceinline__ void tracer_iface_flux(const DevGrid &G, const DevSta
 template <int GD_PER, int NT>
 __global__ void __launch_bounds__(NT) k_gen_densities(DevGrid G, DevState so, DevState sn, DevState td, StepConsts K)
 {
-    __shared__ double hand[64];
+    __shared__ double hand[64], hand_ep[64];
     const int L = G.L, nsh = G.nsh, ncc = G.n_cond, vpl = G.vpl;
     /* the tracer is the fast block index: the blocks of one group of columns
        run side by side on one XCD and share the wind, area and volume columns in L2 */
@@ -1537,7 +1537,9 @@ __global__ void __launch_bounds__(NT) k_gen_densities(DevGrid G, DevState so, De
             }
             const bool up = fi >= 0.0;
             r[t] = rj;
-            d[t] = dj;
+            /* dj itself but for an infinite wind, whose NaN then goes on as in
+               the elimination */
+            d[t] = t > 0 ? dj - ep[t > 0 ? t - 1 : 0]*c_m : dj;
             c[t] = c_m;
             ep[t] = up && !last ? (-q)*fi/dj : 0.0;
             c_m = up ? 0.0 : qlo[t]*fi;
@@ -1550,11 +1552,11 @@ __global__ void __launch_bounds__(NT) k_gen_densities(DevGrid G, DevState so, De
     double x = 0.0;
     for (int s = 0; s < nw; ++s) {
         if (w == s) {
-            if (s > 0) x = hand[lane];
+            if (s > 0) { x = hand[lane]; d[0] -= hand_ep[lane]*c[0]; }
 #pragma unroll
             for (int t = 0; t < GD_PER; ++t)
                 if (j0 + t < L) { x = (r[t] - x*c[t])/d[t]; r[t] = x; }
-            if (s < nw - 1) hand[lane] = x;
+            if (s < nw - 1) { hand[lane] = x; hand_ep[lane] = ep[GD_PER - 1]; }
         }
         __syncthreads();
     }

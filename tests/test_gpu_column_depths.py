@@ -41,3 +41,31 @@ def test_depths_change_no_bit(monkeypatch, res, layers, precision):
     for k in want:
         assert np.isfinite(got[k]).all(), k
         assert np.array_equal(got[k], want[k]), k
+
+
+@pytest.mark.parametrize("layers", [26, 41])
+def test_an_infinite_wind_spreads_alike(monkeypatch, layers):
+    """an infinite vertical wind, up and down, in rows within and at the ends
+    of a wave's rows: the same boxes become not-a-number"""
+    print(f"case: infinite winds, res 3 x {layers} moist", flush=True)
+    grid = get_grid(3, "flat", moist=1, n_layers=layers, n_oro=layers - 2)
+    state, d = oracle_state(grid, moist=True), grid.dims
+    for n, level in enumerate((3, 7, 8, 9, 10, 14, 18, layers - 1)):
+        for cell, sign in ((40 * n + 20, 1.0), (40 * n + 330, -1.0)):
+            state.wind[level * d.vpl + cell] = sign * np.inf
+    from game_archived_amd.rkhevi import DeviceModel
+
+    def tracers():
+        dm = DeviceModel(grid)
+        try:
+            dm.start(state)
+            dm.run(1, 120.0)
+            return np.array(dm.get_state().rho)
+        finally:
+            dm.close()
+
+    got = tracers()
+    monkeypatch.setenv("GAME_GPU_GD_STREAMING", "1")
+    want = tracers()
+    assert np.isnan(want).any() and np.isfinite(want).any()
+    assert np.array_equal(got, want, equal_nan=True)
