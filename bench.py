@@ -69,14 +69,21 @@ def kernel_bytes(name, dims, wb=8):
         # area at w, volume and the (iw dt)/volume table (shared)
         "k_gen_densities": 8 * ((nc - 1) * 3 * S + 3 * W_ + 2 * S),
         # condensate densities, w and area at two interfaces, volume; temperature,
-        # the condensates' c_p table (work) and the output
-        "k_sed_heat": 8 * (4 * S + 2 * W_ + S) + wb * (2 * S + 4 * S),
+        # the c_p tables of ice and liquid (work) and the output
+        "k_sed_heat": 8 * (4 * S + 2 * W_ + S) + wb * (2 * S + 2 * S),
         # TRSK flux: mass flux (edges, w), PV (tangential, rhombus), output (work
-        # arrays); ipw slots 6/7; TRSK tables once
+        # arrays); ipw slots 6/7; TRSK tables once.  With the tendency and the
+        # wind update: kinetic energy, pressure-gradient combination and old
+        # tendency read, kinetic-energy gradient and tendency written (work
+        # arrays), wind old and new
         "k_vorticity_flux_e": wb * (E + (L + 1) * NSH + (L + 1) * NVH + L * NVH + E) + 8 * 2 * S
-                              + 4 * 20 * NVH + 8 * 10 * NVH,
-        "k_vorticity_flux_w": wb * (E + dims.curl // 2 + (L + 1) * NSH) + 8 * 6 * S + 4 * 6 * NSH,
-        "k_pot_vort": 8 * (E + (L + 1) * NSH + S + dims.curl // 2) + wb * (dims.curl + L * NT)
+                              + 4 * 20 * NVH + 8 * 10 * NVH + wb * (S + 4 * E) + 8 * 2 * E,
+        # the same at the w points, with the normal distance; moist: every
+        # density and the gravity metric for the condensates' term
+        "k_vorticity_flux_w": wb * (E + dims.curl // 2 + (L + 1) * NSH) + 8 * 6 * S + 4 * 6 * NSH
+                              + wb * (S + 4 * W_) + 8 * W_ + (8 * (nc * S + W_) + wb * W_ if moist else 0),
+        # with the mass flux (written at edges and w points)
+        "k_pot_vort": 8 * (E + (L + 1) * NSH + S + dims.curl // 2) + wb * (dims.curl + L * NT + V)
                       + 4 * 8 * NVH + 8 * 4 * NVH,
         "k_rel_vort_tri": 8 * (2 * E + L * NT) + wb * L * NT + 4 * 6 * NT,
         # all constituents: rho_k, rhotheta_v, wind and area at edges, volume,
@@ -85,24 +92,21 @@ def kernel_bytes(name, dims, wb=8):
         # launch on average; moist: rates, temperature, heating, sediment heat
         # (work) and exner (state, background)
         "k_scalar_tend": 8 * (S * (nc + 1) + 2 * E + S + S * (nc + 1) + S * (nc - 1) // 2 + (2 * S if moist else 0))
-                         + (wb * (8 + 4) * S if moist else 0) + 4 * 12 * NSH,
-        # tendency (written; read in the second substep only, half a read per
-        # launch on average), pressure-gradient combination, vorticity flux,
-        # kinetic-energy gradient (work arrays), pgc at w; wind old/new
-        "k_vector_tend": wb * (4 * V + V // 2 + W_) + 8 * 2 * E,
-        # exner, theta_bg, theta pert and the gas fraction of the cells
-        "k_pgrad_e": 8 * (4 * S + 2 * E) + wb * 6 * E + 4 * 2 * NVH,
-        "k_pgrad_w": 8 * (4 * S + 3 * W_) + wb * 7 * W_,
+                         + (wb * (8 + 2) * S if moist else 0) + 4 * 12 * NSH,
+        # exner, theta_bg, theta pert and the gas fraction of the cells; with the
+        # first substep's tendency: TRSK flux and kinetic-energy gradient read,
+        # tendency written, wind old and new at the edges
+        "k_pgrad_e": 8 * (4 * S + 2 * E) + wb * 6 * E + 4 * 2 * NVH + wb * 3 * E + 8 * 2 * E,
+        "k_pgrad_w": 8 * (4 * S + 3 * W_) + wb * 7 * W_ + wb * 3 * W_,
         "k_grad_e": wb * (S + E) + 8 * E + 4 * 2 * NVH,
         "k_grad_w": wb * (S + W_) + 8 * W_,
         "k_inner_product": 8 * (V + 8 * S) + wb * S + 4 * 6 * NSH,
-        "k_mass_flux": 8 * (S + E + W_) + wb * (E + W_) + 4 * 2 * NVH,
         "k_phase_trans": 8 * nc * S + wb * (7 + 4) * S,
         # temperature, c_p, gas fraction and phase transitions in one pass
-        "k_temp_phase": 8 * ((4 + nc) * S + S) + wb * (S + 4 * S + 6 * S),
+        "k_temp_phase": 8 * ((4 + nc) * S + S) + wb * (S + 2 * S + 6 * S),
         # theta, exner (background and perturbation), all densities; writes the
         # temperature, the condensates' c_p (work) and the gas fraction
-        "k_temperature": 8 * ((4 + nc) * S + S) + wb * (S + (4 * S if moist else 0)),
+        "k_temperature": 8 * ((4 + nc) * S + S) + wb * (S + (2 * S if moist else 0)),
         "k_lincomb_scalars": 8 * (2 * (nc + 2) * S + (nc + 3) * S),
         "k_lincomb_vector": 8 * 3 * V,
     }
