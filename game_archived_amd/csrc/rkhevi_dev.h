@@ -149,15 +149,21 @@ __device__ __forceinline__ unsigned xcd_linear(unsigned lin, unsigned T)
     const unsigned q = T/N_XCD, r = T%N_XCD, x = lin%N_XCD, k = lin/N_XCD;
     return (x < r) ? x*(q + 1) + k : r*(q + 1) + (x - r)*q + k;
 }
+/* (m % gx, m/gx) by the reciprocal of span_of: ceil(2^32/gx) is at most gx - 1
+   parts of 2^32 too large, so for every 32-bit m the quotient is at most one
+   too large.  2^32 itself, for one block per row (at most 256 columns or edges),
+   has no 32 bits: rcp is 0 there and m the quotient */
+__host__ __device__ __forceinline__ Blk block_at(unsigned m, unsigned gx, unsigned rcp)
+{
+    Blk b;
+    b.y = rcp ? (unsigned)(((unsigned long long)m*rcp) >> 32) : m;
+    b.x = m - b.y*gx;
+    if ((int)b.x < 0) { --b.y; b.x += gx; }
+    return b;
+}
 __device__ __forceinline__ Blk xcd_block(Span sp)
 {
-    const unsigned m = xcd_linear(blockIdx.y*gridDim.x + blockIdx.x, gridDim.x*gridDim.y);
-    /* rcp = ceil(2^32/gridDim.x) overestimates the quotient by one at most (m*gridDim.x < 2^32) */
-    Blk b;
-    b.y = __umulhi(m, sp.rcp);
-    b.x = m - b.y*gridDim.x;
-    if ((int)b.x < 0) { --b.y; b.x += gridDim.x; }
-    return b;
+    return block_at(xcd_linear(blockIdx.y*gridDim.x + blockIdx.x, gridDim.x*gridDim.y), gridDim.x, sp.rcp);
 }
 /* the blocks as they are dispatched: for kernels that mostly stream, where eight
    ranges far apart cost more than neighbours in one L2 give (us per launch,
@@ -172,7 +178,7 @@ static dim3 grid_of(int n, int chunks) { return dim3((unsigned)((n + TPB - 1)/TP
 static Span span_of(int n, int layers, int chunks)
 {
     const unsigned gx = (unsigned)((n + TPB - 1)/TPB);
-    return Span{(layers + chunks - 1)/chunks, gx > 1 ? (unsigned)(((1ULL << 32) + gx - 1)/gx) : 0xffffffffu};
+    return Span{(layers + chunks - 1)/chunks, gx > 1 ? (unsigned)(((1ULL << 32) + gx - 1)/gx) : 0u};
 }
 
 /* layers [l0, l1) of a chunk when n layers are split into chunks of `run`;
