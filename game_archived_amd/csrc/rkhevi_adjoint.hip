@@ -520,7 +520,9 @@ __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const d
 #define TL_ROWS 128
 #define TL_B 8
 static int tl_lanes(int n) { return n <= 64 ? 64 : 32; }
-/* rows j0 .. j0 + TL_B - 1 of column k: lo[j - 1], d[j], up[j], r[j]; rows that
+/* rows j0 .. j0 + TL_B - 1 of column k of the block (the arrays begin at the
+   block's first column, so that any int is a valid column count: the 32-bit
+   offset of at() takes the lane alone): lo[j - 1], d[j], up[j], r[j]; rows that
    the system does not have repeat its last, and a single row has no bands */
 struct TlRows { double lo[TL_B], d[TL_B], up[TL_B], r[TL_B]; };
 __device__ __forceinline__ TlRows tl_load(const double *lo, const double *d, const double *up, const double *r, int n,
@@ -572,9 +574,11 @@ __global__ void __launch_bounds__(64) k_thomas_lds(int n, int ncol, const double
 {
     extern __shared__ double lds[];
     const int lanes = (int)blockDim.x;
-    const unsigned k = xcd_x()*blockDim.x + threadIdx.x;
-    if (k >= (unsigned)ncol) return;
-    double *q = lds + threadIdx.x, *s = q + n*lanes;
+    const unsigned k = threadIdx.x;
+    const i64 k0 = (i64)xcd_x()*lanes;
+    if (k0 + k >= ncol) return;
+    c += k0; d += k0; e += k0; r += k0; x += k0;
+    double *q = lds + k, *s = q + n*lanes;
     tl_down(c, d, e, r, n, ncol, k, q, s, lanes);
     double xj = 0.0;
 #pragma unroll 4
@@ -592,9 +596,11 @@ __global__ void __launch_bounds__(64) k_thomas_adj_lds(int n, int ncol, const do
 {
     extern __shared__ double lds[];
     const int lanes = (int)blockDim.x;
-    const unsigned k = xcd_x()*blockDim.x + threadIdx.x;
-    if (k >= (unsigned)ncol) return;
-    double *q = lds + threadIdx.x, *s = q + n*lanes;
+    const unsigned k = threadIdx.x;
+    const i64 k0 = (i64)xcd_x()*lanes;
+    if (k0 + k >= ncol) return;
+    c += k0; d += k0; e += k0; x += k0; xb += k0; rb += k0; cb += k0; db += k0; eb += k0;
+    double *q = lds + k, *s = q + n*lanes;
     tl_down(e, d, c, xb, n, ncol, k, q, s, lanes);
     /* upwards, the solution's rows loaded TL_B ahead */
     auto load = [&](int j1, double *y) {
@@ -735,7 +741,7 @@ void thomas(int n, int ncol, const double *c, const double *d, const double *e, 
         return;
     }
     const int lanes = tl_lanes(n);
-    const dim3 g((unsigned)((ncol + lanes - 1)/lanes)), b((unsigned)lanes);
+    const dim3 g(((unsigned)ncol + (unsigned)lanes - 1u)/(unsigned)lanes), b((unsigned)lanes);
     const size_t lds = (size_t)2*n*lanes*sizeof(double);
     LAUNCH_SHM("k_thomas", k_thomas_lds, g, b, lds, st, n, ncol, c, d, e, r, x);
 }
@@ -748,7 +754,7 @@ void thomas_adjoint(int n, int ncol, const double *c, const double *d, const dou
         return;
     }
     const int lanes = tl_lanes(n);
-    const dim3 g((unsigned)((ncol + lanes - 1)/lanes)), b((unsigned)lanes);
+    const dim3 g(((unsigned)ncol + (unsigned)lanes - 1u)/(unsigned)lanes), b((unsigned)lanes);
     const size_t lds = (size_t)2*n*lanes*sizeof(double);
     LAUNCH_SHM("k_thomas_adj", k_thomas_adj_lds, g, b, lds, st, n, ncol, c, d, e, x, xb, rb, cb, db, eb);
 }

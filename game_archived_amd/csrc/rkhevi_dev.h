@@ -192,7 +192,9 @@ __device__ __forceinline__ void layer_chunk(int n, unsigned chunk, int run, int 
 /* element i of a row whose address is the same for the whole wave: the row's
    base stays in scalar registers and the lane adds a 32-bit byte offset, so a
    load costs one instruction and the offset is shared by every row read at
-   the same index (a 64-bit element index takes an address pair per load) */
+   the same index (a 64-bit element index takes an address pair per load).  The
+   byte offset has 32 bits: i is below 2^29 for doubles, which a row of any
+   grid that fits the memory is */
 template <typename T>
 __device__ __forceinline__ T at(const T *row, unsigned i)
 {
