@@ -23,7 +23,6 @@
 #include "rkhevi_adjoint.h"
 
 #define ATPB TPB
-#define AGRID(n) dim3((unsigned)(((n) + ATPB - 1)/ATPB))
 
 /* ------------------------------------------------------------------ */
 /* grad^T: fbar(c, l) from gbar at the cell's edges and w points        */
@@ -503,8 +502,8 @@ __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const d
 /* batched three-band solve and its adjoint (element j of column k at    */
 /* j*ncol + k, so lanes read consecutive words)                          */
 /* ------------------------------------------------------------------ */
-/* One column per lane with its quotients and solution in LDS (systems of at
-   most TL_ROWS rows): the rows of the next batch are loaded while the lane
+/* One column per lane with its quotients and solution in LDS (systems of TL_MIN
+   to TL_ROWS rows): the rows of the next batch are loaded while the lane
    eliminates the current ones, so a wave has 32 row loads in flight where the
    walking kernel below waits for four at every row, and the quotients and the
    intermediate solution cost no traffic.  Each block is one wave of `lanes`
@@ -520,6 +519,13 @@ __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const d
 #define TL_ROWS 128
 #define TL_B 8
 static int tl_lanes(int n) { return n <= 64 ? 64 : 32; }
+/* the walking kernel for more rows, and for fewer than four, of which a batch
+   of eight loads each several times (us per solve and adjoint of 1,000,003
+   columns, walking and here: one row 17 and 21, 29 and 38; two 28 and 38, 43
+   and 55; three 38 and 53, 44 and 58; four 54 and 83, 54 and 77); it keeps the
+   quotients in a work array, which the reverse step (two rows or more) has not */
+#define TL_MIN 4
+static bool tl_walk(int n, const double *work) { return n > TL_ROWS || (n < TL_MIN && work); }
 /* rows j0 .. j0 + TL_B - 1 of column k of the block (the arrays begin at the
    block's first column, so that any int is a valid column count: the 32-bit
    offset of at() takes the lane alone): lo[j - 1], d[j], up[j], r[j]; rows that
@@ -631,12 +637,12 @@ __global__ void __launch_bounds__(64) k_thomas_adj_lds(int n, int ncol, const do
     }
 }
 
-/* one column per lane, for systems of more rows */
+/* one column per lane, for systems of more rows and of fewer than TL_MIN */
 __global__ void __launch_bounds__(ATPB) k_thomas(int n, int ncol, const double *c, const double *d, const double *e,
                                                  const double *r, double *x, double *ep)
 {
-    const int k = blockIdx.x*ATPB + threadIdx.x;
-    if (k >= ncol) return;
+    const unsigned k = blockIdx.x*ATPB + threadIdx.x;
+    if (k >= (unsigned)ncol) return;
     /* column_solvers.c:641-667 */
     double epj = (n > 1) ? e[k]/d[k] : 0.0, xj = r[k]/d[k];
     ep[k] = epj;
@@ -662,8 +668,8 @@ __global__ void __launch_bounds__(ATPB) k_thomas_adj(int n, int ncol, const doub
                                                      const double *e, const double *x, const double *xb,
                                                      double *rb, double *cb, double *db, double *eb, double *ep)
 {
-    const int k = blockIdx.x*ATPB + threadIdx.x;
-    if (k >= ncol) return;
+    const unsigned k = blockIdx.x*ATPB + threadIdx.x;
+    if (k >= (unsigned)ncol) return;
     double epj = (n > 1) ? c[k]/d[k] : 0.0, yj = xb[k]/d[k];
     ep[k] = epj;
     rb[k] = yj;
@@ -736,8 +742,8 @@ void inner_product_adjoint(const DevGrid &G, const AdjTables &A, const double *b
 void thomas(int n, int ncol, const double *c, const double *d, const double *e, const double *r, double *x,
             double *work, hipStream_t st)
 {
-    if (n > TL_ROWS) {
-        LAUNCH("k_thomas", k_thomas, AGRID(ncol), dim3(ATPB), st, n, ncol, c, d, e, r, x, work);
+    if (tl_walk(n, work)) {
+        LAUNCH("k_thomas", k_thomas, dim3(((unsigned)ncol + ATPB - 1u)/ATPB), dim3(ATPB), st, n, ncol, c, d, e, r, x, work);
         return;
     }
     const int lanes = tl_lanes(n);
@@ -749,8 +755,8 @@ void thomas(int n, int ncol, const double *c, const double *d, const double *e, 
 void thomas_adjoint(int n, int ncol, const double *c, const double *d, const double *e, const double *x,
                     const double *xb, double *rb, double *cb, double *db, double *eb, double *work, hipStream_t st)
 {
-    if (n > TL_ROWS) {
-        LAUNCH("k_thomas_adj", k_thomas_adj, AGRID(ncol), dim3(ATPB), st, n, ncol, c, d, e, x, xb, rb, cb, db, eb, work);
+    if (tl_walk(n, work)) {
+        LAUNCH("k_thomas_adj", k_thomas_adj, dim3(((unsigned)ncol + ATPB - 1u)/ATPB), dim3(ATPB), st, n, ncol, c, d, e, x, xb, rb, cb, db, eb, work);
         return;
     }
     const int lanes = tl_lanes(n);

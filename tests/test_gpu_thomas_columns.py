@@ -1,4 +1,6 @@
-"""The three-band solve and its adjoint of more columns than a 32-bit byte
+"""The three-band solve and its adjoint of three and four rows, where the
+kernel with one column per lane and a work array gives way to the one with
+quotients in LDS (against the recurrence, equal), and of more columns than a 32-bit byte
 offset reaches (2^29 doubles): every column's solution is its own.  Bands of
 zero and a diagonal of two make the solution half the right-hand side, which
 counts the columns, so every value is exact and no two columns share one."""
@@ -6,6 +8,7 @@ import ctypes as C
 
 import pytest
 
+import test_gpu_thomas_sizes as sizes
 from conftest import get_grid
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +55,9 @@ def test_adjoint(lib):
     assert torch.equal(r_bar, x_bar.mul_(0.5))
     assert torch.equal(d_bar, x_bar.mul_(-0.5))
     assert not bands.any()
+
+
+@pytest.mark.parametrize("n", [3, 4])
+@pytest.mark.parametrize("ncol", [1, 513])
+def test_few_rows(n, ncol):
+    sizes.test_solve_and_adjoint_equal_the_recurrence(n, ncol)
