@@ -15,6 +15,7 @@
 /* threads per block of the kernels with one thread per element of a row */
 #define TPB 256
 #define GAME_MAX_LAYERS 64
+#define SH_COLUMN GAME_MAX_LAYERS
 
 /* src/game_constants.h */
 #define GC_T_0 273.15
@@ -85,8 +86,8 @@ struct DevGrid {
     int round_tendencies;
     /* 1: sound-wave solver with one column per lane; 0: three phases over LDS */
     int vw_streaming;
-    /* 1: sediment heat with one thread per grid box; 0: per chunk of layers */
-    int sh_per_box;
+    /* layers per thread of the sediment heat: 1, 2, 5 or SH_COLUMN, all; 0: by the grid's size */
+    int sh_run;
     /* 1: temperature and phase transitions as two kernels instead of one */
     int unfused_phase;
 };

@@ -1726,15 +1726,21 @@ __global__ void __launch_bounds__(TPB) k_sed_heat(DevGrid G, DevState so, DevSta
    carried to the box below, and the upstream box's density, temperature and
    c_p are loaded once per box and kept for the next interface.  The helper's
    restrict-qualified pointers let the loads of later layers move ahead of the
-   stores of earlier ones. */
-template <typename TW, int NCC, int LT>
+   stores of earlier ones, as many layers of them as a turn of the loop has: UN,
+   eight in the FP64 form and four in the mixed one, whose conversions take
+   registers (us per launch with turns of 4, 8, 13 and, at 26 layers, of the
+   whole column, which the compiler spreads over 64 registers, too few for the
+   loads: res 7 x 26 FP64 83.4, 80.5, 82.0, 79.0 and mixed 67.5, 77.6, 88.0,
+   86.2; res 7 x 24 78.1, 76.3, 74.8 and 62.9, 72.8, 74.6) */
+template <typename TW, int NCC>
 __device__ __forceinline__ void sed_heat_column(const DevGrid &G, const StepConsts &K, int i,
                                                 const double *__restrict__ rho_o, const double *__restrict__ wind_n,
                                                 const double *__restrict__ area, const double *__restrict__ vol,
                                                 const TW *__restrict__ T, const TW *__restrict__ cpc,
                                                 TW *__restrict__ sed_heat)
 {
-    const int nsh = G.nsh, vpl = G.vpl, L = LT;
+    constexpr int UN = sizeof(TW) == sizeof(double) ? 8 : 4;
+    const int nsh = G.nsh, vpl = G.vpl, L = G.L;
     const i64 S = G.s;
     double vsink[NCC];
 #pragma unroll
@@ -1746,7 +1752,7 @@ __device__ __forceinline__ void sed_heat_column(const DevGrid &G, const StepCons
     double fe_m[NCC];
 #pragma unroll
     for (int k = 0; k < NCC; ++k) fe_m[k] = 0.0;
-#pragma unroll
+#pragma unroll UN
     for (int j = 0; j < L; ++j) {
         const i64 b = i + (i64)j*nsh;
         const double v = vol[b];
@@ -1789,13 +1795,13 @@ __device__ __forceinline__ void sed_heat_column(const DevGrid &G, const StepCons
     }
 }
 
-template <typename TW, int NCC, int LT>
+template <typename TW, int NCC>
 __global__ void __launch_bounds__(TPB) k_sed_heat_col(DevGrid G, DevState so, DevState sn, const TW *T, const TW *cpc,
                                                       TW *sed_heat, StepConsts K)
 {
     const int i = (int)(xcd_x()*TPB + threadIdx.x);
     if (i >= G.nsh) return;
-    sed_heat_column<TW, NCC, LT>(G, K, i, so.rho, sn.wind, G.area, G.vol, T, cpc, sed_heat);
+    sed_heat_column<TW, NCC>(G, K, i, so.rho, sn.wind, G.area, G.vol, T, cpc, sed_heat);
 }
 
 /* phase_trans.c:16-311 (surface phase transitions off), one thread per grid box */
@@ -2374,23 +2380,29 @@ static void gen_densities_only(const DevGrid &G, const DevState &so, const DevSt
     else LAUNCH("k_gen_densities", (k_gen_densities<7, 640>), g, b, st, G, so, sn, td, K);
 }
 
-/* A chunk of five layers loads 13 values per box where one of one layer loads
-   26, at 146 registers and three waves per SIMD; a grid that chunks of five
-   leave short of blocks takes two.  us per launch with one, two, five and
-   seven layers: res 5 x 41 9.2, 9.1, 10.5, 10.6; res 6 x 55 57, 43, 34, 35
-   (71 by column); res 7 x 26 FP64 146, 113, 88, 83 and mixed 117, 86, 72, 69.
-   Above 256 blocks of columns one thread per column loads each box once: 77
-   and 64 at res 7 x 26 (38 at res 5, where the 41 blocks leave the chip idle) */
+/* One thread per column loads each box once, from 256 blocks of columns on; a
+   chunk of five layers loads 13 values per box, one of one layer 26, and smaller
+   grids, which columns leave short of blocks, take chunks of five, or of two
+   where five do.  us per launch, FP64 and mixed, in chunks of two and of five
+   and by column:
+     res 5 x 26    10.9  9.7    11.3  9.9    27 and more
+     res 6 x 26                 24.8  22.5    45.5  34.4
+     res 6 x 55    54.9  44.8   44.4  36.8
+     res 7 x 12                 42.6  36.0    38.0  30.4
+     res 7 x 24    95.9  78.0   83.3  66.6    76.3  62.9
+     res 7 x 26   112.9  87.7   89.5  73.6    80.5  67.5
+     res 7 x 41                 134   112     124   104
+     res 7 x 55                 196   154     165   140 */
 template <typename TW>
 static void sed_heat_t(const DevGrid &G, const DevState &so, const DevState &sn, const TW *T, const TW *cpc, TW *sed_heat,
                        const StepConsts &K, hipStream_t st)
 {
     const int bc = (G.nsh + TPB - 1)/TPB;
-    if (G.L == 26 && bc >= 256 && !G.sh_per_box) {
-        LAUNCH("k_sed_heat", (k_sed_heat_col<TW, 4, 26>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K);
+    const int run = G.sh_run ? G.sh_run : (bc >= 256 ? SH_COLUMN : (bc*G.L < 4096 ? 2 : 5));
+    if (run == SH_COLUMN) {
+        LAUNCH("k_sed_heat", (k_sed_heat_col<TW, 4>), grid_of(G.nsh, 1), dim3(TPB), st, G, so, sn, T, cpc, sed_heat, K);
         return;
     }
-    const int run = G.sh_per_box ? 1 : (bc*G.L < 4096 ? 2 : 5);
     const dim3 g = grid_of(G.nsh, (G.L + run - 1)/run), b(TPB);
     const Span sp = span_of(G.nsh, 1, 1);
     if (run == 1) LAUNCH("k_sed_heat", (k_sed_heat<TW, 4, 1>), g, b, st, G, so, sn, T, cpc, sed_heat, K, sp);

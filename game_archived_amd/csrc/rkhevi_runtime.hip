@@ -270,7 +270,15 @@ static int init_model(const game_dims_t *dims, const game_grid_view_t *g, const 
         else if (!strcmp(e, "both")) G.round_tendencies = 3;
     }
     G.vw_streaming = getenv("GAME_GPU_VW_STREAMING") ? 1 : 0;
-    G.sh_per_box = getenv("GAME_GPU_SH_PER_BOX") ? 1 : 0;
+    G.sh_run = getenv("GAME_GPU_SH_PER_BOX") ? 1 : 0;
+    if (const char *e = getenv("GAME_GPU_SH_LAYERS")) {
+        if (!strcmp(e, "all")) G.sh_run = SH_COLUMN;
+        else if (!strcmp(e, "1") || !strcmp(e, "2") || !strcmp(e, "5")) G.sh_run = atoi(e);
+        else {
+            snprintf(g_err, sizeof g_err, "GAME_GPU_SH_LAYERS is %s, not 1, 2, 5 or all", e);
+            return GAME_ERR_ARG;
+        }
+    }
     G.unfused_phase = getenv("GAME_GPU_UNFUSED_PHASE") ? 1 : 0;
     M->use_graphs = getenv("GAME_GPU_NO_GRAPH") ? 0 : 1;
     size_t S = (size_t)d.s, V = (size_t)d.v, NVH = (size_t)d.nvh, NSH = (size_t)d.nsh, NT = (size_t)d.nt;
