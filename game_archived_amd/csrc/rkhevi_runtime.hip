@@ -212,7 +212,10 @@ static void set_layer_splits(DevGrid &G)
     G.split_adj_e = clamp(fill, 4, L);
     if (const char *e = getenv("GAME_GPU_SPLIT_CELL")) {
         int v = atoi(e);
-        if (v >= 1 && v <= L) G.split_cell_w = G.split_adj_c = v;
+        if (v >= 1 && v <= L) {
+            G.split_cell_w = G.split_adj_c = v;
+            G.split_vcc = v < G.n_oro ? v : G.n_oro;
+        }
     }
     if (const char *e = getenv("GAME_GPU_SPLIT_EDGE")) {
         int v = atoi(e);
