@@ -513,9 +513,9 @@ __global__ void __launch_bounds__(ATPB) k_ip_adj(DevGrid G, AdjTables A, const d
    lane per column, 67 and 114 us at 163,842 columns, less).  us per solve and
    per adjoint, walking and here: 26 rows of 163,842 columns 183 together -> 39
    and 58 (4.3 and 5.3 TB/s), 55 rows of 10,243 columns 77 and 105 -> 17 and
-   20.  All rows of a column are read before
-   any output of it is written, and each value is formed as the walking kernel
-   forms it. */
+   20.  Each value is formed as the walking kernel forms it.  The solve here reads
+   all rows of a column before it writes one, the adjoint all rows of the bands
+   and of xb, and of x each row before it writes that row of an output. */
 #define TL_ROWS 128
 #define TL_B 8
 static int tl_lanes(int n) { return n <= 64 ? 64 : 32; }

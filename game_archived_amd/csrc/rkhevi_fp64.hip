@@ -735,11 +735,6 @@ __global__ void __launch_bounds__(TPB) k_grad_w(DevGrid G, const TW *f, TW *out,
     put(out + (i64)lev*G.vpl, h, (TW)(((double)at(lo - G.nsh, h) - (double)at(lo, h))/at(G.nd + (i64)lev*G.vpl, h)));
 }
 
-/* Vertical contravariant corrections (averaging.c:41-95) of the three fields
-   divv_h and divv_h_tracer need in the terrain-following levels L-n_oro..L-1:
-   the wind (tracers, divergences.c:94-145), the gas mass flux and its
-   rhotheta_v flux (divergences.c:41-59); the fluxes are formed on the fly
-   exactly as scalar_times_vector_h forms them (multiplications.c:45-67). */
 /* the slot-major tables of DevGrid, one thread per cell, edge and triangle of
    its number */
 __global__ void __launch_bounds__(TPB) k_tables(DevGrid G, unsigned *c_e, unsigned *c_n, unsigned *c_from, unsigned *e_ti,
@@ -787,7 +782,12 @@ __global__ void __launch_bounds__(TPB) k_vcc_weights(DevGrid G, double *vcw)
     vcw[t] = -0.5*G.ipwT[((i64)l*8 + jj)*G.nsh + h]*G.slope[G.nsh + (i64)l*G.vpl + G.adj[6*h + jj]];
 }
 
-/* MOIST: with the correction of the wind itself, which the tracers take */
+/* Vertical contravariant corrections (averaging.c:41-95) of the three fields
+   divv_h and divv_h_tracer need in the terrain-following levels L-n_oro..L-1:
+   the wind (tracers, divergences.c:94-145), the gas mass flux and its
+   rhotheta_v flux (divergences.c:41-59); the fluxes are formed on the fly
+   exactly as scalar_times_vector_h forms them (multiplications.c:45-67).  MOIST:
+   with the correction of the wind itself, which the tracers take */
 template <bool MOIST>
 __global__ void __launch_bounds__(TPB) k_vcc(DevGrid G, DevState s, double *vcc, Span sp)
 {

@@ -207,7 +207,8 @@ static void set_layer_splits(DevGrid &G)
     const int run_v = bc*G.n_oro <= 1024 ? 1 : 3;
     G.split_vcc = (G.n_oro + run_v - 1)/run_v;
     /* the adjoints: a filled chip, at least four chunks; a cell's chunk forms
-       a layer above and below it again, so it has two layers or more */
+       a layer above and below it again, so beyond four chunks it has two layers
+       or more */
     G.split_adj_c = clamp(1024/bc, 4, (L + 1)/2);
     G.split_adj_e = clamp(fill, 4, L);
     if (const char *e = getenv("GAME_GPU_SPLIT_CELL")) {

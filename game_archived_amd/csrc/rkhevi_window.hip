@@ -456,12 +456,11 @@ void resident_from_tape(int m)
     cl.run();
 }
 
-/* reverse of the momentum advection of (wind, rho) for the cotangent advb of
+/* the reverse of the momentum advection of (wind, rho) for the cotangent advb of
    pot_vort_tend - 0.5 v_squared_grad (vector_tendencies_expl.c:24-35),
-   accumulated into b_wind and b_rho */
-/* the reverse of the momentum advection of (wind, rho); flux and pv are the
-   forward's mass flux and potential vorticity if taped, else null (they are
-   then recomputed).  new_b_wind: b_wind is written, not added to */
+   accumulated into b_wind and b_rho; flux and pv are the forward's mass flux
+   and potential vorticity if taped, else null (they are then recomputed).
+   new_b_wind: b_wind is written, not added to */
 int advection_adjoint(const double *wind, const double *rho, const double *flux, const double *pv,
                       const double *advb, double *b_wind, double *b_rho, int new_b_wind = 0)
 {
@@ -513,10 +512,6 @@ int advection_adjoint(const double *wind, const double *rho, const double *flux,
     return 0;
 }
 
-/* reverse of step n from its tape; w.bS holds the cotangent of the state the
-   step produced (T.out), w.bP the cotangent of the
-   step's pressure gradient nl + l, w.bA that of its second-substep advection;
-   on return w.bS, w.bP, w.bA hold the same for the step before */
 /* the reverse of the gas's scalar tendencies (scalar_tendencies_expl.c:107-176)
    of densities (rho, rt) with the updated wind, with the momentum tendency's
    reverse m (tb: the cotangent of its w tendency); the densities' cotangents
@@ -554,6 +549,10 @@ static void ver_waves_adjoint(const sadj::VwArgs &a, hipStream_t st)
     launch("k_vw_layer_bar", sadj::VwLayerBar{a}, G.s, st);
 }
 
+/* the reverse of a step from its tape; w.bS holds the cotangent of the state the
+   step produced (T.out), w.bP that of the step's pressure gradient nl + l, w.bA
+   that of its second-substep advection; on return w.bS, w.bP, w.bA hold the
+   same for the step before */
 int step_adjoint(const StepTape &T, double dt, int first)
 {
     Window &w = *Wn;

@@ -236,7 +236,10 @@ int game_gpu_set_config(const game_config_t *config);
 /* One RKHEVI step on the device-resident states: replaces manage_rkhevi
    (src/time_stepping/manage_rkhevi.c:20-100).  Reads state_old, updates
    state_new, state_tendency, diagnostics, forcings and irrev in place.
-   `totally_first_step_bool` mirrors config->totally_first_step_bool. */
+   `totally_first_step_bool` mirrors config->totally_first_step_bool: a first
+   step forms the carried forcings anew, but, as the reference with its irrev
+   struct, a moist one reads the sediment heat of the step before it, of an
+   earlier run on the same model too; game_gpu_init clears it. */
 int game_gpu_manage_rkhevi(double delta_t, int totally_first_step_bool);
 
 /* state_out = c0*state_0 + c1*state_1 on the device, theta_v_pert re-derived
